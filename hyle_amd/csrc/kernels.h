@@ -113,6 +113,12 @@ struct SoftmaxParams {
 hipError_t launch_softmax(Elem type, const SoftmaxParams &p, const void *x, const void *mask,
                           void *y, bool vectorised, int compute_units, hipStream_t stream);
 
+// The same rows at any element's address and of any width from one vector on, under a mask with a
+// value per column or none (softmax_unaligned.hip); serves: the widths, sizes and masks it takes.
+bool softmax_unaligned_serves(Elem type, const SoftmaxParams &p);
+hipError_t launch_softmax_unaligned(Elem type, const SoftmaxParams &p, const void *x, const void *mask, void *y,
+                                    hipStream_t stream);
+
 // Softmax along any axis of a strided tensor: rows = outer * inner.
 struct SoftmaxGeneralParams {
   uint64_t outer = 0, inner = 0;

@@ -1763,6 +1763,8 @@ hyle_hip_status hyle_hip_plan_launch(const hyle_hip_plan *plan, const void *cons
       if (rows)
         err = launch_softmax(plan->elem, plan->softmax, inputs[0], mask, outputs[0], true,
                              plan->context->compute_units, stream);
+      else if (plan->softmax_rows_ok && softmax_unaligned_serves(plan->elem, plan->softmax))
+        err = launch_softmax_unaligned(plan->elem, plan->softmax, inputs[0], mask, outputs[0], stream);
       else
         err = launch_softmax_general(plan->elem, plan->softmax_general, inputs[0], mask, outputs[0],
                                      stream);

@@ -1,0 +1,248 @@
+// Row Softmax / LogSoftmax over rows that are no whole number of 16-byte vectors, or start at an
+// address that is none (an odd number of keys, a mask row of odd length, a view one element in):
+// the last axis of a dense tensor, any width from one vector on, arithmetic and the invalid-row
+// rule as in softmax.hip.
+//
+// A lane takes whole 16-byte vectors at element-aligned addresses (gfx950 loads and stores them
+// like any others, a wave's 64 neighbours still cover whole lines), and the vector that would pass
+// the row's end is moved back to end there: no scalar tail, every access inside the row.  The two
+// vectors then share elements, which both compute and store alike and only one counts in the sum.
+// The loads are plain ones, since neighbours share the lines at their seams; the stores stream
+// (bf16 [24, 777, 1013]: 16.8 us with plain stores, 15.0 us).  Bound by HBM from about 1000
+// elements a row on, below that by the vector instructions of a wave's two reductions, which is why
+// short rows share a wave.  MI355X, without a mask / Boolean / additive, before (softmax_general,
+// which walks the strides of every element in three passes) and here:
+//   bf16 [24, 777, 1013]  177 / 190 / 190 -> 15.0 / 15.8 / 17.6 us (5050 / 4850 / 4390 GB/s)
+//   f32  [24, 777, 1013]  179 -> 27.8 us (5440 GB/s)    f32 [12, 777, 7001] Boolean 658 -> 91.7 us (5750 GB/s)
+//   bf16 [24, 777, 3001]  488 -> 39.0 us (5745 GB/s; an aligned row of 3000 in softmax.hip: 45.4)
+//   f16  [24, 777, 100]    41 ->  3.7 us               f32 [8, 1, 1271] 12.6 -> 2.4 us
+// Running the heads of a mask row next to each other on one XCD, which pays for 64 MiB masks
+// (softmax.hip), loses here: bf16 [24, 777, 1013] additive 17.5 -> 20.2 us, f32 [32, 1777, 1777]
+// 149 -> 161 us.
+#include "softmax_math.h"
+
+namespace hyle_hip {
+namespace {
+
+// 16 bytes (or the mask bytes of one vector) at any element's address.
+typedef uint32_t words4_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t word_any __attribute__((aligned(1)));
+
+template <class T, int kLanes, int kVpl, int kThreads, int kMask, bool kLog>
+__global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x, const char *mask, char *y, uint32_t rows,
+                                                                  uint32_t width, float scale, MaskRows mrows) {
+  constexpr uint32_t kVec = Traits<T>::kVec, kSize = Traits<T>::kSize;
+  constexpr int kWords = kVec / 4;
+  constexpr int kGroupsPerBlock = kThreads / kLanes;
+  constexpr int kWaves = kThreads / kWaveLanes;
+  __shared__ float joint_max[kWaves], joint_sum[kWaves];
+  const uint32_t lane = threadIdx.x % kLanes;
+  uint32_t group = threadIdx.x / kLanes;
+  if constexpr (kLanes >= kWaveLanes) group = __builtin_amdgcn_readfirstlane(group);  // the row's address stays scalar
+  const uint32_t wanted_row = blockIdx.x * kGroupsPerBlock + group;
+  const bool row_ok = wanted_row < rows;
+  const uint32_t row = row_ok ? wanted_row : rows - 1;
+  const char *mask_row = nullptr;
+  if constexpr (kMask != kMaskNone) mask_row = mask + mask_row_offset(mrows, row);
+  const char *row_x = x + (size_t)row * width * kSize;
+
+  // Vector `lane + k * kLanes` of the row, moved back to end at the row's end where it would pass
+  // it: `skip` of its elements belong to the vector before it (all of them: nothing is left).
+  uint32_t start[kVpl], skip[kVpl];
+#pragma unroll
+  for (int k = 0; k < kVpl; ++k) {
+    const uint32_t own = (lane + k * kLanes) * kVec;
+    start[k] = own < width - kVec ? own : width - kVec;
+    skip[k] = own - start[k];
+  }
+  uint32_t bits[kVpl][kWords];
+  if constexpr (kMask == kMaskBoolean) {
+#pragma unroll
+    for (int k = 0; k < kVpl; ++k)
+#pragma unroll
+      for (int q = 0; q < kWords; ++q) bits[k][q] = reinterpret_cast<const word_any *>(mask_row + start[k])[q];
+  }
+  u32x4 raw[kVpl], added[kVpl];
+#pragma unroll
+  for (int k = 0; k < kVpl; ++k) {
+    uint32_t from = start[k];
+    if constexpr (kMask == kMaskBoolean) {
+      uint32_t any = 0;
+#pragma unroll
+      for (int q = 0; q < kWords; ++q) any |= bits[k][q];
+      from = any != 0 ? from : 0u;  // nothing kept: no new line is asked for
+    }
+    raw[k] = *reinterpret_cast<const words4_any *>(row_x + (size_t)from * kSize);
+    if constexpr (kMask == kMaskAdditive) added[k] = *reinterpret_cast<const words4_any *>(mask_row + (size_t)start[k] * kSize);
+  }
+#pragma unroll
+  for (int k = 0; k < kVpl; ++k) loads_issued(raw[k]);
+
+  float v[kVpl][kVec];
+  float peak = -INFINITY;
+  bool poisoned = false;
+#pragma unroll
+  for (int k = 0; k < kVpl; ++k) {
+    Traits<T>::unpack(raw[k], v[k]);
+    if constexpr (kMask == kMaskAdditive) {
+      float addend[kVec];
+      Traits<T>::unpack(added[k], addend);
+#pragma unroll
+      for (int j = 0; j < (int)kVec; ++j) v[k][j] = v[k][j] * scale + addend[j];
+    } else if constexpr (kMask == kMaskBoolean) {
+#pragma unroll
+      for (int j = 0; j < (int)kVec; ++j) {
+        const bool keep = ((bits[k][j / 4] >> (8 * (j % 4))) & 0xFFu) != 0;
+        v[k][j] = keep ? v[k][j] * scale : -INFINITY;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < (int)kVec; ++j) v[k][j] *= scale;
+    }
+#pragma unroll
+    for (int j = 0; j < (int)kVec; j += 2) {
+      // f32 only: exp_for of narrow storage lets a NaN through, and the sum takes it to every result
+      if constexpr (kSize == 4) poisoned = poisoned || __builtin_isunordered(v[k][j], v[k][j + 1]);
+      peak = fmaxf(peak, fmaxf(v[k][j], v[k][j + 1]));
+    }
+  }
+  // an infinite maximum of either sign marks the row: +inf poisoned, -inf nothing finite
+  peak = row_max<kLanes>(poisoned ? INFINITY : peak, joint_max);
+  const bool invalid = __builtin_fabsf(peak) == INFINITY;
+  float total = 0.0f, maxima = 0.0f;
+#pragma unroll
+  for (int k = 0; k < kVpl; ++k) {
+    float sum = 0.0f, count = 0.0f;
+#pragma unroll
+    for (int j = 0; j < (int)kVec; ++j) {
+      const float shifted = v[k][j] - peak;
+      if constexpr (kLog) {  // the maxima are counted, not summed (src/compute_provider_cuda/reduction_kernel.cu:178-196)
+        const bool at_peak = shifted == 0.0f;
+        sum += at_peak ? 0.0f : exp_for<T>(shifted);
+        count += at_peak ? 1.0f : 0.0f;
+        v[k][j] = shifted;
+      } else {
+        v[k][j] = exp_for<T>(shifted);
+        sum += v[k][j];
+      }
+    }
+    if (skip[k] != 0) {  // the row's last vectors: elements of two vectors count once
+      sum = 0.0f;
+      count = 0.0f;
+#pragma unroll
+      for (int j = 0; j < (int)kVec; ++j) {
+        const bool mine = (uint32_t)j >= skip[k];
+        if constexpr (kLog) {
+          sum += mine && v[k][j] != 0.0f ? exp_for<T>(v[k][j]) : 0.0f;
+          count += mine && v[k][j] == 0.0f ? 1.0f : 0.0f;
+        } else {
+          sum += mine ? v[k][j] : 0.0f;
+        }
+      }
+    }
+    total += sum;
+    maxima += count;
+  }
+  total = row_sum<kLanes>(total, joint_sum);  // = 2^32 * sum(exp)
+  // joint_max is free again: every wave read it before the barrier of the sum above
+  if constexpr (kLog) maxima = row_sum<kLanes>(maxima, joint_max);
+  float normaliser = kLog ? log1pf((maxima - 1.0f) + total * 2.3283064365386963e-10f) : 1.0f / total;
+  if (invalid) normaliser = __builtin_nanf("");
+  char *row_y = y + (size_t)row * width * kSize;
+#pragma unroll
+  for (int k = 0; k < kVpl; ++k) {
+    if (row_ok && skip[k] < kVec) {
+      float out[kVec];
+#pragma unroll
+      for (int j = 0; j < (int)kVec; ++j) out[j] = kLog ? v[k][j] - normaliser : v[k][j] * normaliser;
+      const u32x4 packed = Traits<T>::pack(out);
+      __builtin_nontemporal_store(packed, reinterpret_cast<words4_any *>(row_y + (size_t)start[k] * kSize));
+    }
+  }
+}
+
+// unaligned_softmax/<lanes>x<vectors per lane>/<threads per block>/<mask>
+template <int kLanes, int kVpl, int kThreads, int kMask> struct UnalignedTag {
+  static std::string text() {
+    return "unaligned_softmax/" + std::to_string(kLanes) + "x" + std::to_string(kVpl) + "/" + std::to_string(kThreads) + "/" + mask_word(kMask);
+  }
+};
+
+template <class T, int kLanes, int kVpl, int kThreads, int kMask>
+void run_mask(const SoftmaxParams &p, const MaskRows &m, const void *x, const void *mask, void *y, hipStream_t s) {
+  constexpr uint32_t kGroupsPerBlock = kThreads / kLanes;
+  const uint32_t rows = (uint32_t)p.shape.rows;
+  const dim3 grid((rows + kGroupsPerBlock - 1) / kGroupsPerBlock);
+  const char *in = static_cast<const char *>(x), *in_mask = static_cast<const char *>(mask);
+  char *out = static_cast<char *>(y);
+  note_variant<UnalignedTag<kLanes, kVpl, kThreads, kMask>>();
+  if (p.log)
+    hipLaunchKernelGGL((softmax_rows_unaligned<T, kLanes, kVpl, kThreads, kMask, true>), grid, dim3(kThreads), 0, s, in, in_mask, out, rows,
+                       p.shape.width, p.scale, m);
+  else
+    hipLaunchKernelGGL((softmax_rows_unaligned<T, kLanes, kVpl, kThreads, kMask, false>), grid, dim3(kThreads), 0, s, in, in_mask, out, rows,
+                       p.shape.width, p.scale, m);
+}
+
+template <class T, int kLanes, int kVpl, int kThreads>
+void run_shape(const SoftmaxParams &p, const void *x, const void *mask, void *y, hipStream_t s) {
+  MaskRows m{};
+  m.outer_rank = p.outer_rank;
+  for (int i = 0; i < kMaxRank; ++i) {
+    m.outer_dims[i] = p.outer_dims[i];
+    m.outer_strides[i] = p.mask_outer_strides[i];
+  }
+  m.inner_stride = p.mask_inner_stride;
+  switch ((int)p.mask_kind) {
+    case kMaskBoolean: return run_mask<T, kLanes, kVpl, kThreads, kMaskBoolean>(p, m, x, mask, y, s);
+    case kMaskAdditive: return run_mask<T, kLanes, kVpl, kThreads, kMaskAdditive>(p, m, x, mask, y, s);
+    default: return run_mask<T, kLanes, kVpl, kThreads, kMaskNone>(p, m, x, mask, y, s);
+  }
+}
+
+// Lanes x vectors for a row of that many vectors, the tightest measured: three vectors a lane where
+// two would leave a third of the lanes idle (bf16 601 additive 64 x 2 14.9 us, 32 x 3 13.4; 3001
+// unmasked 128 x 4 40.0, 128 x 3 39.0), two rows per wave below 64 vectors (f16 203: 64 x 1 7.7 us,
+// 32 x 1 5.3, 16 x 2 5.1; 503 additive 64 x 1 11.7, 32 x 2 11.0), but one row per wave at 65-128
+// (1013 additive 64 x 2 17.9, 32 x 4 19.8).
+template <class T> void run_width(const SoftmaxParams &p, const void *x, const void *mask, void *y, hipStream_t s) {
+  const uint32_t vectors = (p.shape.width + Traits<T>::kVec - 1) / Traits<T>::kVec;
+  if (vectors <= 8) return run_shape<T, 8, 1, 256>(p, x, mask, y, s);
+  if (vectors <= 16) return run_shape<T, 16, 1, 256>(p, x, mask, y, s);
+  if (vectors <= 32) return run_shape<T, 16, 2, 256>(p, x, mask, y, s);
+  if (vectors <= 64) return run_shape<T, 32, 2, 256>(p, x, mask, y, s);
+  if (vectors <= 96) return run_shape<T, 32, 3, 256>(p, x, mask, y, s);
+  if (vectors <= 128) return run_shape<T, 64, 2, 256>(p, x, mask, y, s);
+  if (vectors <= 192) return run_shape<T, 64, 3, 256>(p, x, mask, y, s);
+  if (vectors <= 256) return run_shape<T, 64, 4, 256>(p, x, mask, y, s);
+  if (vectors <= 384) return run_shape<T, 128, 3, 256>(p, x, mask, y, s);
+  if (vectors <= 512) return run_shape<T, 128, 4, 256>(p, x, mask, y, s);
+  if (vectors <= 768) return run_shape<T, 256, 3, 256>(p, x, mask, y, s);
+  if (vectors <= 1024) return run_shape<T, 256, 4, 256>(p, x, mask, y, s);
+  if (vectors <= 1536) return run_shape<T, 512, 3, 512>(p, x, mask, y, s);
+  if (vectors <= 2048) return run_shape<T, 512, 4, 512>(p, x, mask, y, s);
+  return run_shape<T, 1024, 8, 1024>(p, x, mask, y, s);
+}
+
+}  // namespace
+
+bool softmax_unaligned_serves(Elem type, const SoftmaxParams &p) {
+  const uint32_t kvec = (uint32_t)elem_vec(type);
+  if (p.shape.width < kvec || p.shape.width > 8u * 1024u * kvec) return false;
+  // a handful of short rows is one launch's latency either way and stays with the strided kernel
+  // (f32 [6, 129]: 4.3 us there, 2.3 us here, of which 2 us are the dispatch)
+  if (p.shape.rows * p.shape.width < 800) return false;
+  const int64_t unit = (int)p.mask_kind == kMaskBoolean ? 1 : elem_size(type);
+  return (int)p.mask_kind == kMaskNone || p.mask_inner_stride == unit;
+}
+
+hipError_t launch_softmax_unaligned(Elem type, const SoftmaxParams &p, const void *x, const void *mask, void *y, hipStream_t stream) {
+  switch (type) {
+    case Elem::kF32: run_width<F32>(p, x, mask, y, stream); break;
+    case Elem::kF16: run_width<F16>(p, x, mask, y, stream); break;
+    case Elem::kBF16: run_width<BF16>(p, x, mask, y, stream); break;
+  }
+  return hipGetLastError();
+}
+
+}  // namespace hyle_hip

@@ -1,0 +1,55 @@
+"""Softmax / LogSoftmax over rows that are no whole number of 16-byte vectors or start off a 16-byte
+boundary: the launch shapes of softmax_unaligned.hip at both ends of the widths each one takes,
+against the oracle under the bars of test_gpu_softmax_variants.py (f32 1e-5 relative, narrow types one
+unit in the last place, LogSoftmax f32 4e-6 relative + 2e-7)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from hyle_amd import compute as hc
+
+from gpu_support import DEVICE, TYPES, note, run
+from test_gpu_softmax_variants import MASKS, compare_on_device, make_inputs, oracle_softmax
+
+pytestmark = pytest.mark.gpu
+
+# (fewest, most vectors per row, launch shape)
+SHAPES = [(1, 8, "8x1/256"), (9, 16, "16x1/256"), (17, 32, "16x2/256"), (33, 64, "32x2/256"), (65, 96, "32x3/256"),
+          (97, 128, "64x2/256"), (129, 192, "64x3/256"), (193, 256, "64x4/256"), (257, 384, "128x3/256"), (385, 512, "128x4/256"),
+          (513, 768, "256x3/256"), (769, 1024, "256x4/256"), (1025, 1536, "512x3/512"), (1537, 2048, "512x4/512"),
+          (2049, 8192, "1024x8/1024")]
+
+
+def offset_by_one(t):
+    """The same values one element behind a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    flat[1:] = t.reshape(-1)
+    return flat[1:].view(t.shape)
+
+
+def check(tag, q, width, mask_word, shape, log_form, moved, in_place):
+    heads, scale = 2, 0.125 if mask_word != "unmasked" else 1.0
+    note(f"softmax {tag} log={log_form} [{heads}, {q}, {width}] {mask_word} moved={moved} in_place={in_place}: expecting {shape}")
+    x, x_host, mask, mask_host = make_inputs(tag, heads, q, width, mask_word, seed=width + q)
+    if moved:
+        x = offset_by_one(x)
+    want = oracle_softmax(tag, x_host, mask_word, mask_host, scale, log_form)
+    kind = hc.SoftmaxKind.kLogSoftmax if log_form else hc.SoftmaxKind.kSoftmax
+    (out,) = run(hc.Softmax(scale=scale, kind=kind, mask=MASKS[mask_word]), *([x] if mask is None else [x, mask]),
+                 outputs=[x] if in_place else None)
+    assert hc.last_launch_variant() == f"unaligned_softmax/{shape}/{mask_word}"
+    count, text = compare_on_device(tag, out, want, log_form)
+    assert count == 0, f"{count} elements outside the bar, {text}"
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: s[2].replace("/", "-"))
+@pytest.mark.parametrize("tag", ["f32", "bf16", "f16"])
+def test_rows_of_any_width_at_both_ends_of_a_launch_shape(shape, tag):
+    fewest, most, label = shape
+    vec = 16 // TYPES[tag][2].itemsize
+    for width, moved in ((max(vec, (fewest - 1) * vec + 1), fewest == 1), (most * vec - 1, False), (most * vec, True)):
+        q = max(5, 400 // width + 1)
+        for mask_word in ("unmasked", "boolean", "additive"):
+            check(tag, q, width, mask_word, label, False, moved, in_place=mask_word == "boolean")
+        check(tag, q, width, "boolean", label, True, moved, in_place=False)
