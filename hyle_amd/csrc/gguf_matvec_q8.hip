@@ -33,18 +33,11 @@
 #include "device_common.h"
 #include "gguf_decode.h"
 #include "gguf_lines.h"
+#include "gguf_q8_math.h"
 #include "kernels.h"
 
 namespace hyle_hip {
 namespace {
-
-// a * b + c for factors that fit 24 signed bits (v_mad_i32_i24; a full 32-bit multiply is four
-// times slower)
-__device__ __forceinline__ int mad24(int a, int b, int c) { return __mul24(a, b) + c; }
-
-__device__ __forceinline__ int dot4(uint32_t weights, uint32_t codes, int sum) {
-  return __builtin_amdgcn_sdot4((int)weights, (int)codes, sum, false);
-}
 
 // The element of largest magnitude of a block spread over kLanes adjacent lanes; among equal
 // magnitudes the one at the lowest position of the row wins (ggml walks the block in order and
@@ -621,13 +614,6 @@ struct TileGroup {  // what a lane holds of four blocks of its weight row
 __host__ __device__ inline size_t tile_shared_bytes(uint32_t tokens, uint32_t blocks) {
   return (size_t)(1 + tokens) * blocks * 256 + (size_t)tokens * blocks * (32 + 4) +
          (size_t)kWavesPerBlock * kWaveLanes * (tokens >= 4 ? tokens / 4 : 1) * 4;
-}
-
-// Block barrier that orders LDS accesses only: the weight loads issued before it stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // Half a wave quantises an activation block of 256 values (Q8_K), eight values per lane.
@@ -1419,10 +1405,8 @@ hipError_t run_spans(const MatVecParams &p, const void *w, const void *x, void *
 // Q4_K on the matrix unit: K a whole number of blocks, rows and activations made of whole 16-byte
 // vectors, the codes of every activation row within a block's 64 KiB of LDS.
 inline uint32_t tile_tokens(uint32_t m) { return m <= 1 ? 1 : (m <= 4 ? 4 : 8); }
-inline bool tiles_serve(const MatVecParams &p, const void *w, const void *x) {
-  return p.k >= 1024 && p.k % 256 == 0 && p.m <= 8 && p.row_stride % 16 == 0 &&
-         ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0 &&
-         tile_shared_bytes(tile_tokens(p.m), p.k / 256) <= 64 * 1024;
+inline bool tiles_serve(const MatVecParams &p) {
+  return p.k >= 1024 && p.k % 256 == 0 && p.m <= 8 && p.row_stride % 16 == 0 && tile_shared_bytes(tile_tokens(p.m), p.k / 256) <= 64 * 1024;
 }
 template <class TX, int kSets>
 hipError_t run_tiles_m(const MatVecParams &p, const void *w, const void *x, void *y, int compute_units, hipStream_t s) {
@@ -1456,27 +1440,55 @@ hipError_t run_tiles(const MatVecParams &p, const void *w, const void *x, void *
   return run_tiles_m<TX, 2>(p, w, x, y, compute_units, s);
 }
 
+// Q8_0, one activation row, 256 n values: the span kernel with a short last span, up to nine spans.
+inline bool short_span_serves(const MatVecParams &p) {
+  return p.kind == 2 && p.m == 1 && p.k >= 1024 && p.k % 256 == 0 && p.k % 2048 != 0 && (p.k + 2047) / 2048 <= 9 && p.row_stride % 16 == 0;
+}
+// Q8_0 and Q6_K rows of 2048 n values whose codes fit beside the waves' row buffers (12 KiB).
+inline bool whole_spans_serve(const MatVecParams &p) {
+  return p.kind != 0 && p.k != 0 && p.k % 2048 == 0 && p.row_stride % 16 == 0 &&
+         gguf_matvec_q8_shared_bytes(p.m, p.k) + 12 * 1024 <= 64 * 1024;
+}
+// The kernels over rows of whole 16-byte vectors, if weights and activations start on a 16-byte boundary.
+inline bool rows_of_vectors_serve(const MatVecParams &p) {
+  return p.kind == 0 ? tiles_serve(p) : (short_span_serves(p) || whole_spans_serve(p));
+}
+
+// Where the strip kernel (gguf_matvec_strips.hip) is the faster one; `vectors`: weights, activations and
+// the row stride are multiples of 16 bytes.  us, the kernel here / strips:
+//   shapes that walk block by block, from 24 M products on: Q8_0 [1536 -> 8192] x 2 9.5 / 9.0,
+//   [5120 -> 2048] x 2 10.7 / 11.1 and x 4 16.4 / 11.0, Q6_K [5120 -> 8192] x 1 14.4 / 14.0 (below: Q6_K
+//   [5120 -> 2048] x 1 8.7 / 11.5, [1536 -> 2048] x 2 6.2 / 9.0)
+//   tiles: several rows of 4096 values or more and 4096 weight rows: Q4_K [4096 -> 8192] x 2 14.3 / 12.4,
+//   [5120 -> 17408] x 5 44.9 / 21.8 (narrower: [2048 -> 32768] x 4 13.1 / 15.4; one row: [5120 -> 17408] 15.5 / 18.0)
+//   whole spans, from 200 M products on: more than four rows, Q8_0 [4096 -> 32768] x 8 43.7 / 34.8, Q6_K x 6
+//   47.6 / 31.1 ([2048 -> 100000] x 6 Q8_0 48.5 / 50.3, Q6_K 49.3 / 50.2); Q6_K three or four rows of 6144 or
+//   more, [6144 -> 8192] x 4 22.8 / 17.3 ([4096 -> 100000] x 4 69.5 / 71.5, Q8_0 [6144 -> 32768] x 4 42.3 / 46.8)
+bool strips_better(const MatVecParams &p, bool vectors) {
+  if (!gguf_matvec_strips_serve(p)) return false;
+  const uint64_t products = (uint64_t)p.m * p.rows * p.k;
+  if (!vectors || !rows_of_vectors_serve(p)) return products >= 24000000;
+  if (p.kind == 0) return p.m > 1 && p.k >= 4096 && p.rows >= 4096;
+  return products >= 200000000 && ((p.m > 4 && p.k >= 4096) || (p.kind == 1 && p.m > 2 && p.k >= 6144));
+}
+
 template <int kKind, class TX>
 hipError_t run_m(const MatVecParams &p, const void *w, const void *x, void *y, int compute_units, hipStream_t s) {
   if constexpr (kKind == 0) {
     // Q4_K: the matrix unit, or block by block
-    if (tiles_serve(p, w, x)) return run_tiles<TX>(p, w, x, y, compute_units, s);
+    if (tiles_serve(p) && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0) return run_tiles<TX>(p, w, x, y, compute_units, s);
     return run_blocks<kKind, TX>(p, w, x, y, compute_units, s);
   } else {
   if constexpr (kKind == 2) {
     // Q8_0, one activation row, a width of 256 n that is no multiple of 2048 (8 blocks are 17 whole
     // vectors): the span kernel with a short last span, up to nine spans
-    const uint32_t whole = (p.k + 2047) / 2048;
-    if (p.m == 1 && p.k >= 1024 && p.k % 256 == 0 && p.k % 2048 != 0 && whole <= 9 && p.row_stride % 16 == 0 &&
-        ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0)
-      return run_spans<kKind, TX>(p, w, x, y, whole, (p.k % 2048) / 32, compute_units, s);
+    if (short_span_serves(p) && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0)
+      return run_spans<kKind, TX>(p, w, x, y, (p.k + 2047) / 2048, (p.k % 2048) / 32, compute_units, s);
   }
   // the span kernels: rows of 2048 n values made of whole 16-byte vectors, activations on a 16-byte
   // boundary, codes of every activation row in LDS beside the waves' row buffers (12 KiB); everything
   // else walks block by block
-  if (p.k == 0 || p.k % 2048 != 0 || p.row_stride % 16 != 0 ||
-      ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15u) != 0 ||
-      gguf_matvec_q8_shared_bytes(p.m, p.k) + 12 * 1024 > 64 * 1024)
+  if (!whole_spans_serve(p) || ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15u) != 0)
     return run_blocks<kKind, TX>(p, w, x, y, compute_units, s);
   const uint32_t spans = p.k / 2048;
   const uint32_t wanted = (uint32_t)((p.rows + kWavesPerBlock - 1) / kWavesPerBlock);
@@ -1515,13 +1527,12 @@ size_t gguf_matvec_q8_shared_bytes(uint32_t m, uint32_t k) {
 
 bool gguf_matvec_q8_serves(int kind, uint32_t k) { return blocks_row_bytes(kind, k) <= kBlocksSharedBudget; }
 
-uint32_t gguf_matvec_q8_dispatches(int kind, uint32_t m, uint32_t k, uint64_t row_stride) {
+uint32_t gguf_matvec_q8_dispatches(const MatVecParams &p) {
+  const uint32_t m = p.m, k = p.k;
+  const int kind = p.kind;
   if (m == 0 || k == 0) return 1;
-  if (kind == 0) {
-    if (k >= 1024 && k % 256 == 0 && m <= 8 && row_stride % 16 == 0 && tile_shared_bytes(tile_tokens(m), k / 256) <= 64 * 1024) return 1;
-  } else if (k % 2048 == 0 && row_stride % 16 == 0 && gguf_matvec_q8_shared_bytes(m, k) + 12 * 1024 <= 64 * 1024) {
-    return 1;
-  }
+  if (strips_better(p, p.row_stride % 16 == 0)) return gguf_matvec_strips_dispatches(p);
+  if (rows_of_vectors_serve(p)) return 1;
   uint32_t fit = (uint32_t)(kBlocksSharedBudget / blocks_row_bytes(kind, k));
   fit = fit >= 8 ? 8 : (fit >= 4 ? 4 : (fit >= 2 ? 2 : 1));
   return (m + fit - 1) / fit;
@@ -1532,6 +1543,8 @@ uint32_t gguf_matvec_q8_dispatches(int kind, uint32_t m, uint32_t k, uint64_t ro
 hipError_t launch_gguf_matvec_q8(Elem x_type, const MatVecParams &p, const void *weights, const void *x, void *y,
                                  int compute_units, hipStream_t stream) {
   if (p.rows == 0 || p.m == 0) return hipSuccess;
+  const bool vectors = p.row_stride % 16 == 0 && ((reinterpret_cast<uintptr_t>(weights) | reinterpret_cast<uintptr_t>(x)) & 15u) == 0;
+  if (strips_better(p, vectors)) return launch_gguf_matvec_strips(x_type, p, weights, x, y, stream);
   switch (x_type) {
     case Elem::kF32: return run_kind<F32>(p, weights, x, y, compute_units, stream);
     case Elem::kF16: return run_kind<F16>(p, weights, x, y, compute_units, stream);

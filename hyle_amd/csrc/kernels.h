@@ -216,18 +216,22 @@ struct MatVecParams {
   uint64_t row_stride = 0;  // bytes between physical weight rows
   uint8_t kind = 0;
   uint8_t codec = 0;        // HYLE_HIP_ACTIVATIONS_*: 0 exact f32 activations, 1 ggml's 8-bit activation blocks
-  uint32_t compute_units = 256;  // of the plan's device: the grids are three blocks per unit
+  uint32_t compute_units = 256;  // of the plan's device: the grids are one to three blocks per unit
 };
 size_t gguf_matvec_shared_bytes(uint32_t m, uint32_t k);
 // The 8-bit activation route: any whole number of blocks per row at even addresses, M <= 8.
 // Rows of 2048 n values made of whole 16-byte vectors take the span kernels (the codes of all M
-// rows in LDS: gguf_matvec_q8_shared_bytes); other shapes walk block by block, M in groups that
-// fit LDS (gguf_matvec_q8_dispatches launches).  gguf_matvec_q8_serves: one activation row fits.
+// rows in LDS: gguf_matvec_q8_shared_bytes); other shapes walk block by block or, where there is work
+// enough, in strips on the matrix unit, M in groups that fit LDS (gguf_matvec_q8_dispatches launches).  gguf_matvec_q8_serves: one activation row fits.
 size_t gguf_matvec_q8_shared_bytes(uint32_t m, uint32_t k);
 bool gguf_matvec_q8_serves(int kind, uint32_t k);
-uint32_t gguf_matvec_q8_dispatches(int kind, uint32_t m, uint32_t k, uint64_t row_stride);
+uint32_t gguf_matvec_q8_dispatches(const MatVecParams &p);
 hipError_t launch_gguf_matvec_q8(Elem x_type, const MatVecParams &p, const void *weights, const void *x, void *y,
                                  int compute_units, hipStream_t stream);
+// The same products on the matrix unit for many weight rows (gguf_matvec_strips.hip).
+bool gguf_matvec_strips_serve(const MatVecParams &p);
+uint32_t gguf_matvec_strips_dispatches(const MatVecParams &p);
+hipError_t launch_gguf_matvec_strips(Elem x_type, const MatVecParams &p, const void *weights, const void *x, void *y, hipStream_t stream);
 hipError_t launch_gguf_matvec(Elem x_type, const MatVecParams &p, const void *weights, const void *x, void *y,
                               hipStream_t stream);
 

@@ -1141,7 +1141,7 @@ hyle_hip_status admit(hyle_hip_plan *p) {
       p->matvec.kind = matvec_kind;
       if (r.kind2 != HYLE_HIP_ACTIVATIONS_GGML_Q8) p->input_alignment[0] = 1;
       p->dispatches = r.kind2 == HYLE_HIP_ACTIVATIONS_GGML_Q8
-                          ? gguf_matvec_q8_dispatches(matvec_kind, (uint32_t)m, (uint32_t)k, (uint64_t)in[0].byte_strides[1])
+                          ? gguf_matvec_q8_dispatches(p->matvec)
                           : 1;
       return HYLE_HIP_OK;
     }

@@ -1,0 +1,67 @@
+"""The GGUF products with 8-bit activation blocks against many weight rows (gguf_matvec_strips.hip):
+every format, one and two sets of activation rows, both block sizes, one and two blocks per compute
+unit, one to sixteen waves to a tile, rows that are no whole number of 16-byte vectors or start off a
+boundary.  Bar and oracle as in test_gpu_gguf_matvec_q8.py."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from hyle_amd import compute as hc
+
+from gpu_support import context, note
+from test_gpu_gguf_matvec_q8 import KINDS, Q8, check, raw_bytes_for, weights_for
+
+pytestmark = pytest.mark.gpu
+
+# rows, k, activation rows, bytes the weight starts off a boundary, bytes between rows, activation elements off
+CASES = (
+    (4096, 1280, 5, 0, 0, 0),     # five runs, split over fewer waves than a block has
+    (4099, 5120, 7, 0, 0, 0),     # a last block with fewer rows, a tile with rows that repeat
+    (12289, 1536, 2, 0, 0, 0),    # two blocks per compute unit
+    (66000, 256, 2, 0, 0, 0),     # one run: a wave to a tile, no shares
+    (5003, 1792, 4, 2, 6, 1),     # rows at every even offset, activations at an odd element
+    (4097, 2048, 8, 14, 10, 3),
+    (521, 12544, 8, 0, 2, 0),     # eight waves to a block
+    (530, 25600, 3, 6, 0, 1),     # wide rows
+)
+
+
+@pytest.mark.parametrize("x_tag", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("tag", list(KINDS))
+def test_strips_edges(tag, x_tag):
+    rng = np.random.default_rng(1820)
+    for rows, k, m, byte_offset, pad, x_offset in CASES:
+        if tag == "q4_k" and not pad and not byte_offset and (k < 4096 or rows < 4096):
+            byte_offset = 2   # a boundary would take the tile kernel
+        raw = raw_bytes_for(tag, rng, rows, k) if x_tag != "f16" else weights_for(tag, rng, rows, k)
+        padded = np.zeros((rows, raw.shape[1] + pad), np.uint8)
+        padded[:, :raw.shape[1]] = raw
+        x = rng.normal(0, 1.5, (m, k)).astype(np.float32)
+        x[m - 1, :256] = 0.0                                                        # an activation block of zeros
+        x[0, k - 256:] = np.where(np.arange(256) % 2 == 0, -1.25, 1.25)             # equal magnitudes: the first sign decides
+        note(f"q8 matvec strips {tag} x {x_tag} rows {rows} k {k} m {m} off {byte_offset} pad {pad} x off {x_offset}")
+        check(tag, x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad, byte_offset=byte_offset, x_offset=x_offset,
+              kernel=f"gguf_matvec_q8_strips/{tag}/{4 if m <= 4 else 8}-tokens")
+
+
+@pytest.mark.parametrize("tag,k,rows,m,kernel", [
+    ("q6_k", 2304, 24000, 1, "strips/q6_k/4"), ("q6_k", 1280, 4096, 1, "blocks/q6_k/1"), ("q8_0", 4096, 8192, 6, "strips/q8_0/8"),
+    ("q8_0", 4096, 8192, 4, "lines/q8_0/4"), ("q6_k", 6144, 8192, 4, "strips/q6_k/4"), ("q6_k", 6144, 8192, 2, "quads/q6_k/4"),
+    ("q4_k", 4096, 4096, 2, "strips/q4_k/4"), ("q4_k", 3840, 4096, 4, "tiles/q4_k/4")])
+def test_strips_rule(tag, k, rows, m, kernel):
+    rng = np.random.default_rng(1821)
+    note(f"q8 matvec rule {tag} rows {rows} k {k} m {m}")
+    check(tag, "bf16", raw_bytes_for(tag, rng, rows, k), rows, k, rng.normal(0, 1, (m, k) if m > 1 else (k,)).astype(np.float32),
+          kernel="gguf_matvec_q8_" + kernel)
+
+
+def test_strips_activation_rows_in_groups():
+    """Eight activation rows of 17408 Q8_0 values do not fit a block's LDS beside its slots: two groups of four."""
+    rng = np.random.default_rng(1822)
+    rows, k, m = 600, 17408, 8
+    weight = hc.TensorDesc.gguf_weight(hc.GgufQuantizedType.kQ8_0, hc.DataType.kFloat32, k, rows)
+    assert hc.prepare(context(), Q8, weight, hc.TensorDesc.dense(hc.DataType.kFloat32, [m, k])).dispatch_count() == 2
+    note(f"q8 matvec q8_0 [{k} -> {rows}] x {m}: strips, activation rows in groups of four")
+    check("q8_0", "f32", weights_for("q8_0", rng, rows, k), rows, k, rng.normal(0, 1.0, (m, k)).astype(np.float32),
+          kernel="gguf_matvec_q8_strips/q8_0/4-tokens")
