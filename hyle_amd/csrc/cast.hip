@@ -188,6 +188,77 @@ __global__ __launch_bounds__(kBlockThreads) void cast_general(const char *in, vo
   store_element<D::kSize>(out, e, convert_bits<S, D>(load_element<S::kSize>(in + offset)));
 }
 
+// Copy of a strided tensor whose innermost axes are runs of whole units (16, 8, 4 or 2 bytes, as large as
+// the run, the strides and the addresses allow): a unit per lane, its offset from 32-bit divisions
+// over the axes that cannot be folded into one.  Bound by HBM for runs of a cache line or more (a run
+// of 128 bf16: [1024, 16, 128] with its first two axes swapped, 8.4 MB, 3.4 us; element by element 8.5 us).
+template <class Unit>
+__global__ __launch_bounds__(kBlockThreads) void copy_units(const char *in, Unit *out, uint32_t units, CastLayout layout) {
+  const uint32_t e = blockIdx.x * kBlockThreads + threadIdx.x;
+  if (e >= units) return;
+  int64_t offset = 0;
+  uint32_t rest = e;
+  for (int axis = layout.rank - 1; axis > 0; --axis) {
+    const uint32_t above = rest / layout.dims[axis];
+    offset += (int64_t)(rest - above * layout.dims[axis]) * layout.strides[axis];
+    rest = above;
+  }
+  if (layout.rank > 0) offset += (int64_t)rest * layout.strides[0];
+  __builtin_nontemporal_store(*reinterpret_cast<const Unit *>(in + offset), out + e);
+}
+
+struct UnitsTag {
+  static std::string text() { return "copy_units"; }
+};
+
+// The axes of `p` with the inner ones counted in units of `size` bytes and neighbours folded
+// together where the outer one steps over exactly the inner one.  False if no unit from the
+// element's size up (two bytes at least) divides the strides, the run and the addresses.
+bool unit_layout(const CastParams &p, uintptr_t addresses, CastLayout *layout, uint32_t *size, uint64_t *units) {
+  uint64_t dims[kMaxRank];
+  int64_t strides[kMaxRank];
+  int rank = 0;
+  for (int i = 0; i < p.rank; ++i) {
+    if (p.dims[i] == 1) continue;
+    if (rank > 0 && strides[rank - 1] == p.strides[i] * (int64_t)p.dims[i]) {
+      dims[rank - 1] *= p.dims[i];
+      strides[rank - 1] = p.strides[i];
+    } else {
+      dims[rank] = p.dims[i];
+      strides[rank++] = p.strides[i];
+    }
+  }
+  if (rank == 0) return false;
+  const bool run = strides[rank - 1] == (int64_t)p.copy_size;
+  uint64_t marks = addresses;  // every bit that a unit must not reach into
+  for (int i = 0; i < rank - (run ? 1 : 0); ++i) marks |= (uint64_t)strides[i];
+  if (run) marks |= dims[rank - 1] * p.copy_size;
+  uint32_t unit = 16;
+  while (unit > 1 && (marks & (unit - 1)) != 0) unit /= 2;
+  if (!run && unit > p.copy_size) unit = p.copy_size;
+  if (unit < p.copy_size || unit < 2) return false;
+  if (run) {
+    dims[rank - 1] = dims[rank - 1] * p.copy_size / unit;
+    strides[rank - 1] = unit;
+  }
+  *size = unit;
+  *units = p.elements * p.copy_size / unit;
+  if (*units > 0x7FFFFFFFu) return false;
+  layout->rank = rank;
+  for (int i = 0; i < rank; ++i) {
+    layout->dims[i] = (uint32_t)dims[i];
+    layout->strides[i] = strides[i];
+  }
+  return true;
+}
+
+template <class Unit> hipError_t run_units(const void *in, void *out, uint64_t units, const CastLayout &layout, hipStream_t s) {
+  note_variant<UnitsTag>();
+  hipLaunchKernelGGL((copy_units<Unit>), dim3((uint32_t)((units + kBlockThreads - 1) / kBlockThreads)), dim3(kBlockThreads), 0, s,
+                     static_cast<const char *>(in), static_cast<Unit *>(out), (uint32_t)units, layout);
+  return hipGetLastError();
+}
+
 template <int kUnroll, int kThreads, bool kSerial> struct FlatTag {
   static std::string text() {
     return "cast_flat/" + std::to_string(kUnroll) + "x" + std::to_string(kThreads) + (kSerial ? "/serial" : "/batched");
@@ -267,6 +338,17 @@ hipError_t launch_cast(const CastParams &p, const void *in, void *out, bool vect
       CastParams words = p;
       words.elements = bytes / 4;
       return run_pair<CRaw4, CRaw4>(words, in, out, true, stream);
+    }
+    CastLayout layout{};
+    uint32_t size = 0;
+    uint64_t units = 0;
+    if (!p.dense_input && unit_layout(p, reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out), &layout, &size, &units)) {
+      switch (size) {
+        case 2: return run_units<uint16_t>(in, out, units, layout, stream);
+        case 4: return run_units<uint32_t>(in, out, units, layout, stream);
+        case 8: return run_units<u32x2>(in, out, units, layout, stream);
+        default: return run_units<u32x4>(in, out, units, layout, stream);
+      }
     }
     switch (p.copy_size) {
       case 1: return run_pair<CRaw1, CRaw1>(p, in, out, vectorised, stream);
