@@ -684,6 +684,7 @@ class OperationInvocation:
         self._prepared, self._workspace, self._workspace_size = prepared, workspace, workspace_size
         self._in = (C.c_void_p * capi.MAX_INPUTS)()
         self._out = (C.c_void_p * capi.MAX_OUTPUTS)()
+        self._launch = capi.load().hyle_hip_plan_launch
 
     def submit(self, stream: int, inputs: Sequence[int], outputs: Sequence[int]) -> None:
         """Enqueue on HIP stream handle `stream` (0 = default stream) and return at once.
@@ -692,9 +693,8 @@ class OperationInvocation:
             self._in[i] = p
         for i, p in enumerate(outputs):
             self._out[i] = p
-        _check(capi.load().hyle_hip_plan_launch(
-            self._prepared._handle, self._in, len(inputs), self._out, len(outputs),
-            self._workspace, self._workspace_size, stream))
+        _check(self._launch(self._prepared._handle, self._in, len(inputs), self._out, len(outputs),
+                            self._workspace, self._workspace_size, stream))
 
     def wait(self, stream: int, static_scratch: bool = False) -> None:
         """Completion::wait for launches whose kernels can refuse their input (checked Gather):
