@@ -24,8 +24,8 @@
 // goes straight into the lanes (52 us through the slot, 43 us straight).
 //
 // Bound by HBM for a vocabulary, by the quantising of every activation row in every compute unit and
-// by the start of a block below about 30 MB of weights (vector arithmetic: 17408 values of five rows
-// take about 9 of the 36 us).  MI355X, bf16 activations, the kernels that these shapes took before and here:
+// by the start of a block below about 30 MB of weights (vector arithmetic, by instruction count several
+// of the 37 us of five rows of 17408 values).  MI355X, bf16 activations, the kernels that these shapes took before and here:
 //   Q8_0 [5120 -> 17408] x 5   70.2 -> 28.4 us (3330 GB/s)    [17408 -> 5120] x 5  109.8 -> 37.1 us
 //   Q6_K [5120 -> 17408] x 5   70.3 -> 28.2 us                [17408 -> 5120] x 5  112.3 -> 35.7 us
 //   Q4_K [5120 -> 17408] x 5   44.9 -> 21.8 us                [17408 -> 5120] x 5  115.1 -> 31.2 us
