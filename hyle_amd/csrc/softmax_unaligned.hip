@@ -232,6 +232,8 @@ bool softmax_unaligned_serves(Elem type, const SoftmaxParams &p) {
   // a handful of short rows is one launch's latency either way and stays with the strided kernel
   // (f32 [6, 129]: 4.3 us there, 2.3 us here, of which 2 us are the dispatch)
   if (p.shape.rows * p.shape.width < 800) return false;
+  // a launch has fewer than 2^32 threads, and up to 1024 of them serve a row
+  if (p.shape.rows >= (1u << 22) && p.shape.width > 1024u * kvec) return false;
   const int64_t unit = (int)p.mask_kind == kMaskBoolean ? 1 : elem_size(type);
   return (int)p.mask_kind == kMaskNone || p.mask_inner_stride == unit;
 }
