@@ -17,7 +17,12 @@
 // A block of sixteen waves (eight where the codes leave no room for more slots) has a compute unit's
 // LDS, quantises the activation rows once, while its first weight bytes are on their way, and walks its
 // share of the weight rows in tiles of at most sixteen; `1 << split_log2` waves share a tile, each
-// taking every split-th run, and the first adds the shares in wave order.  Q8_0 and Q6_K runs are
+// taking every split-th run, and the first adds the shares.  A lane's chain of up to 224 runs, and the
+// sum over the shares, run in 64 bits: in 32, a chain that is several times as long as one of the
+// kernels that spread a row over 64 lanes was further from the 64-bit sum than theirs in a third of
+// the shapes (f32 Q8_0 [5120 -> 2304] x 6 9.6e-8 relative against 8.2e-8 there, Q4_K [4096 -> 6656] x 4
+// 7.6e-8 against 6.2e-8; in 64 bits 5.3e-8 and 4.5e-8, at most 0.75 of theirs over 87 shapes, for about
+// 1 % of the time).  Q8_0 and Q6_K runs are
 // loaded as the aligned vectors that cover them and redistributed through a wave-private slot: lanes
 // that load their own 16 bytes at 2-byte addresses keep the memory pipe busy several times as long
 // (Q8_0 [2048 -> 151936] 111 us that way, 63 us through the slot).  A Q4_K row is whole vectors and
@@ -139,13 +144,21 @@ __host__ __device__ inline StripLayout strip_layout(int kind, uint32_t m, uint32
   return at;
 }
 
+// The same value, which the compiler can no longer tell: what is worked out from it once a tile is worked
+// out there and takes no register through the runs (one that spills waits for every load in flight when
+// it comes back: Q8_0 [1536 -> 77056] x 8 39 us with nine spilled, 31 us).
+__device__ __forceinline__ uint32_t opaque(uint32_t value) {
+  asm volatile("" : "+v"(value));
+  return value;
+}
+
 // The dots of one run, closed: totals[set][i] gains activation row 4 set + i's part of the lane's groups.
 // `codes`: the lane's operand bases, `scales` / `sums`: the run's, at the lane's first group.
 template <int kKind, int kSets> struct StripDot;
 template <int kSets> struct StripDot<2, kSets> {
   static constexpr uint32_t first_chunk(uint32_t part) { return 2 * part; }
   static __device__ __forceinline__ void add(const Strip<2> &w, uint32_t part, const unsigned char *const (&codes)[kSets],
-                                             const float *scales, const int *, uint32_t run, float (&totals)[kSets][4]) {
+                                             const float *scales, const int *, uint32_t run, double (&totals)[kSets][4]) {
 #pragma unroll
     for (uint32_t j = 0; j < 2; ++j) {
       const float d = f16_to_f32(w.d[j]);
@@ -159,7 +172,7 @@ template <int kSets> struct StripDot<2, kSets> {
         }
         const f32x4 a = *reinterpret_cast<const f32x4 *>(scales + ((size_t)(8 * run + 4 * j + part) * kSets + set) * 4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) totals[set][i] = __builtin_fmaf(d * a[i], (float)dots[i], totals[set][i]);
+        for (int i = 0; i < 4; ++i) totals[set][i] = __builtin_fma((double)(d * a[i]), (double)dots[i], totals[set][i]);
       }
     }
   }
@@ -167,11 +180,11 @@ template <int kSets> struct StripDot<2, kSets> {
 template <int kSets> struct StripDot<1, kSets> {
   static constexpr uint32_t first_chunk(uint32_t part) { return 8 * (part / 2) + part % 2; }
   static __device__ __forceinline__ void add(const Strip<1> &w, uint32_t part, const unsigned char *const (&codes)[kSets],
-                                             const float *scales, const int *, uint32_t run, float (&totals)[kSets][4]) {
+                                             const float *scales, const int *, uint32_t run, double (&totals)[kSets][4]) {
     const u32x4 top = w.top ^ 0xAAAAAAAAu;  // q - 32 modulo 64: bytes of 4 (q - 32) as int8
     const u32x4 q[4] = {((w.low << 2) & 0x3C3C3C3Cu) | ((top << 6) & 0xC0C0C0C0u), ((w.high << 2) & 0x3C3C3C3Cu) | ((top << 4) & 0xC0C0C0C0u),
                         ((w.low >> 2) & 0x3C3C3C3Cu) | ((top << 2) & 0xC0C0C0C0u), ((w.high >> 2) & 0x3C3C3C3Cu) | (top & 0xC0C0C0C0u)};
-    const float step = f16_to_f32(w.d) * 0.25f;
+    const double step = (double)(f16_to_f32(w.d) * 0.25f);
     int scale[4];
 #pragma unroll
     for (int g = 0; g < 4; ++g) scale[g] = (int)(signed char)(w.scales[g / 2] >> (16 * (g % 2) + 8 * (part % 2)));
@@ -188,14 +201,14 @@ template <int kSets> struct StripDot<1, kSets> {
       }
       const f32x4 a = *reinterpret_cast<const f32x4 *>(scales + ((size_t)run * kSets + set) * 4);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) totals[set][i] = __builtin_fmaf(step * a[i], (float)whole[i], totals[set][i]);
+      for (int i = 0; i < 4; ++i) totals[set][i] = __builtin_fma(step * (double)a[i], (double)whole[i], totals[set][i]);
     }
   }
 };
 template <int kSets> struct StripDot<0, kSets> {
   static constexpr uint32_t first_chunk(uint32_t part) { return 4 * part; }
   static __device__ __forceinline__ void add(const Strip<0> &w, uint32_t part, const unsigned char *const (&codes)[kSets],
-                                             const float *scales, const int *sums, uint32_t run, float (&totals)[kSets][4]) {
+                                             const float *scales, const int *sums, uint32_t run, double (&totals)[kSets][4]) {
     // sub-blocks 2 p and 2 p + 1: neighbouring bytes of the table, whole six bits below sub-block 4,
     // from there on four bits in a nibble and two in the top of an earlier byte
     const uint32_t shift = 16 * (part % 2);
@@ -204,7 +217,7 @@ template <int kSets> struct StripDot<0, kSets> {
     const uint32_t sc = packed ? (third & 0x0F0Fu) | ((first >> 2) & 0x3030u) : first & 0x3F3Fu;
     const uint32_t mn = packed ? ((third >> 4) & 0x0F0Fu) | ((second >> 2) & 0x3030u) : second & 0x3F3Fu;
     const int sc_low = (int)(sc & 0xFFu), sc_high = (int)((sc >> 8) & 0xFFu), mn_low = (int)(mn & 0xFFu), mn_high = (int)((mn >> 8) & 0xFFu);
-    const float d = f16_to_f32((uint16_t)w.head.x), dmin = f16_to_f32((uint16_t)(w.head.x >> 16));
+    const double d = (double)f16_to_f32((uint16_t)w.head.x), dmin = (double)f16_to_f32((uint16_t)(w.head.x >> 16));
 #pragma unroll
     for (int set = 0; set < kSets; ++set) {
       i32x4 low = {0, 0, 0, 0}, high = {0, 0, 0, 0};
@@ -222,7 +235,7 @@ template <int kSets> struct StripDot<0, kSets> {
       for (int i = 0; i < 4; ++i) {
         const int scaled = mad24(sc_low, low[i], __mul24(sc_high, high[i]));
         const int minima = mad24(mn_low, sum_low[i], __mul24(mn_high, sum_high[i]));
-        totals[set][i] += a[i] * (d * (float)scaled - dmin * (float)minima);
+        totals[set][i] = __builtin_fma((double)a[i], __builtin_fma(d, (double)scaled, -(dmin * (double)minima)), totals[set][i]);
       }
     }
   }
@@ -330,7 +343,6 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
   const StripLayout layout = strip_layout(kKind, m, k, blockDim.x / kWaveLanes);
   float *scales = reinterpret_cast<float *>(shared + layout.scales);
   int *sums = reinterpret_cast<int *>(shared + layout.sums);
-  float *shares = reinterpret_cast<float *>(shared + layout.shares);
   const uint32_t lane = threadIdx.x % kWaveLanes;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveLanes);
   const uint32_t column = lane % 16, part = lane / 16;
@@ -355,6 +367,7 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
   using Pending = typename Held::Pending;
   uint32_t load_row[Held::kLoads];
   auto aim = [&]() {
+    const uint32_t lane = opaque(threadIdx.x % kWaveLanes), column = lane % 16;
 #pragma unroll
     for (uint32_t i = 0; i < Held::kLoads; ++i)
       load_row[i] = row_at(load_tile, Held::kParked ? min((lane + i * kWaveLanes) / Held::kVectors, kStripRows - 1) : column);
@@ -424,32 +437,40 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
 #pragma unroll
   for (uint32_t set = 0; set < (uint32_t)kSets; ++set)  // activation rows past the last repeat it and are not stored
     base[set] = faces ? kZeroBytes + min(column % 4 + 4 * set, m - 1) * (k + kCodePad) + Dot::first_chunk(part) * 16 : 0u;
-  float totals[kSets][4] = {};
+  double totals[kSets][4] = {};
   uint32_t run = member, tile = slot;
   uint32_t own_row = items != 0 ? (uint32_t)row_at(slot, column) : 0u;  // the lane's weight row
   unsigned char *parked = shared + layout.slots + wave * Held::kSlotBytes;
   // Lane (c, p) of the tile's first wave ends with activation row 4 set + p against weight row c.
   auto finish = [&]() {
+    const uint32_t lane = opaque(threadIdx.x % kWaveLanes), column = lane % 16, part = lane / 16;
     float mine[kSets];
 #pragma unroll
     for (int set = 0; set < kSets; ++set) {
       const bool upper = part >= 2, odd = part % 2 != 0;
-      float pair[2];
+      float own_sum[4], pair[2];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) own_sum[i] = (float)totals[set][i];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        pair[i] = (upper ? totals[set][2 + i] : totals[set][i]) + __shfl_xor(upper ? totals[set][i] : totals[set][2 + i], 32, kWaveLanes);
+        pair[i] = (upper ? own_sum[2 + i] : own_sum[i]) + __shfl_xor(upper ? own_sum[i] : own_sum[2 + i], 32, kWaveLanes);
       mine[set] = (odd ? pair[1] : pair[0]) + __shfl_xor(odd ? pair[0] : pair[1], 16, kWaveLanes);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) totals[set][i] = 0.0f;
+      for (int i = 0; i < 4; ++i) totals[set][i] = 0.0;
     }
     if (split_log2 != 0) {
+      // the wave's own share; those of the waves behind it follow, kSets * kWaveLanes apart
+      float *share = reinterpret_cast<float *>(shared + opaque(layout.shares + (wave * kSets * kWaveLanes + lane) * 4));
 #pragma unroll
-      for (int set = 0; set < kSets; ++set) shares[(wave * kSets + set) * kWaveLanes + lane] = mine[set];
+      for (int set = 0; set < kSets; ++set) share[set * kWaveLanes] = mine[set];
       lds_barrier();
       if (member == 0) {
 #pragma unroll
-        for (int set = 0; set < kSets; ++set)
-          for (uint32_t other = 1; other < split; ++other) mine[set] += shares[((wave + other) * kSets + set) * kWaveLanes + lane];
+        for (int set = 0; set < kSets; ++set) {
+          double whole = (double)mine[set];
+          for (uint32_t other = 1; other < split; ++other) whole += (double)share[(other * kSets + set) * kWaveLanes];
+          mine[set] = (float)whole;
+        }
       }
       lds_barrier();
     }
@@ -489,7 +510,7 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
         finish();
         run = member;
         tile += slots;
-        own_row = (uint32_t)row_at(min(tile, tiles - 1), column);
+        own_row = (uint32_t)row_at(min(tile, tiles - 1), opaque(threadIdx.x % kWaveLanes) % 16);
       }
     }
   }

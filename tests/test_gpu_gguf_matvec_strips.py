@@ -6,10 +6,12 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from hyle_amd import compute as hc
+from oracle import lib as orc
 
-from gpu_support import context, note
+from gpu_support import DEVICE, context, note, run
 from test_gpu_gguf_matvec_q8 import KINDS, Q8, check, raw_bytes_for, weights_for
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +67,33 @@ def test_strips_activation_rows_in_groups():
     note(f"q8 matvec q8_0 [{k} -> {rows}] x {m}: strips, activation rows in groups of four")
     check("q8_0", "f32", weights_for("q8_0", rng, rows, k), rows, k, rng.normal(0, 1.0, (m, k)).astype(np.float32),
           kernel="gguf_matvec_q8_strips/q8_0/4-tokens")
+
+
+@pytest.mark.parametrize("tag,k,rows,m,byte_offset", [
+    ("q8_0", 5120, 2304, 6, 0), ("q8_0", 2560, 8192, 4, 0), ("q6_k", 5120, 3584, 8, 0), ("q6_k", 1024, 8192, 5, 0),
+    ("q4_k", 4096, 6656, 4, 0), ("q4_k", 9984, 3072, 5, 2)])
+def test_strips_are_no_further_from_64_bit_sums(tag, k, rows, m, byte_offset):
+    """f32 products of the strip kernel against those of the kernels that serve the same rows in slices of 256 (too
+    few for strips), both against the oracle's float64 sums over the same 8-bit codes: the strips' error must not be
+    the larger one, over all products (2-norm; summed in 32 bits it was for all of these but the second Q6_K, by 1.04 to 1.2)."""
+    rng = np.random.default_rng(1823)
+    raw = weights_for(tag, rng, rows, k)
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    kind, gguf = KINDS[tag]
+    storage = torch.from_numpy(np.concatenate([np.zeros(byte_offset, np.uint8), raw.reshape(-1)])).to(DEVICE)[byte_offset:].view(rows, -1)
+    activations = torch.from_numpy(x).to(DEVICE)
+
+    def products(first, count):
+        descs = [hc.TensorDesc.gguf_weight(gguf, hc.DataType.kFloat32, k, count), hc.TensorDesc.dense(hc.DataType.kFloat32, [m, k])]
+        (out,) = run(Q8, storage[first:first + count], activations, descs=descs)
+        return out.cpu().numpy().astype(np.float64), hc.last_launch_variant()
+
+    note(f"q8 matvec {tag} [{k} -> {rows}] x {m} off {byte_offset}: strips and slices of 256 rows against float64")
+    whole, label = products(0, rows)
+    assert label.startswith("gguf_matvec_q8_strips"), label
+    slices = [products(first, 256) for first in range(0, rows, 256)]
+    assert all("strips" not in label for _, label in slices)
+    centre, _ = orc.gguf_matvec_q8(kind, raw.reshape(-1), rows, k, x)
+    centre = centre.reshape(m, rows)
+    own, others = np.linalg.norm(whole - centre), np.linalg.norm(np.concatenate([part for part, _ in slices], 1) - centre)
+    assert own <= others, f"{own / others:.3f} of the error of the kernels for few rows"
