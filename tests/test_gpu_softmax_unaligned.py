@@ -53,3 +53,27 @@ def test_rows_of_any_width_at_both_ends_of_a_launch_shape(shape, tag):
         for mask_word in ("unmasked", "boolean", "additive"):
             check(tag, q, width, mask_word, label, False, moved, in_place=mask_word == "boolean")
         check(tag, q, width, "boolean", label, True, moved, in_place=False)
+
+
+@pytest.mark.parametrize("lowest", [-20.0, -85.0])
+@pytest.mark.parametrize("tag", ["bf16", "f16"])
+def test_narrow_rows_are_no_further_from_64_bits_than_the_strided_kernel(tag, lowest):
+    """The exponentials behind a narrow result are 32-bit ones with errors below 2e-6, so few results are on the wrong side of
+    a rounding; counted against float64 there must be no more of them than softmax_general gives for the same rows seen
+    through a stride.  Where both exponentials are as good as each other their last bits still differ: two units of 2^-24 move
+    a share of 2 * 2^-24 / 2^-8 of bf16 results across a rounding, for the better or the worse alike, so the counts may differ
+    by three standard deviations of that (17; a single multiply-add into exp2 has 58 too many at bf16 down to e^-85, 20 too
+    many at f16 down to e^-20)."""
+    rows, width, scale = 1024, 1013, 0.7
+    generator = torch.Generator(device=DEVICE).manual_seed(1840)
+    x = torch.empty((rows, width), device=DEVICE).uniform_(lowest / scale, 0.0, generator=generator).to(TYPES[tag][2])
+    spread = torch.zeros((rows, width, 2), dtype=x.dtype, device=DEVICE)
+    spread[..., 0] = x
+    exact = torch.softmax((x.float() * scale).double(), -1).to(x.dtype)   # one rounding
+    note(f"softmax {tag} [{rows}, {width}] down to {lowest}: dense and strided rows against float64")
+    wrong = []
+    for rows_seen, label in ((x, "unaligned_softmax/"), (spread[..., 0], "softmax_general")):
+        (out,) = run(hc.Softmax(scale=scale), rows_seen)
+        assert hc.last_launch_variant().startswith(label)
+        wrong.append(int((out.view(torch.int16) != exact.view(torch.int16)).sum()))
+    assert wrong[0] <= wrong[1] + 3.0 * (rows * width * 2.0 ** -15) ** 0.5, wrong
