@@ -18,6 +18,7 @@
 //   general  anything else (strides, scattered axes, unaligned bytes): one wave per result,
 //            coordinates by division.  Correct, not tuned.
 #include <algorithm>
+#include <type_traits>
 
 #include "device_common.h"
 #include "kernels.h"
@@ -25,7 +26,6 @@
 namespace hyle_hip {
 namespace {
 
-constexpr uint32_t kBatch = 8;  // 16-byte loads of a lane in flight
 enum : int { kSum = 0, kMean = 1, kMinimum = 2, kMaximum = 3 };
 
 template <int kKind> __device__ __forceinline__ float reduce_identity() {
@@ -40,6 +40,24 @@ template <int kKind> __device__ __forceinline__ float reduce_step(float acc, flo
 template <int kKind> __device__ __forceinline__ float reduce_final(float acc, float divisor) {
   if constexpr (kKind == kMean) return acc / divisor;
   else return acc;
+}
+
+// Calls trip(n) with n = kMost, ..., 4, 2 or 1 as a constant until `steps` steps are done: trips of kMost, then
+// the smallest one that ends it.  A trip is that many 16-byte loads of a lane in flight at once, clamped to
+// the last one there is, so a lane with up to kMost waits for memory once and one with fewer does not load
+// more than it has.  Rows, us in trips of four, two and then one / of eight always / here: f32 [5902, 1968]
+// 9.5 / 8.6 / 8.6, [5003, 2560] 10.1 / 10.4 / 9.4, [16384, 2048] 20.6 / 26.4 / 20.7, [2^20, 64] 143 / 258 / 145,
+// bf16 [65536, 512] 14.6 / 21.9 / 14.8.
+template <uint32_t kLoads> using Loads = std::integral_constant<uint32_t, kLoads>;
+template <uint32_t kMost, class Trip> __device__ __forceinline__ void in_trips(uint32_t steps, Trip trip) {
+  if (steps == 1) return trip(Loads<1>{});
+  if (steps > 2) {
+    for (; steps > kMost; steps -= kMost) trip(Loads<kMost>{});
+    if (kMost > 4 && steps > 4) return trip(Loads<8>{});
+    if (kMost > 2 && steps > 2) return trip(Loads<4>{});
+  }
+  if (steps == 2) trip(Loads<2>{});
+  else if (steps == 1) trip(Loads<1>{});
 }
 
 // ---- rows -------------------------------------------------------------------------------------
@@ -64,24 +82,25 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_rows(const void *x, void
       const size_t base = (size_t)row * (width / kVec);
       const uint32_t last = end / kVec;
       uint32_t vec = begin / kVec + lane;
-      // One trip to memory for a row of up to kBatch vectors a lane, which is what bounds rows that all run
-      // at once (f32 over the last axis, with four, two and then one in flight / with kBatch: [5902, 1968] 14.4 /
-      // 12.2 us, [5003, 2560] 14.1 / 13.6).  A vector past the tile is its last one again and is dropped.
-      for (; vec < last; vec += kBatch * kLanes) {
-        u32x4 raw[kBatch];
+      // a vector past the tile is its last one again and is dropped
+      in_trips<8>(__builtin_amdgcn_readfirstlane((last - begin / kVec + kLanes - 1) / kLanes), [&](auto loads) {
+        constexpr uint32_t kLoads = decltype(loads)::value;
+        if (vec >= last) return;  // nothing left of this lane's
+        u32x4 raw[kLoads];
 #pragma unroll
-        for (uint32_t i = 0; i < kBatch; ++i) raw[i] = load16_stream(x, base + min(vec + i * kLanes, last - 1));
+        for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (i == 0 ? vec : min(vec + i * kLanes, last - 1)));
 #pragma unroll
-        for (uint32_t i = 0; i < kBatch; ++i) loads_issued(raw[i]);
+        for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
 #pragma unroll
-        for (uint32_t i = 0; i < kBatch; ++i) {
-          if (vec + i * kLanes >= last) break;
+        for (uint32_t i = 0; i < kLoads; ++i) {
+          if (i != 0 && vec + i * kLanes >= last) break;
           float v[kVec];
           Traits<TIn>::unpack(raw[i], v);
 #pragma unroll
           for (int j = 0; j < kVec; ++j) acc = reduce_step<kKind>(acc, v[j]);
         }
-      }
+        vec += kLoads * kLanes;
+      });
     } else {
       const size_t base = (size_t)row * width;
       for (uint32_t i = begin + lane; i < end; i += kLanes)
@@ -97,7 +116,7 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_rows(const void *x, void
 // lanes_y along `reduced`.  Grid: x = outer * x_tiles + tile of `inner`, y = segment of `reduced`.
 // The output index of (segment, outer, column) is (segment * outer_count + outer) * inner +
 // column: with one segment that is the final tensor, otherwise f32 partial results.
-template <class TIn, class TOut, int kKind, bool kVector>
+template <class TIn, class TOut, int kKind, bool kVector, uint32_t kMost>
 __global__ __launch_bounds__(kBlockThreads) void reduce_columns(const void *x, void *y,
                                                                 uint32_t outer_count,
                                                                 uint32_t reduced, uint32_t inner,
@@ -121,23 +140,24 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_columns(const void *x, v
     const size_t base = (size_t)outer * reduced * units + unit;  // in units
     uint32_t r = begin + ty;
     if constexpr (kVector) {
-      // kBatch rows of a lane in flight, as above (f32 [586, 1072] over the first axis, both dispatches, two
-      // in flight / kBatch: 9.6 / 8.2 us)
-      for (; r < end; r += kBatch * lanes_y) {
-        u32x4 raw[kBatch];
+      in_trips<kMost>((end - begin + lanes_y - 1) / lanes_y, [&](auto loads) {
+        constexpr uint32_t kLoads = decltype(loads)::value;
+        if (r >= end) return;
+        u32x4 raw[kLoads];
 #pragma unroll
-        for (uint32_t i = 0; i < kBatch; ++i) raw[i] = load16_stream(x, base + (size_t)min(r + i * lanes_y, end - 1) * units);
+        for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (size_t)(i == 0 ? r : min(r + i * lanes_y, end - 1)) * units);
 #pragma unroll
-        for (uint32_t i = 0; i < kBatch; ++i) loads_issued(raw[i]);
+        for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
 #pragma unroll
-        for (uint32_t i = 0; i < kBatch; ++i) {
-          if (r + i * lanes_y >= end) break;
+        for (uint32_t i = 0; i < kLoads; ++i) {
+          if (i != 0 && r + i * lanes_y >= end) break;
           float v[kW];
           Traits<TIn>::unpack(raw[i], v);
 #pragma unroll
           for (int j = 0; j < kW; ++j) acc[j] = reduce_step<kKind>(acc[j], v[j]);
         }
-      }
+        r += kLoads * lanes_y;
+      });
     } else {
       for (; r < end; r += lanes_y)
         acc[0] = reduce_step<kKind>(acc[0], Traits<TIn>::load(x, base + (size_t)r * units));
@@ -221,12 +241,12 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_general(const char *x, v
 // ---- host side --------------------------------------------------------------------------------
 uint32_t ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-// reduce_rows/<block|wave per unit>/<vector|scalar>, reduce_columns/<vector|scalar>, reduce_general[/bytes]
+// reduce_rows/<block|wave per unit>/<vector|scalar>, reduce_columns/<vector/rows in flight|scalar>, reduce_general[/bytes]
 template <bool kBlock, bool kVector> struct RowsTag {
   static std::string text() { return std::string("reduce_rows/") + (kBlock ? "block" : "wave") + (kVector ? "/vector" : "/scalar"); }
 };
-template <bool kVector> struct ColumnsTag {
-  static std::string text() { return std::string("reduce_columns/") + (kVector ? "vector" : "scalar"); }
+template <bool kVector, uint32_t kMost> struct ColumnsTag {
+  static std::string text() { return std::string("reduce_columns/") + (kVector ? "vector/" + std::to_string(kMost) : "scalar"); }
 };
 template <bool kBytewise> struct GeneralTag {
   static std::string text() { return kBytewise ? "reduce_general/bytes" : "reduce_general"; }
@@ -278,14 +298,23 @@ void columns_launch(const void *x, void *y, uint32_t outer, uint32_t reduced, ui
   const uint32_t log2 = lanes_x_log2_for(units, outer);
   const uint32_t x_tiles = ceil_div(units, 1u << log2);
   const dim3 grid(x_tiles * outer, segments, 1);
-  if (vector) note_variant<ColumnsTag<true>>();
-  else note_variant<ColumnsTag<false>>();
-  if (vector)
-    hipLaunchKernelGGL((reduce_columns<TIn, TOut, kKind, true>), grid, dim3(kBlockThreads), 0, s, x, y,
-                       outer, reduced, inner, log2, x_tiles, segment_rows, divisor);
-  else
-    hipLaunchKernelGGL((reduce_columns<TIn, TOut, kKind, false>), grid, dim3(kBlockThreads), 0, s, x, y,
-                       outer, reduced, inner, log2, x_tiles, segment_rows, divisor);
+  // Rows of a lane in flight.  With one or two blocks per compute unit many are needed, with up to five two keep
+  // the memory busy and more get in each other's way; above that a lane has its eight rows and more to walk, and
+  // four are the better again, unless there is no second dispatch because the rows are few.  us, two / four / eight:
+  //   f32 [1024, 2048] 7.2 / 6.4 / 6.2, [586, 1072] 8.2 / 7.2 / 7.1, [2000, 2048] 8.4 / 7.8 / 8.2, [1024, 3072] 7.6 / 7.2 / 7.5
+  //   f32 [64, 131072] 7.5 / 8.5 / 9.4, [3, 256, 8192] middle axis 6.6 / 7.0 / 7.1, bf16 [8192, 2048] 10.4 / 11.1 / 10.9
+  //   f32 [5003, 2560] 15.1 / 14.2 / 14.4, [7000, 2048] 15.7 / 15.1 / 15.2; but [16, 2^20] 15.1 / 17.0 / 17.0
+  const uint64_t blocks = (uint64_t)grid.x * segments;
+  const int most = blocks <= 256 ? 8 : (blocks <= 512 || (blocks >= 1280 && segments > 1) ? 4 : 2);
+#define HYLE_COLUMNS(VECTOR, MOST)                                                                                            \
+  note_variant<ColumnsTag<VECTOR, MOST>>();                                                                                   \
+  hipLaunchKernelGGL((reduce_columns<TIn, TOut, kKind, VECTOR, MOST>), grid, dim3(kBlockThreads), 0, s, x, y, outer, reduced, \
+                     inner, log2, x_tiles, segment_rows, divisor)
+  if (!vector) { HYLE_COLUMNS(false, 1); }
+  else if (most == 8) { HYLE_COLUMNS(true, 8); }
+  else if (most == 4) { HYLE_COLUMNS(true, 4); }
+  else { HYLE_COLUMNS(true, 2); }
+#undef HYLE_COLUMNS
 }
 
 template <class T, int kKind>

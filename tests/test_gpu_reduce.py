@@ -254,3 +254,26 @@ def test_reduce_benchmark_shapes():
             operation = hc.Reduce(kind, hc.Axes.all() if axes is None else hc.Axes.from_(axes), accumulation_type=F32ACC)
             (out,) = run(operation, to_device(x, tag))
             check(kind, tag, to_host(out), x, dims, axes)
+
+
+# [rows, columns] in f32, reduced axis, launch shape: a lane has 1, 2, 3, ... vectors (rows) of its row or column, and
+# the last lanes one fewer; waves and blocks to a row, the three depths of the columns, one and two dispatches
+LOADS = ([([5, 256 * s - 4], 1, "reduce_rows/wave/vector") for s in (1, 2, 3, 4, 5, 7)] +
+         [([3, 1024 * s - 4], 1, "reduce_rows/block/vector") for s in (3, 4, 5, 8, 9, 12, 17)] +
+         [([32 * s - 1, 1028], 0, "reduce_columns/vector/8") for s in (1, 2, 3, 4, 5, 8, 9, 15, 17)] +
+         [([32 * s - 1, 9600], 0, "reduce_columns/vector/4") for s in (1, 3, 5, 6)] +
+         [([32 * s - 1, 19200], 0, "reduce_columns/vector/2") for s in (1, 2, 3)] + [([512, 20480], 0, "reduce_columns/vector/4")])
+
+
+@pytest.mark.parametrize("tag", ["f32", "bf16"])
+def test_reduce_with_every_number_of_loads_a_lane(tag):
+    rng = np.random.default_rng(990)
+    for dims, axis, label in LOADS:
+        if tag == "bf16":   # twice the elements to a vector
+            dims = [dims[0], 2 * dims[1]]
+        for kind in (RK.kSum, RK.kMaximum):
+            x = values_for(rng, dims, tag, plant=kind == RK.kMaximum)
+            note(f"reduce {kind.name} {tag} {dims} over axis {axis}: {label}")
+            (out,) = run(hc.Reduce(kind, hc.Axes.from_([axis]), accumulation_type=F32ACC), to_device(x, tag))
+            assert hc.last_launch_variant().startswith(label), (dims, hc.last_launch_variant())
+            check(kind, tag, to_host(out), x, dims, [axis])
