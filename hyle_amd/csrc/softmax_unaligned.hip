@@ -16,6 +16,7 @@
 //   f32  [24, 777, 1013]  179 -> 27.8 us (5440 GB/s)    f32 [12, 777, 7001] Boolean 658 -> 91.7 us (5750 GB/s)
 //   bf16 [24, 777, 3001]  488 -> 39.0 us (5745 GB/s; an aligned row of 3000 in softmax.hip: 45.4)
 //   f16  [24, 777, 100]    41 ->  3.7 us               f32 [8, 1, 1271] 12.6 -> 2.4 us
+//   f32  [1, 777] 10.3 -> 2.2 us, [6, 129] 4.4 -> 1.9 us, [1, 5] 4.1 -> 1.8 us: no call is too small for it
 // Running the heads of a mask row next to each other on one XCD, which pays for 64 MiB masks
 // (softmax.hip), loses here: bf16 [24, 777, 1013] additive 17.5 -> 20.2 us, f32 [32, 1777, 1777]
 // 149 -> 161 us.
@@ -248,9 +249,6 @@ template <class T> void run_width(const SoftmaxParams &p, const void *x, const v
 bool softmax_unaligned_serves(Elem type, const SoftmaxParams &p) {
   const uint32_t kvec = (uint32_t)elem_vec(type);
   if (p.shape.width < kvec || p.shape.width > 8u * 1024u * kvec) return false;
-  // a handful of short rows is one launch's latency either way and stays with the strided kernel
-  // (f32 [6, 129]: 4.3 us there, 2.3 us here, of which 2 us are the dispatch)
-  if (p.shape.rows * p.shape.width < 800) return false;
   // a launch has fewer than 2^32 threads, and up to 1024 of them serve a row
   if (p.shape.rows >= (1u << 22) && p.shape.width > 1024u * kvec) return false;
   const int64_t unit = (int)p.mask_kind == kMaskBoolean ? 1 : elem_size(type);

@@ -28,8 +28,8 @@ def offset_by_one(t):
     return flat[1:].view(t.shape)
 
 
-def check(tag, q, width, mask_word, shape, log_form, moved, in_place):
-    heads, scale = 2, 0.125 if mask_word != "unmasked" else 1.0
+def check(tag, q, width, mask_word, shape, log_form, moved, in_place, heads=2):
+    scale = 0.125 if mask_word != "unmasked" else 1.0
     note(f"softmax {tag} log={log_form} [{heads}, {q}, {width}] {mask_word} moved={moved} in_place={in_place}: expecting {shape}")
     x, x_host, mask, mask_host = make_inputs(tag, heads, q, width, mask_word, seed=width + q)
     if moved:
@@ -53,6 +53,16 @@ def test_rows_of_any_width_at_both_ends_of_a_launch_shape(shape, tag):
         for mask_word in ("unmasked", "boolean", "additive"):
             check(tag, q, width, mask_word, label, False, moved, in_place=mask_word == "boolean")
         check(tag, q, width, "boolean", label, True, moved, in_place=False)
+
+
+@pytest.mark.parametrize("tag", ["f32", "bf16", "f16"])
+def test_a_few_short_rows(tag):
+    """One head, one to six rows, from a single vector and one element on: no size is too small for these launch shapes."""
+    vec = 16 // TYPES[tag][2].itemsize
+    for q, width in ((1, vec + 1), (2, vec + 1), (1, 129), (6, 129), (1, 777), (4, 197)):
+        shape = next(label for fewest, most, label in SHAPES if fewest <= (width + vec - 1) // vec <= most)
+        for mask_word in ("unmasked", "boolean", "additive"):
+            check(tag, q, width, mask_word, shape, False, width * q % vec == 0, in_place=False, heads=1)
 
 
 @pytest.mark.parametrize("lowest", [-20.0, -85.0])
