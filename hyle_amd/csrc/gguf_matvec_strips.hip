@@ -358,7 +358,7 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
   auto row_of = [&](uint32_t tile, uint32_t r) { return row_begin + tile * tile_rows + r; };
   auto tile_end = [&](uint32_t tile) { return min(row_begin + (tile + 1) * tile_rows, row_end); };
   // rows past a tile's last one are that row again and are not stored
-  // (bytes from the block's first row: below 2^32, see run_strips)
+  // (bytes from the block's first row: below 2^32, see gguf_matvec_strips_serve)
   const uintptr_t own = reinterpret_cast<uintptr_t>(weights) + (uint64_t)row_begin * row_stride;
   auto row_at = [&](uint32_t tile, uint32_t r) { return (min(row_of(tile, r), tile_end(tile) - 1) - row_begin) * (uint32_t)row_stride; };
   uint32_t load_tile = slot, load_run = member, loads_left = items;

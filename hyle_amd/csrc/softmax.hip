@@ -290,6 +290,26 @@ __global__ __launch_bounds__(kBlockThreads) void softmax_general(const char *x, 
 }
 
 // ---- host dispatch ----------------------------------------------------------------------------
+// The leading axes a mask is broadcast over: x rows r and r + period share a mask row,
+// `repeats` times.  repeats = 1 when the mask has no such axes (or there is no mask).
+struct MaskRepeat {
+  uint32_t period, repeats;
+};
+MaskRepeat mask_repeat(const SoftmaxParams &p) {
+  MaskRepeat r{(uint32_t)p.shape.rows, 1};
+  if (p.mask_kind == 0) return r;
+  uint64_t repeats = 1;
+  for (int i = 0; i < p.outer_rank; ++i) {
+    if (p.mask_outer_strides[i] != 0 && p.outer_dims[i] != 1) break;
+    repeats *= p.outer_dims[i];
+  }
+  if (repeats > 1 && p.shape.rows % repeats == 0) {
+    r.repeats = (uint32_t)repeats;
+    r.period = (uint32_t)(p.shape.rows / repeats);
+  }
+  return r;
+}
+
 // softmax_rows/<lanes>x<vectors per lane>/<threads per block>/<mask>/<exact|ragged>[/steered]
 template <int kLanes, int kVpl, int kThreads, int kMask, bool kExact, bool kSteered> struct RowsTag {
   static std::string text() {

@@ -22,6 +22,14 @@
 namespace hyle_hip {
 namespace {
 
+// exp(t) * 2^32 for t <= 0, for results that are stored in 8 or 11 significand bits: one fused
+// multiply-add into the hardware exp2 (about 1e-6 relative; -inf gives 0).  f32 storage keeps the
+// form with the exact residual.
+template <class T> __device__ __forceinline__ float exp_for(float t) {
+  if constexpr (Traits<T>::kSize == 4) return exp_scaled(t);
+  else return __builtin_amdgcn_exp2f(__builtin_fmaf(t, 1.44269504088896340736f, 32.0f));
+}
+
 // kMask: a Boolean mask (one byte per column, 0 = the column is left out) or an additive one (the
 // row's type), a value per column, rows found through `mrows` as in softmax.hip.  A vector whose
 // columns are all left out is not loaded: its lane reads the row's first vector instead (no new

@@ -23,14 +23,6 @@ __device__ __forceinline__ float exp_scaled(float t) {
   return __builtin_fmaf(p, lo * kLn2, p);
 }
 
-// exp(t) * 2^32 for t <= 0, for results that are stored in 8 or 11 significand bits: one fused
-// multiply-add into the hardware exp2 (about 1e-6 relative; -inf gives 0).  f32 storage keeps the
-// form with the exact residual.
-template <class T> __device__ __forceinline__ float exp_for(float t) {
-  if constexpr (Traits<T>::kSize == 4) return exp_scaled(t);
-  else return __builtin_amdgcn_exp2f(__builtin_fmaf(t, 1.44269504088896340736f, 32.0f));
-}
-
 // NaN or +inf: the values that make a softmax row undefined
 // (src/simd/math/activations.cc:181-186).
 __device__ __forceinline__ bool poisons_row(float v) {
@@ -54,26 +46,6 @@ __device__ __forceinline__ int64_t mask_row_offset(const MaskRows &m, uint32_t r
     rest /= extent;
   }
   return offset;
-}
-
-// The leading axes a mask is broadcast over: x rows r and r + period share a mask row,
-// `repeats` times.  repeats = 1 when the mask has no such axes (or there is no mask).
-struct MaskRepeat {
-  uint32_t period, repeats;
-};
-MaskRepeat mask_repeat(const SoftmaxParams &p) {
-  MaskRepeat r{(uint32_t)p.shape.rows, 1};
-  if (p.mask_kind == 0) return r;
-  uint64_t repeats = 1;
-  for (int i = 0; i < p.outer_rank; ++i) {
-    if (p.mask_outer_strides[i] != 0 && p.outer_dims[i] != 1) break;
-    repeats *= p.outer_dims[i];
-  }
-  if (repeats > 1 && p.shape.rows % repeats == 0) {
-    r.repeats = (uint32_t)repeats;
-    r.period = (uint32_t)(p.shape.rows / repeats);
-  }
-  return r;
 }
 
 inline const char *mask_word(int mask) {

@@ -249,8 +249,8 @@ template <class T> void run_width(const SoftmaxParams &p, const void *x, const v
 bool softmax_unaligned_serves(Elem type, const SoftmaxParams &p) {
   const uint32_t kvec = (uint32_t)elem_vec(type);
   if (p.shape.width < kvec || p.shape.width > 8u * 1024u * kvec) return false;
-  // a launch has fewer than 2^32 threads, and up to 1024 of them serve a row
-  if (p.shape.rows >= (1u << 22) && p.shape.width > 1024u * kvec) return false;
+  // A launch has fewer than 2^32 threads, which needs no line here: admission takes at most 2^31 - 1 elements, and a
+  // row of more than one vector has less than two lanes to an element.
   const int64_t unit = (int)p.mask_kind == kMaskBoolean ? 1 : elem_size(type);
   return (int)p.mask_kind == kMaskNone || p.mask_inner_stride == unit;
 }
