@@ -181,10 +181,10 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x
   }
 }
 
-// unaligned_softmax/<lanes>x<vectors per lane>/<threads per block>/<mask>
+// softmax_unaligned/<lanes>x<vectors per lane>/<threads per block>/<mask>
 template <int kLanes, int kVpl, int kThreads, int kMask> struct UnalignedTag {
   static std::string text() {
-    return "unaligned_softmax/" + std::to_string(kLanes) + "x" + std::to_string(kVpl) + "/" + std::to_string(kThreads) + "/" + mask_word(kMask);
+    return "softmax_unaligned/" + std::to_string(kLanes) + "x" + std::to_string(kVpl) + "/" + std::to_string(kThreads) + "/" + mask_word(kMask);
   }
 };
 

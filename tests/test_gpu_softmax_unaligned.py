@@ -28,17 +28,19 @@ def offset_by_one(t):
     return flat[1:].view(t.shape)
 
 
-def check(tag, q, width, mask_word, shape, log_form, moved, in_place, heads=2):
+def check(tag, q, width, mask_word, shape, log_form, moved, in_place, heads=2, mask_moved=False):
     scale = 0.125 if mask_word != "unmasked" else 1.0
-    note(f"softmax {tag} log={log_form} [{heads}, {q}, {width}] {mask_word} moved={moved} in_place={in_place}: expecting {shape}")
+    note(f"softmax {tag} log={log_form} [{heads}, {q}, {width}] {mask_word} moved={moved} {mask_moved} in_place={in_place}: expecting {shape}")
     x, x_host, mask, mask_host = make_inputs(tag, heads, q, width, mask_word, seed=width + q)
-    if moved:
+    if moved:   # x, or a mask under rows that are no whole number of vectors anyway
         x = offset_by_one(x)
+    if mask is not None and (moved or mask_moved):
+        mask = offset_by_one(mask)
     want = oracle_softmax(tag, x_host, mask_word, mask_host, scale, log_form)
     kind = hc.SoftmaxKind.kLogSoftmax if log_form else hc.SoftmaxKind.kSoftmax
     (out,) = run(hc.Softmax(scale=scale, kind=kind, mask=MASKS[mask_word]), *([x] if mask is None else [x, mask]),
                  outputs=[x] if in_place else None)
-    assert hc.last_launch_variant() == f"unaligned_softmax/{shape}/{mask_word}"
+    assert hc.last_launch_variant() == f"softmax_unaligned/{shape}/{mask_word}"
     count, text = compare_on_device(tag, out, want, log_form)
     assert count == 0, f"{count} elements outside the bar, {text}"
 
@@ -52,7 +54,10 @@ def test_rows_of_any_width_at_both_ends_of_a_launch_shape(shape, tag):
         q = max(5, 400 // width + 1)
         for mask_word in ("unmasked", "boolean", "additive"):
             check(tag, q, width, mask_word, label, False, moved, in_place=mask_word == "boolean")
-        check(tag, q, width, "boolean", label, True, moved, in_place=False)
+            check(tag, q, width, mask_word, label, True, moved, in_place=False, mask_moved=True)
+    # rows of whole vectors under a mask that starts one element behind a boundary
+    for mask_word in ("boolean", "additive"):
+        check(tag, max(5, 400 // (most * vec) + 1), most * vec, mask_word, label, False, False, in_place=False, mask_moved=True)
 
 
 @pytest.mark.parametrize("tag", ["f32", "bf16", "f16"])
@@ -82,7 +87,7 @@ def test_narrow_rows_are_no_further_from_64_bits_than_the_strided_kernel(tag, lo
     exact = torch.softmax((x.float() * scale).double(), -1).to(x.dtype)   # one rounding
     note(f"softmax {tag} [{rows}, {width}] down to {lowest}: dense and strided rows against float64")
     wrong = []
-    for rows_seen, label in ((x, "unaligned_softmax/"), (spread[..., 0], "softmax_general")):
+    for rows_seen, label in ((x, "softmax_unaligned/"), (spread[..., 0], "softmax_general")):
         (out,) = run(hc.Softmax(scale=scale), rows_seen)
         assert hc.last_launch_variant().startswith(label)
         wrong.append(int((out.view(torch.int16) != exact.view(torch.int16)).sum()))

@@ -280,6 +280,13 @@ CASES = [
     ("f32", 22, 256, 3072, "boolean", "softmax_rows/256x4/256/boolean/ragged"),
     ("f32", 4, 4096, 4096, "boolean", "softmax_rows/64x16/64/boolean/exact"),
     ("bf16", 2, 3, 70000, "boolean", "softmax_general"),
+] + [
+    # rows that are no whole number of vectors, each shape at its widest
+    ("bf16", 2, 8, 8 * vectors - 1, mask_word, f"softmax_unaligned/{shape}/{mask_word}")
+    for vectors, shape in ((8, "8x1/256"), (16, "16x1/256"), (32, "16x2/256"), (64, "32x2/256"), (96, "32x3/256"), (128, "64x2/256"), (192, "64x3/256"),
+                           (256, "64x4/256"), (384, "128x3/256"), (512, "128x4/256"), (768, "256x3/256"), (1024, "256x4/256"), (1536, "512x3/512"),
+                           (2048, "512x4/512"), (8192, "1024x8/1024"))
+    for mask_word in ("unmasked", "boolean", "additive")
 ]
 
 MASKS = {"unmasked": hc.MaskKind.kNone, "additive": hc.MaskKind.kAdditive, "boolean": hc.MaskKind.kBoolean}
