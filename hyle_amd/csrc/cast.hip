@@ -207,8 +207,9 @@ __global__ __launch_bounds__(kBlockThreads) void copy_units(const char *in, Unit
   __builtin_nontemporal_store(*reinterpret_cast<const Unit *>(in + offset), out + e);
 }
 
-struct UnitsTag {
-  static std::string text() { return "copy_units"; }
+// copy_units/<bytes of a unit>
+template <class Unit> struct UnitsTag {
+  static std::string text() { return "copy_units/" + std::to_string(sizeof(Unit)); }
 };
 
 // The axes of `p` with the inner ones counted in units of `size` bytes and neighbours folded
@@ -253,7 +254,7 @@ bool unit_layout(const CastParams &p, uintptr_t addresses, CastLayout *layout, u
 }
 
 template <class Unit> hipError_t run_units(const void *in, void *out, uint64_t units, const CastLayout &layout, hipStream_t s) {
-  note_variant<UnitsTag>();
+  note_variant<UnitsTag<Unit>>();
   hipLaunchKernelGGL((copy_units<Unit>), dim3((uint32_t)((units + kBlockThreads - 1) / kBlockThreads)), dim3(kBlockThreads), 0, s,
                      static_cast<const char *>(in), static_cast<Unit *>(out), (uint32_t)units, layout);
   return hipGetLastError();
