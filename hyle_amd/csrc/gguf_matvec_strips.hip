@@ -521,9 +521,14 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
 }
 
 inline const char *strip_word(int kind) { return kind == 0 ? "q4_k" : (kind == 1 ? "q6_k" : "q8_0"); }
-// gguf_matvec_q8_strips/<format>/<activation rows>-tokens
-template <int kKind, int kSets> struct StripsTag {
-  static std::string text() { return std::string("gguf_matvec_q8_strips/") + strip_word(kKind) + "/" + std::to_string(4 * kSets) + "-tokens"; }
+// gguf_matvec_q8_strips/<format>/<activation rows>-tokens/<waves of a block: 16, 8, or 8 where two share a compute
+// unit>-waves[/shared: several waves to a tile].  Eight waves for want of LDS nearly always share: one label.
+enum : int { kSixteen = 0, kSixteenShared = 1, kEight = 2, kTwice = 3, kTwiceShared = 4 };
+template <int kKind, int kSets, int kForm> struct StripsTag {
+  static std::string text() {
+    static const char *const forms[] = {"16-waves", "16-waves/shared", "8-waves", "2x8-waves", "2x8-waves/shared"};
+    return std::string("gguf_matvec_q8_strips/") + strip_word(kKind) + "/" + std::to_string(4 * kSets) + "-tokens/" + forms[kForm];
+  }
 };
 
 // Waves of a block whose buffers fit beside the codes of m activation rows: sixteen, eight, or none.
@@ -563,7 +568,11 @@ hipError_t run_strips(const MatVecParams &p, uint32_t m, const void *w, const vo
       split_log2 = log2;
     }
   }
-  note_variant<StripsTag<kKind, kSets>>();
+  if (twice && split_log2 != 0) note_variant<StripsTag<kKind, kSets, kTwiceShared>>();
+  else if (twice) note_variant<StripsTag<kKind, kSets, kTwice>>();
+  else if (waves == 8) note_variant<StripsTag<kKind, kSets, kEight>>();
+  else if (split_log2 != 0) note_variant<StripsTag<kKind, kSets, kSixteenShared>>();
+  else note_variant<StripsTag<kKind, kSets, kSixteen>>();
   hipLaunchKernelGGL((gguf_matvec_q8_strips<kKind, TX, kSets>), dim3(grid), dim3(waves * kWaveLanes), shared, s, static_cast<const unsigned char *>(w), x, y,
                      rows, p.row_stride, p.k, m, block_rows, tile_rows, split_log2);
   return hipGetLastError();

@@ -69,6 +69,38 @@ def test_strips_activation_rows_in_groups():
           kernel="gguf_matvec_q8_strips/q8_0/4-tokens")
 
 
+# rows, k, activation rows, how the launch is laid out: sixteen waves to a block, eight where the codes leave no more
+# room, or eight where two blocks share a compute unit; a wave to a tile or several ("shared")
+FORMS = [(61700, 4352, 4, "16-waves"), (61900, 2304, 8, "16-waves"), (5003, 1792, 4, "16-waves/shared"), (4096, 1280, 5, "16-waves/shared"),
+         (66000, 256, 2, "2x8-waves"), (16400, 256, 6, "2x8-waves"), (12289, 1536, 2, "2x8-waves/shared"), (12289, 1536, 6, "2x8-waves/shared")]
+EIGHT = {"q4_k": [(520, 35072, 4), (520, 17152, 8)], "q6_k": [(520, 24320, 4), (520, 11776, 8)], "q8_0": [(520, 18176, 4), (520, 8704, 8)]}
+
+
+@pytest.mark.parametrize("tag", list(KINDS))
+def test_strips_every_layout_of_a_launch(tag):
+    """The weight repeats 257 distinct rows, so that one meets every place of a tile and of a block: the first 257 products
+    are held against the oracle, all others against those, bit by bit (a row's sums do not depend on its place)."""
+    rng = np.random.default_rng(1824)
+    kind, gguf = KINDS[tag]
+    period = 257
+    for rows, k, m, form in FORMS + [shape + ("8-waves",) for shape in EIGHT[tag]]:
+        raw = weights_for(tag, rng, period, k)
+        x = rng.normal(0, 1, (m, k)).astype(np.float32)
+        row_bytes = raw.shape[1]
+        storage = torch.empty(2 + rows * row_bytes, dtype=torch.uint8, device=DEVICE)[2:]   # two bytes off: no kernel of whole vectors
+        distinct = torch.from_numpy(raw).to(DEVICE)
+        storage.view(rows, row_bytes).copy_(distinct.repeat((rows + period - 1) // period, 1)[:rows])
+        label = f"gguf_matvec_q8_strips/{tag}/{4 if m <= 4 else 8}-tokens/{form}"
+        note(f"q8 matvec {tag} [{k} -> {rows}] x {m}: {label}")
+        descs = [hc.TensorDesc.gguf_weight(gguf, hc.DataType.kFloat32, k, rows), hc.TensorDesc.dense(hc.DataType.kFloat32, [m, k])]
+        (out,) = run(Q8, storage, torch.from_numpy(x).to(DEVICE), descs=descs)
+        assert hc.last_launch_variant() == label, hc.last_launch_variant()
+        got = out.cpu().numpy().reshape(m, rows)
+        centre, bound = orc.gguf_matvec_q8(kind, raw.reshape(-1), period, k, x)
+        assert np.all(np.abs(got[:, :period] - centre.reshape(m, period)) <= bound.reshape(m, period))
+        assert np.array_equal(got, np.take(got, np.arange(rows) % period, 1))
+
+
 @pytest.mark.parametrize("tag,k,rows,m,byte_offset", [
     ("q8_0", 5120, 2304, 6, 0), ("q8_0", 2560, 8192, 4, 0), ("q6_k", 5120, 3584, 8, 0), ("q6_k", 1024, 8192, 5, 0),
     ("q4_k", 4096, 6656, 4, 0), ("q4_k", 9984, 3072, 5, 2)])
