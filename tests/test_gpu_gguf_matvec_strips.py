@@ -129,3 +129,42 @@ def test_strips_are_no_further_from_64_bit_sums(tag, k, rows, m, byte_offset):
     centre = centre.reshape(m, rows)
     own, others = np.linalg.norm(whole - centre), np.linalg.norm(np.concatenate([part for part, _ in slices], 1) - centre)
     assert own <= others, f"{own / others:.3f} of the error of the kernels for few rows"
+
+
+@pytest.mark.parametrize("tag", list(KINDS))
+def test_strips_activations_that_are_no_numbers(tag):
+    """A NaN is no candidate for a block's magnitude and has the code of a zero; an infinity leaves its block no finite
+    scale, so that its activation row's products are NaN; a magnitude whose inverse is none saturates the codes.  In every
+    case as in the kernels that serve few rows, and the other activation rows keep their bits."""
+    rng = np.random.default_rng(1825)
+    kind, gguf = KINDS[tag]
+    rows, k, m = 4352, 1280, 6
+    raw = weights_for(tag, rng, rows, k)
+    storage = torch.from_numpy(np.concatenate([np.zeros(2, np.uint8), raw.reshape(-1)])).to(DEVICE)[2:].view(rows, -1)
+
+    def products(x, first=0, count=rows):
+        descs = [hc.TensorDesc.gguf_weight(gguf, hc.DataType.kFloat32, k, count), hc.TensorDesc.dense(hc.DataType.kFloat32, [m, k])]
+        (out,) = run(Q8, storage[first:first + count], torch.from_numpy(x).to(DEVICE), descs=descs)
+        return out.cpu().numpy(), hc.last_launch_variant()
+
+    clean = rng.normal(0, 1, (m, k)).astype(np.float32)
+    clean[0, [5, 300, 301]] = 0.0
+    clean[1, 512:768] = 0.0
+    odd = clean.copy()
+    odd[0, [5, 300, 301]] = [np.nan, -np.nan, np.nan]
+    odd[1, 512:768] = np.nan                  # a block without a number
+    odd[2, 700] = np.inf
+    odd[3, 256] = -np.inf
+    odd[4, 256:512] = rng.normal(0, 1e-40, 256)   # 127 / magnitude overflows
+    note(f"q8 matvec strips {tag} [{k} -> {rows}] x {m}: NaN, infinities and subnormals among the activations")
+    want, label = products(clean)
+    got, _ = products(odd)
+    assert label.startswith("gguf_matvec_q8_strips")
+    for token in (0, 1, 5):
+        assert np.array_equal(got[token], want[token]), token
+    assert np.isnan(got[2]).all() and np.isnan(got[3]).all()
+    general, label = products(odd, 0, 256)
+    assert "strips" not in label
+    assert np.array_equal(np.isnan(got[:, :256]), np.isnan(general))
+    few = np.abs(np.where(np.isnan(general), 0.0, got[:, :256] - general))
+    assert np.all(few <= 1e-5 * np.nanmax(np.abs(general)))   # both are within gamma(K / 4 + 65, 2^-24) of the same sum of terms
