@@ -18,7 +18,6 @@
 //   general  anything else (strides, scattered axes, unaligned bytes): one wave per result,
 //            coordinates by division.  Correct, not tuned.
 #include <algorithm>
-#include <type_traits>
 
 #include "device_common.h"
 #include "kernels.h"
@@ -36,6 +35,7 @@ template <int kKind> __device__ __forceinline__ float reduce_step(float acc, flo
   else if constexpr (kKind == kMaximum) return max_propagate(acc, v);
   else return acc + v;
 }
+template <int kKind> constexpr bool kExtreme = kKind == kMinimum || kKind == kMaximum;
 // kMean divides once, at the very end; 0 / 0 gives the NaN of an empty mean.
 template <int kKind> __device__ __forceinline__ float reduce_final(float acc, float divisor) {
   if constexpr (kKind == kMean) return acc / divisor;
@@ -43,16 +43,19 @@ template <int kKind> __device__ __forceinline__ float reduce_final(float acc, fl
 }
 
 // Calls trip(n) with n = kMost, ..., 4, 2 or 1 as a constant until `steps` steps are done: trips of kMost, then
-// the smallest one that ends it.  A trip is that many 16-byte loads of a lane in flight at once, clamped to
-// the last one there is, so a lane with up to kMost waits for memory once and one with fewer does not load
+// the smallest one that ends it.  A trip is that many 16-byte loads of a lane in flight at once, clamped in the
+// last one to what there is, so a lane with up to kMost waits for memory once and one with fewer does not load
 // more than it has.  Rows, us in trips of four, two and then one / of eight always / here: f32 [5902, 1968]
-// 9.5 / 8.6 / 8.6, [5003, 2560] 10.1 / 10.4 / 9.4, [16384, 2048] 20.6 / 26.4 / 20.7, [2^20, 64] 143 / 258 / 145,
-// bf16 [65536, 512] 14.6 / 21.9 / 14.8.
-template <uint32_t kLoads> using Loads = std::integral_constant<uint32_t, kLoads>;
+// 9.8 / 8.8 / 8.8, [5003, 2560] 10.2 / 10.4 / 9.5, [16384, 2048] 20.7 / 26.4 / 20.6, [10^6, 64] 143 / 258 / 141,
+// bf16 [65536, 512] 14.5 / 21.7 / 14.4.
+template <uint32_t kLoads, bool kAllThere = false> struct Loads {  // kAllThere: no lane has fewer, nothing to clamp or drop
+  static constexpr uint32_t kCount = kLoads;
+  static constexpr bool kFull = kAllThere;
+};
 template <uint32_t kMost, class Trip> __device__ __forceinline__ void in_trips(uint32_t steps, Trip trip) {
   if (steps == 1) return trip(Loads<1>{});
   if (steps > 2) {
-    for (; steps > kMost; steps -= kMost) trip(Loads<kMost>{});
+    for (; steps > kMost; steps -= kMost) trip(Loads<kMost, true>{});
     if (kMost > 4 && steps > 4) return trip(Loads<8>{});
     if (kMost > 2 && steps > 2) return trip(Loads<4>{});
   }
@@ -83,17 +86,19 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_rows(const void *x, void
       const uint32_t last = end / kVec;
       uint32_t vec = begin / kVec + lane;
       // a vector past the tile is its last one again and is dropped
-      in_trips<8>(__builtin_amdgcn_readfirstlane((last - begin / kVec + kLanes - 1) / kLanes), [&](auto loads) {
-        constexpr uint32_t kLoads = decltype(loads)::value;
-        if (vec >= last) return;  // nothing left of this lane's
+      // an extremum of a block's row: four (all of f32 [4096, 4096] 17.6 us, eight 17.9)
+      in_trips<kExtreme<kKind> && kLanes == kBlockThreads ? 4 : 8>(__builtin_amdgcn_readfirstlane((last - begin / kVec + kLanes - 1) / kLanes), [&](auto loads) {
+        constexpr uint32_t kLoads = decltype(loads)::kCount;
+        constexpr bool kFull = decltype(loads)::kFull;
+        if (!kFull && vec >= last) return;  // nothing left of this lane's
         u32x4 raw[kLoads];
 #pragma unroll
-        for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (i == 0 ? vec : min(vec + i * kLanes, last - 1)));
+        for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (kFull || i == 0 ? vec + i * kLanes : min(vec + i * kLanes, last - 1)));
 #pragma unroll
         for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
 #pragma unroll
         for (uint32_t i = 0; i < kLoads; ++i) {
-          if (i != 0 && vec + i * kLanes >= last) break;
+          if (!kFull && i != 0 && vec + i * kLanes >= last) break;
           float v[kVec];
           Traits<TIn>::unpack(raw[i], v);
 #pragma unroll
@@ -141,16 +146,17 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_columns(const void *x, v
     uint32_t r = begin + ty;
     if constexpr (kVector) {
       in_trips<kMost>((end - begin + lanes_y - 1) / lanes_y, [&](auto loads) {
-        constexpr uint32_t kLoads = decltype(loads)::value;
-        if (r >= end) return;
+        constexpr uint32_t kLoads = decltype(loads)::kCount;
+        constexpr bool kFull = decltype(loads)::kFull;
+        if (!kFull && r >= end) return;
         u32x4 raw[kLoads];
 #pragma unroll
-        for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (size_t)(i == 0 ? r : min(r + i * lanes_y, end - 1)) * units);
+        for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (size_t)(kFull || i == 0 ? r + i * lanes_y : min(r + i * lanes_y, end - 1)) * units);
 #pragma unroll
         for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
 #pragma unroll
         for (uint32_t i = 0; i < kLoads; ++i) {
-          if (i != 0 && r + i * lanes_y >= end) break;
+          if (!kFull && i != 0 && r + i * lanes_y >= end) break;
           float v[kW];
           Traits<TIn>::unpack(raw[i], v);
 #pragma unroll
@@ -304,8 +310,9 @@ void columns_launch(const void *x, void *y, uint32_t outer, uint32_t reduced, ui
   //   f32 [1024, 2048] 7.2 / 6.4 / 6.2, [586, 1072] 8.2 / 7.2 / 7.1, [2000, 2048] 8.4 / 7.8 / 8.2, [1024, 3072] 7.6 / 7.2 / 7.5
   //   f32 [64, 131072] 7.5 / 8.5 / 9.4, [3, 256, 8192] middle axis 6.6 / 7.0 / 7.1, bf16 [8192, 2048] 10.4 / 11.1 / 10.9
   //   f32 [5003, 2560] 15.1 / 14.2 / 14.4, [7000, 2048] 15.7 / 15.1 / 15.2; but [16, 2^20] 15.1 / 17.0 / 17.0
+  // An extremum is six instructions an element and gives memory time enough: two (bf16 [8192, 4096] 23.7, four 26.0).
   const uint64_t blocks = (uint64_t)grid.x * segments;
-  const int most = blocks <= 256 ? 8 : (blocks <= 512 || (blocks >= 1280 && segments > 1) ? 4 : 2);
+  const int most = blocks <= 256 ? 8 : (blocks <= 512 || (blocks >= 1280 && segments > 1 && !kExtreme<kKind>) ? 4 : 2);
 #define HYLE_COLUMNS(VECTOR, MOST)                                                                                            \
   note_variant<ColumnsTag<VECTOR, MOST>>();                                                                                   \
   hipLaunchKernelGGL((reduce_columns<TIn, TOut, kKind, VECTOR, MOST>), grid, dim3(kBlockThreads), 0, s, x, y, outer, reduced, \

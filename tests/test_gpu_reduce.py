@@ -275,5 +275,7 @@ def test_reduce_with_every_number_of_loads_a_lane(tag):
             x = values_for(rng, dims, tag, plant=kind == RK.kMaximum)
             note(f"reduce {kind.name} {tag} {dims} over axis {axis}: {label}")
             (out,) = run(hc.Reduce(kind, hc.Axes.from_([axis]), accumulation_type=F32ACC), to_device(x, tag))
+            if dims[0] == 512 and kind == RK.kMaximum:   # many blocks: four in flight for sums only
+                label = "reduce_columns/vector/2"
             assert hc.last_launch_variant().startswith(label), (dims, hc.last_launch_variant())
             check(kind, tag, to_host(out), x, dims, [axis])
