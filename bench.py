@@ -17,12 +17,13 @@ Inputs are resident in HBM before the timed region.  Shapes whose traffic fits t
 memory-side cache rotate over several buffer sets (> 512 MB in total) so that HBM, not the
 cache, is measured.  `value` is credited bytes per step / step time (algorithmic bytes, less
 the masked loads the softmax skips); `roofline` describes
-the dominant kernel (softmax) timed with HIP events inside the timed region; `per_op` holds
+the dominant kernel (softmax) timed with HIP events inside the timed region; `per_op_us` holds
 each kernel's own figure from an event-timed loop of back-to-back launches; `cpu_baseline`
 times the CPU oracle ("port" of the reference's CPU path) on a bounded sample of the same
 workload on the host cores.
 
-Prints one JSON line.
+Prints one JSON line, kept short enough for whoever keeps the end of a program's output; the whole
+record of each kernel (route, launch shape, bytes, rates) goes to stderr, a JSON object a line.
 """
 from __future__ import annotations
 
@@ -597,6 +598,8 @@ def main() -> int:
     achieved = dominant.credited / dominant_us / 1e3
     # every kernel of the step in short keys (us per launch, GB/s of credited bytes, fraction of the
     # 8 TB/s peak, and against the plain kernel of the same traffic where one was timed)
+    for entry in per_op:
+        print(json.dumps(entry), file=sys.stderr)
     per_config = {}
     for op in step_ops:
         entry = by_name[op.name]
@@ -635,7 +638,7 @@ def main() -> int:
                                        "counter read in this run)",
                      "per_config": per_config, "ceilings": ceilings},
         "cold": cold,
-        "per_op": per_op,
+        "per_op_us": {entry["op"]: entry["us"] for entry in per_op},
     }
     result["device"] = device_state(torch)
     if not args.no_cpu:
