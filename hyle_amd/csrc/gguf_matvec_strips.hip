@@ -28,14 +28,16 @@
 // (Q8_0 [2048 -> 151936] 111 us that way, 63 us through the slot).  A Q4_K row is whole vectors and
 // goes straight into the lanes (52 us through the slot, 43 us straight).
 //
-// Bound by HBM for a vocabulary, by the quantising of every activation row in every compute unit and
-// by the start of a block below about 30 MB of weights (vector arithmetic, by instruction count several
-// of the 37 us of five rows of 17408 values).  MI355X, bf16 activations, the kernels that these shapes took before and here:
-//   Q8_0 [5120 -> 17408] x 5   70.2 -> 28.4 us (3330 GB/s)    [17408 -> 5120] x 5  109.8 -> 37.1 us
-//   Q6_K [5120 -> 17408] x 5   70.3 -> 28.2 us                [17408 -> 5120] x 5  112.3 -> 35.7 us
-//   Q4_K [5120 -> 17408] x 5   44.9 -> 21.8 us                [17408 -> 5120] x 5  115.1 -> 31.2 us
-//   [1536 -> 77056] x 8: Q8_0  104.9 -> 30.2 us (4170 GB/s)   Q6_K 116.8 -> 28.4 us
-//   Q6_K [5120 -> 32768] x 1 / 8   39.3 / 127.5 -> 31.7 / 39.4 us
+// Bound by HBM for a vocabulary.  Below about 100 MB of weights by latency and vector instructions together: at
+// five rows of Q8_0 [5120 -> 17408] a SIMD issues vector instructions in 38 % of the cycles and matrix ones in 4 %, LDS
+// conflicts take 16 % of them and a wave waits for 36 % of its time; at [17408 -> 5120], where the codes leave room for
+// eight waves, vector 43 %, two fifths of it quantising, and HBM delivers 2.5 of 6.8 TB/s.  MI355X, bf16
+// activations, us, the kernels that these shapes took before and here:
+//   Q8_0 [5120 -> 17408] x 5   65.6 -> 28.8 (3290 GB/s)    [17408 -> 5120] x 5   99.9 -> 34.1 (2780 GB/s)
+//   Q6_K [5120 -> 17408] x 5   70.3 -> 27.3                [17408 -> 5120] x 5  112.5 -> 35.7
+//   Q4_K [5120 -> 17408] x 5   44.0 -> 21.4                [17408 -> 5120] x 5  115.3 -> 31.3
+//   [1536 -> 77056] x 8: Q8_0 104.9 -> 31.2 (4030 GB/s)    Q6_K 117.4 -> 29.0
+//   Q6_K [5120 -> 32768] x 1   38.3 -> 31.9
 #include "device_common.h"
 #include "gguf_q8_math.h"
 #include "kernels.h"
@@ -81,7 +83,7 @@ template <int kKind> struct Strip;
 template <> struct Strip<0> {  // rows are whole 16-byte vectors as a rule: loaded straight into the lanes
   static constexpr bool kParked = false;
   // one piece per lane of its own row
-  static constexpr uint32_t kRunBytes = 144, kVectors = 1, kPitch = 0, kLoads = 1, kSlotBytes = 0;
+  static constexpr uint32_t kRunBytes = 144, kVectors = 1, kLoads = 1, kSlotBytes = 0;
   using Pending = Strip;
   u32x4 head, q[2];
   __device__ __forceinline__ void load(const unsigned char *at, uint32_t part) {

@@ -8,14 +8,14 @@
 // the row's end is moved back to end there: no scalar tail, every access inside the row.  The two
 // vectors then share elements, which both compute and store alike and only one counts in the sum.
 // The loads are plain ones, since neighbours share the lines at their seams; the stores stream
-// (bf16 [24, 777, 1013]: 16.8 us with plain stores, 15.0 us).  Bound by HBM from about 1000
+// (bf16 [24, 777, 1013] 1.8 us less than with plain stores).  Bound by HBM from about 1000
 // elements a row on, below that by the vector instructions of a wave's two reductions, which is why
 // short rows share a wave.  MI355X, without a mask / Boolean / additive, before (softmax_general,
 // which walks the strides of every element in three passes) and here:
-//   bf16 [24, 777, 1013]  177 / 190 / 190 -> 15.0 / 15.8 / 17.6 us (5050 / 4850 / 4390 GB/s)
-//   f32  [24, 777, 1013]  179 -> 27.8 us (5440 GB/s)    f32 [12, 777, 7001] Boolean 658 -> 91.7 us (5750 GB/s)
-//   bf16 [24, 777, 3001]  488 -> 39.0 us (5745 GB/s; an aligned row of 3000 in softmax.hip: 45.4)
-//   f16  [24, 777, 100]    41 ->  3.7 us               f32 [8, 1, 1271] 12.6 -> 2.4 us
+//   bf16 [24, 777, 1013]  177 / 189 / 190 -> 13.4 / 14.5 / 15.4 us (5640 / 5300 / 5000 GB/s)
+//   f32  [24, 777, 1013]  180 -> 27.5 us (5500 GB/s)    f32 [12, 777, 7001] Boolean 658 -> 91.0 us (5800 GB/s)
+//   bf16 [24, 777, 3001]  491 -> 35.1 us (6380 GB/s; an aligned row of 3000 in softmax.hip: 45.4)
+//   f16  [24, 777, 100]    42 ->  4.0 us               f32 [8, 1, 1271] 12.7 -> 2.6 us
 //   f32  [1, 777] 10.3 -> 2.2 us, [6, 129] 4.4 -> 1.9 us, [1, 5] 4.1 -> 1.8 us: no call is too small for it
 // Running the heads of a mask row next to each other on one XCD, which pays for 64 MiB masks
 // (softmax.hip), loses here: bf16 [24, 777, 1013] additive 17.5 -> 20.2 us, f32 [32, 1777, 1777]
