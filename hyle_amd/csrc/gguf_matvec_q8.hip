@@ -1455,21 +1455,29 @@ inline bool rows_of_vectors_serve(const MatVecParams &p) {
 }
 
 // Where the strip kernel (gguf_matvec_strips.hip) is the faster one; `vectors`: weights, activations and
-// the row stride are multiples of 16 bytes.  us, the kernel here / strips:
-//   shapes that walk block by block, from 24 M products on: Q8_0 [1536 -> 8192] x 2 9.5 / 9.0,
-//   [5120 -> 2048] x 2 10.7 / 11.1 and x 4 16.4 / 11.0, Q6_K [5120 -> 8192] x 1 14.4 / 14.0 (below: Q6_K
-//   [5120 -> 2048] x 1 8.7 / 11.5, [1536 -> 2048] x 2 6.2 / 9.0)
-//   tiles: several rows of 4096 values or more and 4096 weight rows: Q4_K [4096 -> 8192] x 2 14.3 / 12.4,
-//   [5120 -> 17408] x 5 44.9 / 21.8 (narrower: [2048 -> 32768] x 4 13.1 / 15.4; one row: [5120 -> 17408] 15.5 / 18.0)
-//   whole spans, from 200 M products on: more than four rows, Q8_0 [4096 -> 32768] x 8 43.7 / 34.8, Q6_K x 6
-//   47.6 / 31.1 ([2048 -> 100000] x 6 Q8_0 48.5 / 50.3, Q6_K 49.3 / 50.2); Q6_K three or four rows of 6144 or
-//   more, [6144 -> 8192] x 4 22.8 / 17.3 ([4096 -> 100000] x 4 69.5 / 71.5, Q8_0 [6144 -> 32768] x 4 42.3 / 46.8)
+// the row stride are multiples of 16 bytes.  MI355X, bf16, us, the kernels here / strips:
+//   several activation rows: nearly everywhere, since a compute unit quantises them once.  Q8_0 [2048 -> 16384]
+//   x 2 15.6 / 10.4, [4096 -> 2048] x 8 10.9 / 8.7, Q6_K [1024 -> 2048] x 8 11.9 / 4.7, [6144 -> 8192] x 2 20.2 / 12.9,
+//   Q4_K [1536 -> 3072] x 4 6.0 / 4.6, [7680 -> 2100] x 4 14.0 / 7.8.  Not where narrow Q4_K rows are many (tiles
+//   quantise little there and need no barrier for the tile's end): [2048 -> 6144] x 4 7.1 / 7.5, [2048 -> 65536] x 2
+//   20.1 / 22.9 ([2560 -> 8192] x 2 9.0 / 7.1, [2048 -> 65536] x 8 26.4 / 25.4); nor two rows far wider than the
+//   weight is high, Q8_0 [16384 -> 1024] 10.1 / 11.4 ([8192 -> 2048] 9.5 / 8.1)
+//   one row, where the alternative walks block by block, from 8 M products on, and from 4 M where a row is wide:
+//   Q6_K [1024 -> 8192] 5.8 / 5.4, [2304 -> 2304] 6.9 / 5.6, [7680 -> 2100] 12.9 / 8.2 ([1024 -> 2048] 4.0 / 4.2)
+//   one row of Q4_K tiles: rows of 10240 values or more, [17408 -> 5120] 21.1 / 17.4, and widths that are no
+//   multiple of 2048 with few weight rows, [2560 -> 2560] 5.3 / 4.5, [5120 -> 5120] 8.5 / 7.2 ([2560 -> 5120]
+//   5.7 / 5.8, [4096 -> 2048] 5.2 / 6.4, [8192 -> 8192] 12.1 / 14.6)
 bool strips_better(const MatVecParams &p, bool vectors) {
   if (!gguf_matvec_strips_serve(p)) return false;
-  const uint64_t products = (uint64_t)p.m * p.rows * p.k;
-  if (!vectors || !rows_of_vectors_serve(p)) return products >= 24000000;
-  if (p.kind == 0) return p.m > 1 && p.k >= 4096 && p.rows >= 4096;
-  return products >= 200000000 && ((p.m > 4 && p.k >= 4096) || (p.kind == 1 && p.m > 2 && p.k >= 6144));
+  const bool whole = vectors && rows_of_vectors_serve(p);
+  if (p.m == 1) {
+    const uint64_t products = p.rows * p.k;
+    if (!whole) return products >= 8000000 || (products >= 4000000 && p.k >= 2048);
+    return p.kind == 0 && (p.k >= 10240 || (p.k > 2048 && p.k % 2048 != 0 && (p.rows <= 4096 || p.k >= p.rows)));
+  }
+  if (!whole) return true;
+  if (p.kind == 0) return p.m > 4 || p.k > 2048 || p.rows < 6144;
+  return p.m > 2 || p.k < 8 * p.rows;
 }
 
 template <int kKind, class TX>

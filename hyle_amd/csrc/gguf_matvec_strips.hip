@@ -14,6 +14,13 @@
 // of A rows serves activation rows 4 .. 7 from the same weight registers.  A lane that carries zeros
 // reads them from a row of zeros in LDS: its address does not advance.
 //
+// Q8_0 rows of whole 16-byte vectors need no decoding: a run's 272 bytes go to the matrix unit as they
+// lie, a wave's five windows of four vectors at a time (the fifth holds the seventeenth vector), and the codes
+// are laid out to match, each block's 32 in 48 bytes of LDS at the place its quants have in the three vectors
+// that hold them, zeros round them (at the scale, and at the neighbours' bytes).  Row 4 q + t of A holds the codes of
+// block 4 g + q for the g-th half of a run, so three windows give a lane the dots of one block again; its scale
+// comes out of the windows with two lane swaps.
+//
 // A block of sixteen waves (eight where the codes leave no room for more slots) has a compute unit's
 // LDS, quantises the activation rows once, while its first weight bytes are on their way, and walks its
 // share of the weight rows in tiles of at most sixteen; `1 << split_log2` waves share a tile, each
@@ -22,22 +29,25 @@
 // kernels that spread a row over 64 lanes was further from the 64-bit sum than theirs in a third of
 // the shapes (f32 Q8_0 [5120 -> 2304] x 6 9.6e-8 relative against 8.2e-8 there, Q4_K [4096 -> 6656] x 4
 // 7.6e-8 against 6.2e-8; in 64 bits 5.3e-8 and 4.5e-8, at most 0.75 of theirs over 87 shapes, for about
-// 1 % of the time).  Q8_0 and Q6_K runs are
-// loaded as the aligned vectors that cover them and redistributed through a wave-private slot: lanes
-// that load their own 16 bytes at 2-byte addresses keep the memory pipe busy several times as long
-// (Q8_0 [2048 -> 151936] 111 us that way, 63 us through the slot).  A Q4_K row is whole vectors and
-// goes straight into the lanes (52 us through the slot, 43 us straight).
+// 1 % of the time).  Q8_0 and Q6_K runs are loaded as the aligned vectors that cover them and
+// redistributed through a wave-private slot: lanes that load their own 16 bytes at 2-byte addresses keep the
+// memory pipe busy several times as long (Q8_0 [2048 -> 151936] 111 us that way, 63 us through the slot), and lanes
+// that load their own aligned vectors ask for sixteen half lines at a time (in place, [5120 -> 17408] x 4 24.6 us,
+// through the slot 21.6: the direct form serves where the codes leave no room for slots).  A Q4_K row is whole
+// vectors and goes straight into the lanes (52 us through the slot, 43 us straight).  The loads are plain ones: a run's
+// last line is the next run's first, which another wave asks for (non-temporal: 24.0 us).
 //
-// Bound by HBM for a vocabulary.  Below about 100 MB of weights by latency and vector instructions together: at
-// five rows of Q8_0 [5120 -> 17408] a SIMD issues vector instructions in 38 % of the cycles and matrix ones in 4 %, LDS
-// conflicts take 16 % of them and a wave waits for 36 % of its time; at [17408 -> 5120], where the codes leave room for
-// eight waves, vector 43 %, two fifths of it quantising, and HBM delivers 2.5 of 6.8 TB/s.  MI355X, bf16
-// activations, us, the kernels that these shapes took before and here:
-//   Q8_0 [5120 -> 17408] x 5   65.6 -> 28.8 (3290 GB/s)    [17408 -> 5120] x 5   99.9 -> 34.1 (2780 GB/s)
-//   Q6_K [5120 -> 17408] x 5   70.3 -> 27.3                [17408 -> 5120] x 5  112.5 -> 35.7
-//   Q4_K [5120 -> 17408] x 5   44.0 -> 21.4                [17408 -> 5120] x 5  115.3 -> 31.3
-//   [1536 -> 77056] x 8: Q8_0 104.9 -> 31.2 (4030 GB/s)    Q6_K 117.4 -> 29.0
-//   Q6_K [5120 -> 32768] x 1   38.3 -> 31.9
+// Bound by HBM for a vocabulary ([2560 -> 128758] x 4 5.2 TB/s).  Below about 100 MB of weights by what stands round
+// the stream: of the 24.7 us of Q8_0 [5120 -> 17408] x 5 the block's first code comes after 5, the bare
+// loads take 21, and a second set of activation rows costs 3; at [17408 -> 5120] quantising takes 4.
+// MI355X, bf16 activations, us, with a quantiser of eight values per lane, decoded Q8_0 and non-temporal loads, and here:
+//   Q8_0 [5120 -> 17408] x 5   28.3 -> 24.7 (3830 GB/s)    [17408 -> 5120] x 5   34.2 -> 26.9 (3520 GB/s)
+//   Q6_K [5120 -> 17408] x 5   26.5 -> 22.8                [17408 -> 5120] x 5   34.2 -> 26.9
+//   Q4_K [5120 -> 17408] x 5   21.1 -> 20.0                [17408 -> 5120] x 5   30.4 -> 23.0
+//   [2304 -> 7936] x 2: Q8_0 12.2 -> 8.2                   Q6_K 12.4 -> 8.2
+//   [1536 -> 77056] x 8: Q8_0 31.3 -> 29.7                 Q6_K 29.5 -> 26.1
+#include <type_traits>
+
 #include "device_common.h"
 #include "gguf_q8_math.h"
 #include "kernels.h"
@@ -47,7 +57,7 @@ namespace {
 
 constexpr uint32_t kStripRows = 16, kMostWaves = 16;
 constexpr size_t kStripLds = 160 * 1024;  // of a compute unit, and the most one block can have
-constexpr uint32_t kZeroBytes = 256;      // a lane's operands of one run lie within 256 bytes of its base
+constexpr uint32_t kZeroBytes = 384;      // a lane's operands of one run lie within 384 bytes of its base
 constexpr uint32_t kCodePad = 16;         // between activation rows: neighbours start on other LDS banks
 
 // 16 bytes at any even address.
@@ -70,7 +80,7 @@ template <int kWords> __device__ __forceinline__ void lds_even(const unsigned ch
 // them: kVectors per row (a run starts up to 14 bytes into its first), rows an odd number of vectors
 // apart in LDS, so that the sixteen rows of a column start on different banks.
 template <uint32_t kBytes> struct StripStage {
-  static constexpr bool kParked = true;
+  static constexpr bool kParked = true, kWhole = false;
   static constexpr uint32_t kRunBytes = kBytes, kVectors = (kBytes + 14 + 15) / 16, kPitch = (kVectors | 1u) * 16;
   static constexpr uint32_t kLoads = (kStripRows * kVectors + kWaveLanes - 1) / kWaveLanes, kSlotBytes = kStripRows * kPitch;
   struct Pending {
@@ -81,7 +91,7 @@ template <uint32_t kBytes> struct StripStage {
 // What a lane decodes of one run of its weight row, from the wave's slot; `at`: the run's first byte.
 template <int kKind> struct Strip;
 template <> struct Strip<0> {  // rows are whole 16-byte vectors as a rule: loaded straight into the lanes
-  static constexpr bool kParked = false;
+  static constexpr bool kParked = false, kWhole = false;
   // one piece per lane of its own row
   static constexpr uint32_t kRunBytes = 144, kVectors = 1, kLoads = 1, kSlotBytes = 0;
   using Pending = Strip;
@@ -130,19 +140,49 @@ template <> struct Strip<2> : StripStage<272> {
   }
 };
 
+// Q8_0 rows of whole 16-byte vectors, as they lie in memory: lane (c, p) holds vectors 4 w + p of the run's seventeen
+// (the seventeenth alone in the fifth window, in every part).  Strip<4> loads a tile's runs one after another and parks
+// them, Strip<3> loads straight into the lanes and needs no slots.
+struct StripInPlace {
+  static constexpr uint32_t kRunBytes = 272;
+  u32x4 v[5];
+  __device__ __forceinline__ void take(const unsigned char *at, uint32_t part) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) v[w] = load16(at + 16 * part, 4 * w);
+    v[4] = load16(at, 16);
+  }
+};
+template <> struct Strip<3> : StripInPlace {
+  static constexpr bool kParked = false, kWhole = false;
+  static constexpr uint32_t kVectors = 1, kLoads = 1, kSlotBytes = 0;
+  using Pending = Strip;
+  __device__ __forceinline__ void load(const unsigned char *at, uint32_t part) { take(at, part); }
+};
+template <> struct Strip<4> : StripInPlace {
+  static constexpr bool kParked = true, kWhole = true;
+  static constexpr uint32_t kVectors = 17, kPitch = kVectors * 16, kLoads = (kStripRows * kVectors + kWaveLanes - 1) / kWaveLanes, kSlotBytes = kStripRows * kPitch;
+  struct Pending {
+    u32x4 v[kLoads];
+  };
+  __device__ __forceinline__ void take(const unsigned char *slot, uint32_t at, uint32_t part) { StripInPlace::take(slot + at, part); }
+};
+
 // LDS of a block: zeros | codes [m][k + pad] | scales [activation blocks][4 sets] |
 // Q4_K: sums [sub-blocks][4 sets] | shares [waves][sets][64] | slots [waves]
 struct StripLayout {
   uint32_t scales, sums, shares, slots, bytes;
 };
+// Bytes of an activation row's codes; of a run's.
+__host__ __device__ inline uint32_t strip_run_codes(int kind) { return kind >= 3 ? 384u : 256u; }
+__host__ __device__ inline uint32_t strip_code_pitch(int kind, uint32_t k) { return k / 256 * strip_run_codes(kind) + kCodePad; }
 __host__ __device__ inline StripLayout strip_layout(int kind, uint32_t m, uint32_t k, uint32_t waves) {
   const uint32_t sets = m > 4 ? 2 : 1;
   StripLayout at;
-  at.scales = kZeroBytes + m * (k + kCodePad);
-  at.sums = at.scales + (kind == 2 ? k / 32 : k / 256) * 16 * sets;
+  at.scales = kZeroBytes + m * strip_code_pitch(kind, k);
+  at.sums = at.scales + (kind >= 2 ? k / 32 : k / 256) * 16 * sets;
   at.shares = at.sums + (kind == 0 ? k / 32 * 16 * sets : 0);
   at.slots = at.shares + waves * sets * kWaveLanes * 4;
-  at.bytes = at.slots + waves * (kind == 0 ? Strip<0>::kSlotBytes : (kind == 1 ? Strip<1>::kSlotBytes : Strip<2>::kSlotBytes));
+  at.bytes = at.slots + waves * (kind == 1 ? Strip<1>::kSlotBytes : (kind == 2 ? Strip<2>::kSlotBytes : (kind == 4 ? Strip<4>::kSlotBytes : 0u)));
   return at;
 }
 
@@ -157,9 +197,14 @@ __device__ __forceinline__ uint32_t opaque(uint32_t value) {
 // The dots of one run, closed: totals[set][i] gains activation row 4 set + i's part of the lane's groups.
 // `codes`: the lane's operand bases, `scales` / `sums`: the run's, at the lane's first group.
 template <int kKind, int kSets> struct StripDot;
-template <int kSets> struct StripDot<2, kSets> {
-  static constexpr uint32_t first_chunk(uint32_t part) { return 2 * part; }
-  static __device__ __forceinline__ void add(const Strip<2> &w, uint32_t part, const unsigned char *const (&codes)[kSets],
+// The lane's A row has codes at its k-slots; where they start.
+template <int kStep> struct StripFaces {
+  static constexpr int kBases = 1;
+  static __device__ __forceinline__ bool faces(int, uint32_t column, uint32_t part) { return column / 4 == part; }
+};
+template <int kSets> struct StripDot<2, kSets> : StripFaces<0> {
+  static constexpr uint32_t first_chunk(uint32_t, uint32_t part) { return 2 * part; }
+  static __device__ __forceinline__ void add(const Strip<2> &w, uint32_t part, const unsigned char *const (&codes)[1][kSets],
                                              const float *scales, const int *, uint32_t run, double (&totals)[kSets][4]) {
 #pragma unroll
     for (uint32_t j = 0; j < 2; ++j) {
@@ -169,7 +214,7 @@ template <int kSets> struct StripDot<2, kSets> {
         i32x4 dots = {0, 0, 0, 0};
 #pragma unroll
         for (uint32_t s = 0; s < 2; ++s) {
-          const u32x4 operand = *reinterpret_cast<const u32x4 *>(codes[set] + (8 * j + s) * 16);
+          const u32x4 operand = *reinterpret_cast<const u32x4 *>(codes[0][set] + (8 * j + s) * 16);
           dots = __builtin_amdgcn_mfma_i32_16x16x64_i8((i32x4)operand, (i32x4)w.q[2 * j + s], dots, 0, 0, 0);
         }
         const f32x4 a = *reinterpret_cast<const f32x4 *>(scales + ((size_t)(8 * run + 4 * j + part) * kSets + set) * 4);
@@ -179,9 +224,9 @@ template <int kSets> struct StripDot<2, kSets> {
     }
   }
 };
-template <int kSets> struct StripDot<1, kSets> {
-  static constexpr uint32_t first_chunk(uint32_t part) { return 8 * (part / 2) + part % 2; }
-  static __device__ __forceinline__ void add(const Strip<1> &w, uint32_t part, const unsigned char *const (&codes)[kSets],
+template <int kSets> struct StripDot<1, kSets> : StripFaces<0> {
+  static constexpr uint32_t first_chunk(uint32_t, uint32_t part) { return 8 * (part / 2) + part % 2; }
+  static __device__ __forceinline__ void add(const Strip<1> &w, uint32_t part, const unsigned char *const (&codes)[1][kSets],
                                              const float *scales, const int *, uint32_t run, double (&totals)[kSets][4]) {
     const u32x4 top = w.top ^ 0xAAAAAAAAu;  // q - 32 modulo 64: bytes of 4 (q - 32) as int8
     const u32x4 q[4] = {((w.low << 2) & 0x3C3C3C3Cu) | ((top << 6) & 0xC0C0C0C0u), ((w.high << 2) & 0x3C3C3C3Cu) | ((top << 4) & 0xC0C0C0C0u),
@@ -195,7 +240,7 @@ template <int kSets> struct StripDot<1, kSets> {
       int whole[4] = {0, 0, 0, 0};
 #pragma unroll
       for (uint32_t g = 0; g < 4; ++g) {
-        const u32x4 operand = *reinterpret_cast<const u32x4 *>(codes[set] + 2 * g * 16);
+        const u32x4 operand = *reinterpret_cast<const u32x4 *>(codes[0][set] + 2 * g * 16);
         const i32x4 zero = {0, 0, 0, 0};
         const i32x4 dots = __builtin_amdgcn_mfma_i32_16x16x64_i8((i32x4)operand, (i32x4)q[g], zero, 0, 0, 0);
 #pragma unroll
@@ -207,9 +252,9 @@ template <int kSets> struct StripDot<1, kSets> {
     }
   }
 };
-template <int kSets> struct StripDot<0, kSets> {
-  static constexpr uint32_t first_chunk(uint32_t part) { return 4 * part; }
-  static __device__ __forceinline__ void add(const Strip<0> &w, uint32_t part, const unsigned char *const (&codes)[kSets],
+template <int kSets> struct StripDot<0, kSets> : StripFaces<0> {
+  static constexpr uint32_t first_chunk(uint32_t, uint32_t part) { return 4 * part; }
+  static __device__ __forceinline__ void add(const Strip<0> &w, uint32_t part, const unsigned char *const (&codes)[1][kSets],
                                              const float *scales, const int *sums, uint32_t run, double (&totals)[kSets][4]) {
     // sub-blocks 2 p and 2 p + 1: neighbouring bytes of the table, whole six bits below sub-block 4,
     // from there on four bits in a nibble and two in the top of an earlier byte
@@ -225,8 +270,8 @@ template <int kSets> struct StripDot<0, kSets> {
       i32x4 low = {0, 0, 0, 0}, high = {0, 0, 0, 0};
 #pragma unroll
       for (uint32_t s = 0; s < 2; ++s) {
-        const u32x4 for_low = *reinterpret_cast<const u32x4 *>(codes[set] + s * 16);
-        const u32x4 for_high = *reinterpret_cast<const u32x4 *>(codes[set] + (2 + s) * 16);
+        const u32x4 for_low = *reinterpret_cast<const u32x4 *>(codes[0][set] + s * 16);
+        const u32x4 for_high = *reinterpret_cast<const u32x4 *>(codes[0][set] + (2 + s) * 16);
         low = __builtin_amdgcn_mfma_i32_16x16x64_i8((i32x4)for_low, (i32x4)(w.q[s] & 0x0F0F0F0Fu), low, 0, 0, 0);
         high = __builtin_amdgcn_mfma_i32_16x16x64_i8((i32x4)for_high, (i32x4)((w.q[s] >> 4) & 0x0F0F0F0Fu), high, 0, 0, 0);
       }
@@ -243,85 +288,200 @@ template <int kSets> struct StripDot<0, kSets> {
   }
 };
 
-// Eight neighbouring values of an activation row at any element's address.
+template <int kSets> struct StripDotInPlace {
+  static constexpr int kBases = 3;
+  static __device__ __forceinline__ bool faces(int j, uint32_t column, uint32_t part) { return part + 4 * j - 2 * (column / 4) <= 2u; }
+  static constexpr uint32_t first_chunk(uint32_t column, uint32_t part) { return column / 4 + part; }
+  static __device__ __forceinline__ void add(const StripInPlace &w, uint32_t part, const unsigned char *const (&codes)[3][kSets],
+                                             const float *scales, const int *, uint32_t run, double (&totals)[kSets][4]) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const auto halves = __builtin_amdgcn_permlane32_swap(w.v[2 * g][2 * g], w.v[2 * g + 1][2 * g + 1], false, false);
+      const auto rows = __builtin_amdgcn_permlane16_swap(halves[0], halves[1], false, false);
+      const float d = f16_to_f32((uint16_t)(rows[0] >> (16 * (part % 2))));
+#pragma unroll
+      for (int set = 0; set < kSets; ++set) {
+        i32x4 dots = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const u32x4 operand = *reinterpret_cast<const u32x4 *>(codes[j][set] + (12 * g + 4 * j) * 16);
+          dots = __builtin_amdgcn_mfma_i32_16x16x64_i8((i32x4)operand, (i32x4)w.v[2 * g + j], dots, 0, 0, 0);
+        }
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(scales + ((size_t)(8 * run + 4 * g + part) * kSets + set) * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) totals[set][i] = __builtin_fma((double)(d * a[i]), (double)dots[i], totals[set][i]);
+      }
+    }
+  }
+};
+
+template <int kSets> struct StripDot<3, kSets> : StripDotInPlace<kSets> {};
+template <int kSets> struct StripDot<4, kSets> : StripDotInPlace<kSets> {};
+
+// Sixteen neighbouring values of an activation row at any element's address.
 template <class TX> struct StripValues {
-  static constexpr int kVectors = Traits<TX>::kVec == 8 ? 1 : 2;
+  static constexpr int kVectors = Traits<TX>::kSize;
   u32x4 raw[kVectors];
   __device__ __forceinline__ void load(const void *x, size_t first) {
 #pragma unroll
     for (int h = 0; h < kVectors; ++h)
       raw[h] = *reinterpret_cast<const words4_even *>(static_cast<const char *>(x) + first * Traits<TX>::kSize + 16 * h);
   }
-  __device__ __forceinline__ void values(float (&v)[8]) const {
-    if constexpr (kVectors == 1) {
-      Traits<TX>::unpack(raw[0], v);
-    } else {
+  __device__ __forceinline__ void values(float (&v)[16]) const {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        float piece[4];
-        Traits<TX>::unpack(raw[h], piece);
+    for (int h = 0; h < kVectors; ++h) {
+      float piece[Traits<TX>::kVec];
+      Traits<TX>::unpack(raw[h], piece);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[4 * h + e] = piece[e];
-      }
+      for (int e = 0; e < Traits<TX>::kVec; ++e) v[Traits<TX>::kVec * h + e] = piece[e];
     }
+  }
+  // f32 bits of the largest value that is not negative and of the largest magnitude among the others, 0 where
+  // there is none.  Compared as stored: bit patterns of one sign are in the order of their magnitudes, NaN last.
+  __device__ __forceinline__ void extremes(uint32_t &positive, uint32_t &negative) const {
+    if constexpr (Traits<TX>::kSize == 4) {
+      int above = (int)raw[0].x;
+      uint32_t below = raw[0].x;
+#pragma unroll
+      for (int i = 1; i < 16; ++i) {
+        above = max(above, (int)raw[i / 4][i % 4]);
+        below = max(below, raw[i / 4][i % 4]);
+      }
+      positive = above < 0 ? 0u : (uint32_t)above;
+      negative = (int)below < 0 ? below & 0x7FFFFFFFu : 0u;
+    } else {
+      typedef short i16x2 __attribute__((ext_vector_type(2)));
+      typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+      i16x2 above = __builtin_bit_cast(i16x2, (uint32_t)raw[0].x);
+      u16x2 below = __builtin_bit_cast(u16x2, (uint32_t)raw[0].x);
+#pragma unroll
+      for (int i = 1; i < 8; ++i) {
+        above = __builtin_elementwise_max(above, __builtin_bit_cast(i16x2, (uint32_t)raw[i / 4][i % 4]));
+        below = __builtin_elementwise_max(below, __builtin_bit_cast(u16x2, (uint32_t)raw[i / 4][i % 4]));
+      }
+      const int high = max((int)above.x, (int)above.y);
+      const uint32_t low = max((uint32_t)below.x, (uint32_t)below.y);
+      positive = f32_bits(widened((uint32_t)max(high, 0)));
+      negative = f32_bits(widened((low & 0x8000u) != 0 ? low & 0x7FFFu : 0u));
+    }
+  }
+  static __device__ __forceinline__ float widened(uint32_t half) {
+    if constexpr (std::is_same_v<TX, BF16>) return bits_f32(half << 16);
+    else return f16_to_f32((uint16_t)half);
   }
 };
 
-// Half a wave quantises a run of 256 values of an activation row, eight values per lane u: one Q8_K
-// block, or eight Q8_0 blocks of four lanes each.
-template <int kKind, class TX>
-__device__ __forceinline__ void strip_quantise(const StripValues<TX> &fetched, uint32_t lane, uint32_t *codes, float *scale, uint32_t scale_step,
-                                               int *sums, uint32_t sum_step) {
-  const uint32_t u = lane % 32;
-  float v[8];
-  fetched.values(v);
-  float largest = 0.0f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    largest = __builtin_fmaxf(largest, __builtin_fabsf(v[e]));  // a NaN is no candidate
+// The larger of both over 2 or 16 neighbouring lanes.
+template <int kLanes> __device__ __forceinline__ uint32_t lanes_max(uint32_t v) {
+  v = max(v, (uint32_t)dpp_move<kDppSwap1>((int)v));
+  if constexpr (kLanes == 16) {
+    v = max(v, (uint32_t)dpp_move<kDppSwap2>((int)v));
+    v = max(v, (uint32_t)dpp_move<kDppHalfMirror>((int)v));
+    v = max(v, (uint32_t)dpp_move<kDppRowMirror>((int)v));
   }
-  const float top = group_max<kKind == 2 ? 4 : 32>(largest);
+  return v;
+}
+
+// a / b correctly rounded for a of one or 127 and b from 2^-60 to 2^61: the hardware's reciprocal, a Newton step and
+// a correction of the quotient by its exact remainder (compared with the compiler's division for every such b).  It is
+// six instructions where the full division, which scales its operands, is eleven.
+__device__ __forceinline__ float quotient(float a, float b) {
+  const float rough = __builtin_amdgcn_rcpf(b);
+  const float inverse = __builtin_fmaf(__builtin_fmaf(-b, rough, 1.0f), rough, rough);
+  const float q = a * inverse;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), inverse, q);
+}
+// b / 127 the same way
+__device__ __forceinline__ float over_127(float b) {
+  constexpr float kInverse = 1.0f / 127.0f;
+  const float q = b * kInverse;
+  return __builtin_fmaf(__builtin_fmaf(-127.0f, q, b), kInverse, q);
+}
+
+// Sixteen lanes quantise a run of 256 values of an activation row, sixteen values per lane u: one Q8_K block, or eight
+// Q8_0 blocks of two lanes each.  A block whose largest magnitude lies between 2^-60 and 2^61 and (Q8_K, where its sign
+// counts) is not met with both signs takes the short form, in which a code is the low byte of value * factor + 1.5 * 2^23:
+// rounded to the nearest integer, ties to even, and no more than 127 in magnitude.  Any other block (zeros, NaN,
+// infinities) sends the wave the long way.
+template <int kKind, class TX>
+__device__ __forceinline__ void strip_quantise(const StripValues<TX> &fetched, uint32_t lane, unsigned char *codes, float *scale, uint32_t scale_step,
+                                               int *sums, uint32_t sum_step) {
+  constexpr bool kSmall = kKind >= 2;  // blocks of 32
+  constexpr int kLanes = kSmall ? 2 : 16;
+  const uint32_t u = lane % 16;
+  uint32_t positive, negative;
+  fetched.extremes(positive, negative);
+  if constexpr (kSmall) positive = negative = lanes_max<kLanes>(max(positive, negative));
+  else positive = lanes_max<kLanes>(positive), negative = lanes_max<kLanes>(negative);
+  const uint32_t top_bits = max(positive, negative);
+  const bool regular = top_bits >= (67u << 23) && top_bits < (188u << 23) && (kSmall || positive != negative);
+  float v[16];
+  fetched.values(v);
   float factor = 0.0f, stored = 0.0f;
-  if constexpr (kKind == 2) {
-    if (top != 0.0f) {
-      stored = f16_to_f32(f32_to_f16(top / 127.0f));
-      factor = 127.0f / top;
+  uint32_t words[4];
+  if (__builtin_expect(__ballot(!regular) == 0, 1)) {
+    const float top = bits_f32(top_bits);
+    if constexpr (kSmall) {
+      stored = f16_to_f32(f32_to_f16(over_127(top)));
+      factor = quotient(127.0f, top);
+    } else {
+      factor = quotient(127.0f, top);
+      factor = positive > negative ? -factor : factor;
+      stored = quotient(1.0f, factor);
+    }
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      uint32_t code[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) code[e] = f32_bits(v[4 * w + e] * factor + 12582912.0f);
+      words[w] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(code[3], code[2], 0x0C0C0400u), __builtin_amdgcn_perm(code[1], code[0], 0x0C0C0400u), 0x05040100u);
     }
   } else {
-    // the sign of the block's first value of that magnitude: of the lowest lane that has one
-    bool negative = false;
+    float largest = 0.0f;
 #pragma unroll
-    for (int e = 7; e >= 0; --e) negative = __builtin_fabsf(v[e]) == top ? v[e] < 0.0f : negative;
-    const uint64_t has = __ballot(largest == top), below = __ballot(negative);
-    const uint32_t own_has = (uint32_t)(has >> (lane & 32u)), own_below = (uint32_t)(below >> (lane & 32u));
-    if (top != 0.0f) {
-      const float value = (own_below >> __builtin_ctz(own_has)) & 1u ? -top : top;
-      factor = -127.0f / value;
-      stored = 1.0f / factor;
+    for (int e = 0; e < 16; ++e) largest = __builtin_fmaxf(largest, __builtin_fabsf(v[e]));  // a NaN is no candidate
+    const float top = bits_f32(lanes_max<kLanes>(f32_bits(largest)));
+    if constexpr (kSmall) {
+      if (top != 0.0f) {
+        stored = f16_to_f32(f32_to_f16(top / 127.0f));
+        factor = 127.0f / top;
+      }
+    } else {
+      // the sign of the block's first value of that magnitude: of the lowest lane that has one
+      bool below_zero = false;
+#pragma unroll
+      for (int e = 15; e >= 0; --e) below_zero = __builtin_fabsf(v[e]) == top ? v[e] < 0.0f : below_zero;
+      const uint64_t has = __ballot(largest == top), below = __ballot(below_zero);
+      const uint32_t own_has = (uint32_t)(has >> (lane & 48u)) & 0xFFFFu, own_below = (uint32_t)(below >> (lane & 48u));
+      if (top != 0.0f) {
+        const float value = (own_below >> __builtin_ctz(own_has)) & 1u ? -top : top;
+        factor = -127.0f / value;
+        stored = 1.0f / factor;
+      }
+    }
+    // nearest integer, ties to even, at most 127 (a block of zeros: factor 0); only the low bytes are kept
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      int code[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) code[e] = (int)__builtin_rintf(v[4 * w + e] * factor);
+      const short2v most = {127, 127};
+      const short2v low = __builtin_elementwise_min(__builtin_bit_cast(short2v, __builtin_amdgcn_cvt_pk_i16(code[0], code[1])), most);
+      const short2v high = __builtin_elementwise_min(__builtin_bit_cast(short2v, __builtin_amdgcn_cvt_pk_i16(code[2], code[3])), most);
+      words[w] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, high), __builtin_bit_cast(uint32_t, low), 0x06040200u);
     }
   }
-  // nearest integer, ties to even, at most 127 (a block of zeros: factor 0); only the low bytes are kept
-  uint32_t words[2];
-#pragma unroll
-  for (int w = 0; w < 2; ++w) {
-    int code[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) code[e] = (int)__builtin_rintf(v[4 * w + e] * factor);
-    const short2v most = {127, 127};
-    const short2v low = __builtin_elementwise_min(__builtin_bit_cast(short2v, __builtin_amdgcn_cvt_pk_i16(code[0], code[1])), most);
-    const short2v high = __builtin_elementwise_min(__builtin_bit_cast(short2v, __builtin_amdgcn_cvt_pk_i16(code[2], code[3])), most);
-    words[w] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, high), __builtin_bit_cast(uint32_t, low), 0x06040200u);
-  }
-  codes[2 * u] = words[0];
-  codes[2 * u + 1] = words[1];
+  const u32x4 whole = {words[0], words[1], words[2], words[3]};
+  // Q8_0 in place: 48 bytes per block, its codes where its quants lie in the 48 bytes from its first vector
+  if constexpr (kKind >= 3) *reinterpret_cast<words4_even *>(codes + 50 * (u / 2) + 2 + 16 * (u % 2)) = whole;
+  else reinterpret_cast<u32x4 *>(codes)[u] = whole;
   if constexpr (kKind == 0) {
-    int sum = dot4(0x01010101u, words[0], dot4(0x01010101u, words[1], 0));
-    sum += dpp_move<kDppSwap1>(sum);
-    sum += dpp_move<kDppSwap2>(sum);  // the four lanes of a sub-block
-    if (u % 4 == 0) sums[(u / 4) * sum_step] = sum;
+    int sum = dot4(0x01010101u, words[0], dot4(0x01010101u, words[1], dot4(0x01010101u, words[2], dot4(0x01010101u, words[3], 0))));
+    sum += dpp_move<kDppSwap1>(sum);  // the two lanes of a sub-block
+    if (u % 2 == 0) sums[(u / 2) * sum_step] = sum;
   }
-  if constexpr (kKind == 2) {
-    if (u % 4 == 0) scale[(u / 4) * scale_step] = stored;
+  if constexpr (kSmall) {
+    if (u % 2 == 0) scale[(u / 2) * scale_step] = stored;
   } else {
     if (u == 0) *scale = stored;
   }
@@ -340,7 +500,7 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
                                                                         uint32_t tile_rows, uint32_t split_log2) {
   using Held = Strip<kKind>;
   using Dot = StripDot<kKind, kSets>;
-  constexpr int kDepth = Held::kParked ? 2 : 3;  // runs of a wave in flight
+  constexpr int kDepth = Held::kParked || (kKind == 3 && kSets == 2) ? 2 : 3;  // runs of a wave in flight
   extern __shared__ __align__(16) unsigned char shared[];
   const StripLayout layout = strip_layout(kKind, m, k, blockDim.x / kWaveLanes);
   float *scales = reinterpret_cast<float *>(shared + layout.scales);
@@ -372,16 +532,20 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
     const uint32_t lane = opaque(threadIdx.x % kWaveLanes), column = lane % 16;
 #pragma unroll
     for (uint32_t i = 0; i < Held::kLoads; ++i)
-      load_row[i] = row_at(load_tile, Held::kParked ? min((lane + i * kWaveLanes) / Held::kVectors, kStripRows - 1) : column);
+      load_row[i] = row_at(load_tile, Held::kParked ? min((lane + i * kWaveLanes) / Held::kVectors, kStripRows - 1) : column) +
+                    (Held::kWhole ? (lane + i * kWaveLanes) % Held::kVectors * 16 : 0u);
   };
   auto next_load = [&](Pending &into) {
-    if constexpr (Held::kParked) {
+    if constexpr (Held::kWhole) {
+#pragma unroll
+      for (uint32_t i = 0; i < Held::kLoads; ++i) into.v[i] = load16(reinterpret_cast<const unsigned char *>(own) + (load_row[i] + load_run * Held::kRunBytes), 0);
+    } else if constexpr (Held::kParked) {
 #pragma unroll
       for (uint32_t i = 0; i < Held::kLoads; ++i) {
         const uintptr_t begin = own + (load_row[i] + load_run * Held::kRunBytes);
         const uint32_t wanted = (lane + i * kWaveLanes) % Held::kVectors * 16, last = ((uint32_t)begin & 15u) + Held::kRunBytes - 1;
         // a vector past the run's last byte is the last one again
-        into.v[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((begin & ~(uintptr_t)15) + min(wanted, last & ~15u)));
+        into.v[i] = *reinterpret_cast<const u32x4 *>((begin & ~(uintptr_t)15) + min(wanted, last & ~15u));
       }
     } else {
       into.load(reinterpret_cast<const unsigned char *>(own + (load_row[0] + load_run * Held::kRunBytes)), part);
@@ -397,48 +561,59 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
   };
 
   // ---- the activation rows, quantised once per block -----------------------------------------------
-  // runs go round the block's half waves; the next kBatch of a half wave are on their way
-  constexpr int kBatch = StripValues<TX>::kVectors == 1 ? 4 : 2;
-  const uint32_t halves = blockDim.x / 32;
-  const uint32_t units = m * runs, u = lane % 32;
+  // Four runs at a time per wave, kBatch times on their way: the loads of the first are asked for before the weights',
+  // the wave's first run of weights before they are there, and the rest of the ring behind the quantising: waves
+  // that first queue up every load they can hold wait for the memory pipe to take them (the first code of Q8_0
+  // [2304 -> 7936] x 2 came after 5.4 us that way, after 4.6 us like this).
+  constexpr int kBatch = Traits<TX>::kSize == 2 ? 2 : 1;
+  const uint32_t units = m * runs, step = blockDim.x / 16, u = lane % 16;
   const uint32_t inverse = (1u << 20) / runs + 1;  // unit / runs = unit * inverse >> 20 while units * runs < 2^20 (units <= 8 runs, runs <= 224)
-  auto fetch_batch = [&](uint32_t first, StripValues<TX> (&into)[kBatch]) {
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) into[j].load(x, (size_t)min(first + j * halves, units - 1) * 256 + 8 * u);  // rows are dense
-  };
-  const uint32_t half = threadIdx.x / 32;
+  // a unit past the last is the last one again: the same values to the same places
+  auto fetch = [&](uint32_t first, StripValues<TX> &into) { into.load(x, (size_t)min(first + lane / 16, units - 1) * 256 + 16 * u); };  // rows are dense
+  uint32_t unit = 4 * wave;  // of the wave's first sixteen lanes
   StripValues<TX> ahead[kBatch];
-  fetch_batch(half, ahead);
+#pragma unroll
+  for (int j = 0; j < kBatch; ++j)
+    if (unit + j * step < units) fetch(unit + j * step, ahead[j]);
   Pending ring[kDepth];
   if (items != 0) {
     aim();
-#pragma unroll
-    for (int d = 0; d < kDepth; ++d) next_load(ring[d]);
+    next_load(ring[0]);
   }
-  if (threadIdx.x < kZeroBytes / 16) reinterpret_cast<u32x4 *>(shared)[threadIdx.x] = u32x4{0u, 0u, 0u, 0u};
-  for (uint32_t first = half; first - half < units; first += kBatch * halves) {  // the same trips for both halves of a wave
-    StripValues<TX> now[kBatch];
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) now[j] = ahead[j];
-    fetch_batch(first + kBatch * halves, ahead);
+  {
+    // zeros round the codes where they lie as the weights do, otherwise only the row of zeros
+    const uint32_t clear = (kKind >= 3 ? layout.scales : kZeroBytes) / 16;
+    for (uint32_t i = threadIdx.x; i < clear; i += blockDim.x) reinterpret_cast<u32x4 *>(shared)[i] = u32x4{0u, 0u, 0u, 0u};
+    if constexpr (kKind >= 3) lds_barrier();
+  }
+  while (unit < units) {
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
-      // a unit past the last is the last one again: the same values to the same places
-      const uint32_t unit = min(first + j * halves, units - 1), token = (unit * inverse) >> 20, run = unit - token * runs;
-      strip_quantise<kKind, TX>(now[j], lane, reinterpret_cast<uint32_t *>(shared + kZeroBytes + (size_t)token * (k + kCodePad) + run * 256),
-                                scales + (size_t)(kKind == 2 ? 8 * run : run) * kSets * 4 + token, kSets * 4,
+      if (unit >= units) break;
+      const StripValues<TX> now = ahead[j];
+      if (unit + kBatch * step < units) fetch(unit + kBatch * step, ahead[j]);
+      const uint32_t mine = min(unit + lane / 16, units - 1), token = (mine * inverse) >> 20, run = mine - token * runs;
+      strip_quantise<kKind, TX>(now, lane, shared + kZeroBytes + (size_t)token * strip_code_pitch(kKind, k) + run * strip_run_codes(kKind),
+                                scales + (size_t)(kKind >= 2 ? 8 * run : run) * kSets * 4 + token, kSets * 4,
                                 sums + (size_t)8 * run * kSets * 4 + token, kSets * 4);
+      unit += step;
     }
+  }
+  if (items != 0) {
+#pragma unroll
+    for (int d = 1; d < kDepth; ++d) next_load(ring[d]);
   }
   lds_barrier();
 
   // ---- the weight rows -----------------------------------------------------------------------------
-  const bool faces = column / 4 == part;  // the lane's A row has codes at the lane's k-slots
-  uint32_t base[kSets];
-  const uint32_t advance = faces ? 256u : 0u;
+  // a lane's operands of a run: its activation row's codes from its first chunk on, or, where its A row has none at
+  // its k-slots, the zeros at the start
+  uint32_t base[kSets], faces[Dot::kBases];
+#pragma unroll
+  for (int j = 0; j < Dot::kBases; ++j) faces[j] = Dot::faces(j, column, part) ? 0xFFFFFFFFu : 0u;
 #pragma unroll
   for (uint32_t set = 0; set < (uint32_t)kSets; ++set)  // activation rows past the last repeat it and are not stored
-    base[set] = faces ? kZeroBytes + min(column % 4 + 4 * set, m - 1) * (k + kCodePad) + Dot::first_chunk(part) * 16 : 0u;
+    base[set] = kZeroBytes + min(column % 4 + 4 * set, m - 1) * strip_code_pitch(kKind, k) + Dot::first_chunk(column, part) * 16;
   double totals[kSets][4] = {};
   uint32_t run = member, tile = slot;
   uint32_t own_row = items != 0 ? (uint32_t)row_at(slot, column) : 0u;  // the lane's weight row
@@ -493,19 +668,21 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
         for (uint32_t i = 0; i < Held::kLoads; ++i) {
           const uint32_t piece = lane + i * kWaveLanes;
           if (piece < kStripRows * Held::kVectors)
-            *reinterpret_cast<u32x4 *>(parked + piece / Held::kVectors * Held::kPitch + piece % Held::kVectors * 16) = ring[d].v[i];
+            *reinterpret_cast<u32x4 *>(parked + (Held::kWhole ? piece * 16 : piece / Held::kVectors * Held::kPitch + piece % Held::kVectors * 16)) = ring[d].v[i];
         }
         next_load(ring[d]);
         wave_fence();
-        held.take(parked, column * Held::kPitch + (((uint32_t)own + own_row + run * Held::kRunBytes) & 15u), part);
+        held.take(parked, column * Held::kPitch + (Held::kWhole ? 0u : ((uint32_t)own + own_row + run * Held::kRunBytes) & 15u), part);
         wave_fence();
       } else {
         held = ring[d];
         next_load(ring[d]);
       }
-      const unsigned char *codes[kSets];
+      const unsigned char *codes[Dot::kBases][kSets];
 #pragma unroll
-      for (int set = 0; set < kSets; ++set) codes[set] = shared + base[set] + run * advance;
+      for (int j = 0; j < Dot::kBases; ++j)
+#pragma unroll
+        for (int set = 0; set < kSets; ++set) codes[j][set] = shared + ((base[set] + run * strip_run_codes(kKind)) & faces[j]);
       Dot::add(held, part, codes, scales, sums, run, totals);
       run += split;
       if (run >= runs) {
@@ -529,7 +706,7 @@ enum : int { kSixteen = 0, kSixteenShared = 1, kEight = 2, kTwice = 3, kTwiceSha
 template <int kKind, int kSets, int kForm> struct StripsTag {
   static std::string text() {
     static const char *const forms[] = {"16-waves", "16-waves/shared", "8-waves", "2x8-waves", "2x8-waves/shared"};
-    return std::string("gguf_matvec_q8_strips/") + strip_word(kKind) + "/" + std::to_string(4 * kSets) + "-tokens/" + forms[kForm];
+    return std::string("gguf_matvec_q8_strips/") + strip_word(kKind) + "/" + std::to_string(4 * kSets) + "-tokens/" + forms[kForm] + (kKind == 3 ? "/in-place" : (kKind == 4 ? "/in-place/parked" : ""));
   }
 };
 
@@ -570,11 +747,17 @@ hipError_t run_strips(const MatVecParams &p, uint32_t m, const void *w, const vo
       split_log2 = log2;
     }
   }
-  if (twice && split_log2 != 0) note_variant<StripsTag<kKind, kSets, kTwiceShared>>();
-  else if (twice) note_variant<StripsTag<kKind, kSets, kTwice>>();
-  else if (waves == 8) note_variant<StripsTag<kKind, kSets, kEight>>();
-  else if (split_log2 != 0) note_variant<StripsTag<kKind, kSets, kSixteenShared>>();
-  else note_variant<StripsTag<kKind, kSets, kSixteen>>();
+  if constexpr (kKind == 3) {
+    note_variant<StripsTag<kKind, kSets, kSixteen>>();
+  } else {
+    if constexpr (kKind != 4) {
+      if (!twice && waves == 8) note_variant<StripsTag<kKind, kSets, kEight>>();
+    }
+    if (twice && split_log2 != 0) note_variant<StripsTag<kKind, kSets, kTwiceShared>>();
+    else if (twice) note_variant<StripsTag<kKind, kSets, kTwice>>();
+    else if (waves == kMostWaves && split_log2 != 0) note_variant<StripsTag<kKind, kSets, kSixteenShared>>();
+    else if (waves == kMostWaves) note_variant<StripsTag<kKind, kSets, kSixteen>>();
+  }
   hipLaunchKernelGGL((gguf_matvec_q8_strips<kKind, TX, kSets>), dim3(grid), dim3(waves * kWaveLanes), shared, s, static_cast<const unsigned char *>(w), x, y,
                      rows, p.row_stride, p.k, m, block_rows, tile_rows, split_log2);
   return hipGetLastError();
@@ -593,10 +776,17 @@ template <int kKind, class TX> hipError_t run_groups(const MatVecParams &p, cons
   return hipSuccess;
 }
 
+inline bool in_place_serves(const MatVecParams &p, const void *w) {
+  return p.row_stride % 16 == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0 && strip_waves(3, p.m, p.k) == kMostWaves;
+}
+
 template <class TX> hipError_t run_strips_kind(const MatVecParams &p, const void *w, const void *x, void *y, hipStream_t s) {
   switch (p.kind) {
     case 0: return run_groups<0, TX>(p, w, x, y, s);
     case 1: return run_groups<1, TX>(p, w, x, y, s);
+    case 2:
+      if (in_place_serves(p, w)) return strip_waves(4, p.m, p.k) == kMostWaves ? run_groups<4, TX>(p, w, x, y, s) : run_groups<3, TX>(p, w, x, y, s);
+      [[fallthrough]];
     default: return run_groups<2, TX>(p, w, x, y, s);
   }
 }
@@ -609,6 +799,7 @@ bool gguf_matvec_strips_serve(const MatVecParams &p) {
          strip_waves(p.kind, 1, p.k) != 0 && ((p.rows + units - 1) / units + kStripRows) * p.row_stride < 0xFFFFFFFFull;
 }
 uint32_t gguf_matvec_strips_dispatches(const MatVecParams &p) {
+  if (p.kind == 2 && in_place_serves(p, nullptr)) return 1;
   const uint32_t group = strip_group(p.kind, p.m, p.k);
   return (p.m + group - 1) / group;
 }

@@ -266,7 +266,8 @@ def test_q8_route_q4_k_matrix_unit_widths_tokens_and_shared_tiles(x_tag):
             x[m - 1, 256:512] = 0.0
         tokens = 1 if m == 1 else (4 if m <= 4 else 8)
         note(f"q8 matvec q4_k tiles x {x_tag} rows {rows} k {k} m {m}")
-        check("q4_k", x_tag, raw, rows, k, x, kernel=f"gguf_matvec_q8_tiles/q4_k/{tokens}-tokens")
+        family = "strips" if (rows, m) in ((600, 2), (2100, 1)) else "tiles"   # many weight rows: the strip kernel
+        check("q4_k", x_tag, raw, rows, k, x, kernel=f"gguf_matvec_q8_{family}/q4_k/{4 if family == 'strips' else tokens}-tokens")
     note("q8 matvec q4_k: fewer than four blocks per row, an odd row stride and unaligned activations keep the block-walking kernel")
     raw = raw_bytes_for("q4_k", rng, 20, 768)
     check("q4_k", x_tag, raw, 20, 768, rng.normal(0, 1, 768).astype(np.float32), kernel="gguf_matvec_q8_blocks/q4_k/1-tokens")
@@ -323,4 +324,6 @@ def test_q8_route_q4_k_matrix_unit_seeded_random_shapes():
         padded[:, :raw.shape[1]] = raw
         x = rng.normal(0, 1.5, (m, k) if m > 1 else (k,)).astype(np.float32)
         note(f"q8 matvec q4_k tiles draw {case}: rows {rows} k {k} m {m} x {x_tag} pad {pad}")
-        check("q4_k", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad, kernel=f"gguf_matvec_q8_tiles/q4_k/{tokens}-tokens")
+        strips = rows >= 512 and (m > 1 or k >= 10240 or (k > 2048 and k % 2048 != 0))   # several rows or wide ones against many
+        kernel = f"gguf_matvec_q8_strips/q4_k/{4 if m <= 4 else 8}-tokens" if strips else f"gguf_matvec_q8_tiles/q4_k/{tokens}-tokens"
+        check("q4_k", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad, kernel=kernel)

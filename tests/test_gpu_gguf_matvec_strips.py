@@ -47,10 +47,50 @@ def test_strips_edges(tag, x_tag):
               kernel=f"gguf_matvec_q8_strips/{tag}/{4 if m <= 4 else 8}-tokens")
 
 
+# rows, k, activation rows, the form: Q8_0 rows of whole vectors, whose bytes the matrix unit takes as they lie
+IN_PLACE = (
+    (513, 256, 2, "4-tokens/16-waves/in-place/parked"),  # one run, three weight rows to a block
+    (4099, 1280, 5, "8-tokens/16-waves/shared/in-place/parked"),
+    (4096, 256, 8, "8-tokens/16-waves/in-place/parked"),
+    (66000, 256, 3, "4-tokens/2x8-waves/in-place/parked"),
+    (66000, 256, 8, "8-tokens/2x8-waves/in-place/parked"),
+    (12289, 1792, 2, "4-tokens/2x8-waves/shared/in-place/parked"),
+    (9001, 1280, 7, "8-tokens/2x8-waves/shared/in-place/parked"),
+    (70000, 4352, 4, "4-tokens/2x8-waves/shared/in-place/parked"),  # more tiles than waves
+    (1031, 4096, 8, "8-tokens/16-waves/shared/in-place/parked"),
+    (530, 25600, 3, "4-tokens/16-waves/in-place"),  # no room for slots: straight into the lanes
+    (515, 28672, 3, "4-tokens/16-waves/in-place"),
+    (519, 17408, 5, "8-tokens/16-waves/in-place"),
+)
+
+
+@pytest.mark.parametrize("x_tag", ["f32", "bf16", "f16"])
+def test_strips_q8_0_in_place(x_tag):
+    rng = np.random.default_rng(1823)
+    for rows, k, m, form in IN_PLACE:
+        raw = raw_bytes_for("q8_0", rng, rows, k) if x_tag != "f16" else weights_for("q8_0", rng, rows, k)
+        padded = np.zeros((rows, raw.shape[1] + 16), np.uint8)                       # whole vectors between rows too
+        padded[:, :raw.shape[1]] = raw
+        x = rng.normal(0, 1.5, (m, k)).astype(np.float32)
+        x[m - 1, :32], x[0, k - 32:] = 0.0, -3.0                                    # a block of zeros, one of equal values
+        note(f"q8 matvec strips in place x {x_tag} rows {rows} k {k} m {m}")
+        check("q8_0", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + 16, kernel=f"gguf_matvec_q8_strips/q8_0/{form}")
+
+
+def test_strips_decoded_q8_0_off_a_boundary_in_every_form():
+    rng = np.random.default_rng(1824)
+    for rows, k, m in ((66000, 256, 2), (66000, 256, 5), (12289, 1536, 2), (9001, 1280, 7), (70000, 4352, 4), (70000, 4352, 5), (4096, 1280, 5), (600, 1536, 3)):
+        raw = raw_bytes_for("q8_0", rng, rows, k)
+        note(f"q8 matvec strips q8_0 rows {rows} k {k} m {m}, two bytes off")
+        check("q8_0", "bf16", raw, rows, k, rng.normal(0, 1, (m, k)).astype(np.float32), byte_offset=2, kernel="gguf_matvec_q8_strips/q8_0/")
+
+
 @pytest.mark.parametrize("tag,k,rows,m,kernel", [
     ("q6_k", 2304, 24000, 1, "strips/q6_k/4"), ("q6_k", 1280, 4096, 1, "blocks/q6_k/1"), ("q8_0", 4096, 8192, 6, "strips/q8_0/8"),
-    ("q8_0", 4096, 8192, 4, "lines/q8_0/4"), ("q6_k", 6144, 8192, 4, "strips/q6_k/4"), ("q6_k", 6144, 8192, 2, "quads/q6_k/4"),
-    ("q4_k", 4096, 4096, 2, "strips/q4_k/4"), ("q4_k", 3840, 4096, 4, "tiles/q4_k/4")])
+    ("q8_0", 4096, 8192, 4, "strips/q8_0/4"), ("q8_0", 16384, 1024, 2, "lines/q8_0/2"), ("q6_k", 6144, 8192, 4, "strips/q6_k/4"),
+    ("q6_k", 6144, 511, 2, "quads/q6_k/4"), ("q6_k", 2304, 2304, 1, "strips/q6_k/4"), ("q6_k", 4096, 8192, 1, "spans/q6_k/2"),
+    ("q4_k", 4096, 4096, 2, "strips/q4_k/4"), ("q4_k", 2048, 8192, 4, "tiles/q4_k/4"), ("q4_k", 2048, 8192, 5, "strips/q4_k/8"),
+    ("q4_k", 3840, 4096, 1, "strips/q4_k/4"), ("q4_k", 2560, 5120, 1, "tiles/q4_k/1"), ("q4_k", 10240, 16384, 1, "strips/q4_k/4")])
 def test_strips_rule(tag, k, rows, m, kernel):
     rng = np.random.default_rng(1821)
     note(f"q8 matvec rule {tag} rows {rows} k {k} m {m}")
@@ -168,3 +208,18 @@ def test_strips_activations_that_are_no_numbers(tag):
     assert np.array_equal(np.isnan(got[:, :256]), np.isnan(general))
     few = np.abs(np.where(np.isnan(general), 0.0, got[:, :256] - general))
     assert np.all(few <= 1e-5 * np.nanmax(np.abs(general)))   # both are within gamma(K / 4 + 65, 2^-24) of the same sum of terms
+
+
+@pytest.mark.parametrize("tag", ["q4_k", "q6_k"])
+def test_strips_activation_blocks_on_both_sides_of_the_short_form(tag):
+    """Magnitudes below 2^-60 and from 2^61 on divide in full: whole waves of such blocks, and blocks that share a
+    wave with ordinary ones."""
+    rng = np.random.default_rng(1825)
+    rows, k = 1030, 4096
+    x = rng.normal(0, 1, (4, k)).astype(np.float32)
+    x[0] *= np.float32(2.0 ** -70)
+    x[1] *= np.repeat(np.float32([2.0 ** -62, 1, 2.0 ** -59, 2.0 ** 20]), k // 4)
+    x[2] *= np.repeat(np.float32([2.0 ** 58, 2.0 ** 61, 2.0 ** 64, 2.0 ** 60]), k // 4)
+    x[3] *= np.tile(np.repeat(np.float32([2.0 ** -65, 2.0 ** -60]), 256), k // 512)
+    note(f"q8 matvec strips {tag}: activation blocks below 2^-60 and above 2^61")
+    check(tag, "f32", weights_for(tag, rng, rows, k), rows, k, x, kernel=f"gguf_matvec_q8_strips/{tag}/4-tokens")
