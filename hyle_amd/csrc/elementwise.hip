@@ -505,13 +505,16 @@ hipError_t run_flat_as(const EwFlat &p, Operand a, Operand b, Operand c, void *o
 }
 
 // Launch shape from the HBM traffic of the launch (streams as long as the output, the output
-// included), as measured on MI355X.  Inputs all as long as the output: R[8192,2048] += Y bf16
-// (101 MB) takes 16.5 us with 8 vectors per lane taken serially in blocks of 512 threads,
-// against 17.1 (4 at once, 256 threads) and 17.8 (1 vector per lane); SwiGLU over [8192,6144]
-// bf16 (302 MB) takes 46.9 us with 4 vectors at once against 47.5 (1 vector) and 49-53 for the
-// serial forms.  With broadcast operands: (A[4096,2048] + b) * s f32 (67 MB) takes 11.3 us
+// included), as measured on MI355X.  Inputs all as long as the output: one vector per lane in blocks of
+// one wave, so that a wave waits for its own loads only, starts when any slot is free and leaves no block
+// half done, and a small launch is spread over all compute units.  SwiGLU bf16, us, against blocks
+// of 512 threads that take four or eight vectors one after another: 0.2 MB 2.0 / 4.1, 8 MB 3.1 / 5.4, 60 MB 11.0 /
+// 14.5, 110 MB 18.4 / 24; blocks of 256 threads with four vectors at once: 300 MB 45.9 / 47.0, 600 MB 90.2 / 92.9.
+// Between 44 and 50 MB the launch fits the chip at once in the serial form, whose reads then end before its
+// writes begin: add f32 50 MB 8.6 against 9.4, 45 MB 8.2 / 8.6 (55 MB 11.4 / 10.3, 36 MB 7.1 / 7.3).
+// With broadcast operands: (A[4096,2048] + b) * s f32 (67 MB) takes 11.3 us
 // with 4 vectors per lane in blocks of 1024 threads against 11.8 (256 threads) and 12.9
-// (8 vectors).
+// (8 vectors); below 24 MB one vector per lane, A[512,2048] + b f32 2.9 against 5.1.
 template <class T, class Fn>
 hipError_t run_vec(const EwFlat &p, Operand a, Operand b, Operand c, void *out, hipStream_t s) {
   uint64_t streams = 1;  // the output
@@ -522,12 +525,11 @@ hipError_t run_vec(const EwFlat &p, Operand a, Operand b, Operand c, void *out, 
   }
   const uint64_t traffic = streams * p.elements * Traits<T>::kSize;
   if (!all_full) {
-    if (traffic > (80ull << 20)) return run_flat_as<T, Fn, 1, 256>(p, a, b, c, out, s);
+    if (traffic > (80ull << 20) || traffic < (24ull << 20)) return run_flat_as<T, Fn, 1, 256>(p, a, b, c, out, s);
     return run_flat_as<T, Fn, 4, 1024>(p, a, b, c, out, s);
   }
-  if (traffic > (110ull << 20)) return run_full_as<T, Fn, 4, 256, false>(p, a, b, c, out, s);
-  if (traffic > (48ull << 20)) return run_full_as<T, Fn, 8, 512, true>(p, a, b, c, out, s);
-  return run_full_as<T, Fn, 4, 512, true>(p, a, b, c, out, s);
+  if (traffic > (42ull << 20) && traffic <= (48ull << 20)) return run_full_as<T, Fn, 4, 512, true>(p, a, b, c, out, s);
+  return run_full_as<T, Fn, 1, 64, false>(p, a, b, c, out, s);
 }
 
 template <class T, int kKind0>
