@@ -191,10 +191,11 @@ __global__ __launch_bounds__(kBlockThreads) void cast_general(const char *in, vo
 // Copy of a strided tensor whose innermost axes are runs of whole units (16, 8, 4 or 2 bytes, as large as
 // the run, the strides and the addresses allow): a unit per lane, its offset from 32-bit divisions
 // over the axes that cannot be folded into one.  Bound by HBM for runs of a cache line or more (a run
-// of 128 bf16: [1024, 16, 128] with its first two axes swapped, 8.4 MB, 3.4 us; element by element 8.5 us).
+// of 128 bf16: [1024, 16, 128] with its first two axes swapped, 8.4 MB, 3.3 us; element by element 8.5 us).
+// Blocks of one wave: [4096, 32, 128], 67 MB, 13.2 us against 15.0 in blocks of four.
 template <class Unit>
-__global__ __launch_bounds__(kBlockThreads) void copy_units(const char *in, Unit *out, uint32_t units, CastLayout layout) {
-  const uint32_t e = blockIdx.x * kBlockThreads + threadIdx.x;
+__global__ __launch_bounds__(kWaveLanes) void copy_units(const char *in, Unit *out, uint32_t units, CastLayout layout) {
+  const uint32_t e = blockIdx.x * kWaveLanes + threadIdx.x;
   if (e >= units) return;
   int64_t offset = 0;
   uint32_t rest = e;
@@ -255,7 +256,7 @@ bool unit_layout(const CastParams &p, uintptr_t addresses, CastLayout *layout, u
 
 template <class Unit> hipError_t run_units(const void *in, void *out, uint64_t units, const CastLayout &layout, hipStream_t s) {
   note_variant<UnitsTag<Unit>>();
-  hipLaunchKernelGGL((copy_units<Unit>), dim3((uint32_t)((units + kBlockThreads - 1) / kBlockThreads)), dim3(kBlockThreads), 0, s,
+  hipLaunchKernelGGL((copy_units<Unit>), dim3((uint32_t)((units + kWaveLanes - 1) / kWaveLanes)), dim3(kWaveLanes), 0, s,
                      static_cast<const char *>(in), static_cast<Unit *>(out), (uint32_t)units, layout);
   return hipGetLastError();
 }
@@ -284,15 +285,18 @@ hipError_t run_flat_as(const void *in, void *out, uint64_t elements, hipStream_t
 template <class S, class D>
 hipError_t run_pair(const CastParams &p, const void *in, void *out, bool vectorised, hipStream_t s) {
   if (p.dense_input && vectorised) {
-    // Launch shape from the traffic, as for the elementwise kernels: fat blocks that take their
-    // groups one after another below about 110 MB, several groups at once per lane above.
+    // Launch shape from the traffic: one group per lane below about 24 MB, where the launch is spread
+    // over all compute units and ends with its one wait; fat blocks that take their groups one after
+    // another up to about 110 MB, blocks of one wave above.
     const uint64_t traffic = p.elements * (uint64_t)(S::kSize + D::kSize);
     // Measured on MI355X, [8192, 2048]: f32 -> bf16 16.6 us and bf16 -> f32 17.3 us with 8
     // groups per lane taken serially in blocks of 512 threads, against 18.9 / 17.6 us with one
-    // group per lane; a 201 MB copy 32.6 us with one group per lane against 35-37 us serially.
-    if (traffic > (110ull << 20)) return run_flat_as<S, D, 1, 256, false>(in, out, p.elements, s);
+    // group per lane; f32 -> bf16 of 300 MB 44.9 us with one group per lane in blocks of 64 threads, 49.9 us in
+    // blocks of 256, 53 serially; of 4 MB 2.4 us with one group per lane, 3.7 serially.
+    if (traffic > (110ull << 20)) return run_flat_as<S, D, 1, 64, false>(in, out, p.elements, s);
     if (traffic > (48ull << 20)) return run_flat_as<S, D, 8, 512, true>(in, out, p.elements, s);
-    return run_flat_as<S, D, 4, 512, true>(in, out, p.elements, s);
+    if (traffic > (24ull << 20)) return run_flat_as<S, D, 4, 512, true>(in, out, p.elements, s);
+    return run_flat_as<S, D, 1, 256, false>(in, out, p.elements, s);
   }
   CastLayout layout{};
   layout.rank = p.rank;

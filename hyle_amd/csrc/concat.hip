@@ -20,22 +20,21 @@ struct ConcatOperands {
 };
 
 // Dense inputs: kUnit bytes per thread step (16 when every run, offset and pointer allows it,
-// otherwise the element size).  grid.y is the input; a block takes up to kRunSteps * 256 units of
+// otherwise the element size).  grid.y is the input; a block takes up to kSteps units per thread of
 // one run, so the run and the place in it come from one division per block.
-constexpr uint32_t kRunSteps = 4;
-template <int kUnit>
+template <int kUnit, uint32_t kSteps>
 __global__ __launch_bounds__(kBlockThreads) void concat_runs(ConcatOperands p, unsigned char *out) {
   const uint32_t input = blockIdx.y;
   const uint32_t units_per_run = (uint32_t)(p.run_bytes[input] / kUnit);
   if (units_per_run == 0) return;
-  const uint32_t blocks_per_run = (units_per_run + kRunSteps * kBlockThreads - 1) / (kRunSteps * kBlockThreads);
+  const uint32_t blocks_per_run = (units_per_run + kSteps * blockDim.x - 1) / (kSteps * blockDim.x);
   const uint32_t run = blockIdx.x / blocks_per_run, piece = blockIdx.x - run * blocks_per_run;
   if (run >= p.outer) return;
   const unsigned char *from = p.base[input] + (uint64_t)run * p.run_bytes[input];
   unsigned char *to = out + (uint64_t)run * p.out_pitch + p.offset_bytes[input];
 #pragma unroll
-  for (uint32_t j = 0; j < kRunSteps; ++j) {
-    const uint32_t u = (piece * kRunSteps + j) * kBlockThreads + threadIdx.x;
+  for (uint32_t j = 0; j < kSteps; ++j) {
+    const uint32_t u = (piece * kSteps + j) * blockDim.x + threadIdx.x;
     if (u >= units_per_run) break;
     if constexpr (kUnit == 16) store16_stream(to, u, load16_stream(from, u));
     else if constexpr (kUnit == 8) reinterpret_cast<uint64_t *>(to)[u] = reinterpret_cast<const uint64_t *>(from)[u];
@@ -83,6 +82,13 @@ uint32_t blocks_for(uint64_t units) {
   return (uint32_t)(blocks < 1 ? 1 : (blocks > 16384 ? 16384 : blocks));
 }
 
+template <int kUnit, uint32_t kSteps>
+void run_runs(const ConcatOperands &c, uint32_t inputs, uint32_t threads, unsigned char *out, hipStream_t s) {
+  uint64_t blocks = 1;  // of the input that needs most
+  for (uint32_t i = 0; i < inputs; ++i) blocks = std::max<uint64_t>(blocks, (c.run_bytes[i] / kUnit + kSteps * threads - 1) / (kSteps * threads) * c.outer);
+  hipLaunchKernelGGL((concat_runs<kUnit, kSteps>), dim3((uint32_t)blocks, inputs), dim3(threads), 0, s, c, out);
+}
+
 }  // namespace
 
 // Launch-shape labels
@@ -109,18 +115,22 @@ hipError_t launch_concat(const ConcatParams &p, const void *const *inputs, void 
         wide = wide && (c.run_bytes[i] | c.offset_bytes[i] | reinterpret_cast<uintptr_t>(inputs[i])) % 16 == 0;
     }
     const int unit = wide ? 16 : p.size;
-    uint64_t blocks = 1;  // of the input that needs most
-    for (uint32_t i = 0; i < p.inputs; ++i) {
-      const uint64_t units_per_run = c.run_bytes[i] / unit;
-      blocks = std::max<uint64_t>(blocks, (units_per_run + kRunSteps * kBlockThreads - 1) / (kRunSteps * kBlockThreads) * p.outer);
-    }
-    const dim3 grid((uint32_t)blocks, p.inputs), block(kBlockThreads);
+    // One unit per thread below 16 MB of output, where the launch is spread thin and each step would be a
+    // wait of its own ([10, 22 + 1132, 64] f32, 3 MB, 2.5 us against 3.8 with four); four up to 64 MB
+    // ([16, 3072 + 1024, 128] bf16, 17 MB, 7.6 us against 7.9 with two); two in blocks of 128 threads above
+    // ([32, 8000 + 3000, 256] bf16, 180 MB, 58.5 us against 63.7 with four in blocks of 256, 71 with one in blocks of 64).
+    const uint64_t bytes = p.elements * p.size;
     switch (unit) {
-      case 16: note_variant<ConcatTag<16, true>>(); hipLaunchKernelGGL((concat_runs<16>), grid, block, 0, stream, c, o); break;
-      case 8: note_variant<ConcatTag<8, true>>(); hipLaunchKernelGGL((concat_runs<8>), grid, block, 0, stream, c, o); break;
-      case 4: note_variant<ConcatTag<4, true>>(); hipLaunchKernelGGL((concat_runs<4>), grid, block, 0, stream, c, o); break;
-      case 2: note_variant<ConcatTag<2, true>>(); hipLaunchKernelGGL((concat_runs<2>), grid, block, 0, stream, c, o); break;
-      default: note_variant<ConcatTag<1, true>>(); hipLaunchKernelGGL((concat_runs<1>), grid, block, 0, stream, c, o); break;
+      case 16:
+        note_variant<ConcatTag<16, true>>();
+        if (bytes < (16ull << 20)) run_runs<16, 1>(c, p.inputs, 256, o, stream);
+        else if (bytes < (64ull << 20)) run_runs<16, 4>(c, p.inputs, 256, o, stream);
+        else run_runs<16, 2>(c, p.inputs, 128, o, stream);
+        break;
+      case 8: note_variant<ConcatTag<8, true>>(); run_runs<8, 4>(c, p.inputs, 256, o, stream); break;
+      case 4: note_variant<ConcatTag<4, true>>(); run_runs<4, 4>(c, p.inputs, 256, o, stream); break;
+      case 2: note_variant<ConcatTag<2, true>>(); run_runs<2, 4>(c, p.inputs, 256, o, stream); break;
+      default: note_variant<ConcatTag<1, true>>(); run_runs<1, 4>(c, p.inputs, 256, o, stream); break;
     }
     return hipGetLastError();
   }

@@ -24,7 +24,7 @@ pytestmark = pytest.mark.gpu
 SUITE = ("test_gpu_parity", "test_gpu_softmax_variants", "test_gpu_norm_variants", "test_gpu_reduce", "test_gpu_cast_copy",
          "test_gpu_k_quants", "test_gpu_gguf_matvec_q8", "test_gpu_gguf_matvec", "test_gpu_topk", "test_gpu_unary_gated",
          "test_gpu_fill_select", "test_gpu_concat", "test_gpu_gather", "test_gpu_rope", "test_gpu_sampling", "test_gpu_storage_types",
-         "test_gpu_softmax_unaligned", "test_gpu_gguf_matvec_strips", "test_gpu_copy_units")
+         "test_gpu_softmax_unaligned", "test_gpu_gguf_matvec_strips", "test_gpu_copy_units", "test_gpu_streaming_shapes")
 
 
 def test_every_launch_shape_compiled_into_the_library_was_launched_by_a_test():
