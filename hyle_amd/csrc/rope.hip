@@ -121,16 +121,6 @@ __global__ __launch_bounds__(kBlockThreads) void rope_steps(RopeOperands p, cons
   constexpr int kPairs = kHalfSplit ? kVec : kVec / 2;
   const uint32_t first_step = blockIdx.x * steps_per_block;
   const uint32_t own = steps - first_step < steps_per_block ? steps - first_step : steps_per_block;
-  for (uint32_t i = threadIdx.x; i < own * p.pairs; i += kBlockThreads) {
-    const uint32_t local = i / p.pairs, pair = i - local * p.pairs;
-    const uint32_t step_index = first_step + local, step = step_index % p.sequence;
-    const uint32_t position_at = p.batched_positions ? step_index : step;
-    const float position = p.wide_positions ? (float)static_cast<const int64_t *>(p.positions)[position_at]
-                                            : (float)static_cast<const int32_t *>(p.positions)[position_at];
-    const float frequency = p.frequencies[(p.stepped_frequencies ? step * p.pairs : 0u) + pair];
-    sincosf(frequency * position, &table[(2 * local + 1) * p.pairs + pair], &table[2 * local * p.pairs + pair]);
-  }
-  __syncthreads();
   const uint32_t rotating = (kHalfSplit ? p.pairs : p.rotary) / kVec, partner = p.pairs / kVec;
   const uint32_t per_step = p.inner * places, total = own * per_step;
   // a unit is one place of one row; its loads are issued one unit ahead of its arithmetic
@@ -157,9 +147,20 @@ __global__ __launch_bounds__(kBlockThreads) void rope_steps(RopeOperands p, cons
     }
     return unit;
   };
+  // (the first one's before the phases; a thread without one asks for the block's first)
   uint32_t u = threadIdx.x;
+  Unit current = fetch(u < total ? u : 0);
+  for (uint32_t i = threadIdx.x; i < own * p.pairs; i += kBlockThreads) {
+    const uint32_t local = i / p.pairs, pair = i - local * p.pairs;
+    const uint32_t step_index = first_step + local, step = step_index % p.sequence;
+    const uint32_t position_at = p.batched_positions ? step_index : step;
+    const float position = p.wide_positions ? (float)static_cast<const int64_t *>(p.positions)[position_at]
+                                            : (float)static_cast<const int32_t *>(p.positions)[position_at];
+    const float frequency = p.frequencies[(p.stepped_frequencies ? step * p.pairs : 0u) + pair];
+    sincosf(frequency * position, &table[(2 * local + 1) * p.pairs + pair], &table[2 * local * p.pairs + pair]);
+  }
+  __syncthreads();
   if (u >= total) return;
-  Unit current = fetch(u);
   while (true) {
     const uint32_t following = u + kBlockThreads;
     Unit next = current;
@@ -242,12 +243,16 @@ hipError_t run_rope(const RopeParams &p, const void *in, const void *positions, 
     const uint64_t units = p.rows / p.inner * groups * places;  // at most INT32_MAX elements / kVec
     const uint64_t steps = p.rows / p.inner;
     if (p.rotary / 2 <= 2048) {
-      // The steps that give a block about 512 places, two per thread with the second one's loads
-      // issued before the first one's arithmetic.  Measured on MI355X for [1, 8192, 16, 128] bf16,
-      // half-split: 13.5 us so (14.2 / 13.6 / 13.8 / 15.3 us with 128 / 256 / 1024 / 2048 places);
-      // 14.9 us when every thread takes cos and sin itself for eight rows, 31.2 us when it does
+      // The steps that give a block about 256 places, one per thread, its loads issued before the phases are taken;
+      // 512, two per thread, where 256 would leave a quarter of the threads without one and the launch is large
+      // enough for that to count.  Measured on MI355X, 256 / 512 places: [1, 8192, 16, 128] bf16 half-split
+      // 13.2 / 13.9 us, [1, 4138, 14, 96] bf16 6.0 / 8.1, [1, 1981, 21, 64] f32 rotary 32 5.2 / 7.4, [1, 1037, 20, 80] f16
+      // rotary 32 (160 of 256 threads) 4.4 / 5.3, but [1, 6606, 20, 128] f16 (160 of 256) 15.8 / 15.1; 16.0 with 128
+      // places, 14.9 us for the first when every thread takes cos and sin itself for eight rows, 31.2 us when it does
       // so for each row; the plain copy of the same bytes 11.1 us.
-      uint32_t per_block = 512 / (p.inner * places);
+      const uint32_t per_step = p.inner * places;
+      const bool idle = 256 / per_step * per_step < 192 && p.rows * p.depth * Traits<T>::kSize > (16ull << 20);
+      uint32_t per_block = (idle ? 512 : 256) / per_step;
       per_block = per_block < 1 ? 1 : per_block;
       while (per_block > 1 && (size_t)per_block * p.rotary * sizeof(float) > 32768) --per_block;
       const size_t lds = (size_t)per_block * p.rotary * sizeof(float);
