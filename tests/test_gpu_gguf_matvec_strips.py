@@ -51,6 +51,7 @@ def test_strips_edges(tag, x_tag):
 IN_PLACE = (
     (513, 256, 2, "4-tokens/16-waves/in-place/parked"),  # one run, three weight rows to a block
     (4099, 1280, 5, "8-tokens/16-waves/shared/in-place/parked"),
+    (2050, 5120, 4, "4-tokens/16-waves/shared/in-place/parked"),
     (4096, 256, 8, "8-tokens/16-waves/in-place/parked"),
     (66000, 256, 3, "4-tokens/2x8-waves/in-place/parked"),
     (66000, 256, 8, "8-tokens/2x8-waves/in-place/parked"),
