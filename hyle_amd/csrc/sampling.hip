@@ -356,7 +356,163 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
   }
 }
 
+// Rows of up to 256 elements, a few of them (what TopK leaves of a vocabulary): one wave per row does
+// the work of both dispatches above in one, with the same sums in the same order -- a lane's own first,
+// then the lanes of what would be each wave of a block (kWaves of them hold elements), then the waves --
+// so that every index and score is the one the two dispatches give.  The status word is written once, by
+// the launch's last block, which looks at all rows itself: rows cannot clear a word that others set.
+// Bound by latency.  MI355X, us, two dispatches / one: [5, 40] bf16 7.7 / 3.3, [64, 100] f32 7.7 / 3.5, [250, 64] bf16
+// 8.0 / 5.9.
+constexpr int kShortWidth = 256;             // TopK's select route serves as many
+constexpr int kShortWaves = 16;              // that share the status block's rows
+constexpr uint32_t kShortRows = 256;         // four turns of the status block
+
+template <class T, bool kVector, bool kScored>
+__global__ __launch_bounds__(kShortWaves *kWaveLanes) void categorical_short(const void *logits, const uint32_t *identities,
+                                                                            uint32_t rows, uint32_t width, int32_t *indices,
+                                                                            float *scores, uint32_t *status) {
+  constexpr float kInfinity = __builtin_huge_valf();
+  const uint32_t lane = threadIdx.x % kWaveLanes, wave = threadIdx.x / kWaveLanes;
+  if (blockIdx.x == gridDim.x - 1) {
+    // four rows of a wave at a time, sixteen loads of a lane in flight; a place past the row is its last one again
+    constexpr int kRows = 4, kPieces = kShortWidth / kWaveLanes;
+    bool refused = false;
+    for (uint32_t first = wave; first < rows; first += kShortWaves * kRows) {
+      float v[kRows][kPieces];
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) {
+        const uint32_t row = min(first + r * kShortWaves, rows - 1);
+        const unsigned char *base = static_cast<const unsigned char *>(logits) + (size_t)row * width * Traits<T>::kSize;
+#pragma unroll
+        for (int piece = 0; piece < kPieces; ++piece) v[r][piece] = Traits<T>::load(base, min(piece * kWaveLanes + lane, width - 1));
+      }
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) {
+        bool finite = false;
+#pragma unroll
+        for (int piece = 0; piece < kPieces; ++piece) {
+          refused = refused || invalid_weight(v[r][piece]);
+          finite = finite || v[r][piece] > -kInfinity;
+        }
+        refused = refused || __ballot(finite) == 0;
+      }
+    }
+    const int any = __syncthreads_or(refused ? 1 : 0);
+    if (threadIdx.x == 0) *status = any ? kStatusInvalidNumericInput : 0u;
+    return;
+  }
+  // one row to a block: sixteen on a compute unit wait for each other's 64-bit sums ([64, 100] f32 5.2 us, 3.5 like this)
+  if (wave != 0) return;  // no barrier below
+  const uint32_t row = blockIdx.x;
+  const void *base = static_cast<const unsigned char *>(logits) + (size_t)row * width * Traits<T>::kSize;
+  const uint32_t *identity = identities + (size_t)row * 4;
+  const uint32_t key0 = identity[0], key1 = identity[1], draw0 = identity[2], draw1 = identity[3];
+  // The tile's order: vector `lane`, or elements lane, 64 + lane, ...; and sixteen consecutive elements per
+  // lane for the scan.  Places past the row read as -inf.
+  constexpr int kVec = kVector ? Traits<T>::kVec : 1;
+  constexpr int kWaves = kVector ? 1 : kShortWidth / kWaveLanes;
+  float tile[kWaves][kVec], v[kPerThread];
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const uint32_t at = (w * kWaveLanes + lane) * kVec;  // width is a multiple of kVec
+    if constexpr (kVector) {
+      Traits<T>::unpack(load16(base, at < width ? at / kVec : 0), tile[w]);
+    } else {
+      tile[w][0] = Traits<T>::load(base, at < width ? at : 0);
+    }
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) tile[w][e] = at < width ? tile[w][e] : -kInfinity;
+  }
+#pragma unroll
+  for (int j = 0; j < kPerThread / kVec; ++j) {
+    const uint32_t at = lane * kPerThread + j * kVec;
+    float part[kVec];
+    if constexpr (kVector) {
+      Traits<T>::unpack(load16(base, at < width ? at / kVec : 0), part);
+    } else {
+      part[0] = Traits<T>::load(base, at < width ? at : 0);
+    }
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) v[j * kVec + e] = at < width ? part[e] : -kInfinity;
+  }
+  const PhiloxWords draw = philox_block(key0, key1, draw0, draw1, 0);
+  const double uniform = ((double)draw.x0 * 0x1p20 + (double)(draw.x1 >> 12) + 0.5) * 0x1p-52;
+  bool invalid = false;
+  float maximum = -kInfinity;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) {
+      invalid = invalid || invalid_weight(tile[w][e]);
+      maximum = fmaxf(maximum, tile[w][e]);
+    }
+  maximum = row_max<kWaveLanes>(maximum, nullptr);
+  if (__ballot(invalid) != 0 || !(maximum > -kInfinity)) return;
+  double total = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    double mass = 0;
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) mass += (double)exp_nonpositive(tile[w][e] - maximum);
+    total += wave_sum(mass);
+  }
+  // the row is one tile, whose scale is exp(0)
+  const double threshold = total * uniform;
+  if (!(total > threshold)) {
+    // rounding left the threshold at the total: the last element equal to the maximum
+    int last = 0;
+    for (uint32_t c = lane; c < width; c += kWaveLanes)
+      if (Traits<T>::load(base, c) == maximum) last = (int)c;
+#pragma unroll
+    for (int step = 1; step < kWaveLanes; step *= 2) last = max(last, __shfl_xor(last, step, kWaveLanes));
+    if (lane == 0) {
+      indices[row] = last;
+      if constexpr (kScored) scores[row] = -logf((float)total);
+    }
+    return;
+  }
+  float weights[kPerThread];
+  double mass = 0;
+#pragma unroll
+  for (int i = 0; i < kPerThread; ++i) {
+    weights[i] = exp_nonpositive(v[i] - maximum);
+    mass += (double)weights[i];
+  }
+  double through = mass;
+#pragma unroll
+  for (int step = 1; step < kShortWidth / kPerThread; step *= 2) {  // sixteen lanes hold the row
+    const double below = __shfl_up(through, step, kWaveLanes);
+    if (lane >= (uint32_t)step) through += below;
+  }
+  const double previous = __shfl_up(through, 1, kWaveLanes), before = lane == 0 ? 0 : previous;
+  const double all = __shfl(through, kShortWidth / kPerThread - 1, kWaveLanes);
+  const bool last_mass = !(all > threshold) && mass > 0 && through == all;
+  if (lane < kShortWidth / kPerThread && ((!(before > threshold) && through > threshold) || last_mass)) {
+    double running = before;
+    int selected = -1, last_positive = -1;
+#pragma unroll
+    for (int i = 0; i < kPerThread; ++i) {
+      running += (double)weights[i];
+      if (weights[i] > 0) last_positive = i;
+      if (selected < 0 && running > threshold) selected = i;
+    }
+    if (selected < 0) selected = last_positive;
+    float chosen = v[0];
+#pragma unroll
+    for (int i = 1; i < kPerThread; ++i) chosen = selected == i ? v[i] : chosen;
+    indices[row] = (int32_t)(lane * kPerThread + selected);
+    if constexpr (kScored) {
+      const float total32 = (float)total;
+      const double log_total = (double)logf(total32) + (total - (double)total32) / (double)total32;
+      scores[row] = (float)((double)chosen - (double)maximum - log_total);
+    }
+  }
+}
+
 // Launch-shape labels
+template <bool kVector, bool kScored> struct CategoricalShortTag {
+  static std::string text() { return std::string("categorical_short/") + (kVector ? "vector" : "scalar") + (kScored ? "/scored" : ""); }
+};
 template <bool kVector> struct CategoricalTilesTag {
   static std::string text() { return std::string("categorical_tiles/") + (kVector ? "vector" : "scalar"); }
 };
@@ -367,11 +523,29 @@ template <int kForm> struct RandomBitsTag {  // 0 rows of blocks, 1 flat
   static std::string text() { return kForm == 0 ? "random_bits_rows" : "random_bits"; }
 };
 
+// One wave per row while the status block's walk over all rows stays as short as a row's own chain.
+bool short_rows(const CategoricalParams &p) {
+  return p.width <= (uint32_t)kShortWidth && p.rows <= kShortRows;
+}
+
 template <class T, bool kVector>
 hipError_t run_categorical(const CategoricalParams &p, const void *logits, const uint32_t *identities, int32_t *indices,
                            float *scores, void *workspace, hipStream_t stream) {
   CategoricalTile *parts = static_cast<CategoricalTile *>(workspace);
   uint32_t *status = reinterpret_cast<uint32_t *>(static_cast<unsigned char *>(workspace) + p.status_offset);
+  if (short_rows(p)) {
+    const dim3 grid(p.rows + 1), waves(kShortWaves * kWaveLanes);
+    if (p.scored) {
+      note_variant<CategoricalShortTag<kVector, true>>();
+      hipLaunchKernelGGL((categorical_short<T, kVector, true>), grid, waves, 0, stream, logits, identities, p.rows, p.width,
+                         indices, scores, status);
+    } else {
+      note_variant<CategoricalShortTag<kVector, false>>();
+      hipLaunchKernelGGL((categorical_short<T, kVector, false>), grid, waves, 0, stream, logits, identities, p.rows, p.width,
+                         indices, scores, status);
+    }
+    return hipGetLastError();
+  }
   const dim3 block(kBlockThreads);
   note_variant<CategoricalTilesTag<kVector>>();
   hipLaunchKernelGGL((categorical_tiles<T, kVector>), dim3(p.rows * p.tiles), block, 0, stream, logits, p.width, p.tiles, parts,

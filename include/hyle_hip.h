@@ -304,7 +304,8 @@ HYLE_HIP_API hyle_hip_status hyle_hip_plan_outputs(const hyle_hip_plan *plan,
 HYLE_HIP_API int hyle_hip_plan_alias_support(const hyle_hip_plan *plan, uint32_t output_index,
                                              uint32_t input_index);
 /* ProviderRouteCostFacts::dispatch_count
- * (include/hyle/compute/prepared_operation.h:51-67): kernels one launch enqueues. */
+ * (include/hyle/compute/prepared_operation.h:51-67): kernels one launch enqueues (of a Categorical: at
+ * most, since a few short rows take one). */
 HYLE_HIP_API uint32_t hyle_hip_plan_dispatch_count(const hyle_hip_plan *plan);
 /* Name of the kernel route the plan selected (diagnostics, profiling). */
 HYLE_HIP_API const char *hyle_hip_plan_route_name(const hyle_hip_plan *plan);

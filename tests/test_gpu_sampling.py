@@ -145,6 +145,42 @@ def test_categorical_is_the_oracles_inverse_cdf(type_id, rows, width):
     assert check_against_float64(values, ids, picked, scores, oracle_picked) > 0.9   # rows pinned to the oracle's index
 
 
+@pytest.mark.parametrize("type_id", [orc.F32, orc.F16, orc.BF16])
+def test_categorical_of_short_rows_is_the_draw_of_long_rows(type_id):
+    """Up to 256 rows of up to 256 elements take one dispatch: the oracle's inverse CDF, and bit for bit what the two
+    dispatches give for the same rows (the same rows in front of enough others)."""
+    rng = np.random.default_rng(31 + type_id)
+    for rows, width in ((1, 1), (2, 20), (5, 40), (17, 63), (64, 64), (63, 65), (26, 100), (65, 129), (256, 250), (3, 255), (256, 256)):
+        values = rng.normal(0, 4, (rows, width)).astype(np.float32)
+        values[:, 1:][rng.random((rows, width - 1)) < 0.2] = -np.inf
+        stored = values if type_id == orc.F32 else orc.from_f32(type_id, values)
+        values = values if type_id == orc.F32 else orc.to_f32(type_id, stored)
+        ids = rng.integers(0, 1 << 32, (rows, 4), dtype=np.uint64).astype(np.uint32)
+        many = np.concatenate([stored] * (257 // rows + 1))
+        many_ids = np.concatenate([ids] * (257 // rows + 1))
+        for scored in (True, False):
+            note(f"categorical short type {type_id} rows {rows} width {width} scored {scored}")
+            status, picked, scores = categorical_on_device(type_id, stored, ids, scored)
+            assert status == 0 and hc.last_launch_variant().startswith("categorical_short/")
+            status, long_picked, long_scores = categorical_on_device(type_id, many, many_ids, scored)
+            assert status == 0 and "categorical_tiles" in hc.last_launch_variant()
+            assert np.array_equal(picked, long_picked[:rows])
+            if scored:
+                assert np.array_equal(scores.view(np.uint32), long_scores[:rows].view(np.uint32))
+                check_against_float64(values, ids, picked, scores, orc.categorical(type_id, stored, ids)[1])
+
+
+def test_categorical_short_rows_refuse_what_long_rows_refuse():
+    for rows, width, at in ((1, 1, (0, 0)), (64, 100, (63, 99)), (256, 256, (255, 255)), (70, 65, (64, 64))):
+        for invalid in (np.nan, np.inf, -np.inf):
+            note(f"categorical short refusal {invalid} rows {rows} width {width}")
+            values = np.zeros((rows, width), np.float32)
+            values[at[0], at[1] if invalid != -np.inf else slice(None)] = invalid
+            status, picked, _ = categorical_on_device(orc.F32, values, fixture_identities(rows, 3), False)
+            assert status == capi.INVALID_ARGUMENT and picked[at[0]] == -7
+            assert ((picked >= 0) | (np.arange(rows) == at[0])).all()
+
+
 def test_categorical_one_positive_mass_in_a_full_vocabulary():
     width = 248320
     for rows in (1, 16):
