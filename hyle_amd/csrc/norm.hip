@@ -146,6 +146,9 @@ hipError_t launch_norm(Elem type, const NormParams &p, const void *x, const void
     const bool launched = p.layer ? launch_norm_exact_layer(type, p, x, w, b, y, stream)
                                   : launch_norm_exact_rms(type, p, x, w, y, stream);
     if (launched) return hipGetLastError();
+    const bool tail = p.layer ? launch_norm_tail_layer(type, p, x, w, b, y, stream)
+                              : launch_norm_tail_rms(type, p, x, w, y, stream);
+    if (tail) return hipGetLastError();
   }
   const Bound io{x, w, b, y};
   return p.layer ? run_typed<true>(type, p, io, vectorised, stream)

@@ -28,6 +28,11 @@ __device__ __forceinline__ void load_weight(const void *w, uint32_t vec, float (
   }
 }
 
+template <int kVec> __device__ __forceinline__ float tree_sum(const float (&v)[kVec]) {
+  if constexpr (kVec == 8) return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  else return (v[0] + v[1]) + (v[2] + v[3]);
+}
+
 enum : int { kPlain = 0, kScale = 1, kScaleBias = 2 };  // learned parameters of a launch
 
 // `kRows` consecutive rows share one group of lanes.  Loads carry no branches (a lane outside
@@ -43,27 +48,26 @@ enum : int { kPlain = 0, kScale = 1, kScaleBias = 2 };  // learned parameters of
 // sixteen.  One such instruction per element is 0.44 us of every SIMD's time for 16.7 M
 // elements, which the loads do not hide once all waves of a launch are resident together and
 // move through their phases side by side.
-template <class T, class W, int kLanes, int kVpl, int kThreads, int kRows, bool kLayer, int kParameters, bool kExact>
-__global__ __launch_bounds__(kThreads) void norm_rows(const void *x, const void *w, const void *b,
-                                                      void *y, uint32_t rows, uint32_t row_vectors,
-                                                      float width, float epsilon) {
+// `kTail` launches (norm_tail.h) cover their rows, and only the last vector of a lane is masked.
+template <class T, class W, int kLanes, int kVpl, int kThreads, int kRows, bool kLayer, int kParameters, bool kExact,
+          bool kTail>
+__device__ __forceinline__ void norm_group(const void *x, const void *w, const void *b, void *y, uint32_t first_row, uint32_t rows,
+                                           uint32_t row_vectors, float width, float epsilon) {
   constexpr int parameters = kParameters;
   constexpr int kVec = Traits<T>::kVec;
-  constexpr int kGroupsPerBlock = kThreads / kLanes;
   __shared__ float joint[kLayer ? 2 : 1][kRows][kThreads / kWaveLanes];
   const uint32_t lane = threadIdx.x % kLanes;
-  const uint32_t first_row = (blockIdx.x * kGroupsPerBlock + threadIdx.x / kLanes) * kRows;
 
   u32x4 raw[kRows][kVpl];
   uint32_t vec[kVpl];
 #pragma unroll
   for (int k = 0; k < kVpl; ++k) {
     const uint32_t wanted = lane + k * kLanes;
-    vec[k] = kExact || wanted < row_vectors ? wanted : row_vectors - 1;
+    vec[k] = kExact || (kTail && k < kVpl - 1) || wanted < row_vectors ? wanted : row_vectors - 1;
   }
 #pragma unroll
   for (int r = 0; r < kRows; ++r) {
-    const uint32_t row = kExact || first_row + r < rows ? first_row + r : rows - 1;
+    const uint32_t row = kExact || kTail || first_row + r < rows ? first_row + r : rows - 1;
     const size_t row_base = (size_t)row * row_vectors;
 #pragma unroll
     for (int k = 0; k < kVpl; ++k) raw[r][k] = load16_stream(x, row_base + vec[k]);
@@ -88,29 +92,40 @@ __global__ __launch_bounds__(kThreads) void norm_rows(const void *x, const void 
     bool ok[kVpl];
 #pragma unroll
     for (int k = 0; k < kVpl; ++k) {
-      ok[k] = kExact || (first_row + r < rows && lane + k * kLanes < row_vectors);
+      ok[k] = kExact || (kTail && k < kVpl - 1) || ((kTail || first_row + r < rows) && lane + k * kLanes < row_vectors);
       Traits<T>::unpack(raw[r][k], v[r][k]);
     }
     if constexpr (kLayer) {
       float sum = 0.0f;
+      if constexpr (kTail) {  // a sum per element of a vector: shorter chains, and fewer roundings in each
+        float sums[kVec] = {};
 #pragma unroll
-      for (int k = 0; k < kVpl; ++k)
+        for (int k = 0; k < kVpl; ++k)
 #pragma unroll
-        for (int j = 0; j < kVec; ++j) sum += ok[k] ? v[r][k][j] : 0.0f;
+          for (int j = 0; j < kVec; ++j) sums[j] += ok[k] ? v[r][k][j] : 0.0f;
+        sum = tree_sum(sums);
+      } else {
+#pragma unroll
+        for (int k = 0; k < kVpl; ++k)
+#pragma unroll
+          for (int j = 0; j < kVec; ++j) sum += ok[k] ? v[r][k][j] : 0.0f;
+      }
       const float mean = row_sum<kLanes>(sum, joint[1][r]) / width;
 #pragma unroll
       for (int k = 0; k < kVpl; ++k)
 #pragma unroll
         for (int j = 0; j < kVec; ++j) v[r][k][j] -= mean;
     }
-    float squares = 0.0f;
+    float squares = 0.0f, parts[kVec] = {};
 #pragma unroll
     for (int k = 0; k < kVpl; ++k)
 #pragma unroll
       for (int j = 0; j < kVec; ++j) {
         v[r][k][j] = ok[k] ? v[r][k][j] : 0.0f;
-        squares = __builtin_fmaf(v[r][k][j], v[r][k][j], squares);
+        float &sum = kTail ? parts[j] : squares;
+        sum = __builtin_fmaf(v[r][k][j], v[r][k][j], sum);
       }
+    if constexpr (kTail) squares = tree_sum(parts);
     squares = row_sum<kLanes>(squares, joint[0][r]);
     inverse[r] = 1.0f / sqrtf(squares / width + epsilon);
   }
@@ -120,7 +135,7 @@ __global__ __launch_bounds__(kThreads) void norm_rows(const void *x, const void 
     const size_t row_base = (size_t)row * row_vectors;
 #pragma unroll
     for (int k = 0; k < kVpl; ++k) {
-      if (kExact || (row < rows && lane + k * kLanes < row_vectors)) {
+      if (kExact || (kTail && k < kVpl - 1) || ((kTail || row < rows) && lane + k * kLanes < row_vectors)) {
         float out[kVec];
 #pragma unroll
         for (int j = 0; j < kVec; ++j) {
@@ -132,6 +147,27 @@ __global__ __launch_bounds__(kThreads) void norm_rows(const void *x, const void 
       }
     }
   }
+}
+
+template <class T, class W, int kLanes, int kVpl, int kThreads, int kRows, bool kLayer, int kParameters, bool kExact, bool kTail = false>
+__global__ __launch_bounds__(kThreads) void norm_rows(const void *x, const void *w, const void *b,
+                                                      void *y, uint32_t rows, uint32_t row_vectors,
+                                                      float width, float epsilon) {
+  constexpr int kGroupsPerBlock = kThreads / kLanes;
+  uint32_t group = blockIdx.x * kGroupsPerBlock + threadIdx.x / kLanes;
+  if constexpr (kTail) {
+    static_assert(!kExact && kLanes == kWaveLanes, "a wave goes its own way: no barrier follows");
+    group = __builtin_amdgcn_readfirstlane(group);
+    const uint32_t first_row = group * kRows;
+    if (first_row >= rows) return;
+    if (kRows > 1 && first_row + kRows > rows) {  // the last rows one by one
+      for (uint32_t row = first_row; row < rows; ++row)
+        norm_group<T, W, kLanes, kVpl, kThreads, 1, kLayer, kParameters, false, true>(x, w, b, y, row, rows, row_vectors, width, epsilon);
+      return;
+    }
+  }
+  norm_group<T, W, kLanes, kVpl, kThreads, kRows, kLayer, kParameters, kExact, kTail>(x, w, b, y, group * kRows, rows, row_vectors,
+                                                                                      width, epsilon);
 }
 
 struct Bound {
@@ -177,5 +213,9 @@ bool run_exact(const NormParams &p, const Bound &io, int parameters, hipStream_t
 bool launch_norm_exact_rms(Elem type, const NormParams &p, const void *x, const void *w, void *y, hipStream_t stream);
 bool launch_norm_exact_layer(Elem type, const NormParams &p, const void *x, const void *w, const void *b, void *y,
                              hipStream_t stream);
+// Rows of 65 to 768 vectors (norm_tail.h).  False: nothing was launched.
+bool launch_norm_tail_rms(Elem type, const NormParams &p, const void *x, const void *w, void *y, hipStream_t stream);
+bool launch_norm_tail_layer(Elem type, const NormParams &p, const void *x, const void *w, const void *b, void *y,
+                            hipStream_t stream);
 
 }  // namespace hyle_hip

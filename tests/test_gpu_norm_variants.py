@@ -169,6 +169,18 @@ CASES = [
     ("layer", "bf16", 4, 16384, "norm_rows_exact/layer/256x8/256/2"),
 ]
 
+# One wave per row (norm_tail.h): widths on both sides of a lane's last vector, few rows, and for two rows per wave an
+# odd number of them in 20 to 64 MB.
+for _k in range(2, 13):
+    for _operator in ("layer", "rms"):
+        _shape = f"norm_rows_tail/{_operator}/64x{_k}/" + ("256/1" if _k == 2 else "64/1")
+        CASES += [(_operator, "f32", 17, 256 * (_k - 1) + 4, _shape), (_operator, "bf16", 19, 512 * _k - 8, _shape)]
+        if _k > 2 and (_operator, _k) != ("rms", 4):
+            CASES.append((_operator, "f32", (21 << 18) // (256 * _k - 4) | 1, 256 * _k - 4, f"norm_rows_tail/{_operator}/64x{_k}/64/2"))
+CASES += [("rms", "f32", 1, 1024, "norm_rows_tail/rms/64x4/64/1"), ("layer", "bf16", 1, 1032, "norm_rows_tail/layer/64x3/64/1"),
+          ("layer", "bf16", 5, 1536, "norm_rows_tail/layer/64x3/64/1"), ("rms", "bf16", 4097, 2568, "norm_rows_tail/rms/64x6/64/2"),
+          ("rms", "bf16", 4001, 5640, "norm_rows_tail/rms/64x12/64/2")]
+
 reached = set()
 
 
