@@ -353,9 +353,13 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_lines(const unsi
 // tail_lanes: how many lanes of the last span's wave have a block of the row (64 unless the row is
 // a Q8_0 row whose width is a multiple of 256 but not of 2048: a lane is a block of 32 values
 // there, and the last span then holds 8, 16, ... 56 blocks in 17, 34, ... 119 whole vectors).
-template <int kKind, class TX, int kSpans, bool kShort>
+//
+// A block's rows follow one another in memory.  kStream: non-temporal loads, for weights that outgrow the memory-side
+// cache; below, plain ones, by which the line that two rows or two spans share is fetched once.
+template <int kKind, class TX, int kSpans, bool kShort, bool kStream>
 __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(const unsigned char *weights, const void *x, void *y,
-                                                                          uint32_t rows, uint64_t row_stride, uint32_t tail_lanes) {
+                                                                          uint32_t all_rows, uint32_t block_rows, uint64_t row_stride,
+                                                                          uint32_t tail_lanes) {
   static_assert(!kShort || kKind == 2, "only Q8_0 rows have short last spans");
   using Row = LinesRow<kKind, 1>;
   using Kind = Lines<kKind>;
@@ -366,7 +370,7 @@ __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(cons
   const uint32_t span = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveLanes);
   unsigned char *slot = slots[span];
   const typename Kind::Lane at = Kind::lane_of(0, lane);
-  const uint32_t stride = gridDim.x, first = blockIdx.x;  // first < rows: the grid has at most `rows` blocks
+  const uint32_t first = blockIdx.x * block_rows, rows = min(first + block_rows, all_rows);  // first < all_rows
   const unsigned char *mine = weights + (size_t)span * kSpanBytes;
   // (whole spans: constants, and the compiler drops what depends on them)
   const uint32_t live_lanes = kShort && span == (uint32_t)kSpans - 1 ? tail_lanes : (uint32_t)kWaveLanes;
@@ -375,21 +379,21 @@ __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(cons
   Row ring[kLinesDepth];
 #pragma unroll
   for (int d = 0; d < kLinesDepth; ++d) {
-    const uint64_t wanted = (uint64_t)first + (uint64_t)d * stride;
-    ring[d] = Row::load(mine + (size_t)(wanted < rows ? (uint32_t)wanted : first) * row_stride, lane, vectors);
+    const uint32_t wanted = first + d;
+    ring[d] = Row::template load<kStream>(mine + (size_t)(wanted < rows ? wanted : first) * row_stride, lane, vectors);
   }
   const LaneCodes held = quantise_span<kKind, TX>(x, 0, span, lane, live);  // while the first rows are on their way
-  for (uint64_t base = first; base < rows; base += (uint64_t)kLinesDepth * stride) {
+  for (uint32_t base = first; base < rows; base += kLinesDepth) {
     float totals[kLinesDepth] = {};
 #pragma unroll
     for (int d = 0; d < kLinesDepth; ++d) {
-      const uint64_t row = base + (uint64_t)d * stride;
+      const uint32_t row = base + d;
       if (row >= rows) break;
 #pragma unroll
       for (int i = 0; i < Row::kLoads; ++i)
         *reinterpret_cast<u32x4 *>(slot + (size_t)(lane + i * kWaveLanes) * 16) = ring[d].v[i];
-      const uint64_t wanted = row + (uint64_t)kLinesDepth * stride;
-      ring[d] = Row::load(mine + (size_t)(wanted < rows ? (uint32_t)wanted : first) * row_stride, lane, vectors);
+      const uint32_t wanted = row + kLinesDepth;
+      ring[d] = Row::template load<kStream>(mine + (size_t)(wanted < rows ? wanted : first) * row_stride, lane, vectors);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -403,12 +407,12 @@ __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(cons
     static_assert(kLinesDepth == 4, "the joint sum is taken over four rows");
     const float share = joint_sum<kLinesDepth>(totals, lane);  // lane l < 4: row l over the wave
     if constexpr (kSpans == 1) {
-      const uint64_t row = base + (uint64_t)lane * stride;
+      const uint32_t row = base + lane;
       if (lane < (uint32_t)kLinesDepth && row < rows) Traits<TX>::store(y, (size_t)row, share);
     } else {
       if (lane < (uint32_t)kLinesDepth) shares[span][lane] = share;
       __syncthreads();
-      const uint64_t row = base + (uint64_t)lane * stride;
+      const uint32_t row = base + lane;
       if (span == 0 && lane < (uint32_t)kLinesDepth && row < rows) {
         float whole = shares[0][lane];
 #pragma unroll
@@ -1360,18 +1364,34 @@ hipError_t run_registers(const MatVecParams &p, const void *w, const void *x, vo
 // One activation row: a wave per span.  Eight waves per compute unit measured best or equal in
 // 25 of 27 shapes (three formats, K = 2048 ... 12288, 1024 ... 151936 rows: 0-30 % below the
 // kernel that parks the codes in LDS first).
+//
+// A block takes neighbouring rows.  MI355X, bf16, us, rows dealt out one by one with non-temporal loads / neighbouring
+// rows, non-temporal / plain:
+//   Q6_K [6144 -> 2048] 5.9 / 5.6 / 5.2   [4096 -> 8192] 8.7 / 8.4 / 7.9   [2048 -> 2048] 4.7 / 4.7 / 4.2
+//   Q8_0 [5120 -> 17408] (95 MB) 18.0 / 17.9 / 16.8   [17408 -> 5120] 18.9 / 18.4 / 17.6   [7168 -> 3072] 7.8 / 7.5 / 6.8
+//   Q6_K [2048 -> 151936] (255 MB) 47.8 / 46.2 / 51.0   Q8_0 [2048 -> 100000] (218 MB) 36.5 / 36.3 / 42.2   [2560 -> 77056]
+//   (210 MB) 38.2 / 37.7 / 40.1
+// (16 waves per compute unit with plain loads: 5.6, 8.5, 4.2, 17.8, 17.6, 7.2, 52, 43, 41)
+constexpr uint64_t kSpansStream = 128ull << 20;
+
 template <int kKind, class TX>
 hipError_t run_spans(const MatVecParams &p, const void *w, const void *x, void *y, uint32_t spans, uint32_t tail_lanes,
                      int compute_units, hipStream_t s) {
   const uint32_t units = (uint32_t)(compute_units > 0 ? compute_units : 256);
   const uint32_t most = units * (spans <= 8 ? 8u / spans : 1u);
-  const dim3 blocks((uint32_t)p.rows < most ? (uint32_t)p.rows : most);
+  const uint32_t block_rows = ((uint32_t)p.rows + most - 1) / most;
+  const dim3 blocks(((uint32_t)p.rows + block_rows - 1) / block_rows);
   const unsigned char *in = static_cast<const unsigned char *>(w);
   const uint32_t rows = (uint32_t)p.rows;
-#define HYLE_SPANS(N, SHORT)                                                                                             \
-  note_variant<SpansTag<kKind, N, SHORT>>();                                                                             \
-  hipLaunchKernelGGL((gguf_matvec_q8_spans<kKind, TX, N, SHORT>), blocks, dim3(N * kWaveLanes), 0, s, in, x, y, rows,      \
-                     p.row_stride, tail_lanes)
+  const bool stream = p.rows * p.row_stride > kSpansStream;
+#define HYLE_SPANS(N, SHORT)                                                                                                       \
+  note_variant<SpansTag<kKind, N, SHORT>>();                                                                                       \
+  if (stream)                                                                                                                      \
+    hipLaunchKernelGGL((gguf_matvec_q8_spans<kKind, TX, N, SHORT, true>), blocks, dim3(N * kWaveLanes), 0, s, in, x, y, rows,       \
+                       block_rows, p.row_stride, tail_lanes);                                                                      \
+  else                                                                                                                             \
+    hipLaunchKernelGGL((gguf_matvec_q8_spans<kKind, TX, N, SHORT, false>), blocks, dim3(N * kWaveLanes), 0, s, in, x, y, rows,      \
+                       block_rows, p.row_stride, tail_lanes)
   if (tail_lanes == kWaveLanes) {
     switch (spans) {
       case 1: HYLE_SPANS(1, false); break;

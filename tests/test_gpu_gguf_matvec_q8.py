@@ -327,3 +327,16 @@ def test_q8_route_q4_k_matrix_unit_seeded_random_shapes():
         strips = rows >= 512 and (m > 1 or k >= 10240 or (k > 2048 and k % 2048 != 0))   # several rows or wide ones against many
         kernel = f"gguf_matvec_q8_strips/q4_k/{4 if m <= 4 else 8}-tokens" if strips else f"gguf_matvec_q8_tiles/q4_k/{tokens}-tokens"
         check("q4_k", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad, kernel=kernel)
+
+
+@pytest.mark.parametrize("tag,rows,k,kernel", [("q6_k", 10247, 2048, "1-spans"), ("q6_k", 8195, 4096, "2-spans"), ("q8_0", 8221, 2048, "1-spans"),
+                                               ("q8_0", 8193, 3328, "2-spans/short")])
+def test_q8_route_one_row_against_more_than_128_mb(tag, rows, k, kernel):
+    """Blocks of several neighbouring rows, the last one short, loaded past the caches; the stride is what makes it large."""
+    rng = np.random.default_rng(1811)
+    raw = weights_for(tag, rng, rows, k)
+    stride = 16400
+    padded = np.zeros((rows, stride), np.uint8)
+    padded[:, :raw.shape[1]] = raw
+    note(f"q8 matvec {tag} rows {rows} k {k}: {rows * stride >> 20} MB")
+    check(tag, "bf16", padded, rows, k, rng.normal(0, 1.5, (k,)).astype(np.float32), row_stride=stride, kernel=f"gguf_matvec_q8_spans/{tag}/{kernel}")
