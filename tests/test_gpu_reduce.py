@@ -279,3 +279,24 @@ def test_reduce_with_every_number_of_loads_a_lane(tag):
                 label = "reduce_columns/vector/2"
             assert hc.last_launch_variant().startswith(label), (dims, hc.last_launch_variant())
             check(kind, tag, to_host(out), x, dims, [axis])
+
+
+@pytest.mark.parametrize("dims,axis,label", [([37, 260], 1, "reduce_rows/wave/vector"), ([5, 4100], 1, "reduce_rows/block/vector"),
+                                             ([3, 300000], 1, "reduce_rows/block/vector"), ([300, 96], 0, "reduce_columns/vector"),
+                                             ([9000, 64], 0, "reduce_columns/vector")])
+def test_reduce_extrema_keep_the_bits_of_a_nan_and_tell_the_zeros_apart(dims, axis, label):
+    rng = np.random.default_rng(991)
+    for kind, side in ((RK.kMaximum, -1.0), (RK.kMinimum, 1.0)):
+        x = (side * np.abs(rng.normal(1, 0.2, dims))).astype(np.float32)
+        lanes = x if axis == 1 else x.T
+        lanes[0, ::7] = -0.0                    # zeros of both signs are the extremum: +0 of a maximum, -0 of a minimum
+        lanes[0, 3::7] = 0.0
+        bits = lanes.view(np.uint32) if axis == 1 else x.view(np.uint32).T
+        bits[2, 17] = 0x7FA00123                # a signalling NaN
+        bits[1, lanes.shape[1] - 1] = 0xFFC00007
+        note(f"reduce {kind.name} {dims} over axis {axis} with NaNs and zeros")
+        (out,) = run(hc.Reduce(kind, hc.Axes.from_([axis]), accumulation_type=F32ACC), to_device(x, "f32"))
+        assert hc.last_launch_variant().startswith(label)
+        got = to_host(out).view(np.uint32)
+        assert got[0] == (0 if kind == RK.kMaximum else 0x80000000) and got[2] == 0x7FA00123 and got[1] == 0xFFC00007
+        check(kind, "f32", to_host(out), x, dims, [axis])
