@@ -170,6 +170,22 @@ def test_categorical_of_short_rows_is_the_draw_of_long_rows(type_id):
                 check_against_float64(values, ids, picked, scores, orc.categorical(type_id, stored, ids)[1])
 
 
+@pytest.mark.parametrize("type_id,rows,width", [(orc.F32, 2, 300001), (orc.F32, 3, 262148), (orc.BF16, 2, 262145), (orc.F32, 2, 262144),
+                                                (orc.F16, 5, 257), (orc.BF16, 300, 4097)])
+def test_categorical_on_both_sides_of_64_tiles(type_id, rows, width):
+    rng = np.random.default_rng(width)
+    values = rng.normal(0, 3, (rows, width)).astype(np.float32)
+    values[0, :min(4096, width - 1)] = -np.inf                                                    # a tile without mass in front
+    stored = values if type_id == orc.F32 else orc.from_f32(type_id, values)
+    values = values if type_id == orc.F32 else orc.to_f32(type_id, stored)
+    ids = rng.integers(0, 1 << 32, (rows, 4), dtype=np.uint64).astype(np.uint32)
+    for scored in (True, False):
+        note(f"categorical tiles type {type_id} rows {rows} width {width} scored {scored}")
+        status, picked, scores = categorical_on_device(type_id, stored, ids, scored)
+        assert status == 0 and hc.last_launch_variant().endswith("/many-tiles") == (width > 262144)
+        check_against_float64(values, ids, picked, scores, orc.categorical(type_id, stored, ids)[1])
+
+
 def test_categorical_short_rows_refuse_what_long_rows_refuse():
     for rows, width, at in ((1, 1, (0, 0)), (64, 100, (63, 99)), (256, 256, (255, 255)), (70, 65, (64, 64))):
         for invalid in (np.nan, np.inf, -np.inf):
