@@ -239,6 +239,26 @@ def test_few_checked_indices_take_one_dispatch():
         assert status == capi.OUT_OF_RANGE and (got.view(np.uint8) == 0x33).all()
 
 
+def test_up_to_1536_checked_rows_of_whole_units_take_one_dispatch():
+    """Also where the source lies off a 16-byte boundary, so that the units are narrower than the plan took them for."""
+    rows = 700
+    for count, width, lead in ((1536, 1280, 0), (1037, 2560, 0), (1037, 264, 2), (900, 2048, 4), (1025, 8, 0)):
+        values = np.random.default_rng(count).integers(0, 1 << 16, (rows, width), dtype=np.uint64).astype(np.uint16)
+        storage = np.concatenate([np.zeros(lead, np.uint8), values.view(np.uint8).reshape(-1)])
+        plan = hc.prepare(context(), hc.Gather(0), hc.TensorDesc.dense(DT.kFloat16, [rows, width]), hc.TensorDesc.dense(DT.kInt32, [count]))
+        assert plan.dispatch_count() == 1
+        ids = np.random.default_rng(width).integers(0, rows, count).astype(np.int32)
+        note(f"gather {count} checked rows of {2 * width} bytes, {lead} off a boundary, one dispatch")
+        status, got = gather_on_device(DT.kFloat16, 2, storage, lead, [rows, width], None, True, 0, ids, 0, [count], None, True, False)
+        assert status == 0 and np.array_equal(got, values[ids])
+        for place, value in ((0, -1), (count - 1, rows)):
+            bad = ids.copy()
+            bad[place] = value
+            status, got = gather_on_device(DT.kFloat16, 2, storage, lead, [rows, width], None, True, 0, bad, 0, [count], None, True, False,
+                                           poison=0x77)
+            assert status == capi.OUT_OF_RANGE and (got.view(np.uint8) == 0x77).all()
+
+
 def test_many_long_checked_rows_check_themselves_while_they_load():
     """A launch large enough for the blocks of sixteen chunks takes one dispatch up to 16384 indices: valid
     indices move every row, one bad index (negative, past the axis, first or last) moves none; both index
