@@ -830,13 +830,15 @@ void select_tiles_launch(const TopKParams &p, const Addressing &a, const char *i
   note_variant<SelectTag<kE, VEC, BYTES, FINAL>>();                                                         \
   hipLaunchKernelGGL((topk_select<T, kE, VEC, BYTES, FINAL>), grid, block, 0, s, in, values, indices, lists, a, \
                      p.tiles, largest)
-  // tiles of 2048 elements are chosen only for rows that one of them covers (topk_plan): no lists there
-  if (vector) {
-    if (final) { HYLE_SELECT(true, false, true); }
-    else if constexpr (kE != 8) { HYLE_SELECT(true, false, false); }
-  } else {
-    if (final) { HYLE_SELECT(false, kBytewise, true); }
-    else if constexpr (kE != 8) { HYLE_SELECT(false, kBytewise, false); }
+  // tiles of 2048 elements are chosen only for rows that one of them covers (topk_plan): no lists there; tiles of
+  // 4096 only for rows of three or more
+  if constexpr (kE != 16) {
+    if (final && vector) { HYLE_SELECT(true, false, true); }
+    else if (final) { HYLE_SELECT(false, kBytewise, true); }
+  }
+  if constexpr (kE != 8) {
+    if (!final && vector) { HYLE_SELECT(true, false, false); }
+    else if (!final) { HYLE_SELECT(false, kBytewise, false); }
   }
 #undef HYLE_SELECT
 }
@@ -889,6 +891,8 @@ hipError_t run(const TopKParams &p, const void *x, void *values, int32_t *indice
   if (p.select) {
     if (p.tile_elements == kBlockThreads * 32)
       select_tiles_launch<T, 32, kBytewise>(p, a, in, values, indices, lists_a, vector, s);
+    else if (p.tile_elements == kBlockThreads * 16)
+      select_tiles_launch<T, 16, kBytewise>(p, a, in, values, indices, lists_a, vector, s);
     else
       select_tiles_launch<T, 8, kBytewise>(p, a, in, values, indices, lists_a, vector, s);
     uint32_t lists = p.tiles;
@@ -977,13 +981,25 @@ hipError_t run(const TopKParams &p, const void *x, void *values, int32_t *indice
 
 uint32_t topk_max_count() { return kTile / 2; }  // above it: sorted runs merged in pairs
 
+// Tiles of 4096 elements: twice the blocks, and half the comparisons of each, where tiles of 8192 leave the chip idle.  The
+// ranking dispatch then has twice the lists: not with more than 32, of which it has two samples each, nor for counts
+// above 64, whose bound four waves with half the elements find less sharply.  MI355X, us, tiles of 8192 / 4096:
+//   bf16 [3, 50001] 64 best 12.3 / 11.1, [2, 77255] 20 10.1 / 9.1, f16 [7, 62798] 40 11.8 / 10.5, f32 [1, 128000] 64 11.5 / 10.8,
+//   [16, 120000] 40 11.7 / 11.3, [64, 62800] 20 11.7 / 11.4; but f32 [3, 151936] 20 9.4 / 12.1, bf16 [1, 151936] 64 12.1 / 22.9,
+//   [60, 32000] 100 16.4 / 18.0, [30, 130000] 100 17.1 / 19.5
+bool few_select_blocks(const TopKParams &p) {
+  const uint64_t tiles = (p.width + kBlockThreads * 16 - 1) / (kBlockThreads * 16);
+  return p.width > kBlockThreads * 32 && tiles <= 32 && p.rows * tiles <= 1024 && p.count <= kWaveLanes;
+}
+
 void topk_plan(TopKParams *p) {
   p->select = p->count <= kSelectMax;
   if (p->select) {
-    // 8192-element tiles for long rows (32 elements per thread: the per-block work of finding the
+    // 8192-element tiles for long rows (4096 in a small launch; 32 elements per thread: the per-block work of finding the
     // bound is paid once per tile), 2048 otherwise; merges take as many
     // lists as 4096 keys hold (2048 when that already covers every tile of a row): 32 KiB of LDS.
     p->tile_elements = p->width > kTile ? kBlockThreads * 32 : kBlockThreads * 8;
+    if (few_select_blocks(*p)) p->tile_elements = kBlockThreads * 16;
     p->tiles = (p->width + p->tile_elements - 1) / p->tile_elements;
     p->fan = (p->tiles * p->count <= kBlockThreads * 8 ? kBlockThreads * 8 : kBlockThreads * 16) / p->count;
   } else {

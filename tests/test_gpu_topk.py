@@ -251,3 +251,38 @@ def test_topk_rows_at_odd_addresses_on_every_route(tag):
         note(f"topk {tag} {dims} rows {row_bytes} bytes apart, count {count}")
         outputs = run(hc.TopK(count=count), torch.from_numpy(raw).to(DEVICE), descs=[desc])
         check(tag, raw, dims, count, 1, True, outputs, [row_bytes, size])
+
+
+@pytest.mark.parametrize("tag", ["f32", "bf16"])
+def test_topk_tiles_of_4096_and_of_8192_elements(tag):
+    """Both sides of the rule that halves a tile: width, lists, blocks and count; ties, NaNs and ordered rows; a layout of each access."""
+    rng = np.random.default_rng(1160)
+    size = 4 if tag == "f32" else 2
+    for rows, width, count, tile in ((3, 8193, 1 + 40, 16), (2, 8192, 40, 32), (2, 131072, 64, 16), (2, 131073, 20, 32), (1, 12288, 64, 16),
+                                     (1, 12288, 65, 32), (128, 32768, 2, 16), (129, 32768, 2, 32)):
+        values = rng.normal(0, 3, (rows, width)).astype(np.float32)
+        values[0] = np.sort(values[0])                                     # the best ones last
+        values[-1, ::2] = np.nan
+        stored = host_values(values, tag)
+        for largest in (True, False):
+            note(f"topk {tag} [{rows}, {width}] count {count} largest {largest}: tiles of {256 * tile}")
+            outputs = run(hc.TopK(count=count, largest=largest), to_device(stored, tag))
+            assert hc.last_launch_variant().startswith(f"topk_select/{tile}x256/"), hc.last_launch_variant()
+            check(tag, stored, [rows, width], count, -1, largest, outputs)
+    stored = tied_values(rng, [2, 30001], tag)
+    row_bytes = 30001 * size + 3
+    raw = np.zeros(2 * row_bytes + 8, np.uint8)
+    for r in range(2):
+        raw[r * row_bytes:r * row_bytes + 30001 * size] = stored[r].view(np.uint8)
+    desc = hc.TensorDesc.strided_bytes(TYPES[tag][0], [2, 30001], [row_bytes, size])
+    for count, tile in ((33, 16), (100, 32)):
+        note(f"topk {tag} [2, 30001] at odd addresses, count {count}")
+        outputs = run(hc.TopK(count=count), torch.from_numpy(raw).to(DEVICE), descs=[desc])
+        assert hc.last_launch_variant().startswith(f"topk_select/{tile}x256/bytes"), hc.last_launch_variant()
+        check(tag, raw, [2, 30001], count, 1, True, outputs, [row_bytes, size])
+    note(f"topk {tag} axis 0 of [20000, 3] and [20001, 2]")
+    for dims in ([20000, 3], [20001, 2]):
+        stored = tied_values(rng, dims, tag)
+        outputs = run(hc.TopK(count=50, axis=0), to_device(stored, tag))
+        assert "topk_select/16x256/scalar" in hc.last_launch_variant()
+        check(tag, stored, dims, 50, 0, True, outputs)
