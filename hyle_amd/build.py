@@ -9,12 +9,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libhyle_hip.so")
+SUBMIT = os.path.join(HERE, "_submit.so")
 
 SOURCES = ["plan.hip", "elementwise.hip", "norm.hip", "norm_exact_rms.hip", "norm_exact_layer.hip", "norm_tail_rms.hip", "norm_tail_layer.hip", "softmax.hip", "softmax_exact.hip", "softmax_unaligned.hip", "reduce.hip", "argmax.hip", "topk.hip", "q8_0.hip", "gguf_k.hip", "gguf_matvec.hip", "gguf_matvec_q8.hip", "gguf_matvec_strips.hip", "cast.hip", "select_fill.hip", "concat.hip", "gather.hip", "sampling.hip", "rope.hip", "file_stream.hip", "backend.hip"]
 
@@ -47,6 +49,19 @@ def _compile(source: str) -> str:
     return obj
 
 
+def _build_submit() -> None:
+    """The CPython extension that passes a submit's arguments on (csrc/submit.cc): host code, by g++."""
+    headers = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(headers, "Python.h")):
+        sys.stderr.write("no Python.h: submits go through ctypes\n")
+        return
+    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-fvisibility=hidden", "-I" + headers,
+           "-I" + os.path.join(os.path.dirname(HERE), "include"), os.path.join(CSRC, "submit.cc"), "-o", SUBMIT]
+    done = subprocess.run(cmd, capture_output=True, text=True)
+    if done.returncode != 0:
+        raise RuntimeError(f"g++ failed on submit.cc:\n{done.stderr}")
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(OBJ, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
@@ -55,6 +70,7 @@ def build(verbose: bool = True) -> str:
     done = subprocess.run(link, capture_output=True, text=True)
     if done.returncode != 0:
         raise RuntimeError(f"link failed:\n{done.stderr}")
+    _build_submit()
     if verbose:
         print(f"built {LIB} ({os.path.getsize(LIB)} bytes)")
     return LIB

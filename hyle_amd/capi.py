@@ -6,6 +6,7 @@ not been built the import fails loudly rather than falling back to any CPU path.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -185,6 +186,21 @@ def load() -> C.CDLL:
         raise RuntimeError("libhyle_hip.so ABI version differs from hyle_amd/capi.py")
     _lib = lib
     return lib
+
+
+@functools.lru_cache(maxsize=None)
+def launcher():
+    """launch(plan, inputs, outputs, workspace, workspace size, stream) -> status code: hyle_hip_plan_launch through the
+    extension of csrc/submit.cc, or through ctypes where that was not built (no Python headers)."""
+    function = load().hyle_hip_plan_launch
+    try:
+        from . import _submit
+    except ImportError:
+        def launch(plan, inputs, outputs, workspace, workspace_size, stream):
+            return function(plan, (C.c_void_p * MAX_INPUTS)(*inputs), len(inputs), (C.c_void_p * MAX_OUTPUTS)(*outputs),
+                            len(outputs), workspace, workspace_size, stream)
+        return launch
+    return functools.partial(_submit.launch, C.cast(function, C.c_void_p).value)
 
 
 def last_error() -> str:

@@ -684,17 +684,14 @@ class OperationInvocation:
         self._prepared, self._workspace, self._workspace_size = prepared, workspace, workspace_size
         self._in = (C.c_void_p * capi.MAX_INPUTS)()
         self._out = (C.c_void_p * capi.MAX_OUTPUTS)()
-        self._launch = capi.load().hyle_hip_plan_launch
+        self._launch = capi.launcher()
 
     def submit(self, stream: int, inputs: Sequence[int], outputs: Sequence[int]) -> None:
         """Enqueue on HIP stream handle `stream` (0 = default stream) and return at once.
         `inputs` / `outputs` are device addresses."""
-        for i, p in enumerate(inputs):
-            self._in[i] = p
-        for i, p in enumerate(outputs):
-            self._out[i] = p
-        _check(self._launch(self._prepared._handle, self._in, len(inputs), self._out, len(outputs),
-                            self._workspace, self._workspace_size, stream))
+        code = self._launch(self._prepared._handle, inputs, outputs, self._workspace, self._workspace_size, stream)
+        if code != capi.OK:
+            _check(code)
 
     def wait(self, stream: int, static_scratch: bool = False) -> None:
         """Completion::wait for launches whose kernels can refuse their input (checked Gather):
