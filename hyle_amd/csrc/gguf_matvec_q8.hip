@@ -354,8 +354,10 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_lines(const unsi
 // a Q8_0 row whose width is a multiple of 256 but not of 2048: a lane is a block of 32 values
 // there, and the last span then holds 8, 16, ... 56 blocks in 17, 34, ... 119 whole vectors).
 //
-// A block's rows follow one another in memory.  kStream: non-temporal loads, for weights that outgrow the memory-side
-// cache; below, plain ones, by which the line that two rows or two spans share is fetched once.
+// A block's rows follow one another in memory, and its loads are plain ones, by which the line that two rows or two spans
+// share is fetched once.  kStream, for weights that outgrow the caches: non-temporal loads, and a block takes every
+// gridDim.x-th four rows, so that the blocks walk the weights together.  (A row is 1680 bytes or more: row numbers stay far
+// below 2^32.)
 template <int kKind, class TX, int kSpans, bool kShort, bool kStream>
 __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(const unsigned char *weights, const void *x, void *y,
                                                                           uint32_t all_rows, uint32_t block_rows, uint64_t row_stride,
@@ -370,7 +372,8 @@ __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(cons
   const uint32_t span = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveLanes);
   unsigned char *slot = slots[span];
   const typename Kind::Lane at = Kind::lane_of(0, lane);
-  const uint32_t first = blockIdx.x * block_rows, rows = min(first + block_rows, all_rows);  // first < all_rows
+  const uint32_t first = blockIdx.x * (kStream ? (uint32_t)kLinesDepth : block_rows);  // < all_rows
+  const uint32_t rows = kStream ? all_rows : min(first + block_rows, all_rows), step = kLinesDepth * (kStream ? gridDim.x : 1u);
   const unsigned char *mine = weights + (size_t)span * kSpanBytes;
   // (whole spans: constants, and the compiler drops what depends on them)
   const uint32_t live_lanes = kShort && span == (uint32_t)kSpans - 1 ? tail_lanes : (uint32_t)kWaveLanes;
@@ -383,7 +386,7 @@ __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(cons
     ring[d] = Row::template load<kStream>(mine + (size_t)(wanted < rows ? wanted : first) * row_stride, lane, vectors);
   }
   const LaneCodes held = quantise_span<kKind, TX>(x, 0, span, lane, live);  // while the first rows are on their way
-  for (uint32_t base = first; base < rows; base += kLinesDepth) {
+  for (uint32_t base = first; base < rows; base += step) {
     float totals[kLinesDepth] = {};
 #pragma unroll
     for (int d = 0; d < kLinesDepth; ++d) {
@@ -392,7 +395,7 @@ __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(cons
 #pragma unroll
       for (int i = 0; i < Row::kLoads; ++i)
         *reinterpret_cast<u32x4 *>(slot + (size_t)(lane + i * kWaveLanes) * 16) = ring[d].v[i];
-      const uint32_t wanted = row + kLinesDepth;
+      const uint32_t wanted = row + step;
       ring[d] = Row::template load<kStream>(mine + (size_t)(wanted < rows ? wanted : first) * row_stride, lane, vectors);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -1369,8 +1372,10 @@ hipError_t run_registers(const MatVecParams &p, const void *w, const void *x, vo
 // rows, non-temporal / plain:
 //   Q6_K [6144 -> 2048] 5.9 / 5.6 / 5.2   [4096 -> 8192] 8.7 / 8.4 / 7.9   [2048 -> 2048] 4.7 / 4.7 / 4.2
 //   Q8_0 [5120 -> 17408] (95 MB) 18.0 / 17.9 / 16.8   [17408 -> 5120] 18.9 / 18.4 / 17.6   [7168 -> 3072] 7.8 / 7.5 / 6.8
-//   Q6_K [2048 -> 151936] (255 MB) 47.8 / 46.2 / 51.0   Q8_0 [2048 -> 100000] (218 MB) 36.5 / 36.3 / 42.2   [2560 -> 77056]
-//   (210 MB) 38.2 / 37.7 / 40.1
+//   Q6_K [2048 -> 151936] (255 MB) 47.8 / 46.2 / 51.0   Q8_0 [2048 -> 100000] (218 MB) 36.5 / 36.3 / 42.2
+// Large ones non-temporally, one by one / one run of rows to a block / four rows to a block in turn:
+//   Q8_0 [2048 -> 151936] (331 MB) 53.4 / 56.7 / 52.4   [1024 -> 151936] 35.4 / 37.9 / 34.4   [2560 -> 77056] 38.6 / 37.3 / 37.0
+//   Q6_K [2048 -> 151936] 47.1 / 46.4 / 46.4   f16 [2048 -> 100001] 33.0 / 32.7 / 31.8
 // (16 waves per compute unit with plain loads: 5.6, 8.5, 4.2, 17.8, 17.6, 7.2, 52, 43, 41)
 constexpr uint64_t kSpansStream = 128ull << 20;
 
@@ -1380,10 +1385,11 @@ hipError_t run_spans(const MatVecParams &p, const void *w, const void *x, void *
   const uint32_t units = (uint32_t)(compute_units > 0 ? compute_units : 256);
   const uint32_t most = units * (spans <= 8 ? 8u / spans : 1u);
   const uint32_t block_rows = ((uint32_t)p.rows + most - 1) / most;
-  const dim3 blocks(((uint32_t)p.rows + block_rows - 1) / block_rows);
+  const bool stream = p.rows * p.row_stride > kSpansStream;
+  const uint32_t fours = ((uint32_t)p.rows + kLinesDepth - 1) / kLinesDepth;
+  const dim3 blocks(stream ? (fours < most ? fours : most) : ((uint32_t)p.rows + block_rows - 1) / block_rows);
   const unsigned char *in = static_cast<const unsigned char *>(w);
   const uint32_t rows = (uint32_t)p.rows;
-  const bool stream = p.rows * p.row_stride > kSpansStream;
 #define HYLE_SPANS(N, SHORT)                                                                                                       \
   note_variant<SpansTag<kKind, N, SHORT>>();                                                                                       \
   if (stream)                                                                                                                      \
