@@ -1,7 +1,8 @@
 // The row kernel of RMSNorm and LayerNorm and what its launchers share: included by norm.hip (the
-// launch shapes that mask lanes and rows outside the tensor) and by norm_exact_rms.hip /
-// norm_exact_layer.hip (the shapes that cover it exactly), which are separate files so that their
-// many instantiations compile side by side.
+// launch shapes that mask lanes and rows outside the tensor), by norm_exact_rms.hip /
+// norm_exact_layer.hip (the shapes that cover it exactly) and by norm_tail_rms.hip /
+// norm_tail_layer.hip (one wave per row, only the last vector masked), which are separate files so
+// that their many instantiations compile side by side.
 #pragma once
 
 #include <type_traits>

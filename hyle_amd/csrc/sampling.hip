@@ -11,7 +11,8 @@
 // first whose running mass exceeds u * total, masses being exp(x - max) summed in double.  The
 // first dispatch leaves per tile of 4096 elements its maximum, its mass relative to that maximum
 // and whether it holds NaN or +Inf; the second, one block per row, folds the tiles, finds the
-// tile in which the running mass crosses the threshold and scans only that tile again.  A row
+// tile in which the running mass crosses the threshold and scans only that tile again.  A few rows of
+// up to 256 elements take one dispatch, a wave per row.  A row
 // with NaN, +Inf or no finite element writes nothing and sets the status word, which the host
 // reports as InvalidArgument (sampling.cc:119-135,203-206).
 #include <type_traits>
