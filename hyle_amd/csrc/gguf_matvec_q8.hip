@@ -1486,7 +1486,9 @@ inline bool rows_of_vectors_serve(const MatVecParams &p) {
 //   x 2 15.6 / 10.4, [4096 -> 2048] x 8 10.9 / 8.7, Q6_K [1024 -> 2048] x 8 11.9 / 4.7, [6144 -> 8192] x 2 20.2 / 12.9,
 //   Q4_K [1536 -> 3072] x 4 6.0 / 4.6, [7680 -> 2100] x 4 14.0 / 7.8.  Not where narrow Q4_K rows are many (tiles
 //   quantise little there and need no barrier for the tile's end): [2048 -> 6144] x 4 7.1 / 7.5, [2048 -> 65536] x 2
-//   20.1 / 22.9 ([2560 -> 8192] x 2 9.0 / 7.1, [2048 -> 65536] x 8 26.4 / 25.4); nor two rows far wider than the
+//   20.1 / 22.9 ([2560 -> 8192] x 2 9.0 / 7.1, [2048 -> 65536] x 8 26.4 / 25.4, [2048 -> 80000] x 8 30.5 / 27.2), [2048 -> 100000] x 6
+//   39.6 / 41.9, [2048 -> 151936] x 5 54.9 / 58.2 and Q6_K [2048 -> 100000] x 2 38.0 / 42.0, [2048 -> 151936] x 2 55.2 / 59.2
+//   ([2048 -> 65536] x 2 29.4 / 25.2, Q4_K [1792 -> 120000] x 8 41.0 / 36.9); nor two rows far wider than the
 //   weight is high, Q8_0 [16384 -> 1024] 10.1 / 11.4 ([8192 -> 2048] 9.5 / 8.1)
 //   one row, where the alternative walks block by block, from 8 M products on, and from 4 M where a row is wide:
 //   Q6_K [1024 -> 8192] 5.8 / 5.4, [2304 -> 2304] 6.9 / 5.6, [7680 -> 2100] 12.9 / 8.2 ([1024 -> 2048] 4.0 / 4.2)
@@ -1502,7 +1504,10 @@ bool strips_better(const MatVecParams &p, bool vectors) {
     return p.kind == 0 && (p.k >= 10240 || (p.k > 2048 && p.k % 2048 != 0 && (p.rows <= 4096 || p.k >= p.rows)));
   }
   if (!whole) return true;
-  if (p.kind == 0) return p.m > 4 || p.k > 2048 || p.rows < 6144;
+  // one span of a vocabulary: the tile and quad kernels keep its codes at hand and have no tiles left over
+  const bool span_of_many = p.k > 1792 && p.k <= 2048 && p.rows >= 90000;
+  if (p.kind == 0) return (p.m > 4 && !span_of_many) || p.k > 2048 || p.rows < 6144;
+  if (p.kind == 1 && p.m <= 4 && span_of_many) return false;
   return p.m > 2 || p.k < 8 * p.rows;
 }
 

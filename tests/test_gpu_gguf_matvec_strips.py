@@ -224,3 +224,11 @@ def test_strips_activation_blocks_on_both_sides_of_the_short_form(tag):
     x[3] *= np.tile(np.repeat(np.float32([2.0 ** -65, 2.0 ** -60]), 256), k // 512)
     note(f"q8 matvec strips {tag}: activation blocks below 2^-60 and above 2^61")
     check(tag, "f32", weights_for(tag, rng, rows, k), rows, k, x, kernel=f"gguf_matvec_q8_strips/{tag}/4-tokens")
+
+
+@pytest.mark.parametrize("tag,rows,m,kernel", [("q4_k", 89999, 5, "strips/q4_k/8"), ("q4_k", 90000, 5, "tiles/q4_k/8"), ("q6_k", 89999, 2, "strips/q6_k/4"),
+                                               ("q6_k", 90000, 2, "quads/q6_k/4")])
+def test_strips_rule_for_one_span_of_a_vocabulary(tag, rows, m, kernel):
+    rng = np.random.default_rng(1825)
+    note(f"q8 matvec rule {tag} rows {rows} k 2048 m {m}")
+    check(tag, "bf16", raw_bytes_for(tag, rng, rows, 2048), rows, 2048, rng.normal(0, 1, (m, 2048)).astype(np.float32), kernel="gguf_matvec_q8_" + kernel)
