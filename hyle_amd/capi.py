@@ -188,19 +188,24 @@ def load() -> C.CDLL:
     return lib
 
 
+def launch_through_ctypes(plan, inputs, outputs, workspace, workspace_size, stream) -> int:
+    """hyle_hip_plan_launch with whatever ctypes takes for an address -> status code."""
+    return load().hyle_hip_plan_launch(plan, (C.c_void_p * MAX_INPUTS)(*inputs), len(inputs), (C.c_void_p * MAX_OUTPUTS)(*outputs),
+                                       len(outputs), workspace, workspace_size, stream)
+
+
 @functools.lru_cache(maxsize=None)
 def launcher():
     """launch(plan, inputs, outputs, workspace, workspace size, stream) -> status code: hyle_hip_plan_launch through the
-    extension of csrc/submit.cc, or through ctypes where that was not built (no Python headers)."""
-    function = load().hyle_hip_plan_launch
+    extension of csrc/submit.cc, which raises TypeError before it launches anything where an address is neither an int,
+    None nor a c_void_p; through ctypes where the extension was not built (no Python headers)."""
     try:
         from . import _submit
     except ImportError:
-        def launch(plan, inputs, outputs, workspace, workspace_size, stream):
-            return function(plan, (C.c_void_p * MAX_INPUTS)(*inputs), len(inputs), (C.c_void_p * MAX_OUTPUTS)(*outputs),
-                            len(outputs), workspace, workspace_size, stream)
-        return launch
-    return functools.partial(_submit.launch, C.cast(function, C.c_void_p).value)
+        if os.path.exists(os.path.join(HERE, "_submit.so")):  # built, and broken
+            raise
+        return launch_through_ctypes
+    return functools.partial(_submit.launch, C.cast(load().hyle_hip_plan_launch, C.c_void_p).value)
 
 
 def last_error() -> str:

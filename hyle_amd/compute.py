@@ -689,7 +689,10 @@ class OperationInvocation:
     def submit(self, stream: int, inputs: Sequence[int], outputs: Sequence[int]) -> None:
         """Enqueue on HIP stream handle `stream` (0 = default stream) and return at once.
         `inputs` / `outputs` are device addresses."""
-        code = self._launch(self._prepared._handle, inputs, outputs, self._workspace, self._workspace_size, stream)
+        try:
+            code = self._launch(self._prepared._handle, inputs, outputs, self._workspace, self._workspace_size, stream)
+        except TypeError:  # nothing was launched: a stream object that converts itself, or what ctypes refuses too
+            code = capi.launch_through_ctypes(self._prepared._handle, inputs, outputs, self._workspace, self._workspace_size, stream)
         if code != capi.OK:
             _check(code)
 

@@ -11,7 +11,9 @@ namespace {
 
 constexpr Py_ssize_t kMostInputs = HYLE_HIP_MAX_INPUTS, kMostOutputs = HYLE_HIP_MAX_OUTPUTS;
 
-// An address: an int, None for null, or a ctypes pointer value of either.
+PyObject *pointer_type = nullptr;  // ctypes.c_void_p
+
+// An address: an int, None for null, or a c_void_p of either.  Anything else is refused here; the caller then asks ctypes.
 bool address_of(PyObject *object, void **out) {
   if (PyLong_Check(object)) {
     *out = reinterpret_cast<void *>(PyLong_AsUnsignedLongLongMask(object));
@@ -19,18 +21,21 @@ bool address_of(PyObject *object, void **out) {
   }
   *out = nullptr;
   if (object == Py_None) return true;
-  PyObject *value = PyObject_GetAttrString(object, "value");
-  const bool fine = value != nullptr && (value == Py_None || PyLong_Check(value));
-  if (fine && value != Py_None) *out = reinterpret_cast<void *>(PyLong_AsUnsignedLongLongMask(value));
-  Py_XDECREF(value);
-  if (!fine) {
-    PyErr_Clear();
+  const int pointer = PyObject_IsInstance(object, pointer_type);
+  if (pointer < 0) return false;
+  if (pointer == 0) {
     PyErr_Format(PyExc_TypeError, "cannot be converted to pointer: %.100s", Py_TYPE(object)->tp_name);
+    return false;
   }
-  return fine;
+  PyObject *value = PyObject_GetAttrString(object, "value");
+  if (value == nullptr) return false;
+  if (value != Py_None) *out = reinterpret_cast<void *>(PyLong_AsUnsignedLongLongMask(value));
+  Py_DECREF(value);
+  return !PyErr_Occurred();
 }
 
 bool addresses_of(PyObject *sequence, void **out, Py_ssize_t most, uint32_t *count) {
+  if (PyObject_Size(sequence) < 0) return false;  // an iterator is no sequence
   PyObject *items = PySequence_Fast(sequence, "a sequence of device addresses is expected");
   if (items == nullptr) return false;
   const Py_ssize_t size = PySequence_Fast_GET_SIZE(items);
@@ -69,4 +74,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_submit", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__submit() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__submit() {
+  PyObject *ctypes = PyImport_ImportModule("ctypes");
+  if (ctypes == nullptr) return nullptr;
+  pointer_type = PyObject_GetAttrString(ctypes, "c_void_p");
+  Py_DECREF(ctypes);
+  return pointer_type == nullptr ? nullptr : PyModule_Create(&module);
+}
