@@ -31,7 +31,8 @@ class StreamObject:
 
 @pytest.fixture(params=["extension", "ctypes"])
 def invocation(request, monkeypatch):
-    monkeypatch.setattr(capi, "load", lambda: SimpleNamespace(hyle_hip_plan_launch=noting))
+    library = SimpleNamespace(hyle_hip_plan_launch=noting, hyle_hip_last_launch_variant=lambda: b"")   # the GPU tests ask for the label
+    monkeypatch.setattr(capi, "load", lambda: library)
     if request.param == "ctypes":                                      # as if it had not been built
         monkeypatch.setitem(sys.modules, "hyle_amd._submit", None)
         monkeypatch.delattr("hyle_amd._submit", raising=False)
