@@ -178,8 +178,9 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_tiles(const void *l
 
 // Scan of one double per thread over the block, in thread order: returns the sum of the threads
 // below (exactly the inclusive value the thread below holds) and leaves the inclusive value and
-// the block's total in `through` and `total`.  Two barriers.
-__device__ __forceinline__ double block_scan(double v, double *wave_totals, double *through, double *total) {
+// the block's total in `through` and `total`.  Two barriers; `vote` comes between them, with both sums known.
+template <class Vote>
+__device__ __forceinline__ double block_scan(double v, double *wave_totals, double *through, double *total, Vote vote) {
   const int lane = threadIdx.x & (kWaveLanes - 1), wave = threadIdx.x / kWaveLanes;
 #pragma unroll
   for (int step = 1; step < kWaveLanes; step *= 2) {
@@ -195,9 +196,10 @@ __device__ __forceinline__ double block_scan(double v, double *wave_totals, doub
     if (w < wave) before += wave_totals[w];
     all += wave_totals[w];
   }
-  __syncthreads();
   *total = all;
   *through = v + before;
+  vote();
+  __syncthreads();
   return lane == 0 ? before : previous + before;
 }
 
@@ -228,6 +230,24 @@ __device__ __forceinline__ void load_consecutive(const void *row, uint32_t first
   }
 }
 
+// Who holds the crossing.  A scan's running sums are associated differently from lane to lane, so they need not be
+// monotone in their last bit: a lane without mass may see the threshold between its neighbour's sum and its own, two
+// lanes may both see it between theirs, and none may.  Everywhere below the lowest lane with mass of its own whose
+// running sum exceeds the threshold answers, with its first element that has mass and carries the sum past it.
+
+// Of a lane's consecutive weights (one at least is mass); `before`: the running sum in front of them.
+__device__ __forceinline__ int crossing_element(const float (&weights)[kPerThread], double before, double threshold) {
+  double running = before;
+  int selected = -1, last_positive = 0;
+#pragma unroll
+  for (int i = 0; i < kPerThread; ++i) {
+    running += (double)weights[i];
+    if (weights[i] > 0) last_positive = i;
+    if (selected < 0 && weights[i] > 0 && running > threshold) selected = i;
+  }
+  return selected < 0 ? last_positive : selected;  // (the scan's sum and this walk's differ in their last bit)
+}
+
 // What the thread that holds the crossing tile tells the block.
 struct Crossing {
   double residual;   // the threshold less the mass before the tile, on the row's scale
@@ -242,7 +262,8 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
   __shared__ float joint[kBlockThreads / kWaveLanes];
   __shared__ double wave_totals[kBlockThreads / kWaveLanes];
   __shared__ Crossing found_crossing;
-  __shared__ uint32_t found, claim;
+  __shared__ uint32_t found, claim, crossing_of[kBlockThreads / kWaveLanes], last_of[kBlockThreads / kWaveLanes];
+  constexpr uint32_t kNobody = 0xFFFFFFFFu;
   constexpr float kInfinity = __builtin_huge_valf();
   const uint32_t row = blockIdx.x, lane = threadIdx.x % kWaveLanes;
   const CategoricalTile *mine = parts + (size_t)row * tiles;
@@ -274,7 +295,7 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
     const double previous = __shfl_up(through, 1, kWaveLanes), before = lane == 0 ? 0.0 : previous;
     total = __shfl(through, kWaveLanes - 1, kWaveLanes);
     const double threshold = total * uniform;
-    const uint64_t candidates = __ballot(own > 0 && !(before > threshold) && through > threshold);
+    const uint64_t candidates = __ballot(own > 0 && through > threshold);
     const int holder = candidates != 0 ? __builtin_ctzll(candidates) : 0;
     const double residual = before + own > threshold ? threshold - before : 0.0;
     crossing = Crossing{__shfl(residual, holder, kWaveLanes), candidates != 0 ? (uint32_t)holder : 0xFFFFFFFFu,
@@ -295,7 +316,7 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
     double own = 0;
     for (uint32_t t = begin; t < end; ++t) own += mine[t].mass * (double)scale_of(t);
     double through = 0;
-    const double before = block_scan(own, wave_totals, &through, &total);
+    const double before = block_scan(own, wave_totals, &through, &total, [] {});
     const PhiloxWords draw = philox_block(key0, key1, draw0, draw1, 0);
     // the 52-bit midpoint is exact in double at both ends (sampling.cc:155-158)
     const double uniform = ((double)draw.x0 * 0x1p20 + (double)(draw.x1 >> 12) + 0.5) * 0x1p-52;
@@ -305,11 +326,7 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
       claim = 0xFFFFFFFFu;
     }
     __syncthreads();
-    // The scan's running sums are associated differently from lane to lane, so they need not be
-    // monotone in their last bit: a thread without mass may see the threshold between its equal
-    // `before` and `through`, and two neighbours may both see it.  Only threads with mass of their
-    // own may hold the crossing, and the lowest of them answers.
-    const bool candidate = own > 0 && !(before > threshold) && through > threshold;
+    const bool candidate = own > 0 && through > threshold;
     if (candidate) atomicMin(&claim, threadIdx.x);
     __syncthreads();
     if (candidate && claim == threadIdx.x) {  // the first tile whose running mass exceeds the threshold is here
@@ -317,7 +334,8 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
       uint32_t tile = 0xFFFFFFFFu, last_with_mass = 0xFFFFFFFFu;
       for (uint32_t t = begin; t < end; ++t) {
         const double share = mine[t].mass * (double)scale_of(t);
-        if (share > 0) last_with_mass = t;
+        if (!(share > 0)) continue;
+        last_with_mass = t;
         if (running + share > threshold) {
           tile = t;
           break;
@@ -364,20 +382,22 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
     mass += (double)weights[i];
   }
   double tile_total = 0, mass_through = 0;
-  const double mass_before = block_scan(mass, wave_totals, &mass_through, &tile_total);
-  // exactly one thread holds the crossing; none when rounding left the residual at the tile's total,
-  // and then the thread with the tile's last mass answers
-  const bool last_mass = !(tile_total > residual) && mass > 0 && mass_through == tile_total;
-  if ((!(mass_before > residual) && mass_through > residual) || last_mass) {
-    double running = mass_before;
-    int selected = -1, last_positive = -1;
-#pragma unroll
-    for (int i = 0; i < kPerThread; ++i) {
-      running += (double)weights[i];
-      if (weights[i] > 0) last_positive = i;
-      if (selected < 0 && running > residual) selected = i;
+  const double mass_before = block_scan(mass, wave_totals, &mass_through, &tile_total, [&] {
+    // per wave: who holds the crossing, and the last with mass, who answers when rounding left the residual at the tile's total
+    const uint64_t crossed = __ballot(mass > 0 && mass_through > residual), massive = __ballot(mass > 0);
+    if (lane == 0) {
+      crossing_of[threadIdx.x / kWaveLanes] = crossed != 0 ? threadIdx.x + (uint32_t)__builtin_ctzll(crossed) : kNobody;
+      last_of[threadIdx.x / kWaveLanes] = massive != 0 ? threadIdx.x + (uint32_t)(kWaveLanes - 1 - __builtin_clzll(massive)) : 0u;
     }
-    if (selected < 0) selected = last_positive;
+  });
+  uint32_t answering = kNobody, last = 0;
+#pragma unroll
+  for (int w = 0; w < kBlockThreads / kWaveLanes; ++w) {
+    answering = min(answering, crossing_of[w]);
+    last = max(last, last_of[w]);
+  }
+  if (threadIdx.x == (answering != kNobody ? answering : last)) {
+    const int selected = crossing_element(weights, mass_before, residual);
     float chosen = v[0];
 #pragma unroll
     for (int i = 1; i < kPerThread; ++i) chosen = selected == i ? v[i] : chosen;
@@ -520,18 +540,10 @@ __global__ __launch_bounds__(kShortWaves *kWaveLanes) void categorical_short(con
     if (lane >= (uint32_t)step) through += below;
   }
   const double previous = __shfl_up(through, 1, kWaveLanes), before = lane == 0 ? 0 : previous;
-  const double all = __shfl(through, kShortWidth / kPerThread - 1, kWaveLanes);
-  const bool last_mass = !(all > threshold) && mass > 0 && through == all;
-  if (lane < kShortWidth / kPerThread && ((!(before > threshold) && through > threshold) || last_mass)) {
-    double running = before;
-    int selected = -1, last_positive = -1;
-#pragma unroll
-    for (int i = 0; i < kPerThread; ++i) {
-      running += (double)weights[i];
-      if (weights[i] > 0) last_positive = i;
-      if (selected < 0 && running > threshold) selected = i;
-    }
-    if (selected < 0) selected = last_positive;
+  // (lanes past the sixteen have no mass)  None crossed: rounding left the threshold at the scan's total, the last with mass
+  const uint64_t crossed = __ballot(mass > 0 && through > threshold), massive = __ballot(mass > 0);
+  if (lane == (uint32_t)(crossed != 0 ? __builtin_ctzll(crossed) : kWaveLanes - 1 - __builtin_clzll(massive))) {
+    const int selected = crossing_element(weights, before, threshold);
     float chosen = v[0];
 #pragma unroll
     for (int i = 1; i < kPerThread; ++i) chosen = selected == i ? v[i] : chosen;

@@ -71,3 +71,57 @@ def inverse_cdf_bounds(values: np.ndarray, identities: np.ndarray, slack: float 
         low[r] = positive[np.searchsorted(positive, min(first, width - 1), side="left").clip(0, positive.size - 1)]
         high[r] = positive[np.searchsorted(positive, min(last, width - 1), side="left").clip(0, positive.size - 1)]
     return low, high, scores
+
+
+def running_sums(masses: np.ndarray) -> np.ndarray:
+    """[rows, lanes] f64 -> what each lane holds after a scan that adds the sum 1, 2, 4, ... lanes below."""
+    through = masses.astype(np.float64).copy()
+    step = 1
+    while step < through.shape[1]:
+        through[:, step:] = through[:, step:] + through[:, :-step].copy()
+        step *= 2
+    return through
+
+
+def rows_with_a_threshold_between_sums(mass_of, identities: np.ndarray, seed: int):
+    """float32 logits [n, 256] and their identities whose threshold falls where the running sums of sixteen elements
+    a lane are not monotone: lane 7 has no mass (-inf), its own sum is above lane 6's by the last bit, and the threshold
+    lies from lane 6's sum to below lane 7's.  `mass_of(float32 array)`: the kernel's exp of values up to 0, as float32.
+    Only the rows for which the arithmetic lands there; the last element in front of lane 7 has no mass either."""
+    rng = np.random.default_rng(seed)
+    rows, lanes, hole = identities.shape[0], 16, 7
+    words = philox_array(np.stack([np.zeros(rows, np.uint32)] * 2 + [identities[:, 2], identities[:, 3]], axis=1), identities[:, :2])
+    uniform = np.array([uniform_of(w) for w in words])
+    t = np.full((rows, lanes, 16), -np.inf, np.float32)
+    t[:, :hole] = -rng.uniform(0, 5, (rows, hole, 16)) ** 2  # so far apart that sums round
+    t[:, 0, 0], t[:, hole - 1, 15] = 0, -np.inf
+    lane_mass = lambda: np.add.accumulate(mass_of(t).astype(np.float64), axis=2)[:, :, -1]
+    front = running_sums(lane_mass())[:, hole - 1]
+    # what lies behind the hole: bulk, then ever smaller masses that close what is left of the wanted sum
+    wanted = front / uniform - front
+    place = (hole + 1) * 16
+    flat = t.reshape(rows, 256)
+    for _ in range(256 - place - 8):
+        bulk = wanted > 1.0
+        flat[bulk, place] = np.float32(-0.1)
+        wanted[bulk] -= mass_of(flat[bulk, place]).astype(np.float64)
+        place += 1
+    for _ in range(8):
+        start = np.log(np.maximum(wanted, 1e-300)).astype(np.float32)
+        steps = np.arange(-8, 9, dtype=np.int64)[None, :]
+        near = (start.view(np.int32).astype(np.int64)[:, None] + steps).astype(np.int32).view(np.float32)
+        masses = mass_of(near).astype(np.float64)
+        masses[~((near < 0) & (near > -60) & (masses <= wanted[:, None]))] = -1.0
+        best = masses.argmax(axis=1)
+        found = masses[np.arange(rows), best] > 0
+        flat[found, place] = near[np.arange(rows), best][found]
+        wanted[found] -= masses[np.arange(rows), best][found]
+        place += 1
+    # the row's total as the kernel takes it: four elements a lane, then pairs 1, 2, 4, ... lanes apart
+    total = np.add.accumulate(mass_of(flat).astype(np.float64).reshape(rows, 64, 4), axis=2)[:, :, -1]
+    while total.shape[1] > 1:
+        total = total[:, 0::2] + total[:, 1::2]
+    threshold = total[:, 0] * uniform
+    through = running_sums(lane_mass())
+    armed = (through[:, hole - 1] <= threshold) & (threshold < through[:, hole])
+    return flat[armed], identities[armed]

@@ -18,7 +18,7 @@ from hyle_amd import compute as hc
 from oracle import lib as orc
 
 from gpu_support import DEVICE, context, note
-from sampling_support import fixture_identities, fixture_logits, inverse_cdf_bounds
+from sampling_support import fixture_identities, fixture_logits, inverse_cdf_bounds, rows_with_a_threshold_between_sums
 
 pytestmark = pytest.mark.gpu
 
@@ -184,6 +184,31 @@ def test_categorical_on_both_sides_of_64_tiles(type_id, rows, width):
         status, picked, scores = categorical_on_device(type_id, stored, ids, scored)
         assert status == 0 and hc.last_launch_variant().endswith("/many-tiles") == (width > 262144)
         check_against_float64(values, ids, picked, scores, orc.categorical(type_id, stored, ids)[1])
+
+
+def test_categorical_never_answers_with_a_lane_without_mass():
+    """Thresholds between a lane's running sum and the larger one of its neighbour without mass: the neighbour must not
+    answer, in one dispatch and in two."""
+    def mass_of(values):                                    # the kernels' exp of values up to 0
+        t = torch.from_numpy(np.ascontiguousarray(values)).to(DEVICE).clamp(min=-200.0)
+        high = t * np.float32(1.44269504088896340736)
+        low = (t.double() * float(np.float32(1.44269504088896340736)) - high.double()).float()
+        p = torch.exp2(high)
+        return (p.double() + p.double() * (low * np.float32(0.69314718055994530942)).double()).float().cpu().numpy()
+
+    ids = np.random.default_rng(3).integers(0, 1 << 32, (4096, 4), dtype=np.uint64).astype(np.uint32)
+    values, ids = rows_with_a_threshold_between_sums(mass_of, ids, 1)
+    values, ids = values[:256], ids[:256]
+    assert len(values) >= 50
+    behind = 128 + np.isfinite(values[:, 128:]).argmax(axis=1)
+    for label, rows in (("categorical_short/vector/scored", len(values)), ("categorical_tiles", 257)):
+        note(f"categorical {label}: {len(values)} thresholds at a lane without mass")
+        stored, keys = (np.resize(a, (rows, a.shape[1])) for a in (values, ids))
+        status, picked, scores = categorical_on_device(orc.F32, stored, keys, True)
+        assert status == 0 and label in hc.last_launch_variant()
+        assert np.isfinite(stored[np.arange(rows), picked]).all() and np.isfinite(scores).all()
+        assert np.array_equal(picked, np.resize(behind, rows))
+        check_against_float64(stored, keys, picked, scores, orc.categorical(orc.F32, stored, keys)[1])
 
 
 def test_categorical_short_rows_refuse_what_long_rows_refuse():
