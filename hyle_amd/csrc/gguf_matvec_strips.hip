@@ -382,14 +382,15 @@ template <int kLanes> __device__ __forceinline__ uint32_t lanes_max(uint32_t v) 
   return v;
 }
 
-// a / b correctly rounded for a of one or 127 and b from 2^-60 to 2^61: the hardware's reciprocal, a Newton step and
-// a correction of the quotient by its exact remainder (compared with the compiler's division for every such b).  It is
-// six instructions where the full division, which scales its operands, is eleven.
-__device__ __forceinline__ float quotient(float a, float b) {
+// 127 / b correctly rounded for b from 2^-60 to 2^61: the hardware's reciprocal, a Newton step and a correction of
+// the quotient by its exact remainder, right for every mantissa of b with a reciprocal up to one unit off.  It is
+// six instructions where the full division, which scales its operands, is eleven.  (1 / b is not to be had this way: for
+// a mantissa of all ones the step ends one unit short.)
+__device__ __forceinline__ float quotient_of_127(float b) {
   const float rough = __builtin_amdgcn_rcpf(b);
   const float inverse = __builtin_fmaf(__builtin_fmaf(-b, rough, 1.0f), rough, rough);
-  const float q = a * inverse;
-  return __builtin_fmaf(__builtin_fmaf(-b, q, a), inverse, q);
+  const float q = 127.0f * inverse;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, 127.0f), inverse, q);
 }
 // b / 127 the same way
 __device__ __forceinline__ float over_127(float b) {
@@ -423,11 +424,11 @@ __device__ __forceinline__ void strip_quantise(const StripValues<TX> &fetched, u
     const float top = bits_f32(top_bits);
     if constexpr (kSmall) {
       stored = f16_to_f32(f32_to_f16(over_127(top)));
-      factor = quotient(127.0f, top);
+      factor = quotient_of_127(top);
     } else {
-      factor = quotient(127.0f, top);
+      factor = quotient_of_127(top);
       factor = positive > negative ? -factor : factor;
-      stored = quotient(1.0f, factor);
+      stored = 1.0f / factor;
     }
 #pragma unroll
     for (int w = 0; w < 4; ++w) {

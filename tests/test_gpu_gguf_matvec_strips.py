@@ -12,6 +12,7 @@ from hyle_amd import compute as hc
 from oracle import lib as orc
 
 from gpu_support import DEVICE, context, note, run
+from k_quant_support import pack_q6_k
 from test_gpu_gguf_matvec_q8 import KINDS, Q8, check, raw_bytes_for, weights_for
 
 pytestmark = pytest.mark.gpu
@@ -232,3 +233,33 @@ def test_strips_rule_for_one_span_of_a_vocabulary(tag, rows, m, kernel):
     rng = np.random.default_rng(1825)
     note(f"q8 matvec rule {tag} rows {rows} k 2048 m {m}")
     check(tag, "bf16", raw_bytes_for(tag, rng, rows, 2048), rows, 2048, rng.normal(0, 1, (m, 2048)).astype(np.float32), kernel="gguf_matvec_q8_" + kernel)
+
+
+def test_strips_scales_of_activation_blocks_are_exact_quotients():
+    """A weight row picks one activation block's largest value, whose code is 127: the product is 127 times the block's
+    scale, 1 / (127 / largest) in f32, rounded once.  Among the largest values those whose factor has a mantissa of all
+    ones, where a quotient by a corrected reciprocal ends one unit short."""
+    blocks, m, rows = 16, 8, 512
+    raw = np.zeros((rows, blocks, 210), np.uint8)
+    quants = np.full(256, 32)
+    quants[5] = 33
+    for r in range(rows):
+        raw[r, :] = pack_q6_k(np.float16(0), np.ones(16), np.full(256, 32))
+        raw[r, r % blocks] = pack_q6_k(np.float16(1), np.ones(16), quants)
+    rng = np.random.default_rng(1826)
+    for draw in range(4):
+        largest = (rng.integers(0, 1 << 23, (m, blocks), dtype=np.uint32) | np.uint32(127 << 23)).view(np.float32)
+        largest[:, ::4] = np.nextafter(np.float32(63.5), np.float32(64))        # 127 / largest is 2 - 2^-23
+        largest *= np.float32(2) ** rng.integers(-59, 50, (m, blocks)).astype(np.float32)
+        largest *= rng.choice(np.float32([-1, 1]), (m, blocks))
+        x = np.zeros((m, blocks, 256), np.float32)
+        x[:, :, 5], x[:, :, 77] = largest, largest * np.float32(0.5)
+        factor = np.float32(-127) / largest
+        assert (np.abs(factor[:, ::4]).view(np.uint32) & np.uint32(0x7FFFFF) == np.uint32(0x7FFFFF)).all()
+        note(f"q8 matvec strips: scales of activation blocks, draw {draw}")
+        descs = [hc.TensorDesc.gguf_weight(KINDS["q6_k"][1], hc.DataType.kFloat32, 256 * blocks, rows),
+                 hc.TensorDesc.dense(hc.DataType.kFloat32, [m, 256 * blocks])]
+        (out,) = run(Q8, torch.from_numpy(raw.reshape(-1)).to(DEVICE), torch.from_numpy(x.reshape(m, -1)).to(DEVICE), descs=descs)
+        assert hc.last_launch_variant().startswith("gguf_matvec_q8_strips/q6_k/8")
+        wanted = np.float32(-127) * (np.float32(1) / factor)
+        assert np.array_equal(out.cpu().numpy(), np.tile(wanted, (1, rows // blocks)))

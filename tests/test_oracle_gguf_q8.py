@@ -141,3 +141,26 @@ def test_centre_is_the_product_with_the_dequantised_activations_and_the_bound_ha
             step = np.repeat(np.abs(scales), 32 if kind == orc.Q8_0 else 256).astype(np.float64)
             slack = np.abs(weights) @ (0.5 * step * (1 + 1e-6) + np.abs(x[i]) * 2.0 ** -11)
             assert np.all(np.abs(centre[i] - exact) <= slack)
+
+
+def test_short_divisions_of_the_activation_blocks_are_exact():
+    """127 / b from a reciprocal one unit off on either side, and b / 127, as the strip kernel takes them: correctly
+    rounded for every mantissa of b (the kernel's range of exponents only scales the steps by powers of two).  Each
+    fused step is taken in 64-bit mantissas, which hold its product, and rounded once more to 24."""
+    def fused(a, b, c):
+        return (a.astype(np.longdouble) * b + c).astype(np.float32)
+
+    one = np.float32(1)
+    for first in range(0, 1 << 23, 1 << 21):
+        b = (np.arange(first, first + (1 << 21), dtype=np.uint32) | np.uint32(0x3F800000)).view(np.float32)
+        wanted = rn(127.0 / b.astype(np.float64))       # a quotient of 24-bit numbers is no closer than 2^-49 to a tie
+        nearest = rn(1.0 / b.astype(np.float64))
+        for unit in (-1, 0, 1):
+            rough = (nearest.view(np.int32) + np.int32(unit)).view(np.float32)
+            inverse = fused(fused(-b, rough, one), rough, rough)
+            q = rn(127.0 * inverse.astype(np.float64))
+            assert np.array_equal(fused(fused(-b, q, np.float32(127)), inverse, q), wanted), (first, unit)
+        inverse = np.float32(1) / np.float32(127)
+        q = rn(b.astype(np.float64) * float(inverse))
+        got = fused(fused(np.full_like(b, -127), q, b), np.full_like(b, inverse), q)
+        assert np.array_equal(got, rn(b.astype(np.float64) / 127.0)), first
