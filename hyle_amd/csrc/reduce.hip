@@ -36,8 +36,8 @@ template <int kKind> __device__ __forceinline__ float reduce_step(float acc, flo
   else return acc + v;
 }
 // The same extremum in one instruction for two elements (v_maximum3_f32, v_minimum3_f32: a NaN propagates, +0 ranks
-// above -0) instead of six for one, except that a NaN comes back quiet: who meets one takes reduce_step over the same
-// elements again.  MI355X, us: max over rows of f32 [5003, 2560] 12.4 -> 9.9, bf16 [5003, 2560] 9.5 -> 6.0, f16
+// above -0) instead of six for one, except that a NaN comes back quiet: a lane whose trip ends in its first one takes
+// reduce_step over the same registers, and a lane that has one keeps it.  MI355X, us: max over rows of f32 [5003, 2560] 12.4 -> 9.9, bf16 [5003, 2560] 9.5 -> 6.0, f16
 // [2000, 5000] 8.2 -> 5.8, f32 [4096, 4096] 13.8 -> 11.7.
 template <int kKind> __device__ __forceinline__ float reduce_step_quick(float acc, float v) {
   if constexpr (kKind == kMinimum) return __builtin_elementwise_minimum(acc, v);
@@ -93,36 +93,33 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_rows(const void *x, void
       // width and tile_width are multiples of the vector width
       const size_t base = (size_t)row * (width / kVec);
       const uint32_t last = end / kVec;
-      auto walk = [&](auto step) {
-        uint32_t vec = begin / kVec + lane;
-        // a vector past the tile is its last one again and is dropped
-        in_trips<8>(__builtin_amdgcn_readfirstlane((last - begin / kVec + kLanes - 1) / kLanes), [&](auto loads) {
-          constexpr uint32_t kLoads = decltype(loads)::kCount;
-          constexpr bool kFull = decltype(loads)::kFull;
-          if (!kFull && vec >= last) return;  // nothing left of this lane's
-          u32x4 raw[kLoads];
+      uint32_t vec = begin / kVec + lane;
+      // a vector past the tile is its last one again and is dropped
+      in_trips<8>(__builtin_amdgcn_readfirstlane((last - begin / kVec + kLanes - 1) / kLanes), [&](auto loads) {
+        constexpr uint32_t kLoads = decltype(loads)::kCount;
+        constexpr bool kFull = decltype(loads)::kFull;
+        if (!kFull && vec >= last) return;  // nothing left of this lane's
+        u32x4 raw[kLoads];
 #pragma unroll
-          for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (kFull || i == 0 ? vec + i * kLanes : min(vec + i * kLanes, last - 1)));
+        for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (kFull || i == 0 ? vec + i * kLanes : min(vec + i * kLanes, last - 1)));
 #pragma unroll
-          for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
+        for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
+        auto taken = [&](float from, auto step) {
 #pragma unroll
           for (uint32_t i = 0; i < kLoads; ++i) {
             if (!kFull && i != 0 && vec + i * kLanes >= last) break;
             float v[kVec];
             Traits<TIn>::unpack(raw[i], v);
 #pragma unroll
-            for (int j = 0; j < kVec; ++j) acc = step(acc, v[j]);
+            for (int j = 0; j < kVec; ++j) from = step(from, v[j]);
           }
-          vec += kLoads * kLanes;
-        });
-      };
-      walk([](float a, float v) { return reduce_step_quick<kKind>(a, v); });
-      if constexpr (kExtreme<kKind>) {
-        if (__ballot(acc != acc) != 0) {  // (the trips want whole waves)
-          acc = reduce_identity<kKind>();
-          walk([](float a, float v) { return reduce_step<kKind>(a, v); });
-        }
-      }
+          return from;
+        };
+        const float quick = taken(acc, [](float a, float v) { return reduce_step_quick<kKind>(a, v); });
+        if (!kExtreme<kKind> || quick == quick) acc = quick;
+        else if (acc == acc) acc = taken(acc, [](float a, float v) { return reduce_step<kKind>(a, v); });
+        vec += kLoads * kLanes;
+      });
     } else {
       const size_t base = (size_t)row * width;
       for (uint32_t i = begin + lane; i < end; i += kLanes)
@@ -161,39 +158,53 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_columns(const void *x, v
   if (active) {
     const size_t base = (size_t)outer * reduced * units + unit;  // in units
     if constexpr (kVector) {
-      auto walk = [&](auto step) {
-        uint32_t r = begin + ty;
-        in_trips<kMost>((end - begin + lanes_y - 1) / lanes_y, [&](auto loads) {
-          constexpr uint32_t kLoads = decltype(loads)::kCount;
-          constexpr bool kFull = decltype(loads)::kFull;
-          if (!kFull && r >= end) return;
-          u32x4 raw[kLoads];
+      uint32_t r = begin + ty;
+      in_trips<kMost>((end - begin + lanes_y - 1) / lanes_y, [&](auto loads) {
+        constexpr uint32_t kLoads = decltype(loads)::kCount;
+        constexpr bool kFull = decltype(loads)::kFull;
+        if (!kFull && r >= end) return;
+        u32x4 raw[kLoads];
 #pragma unroll
-          for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (size_t)(kFull || i == 0 ? r + i * lanes_y : min(r + i * lanes_y, end - 1)) * units);
+        for (uint32_t i = 0; i < kLoads; ++i) raw[i] = load16_stream(x, base + (size_t)(kFull || i == 0 ? r + i * lanes_y : min(r + i * lanes_y, end - 1)) * units);
 #pragma unroll
-          for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
+        for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
+        auto take = [&](float (&into)[kW], auto step) {
 #pragma unroll
           for (uint32_t i = 0; i < kLoads; ++i) {
             if (!kFull && i != 0 && r + i * lanes_y >= end) break;
             float v[kW];
             Traits<TIn>::unpack(raw[i], v);
 #pragma unroll
-            for (int j = 0; j < kW; ++j) acc[j] = step(acc[j], v[j]);
+            for (int j = 0; j < kW; ++j) into[j] = step(into[j], v[j]);
           }
-          r += kLoads * lanes_y;
-        });
-      };
-      walk([](float a, float v) { return reduce_step_quick<kKind>(a, v); });
-      if constexpr (kExtreme<kKind>) {
-        bool nan = false;
+        };
+        if constexpr (kExtreme<kKind>) {
+          float quick[kW];
 #pragma unroll
-        for (int j = 0; j < kW; ++j) nan = nan || acc[j] != acc[j];
-        if (nan) {
+          for (int j = 0; j < kW; ++j) quick[j] = acc[j];
+          take(quick, [](float a, float v) { return reduce_step_quick<kKind>(a, v); });
+          float any = quick[0];  // NaN if one of them is
 #pragma unroll
-          for (int j = 0; j < kW; ++j) acc[j] = reduce_identity<kKind>();
-          walk([](float a, float v) { return reduce_step<kKind>(a, v); });
+          for (int j = 1; j < kW; ++j) any = reduce_step_quick<kKind>(any, quick[j]);
+          if (any == any) {
+#pragma unroll
+            for (int j = 0; j < kW; ++j) acc[j] = quick[j];
+          } else {
+            bool first = false;
+#pragma unroll
+            for (int j = 0; j < kW; ++j) first = first || (quick[j] != quick[j] && acc[j] == acc[j]);
+            if (first) {
+              take(acc, [](float a, float v) { return reduce_step<kKind>(a, v); });
+            } else {
+#pragma unroll
+              for (int j = 0; j < kW; ++j) acc[j] = quick[j] == quick[j] ? quick[j] : acc[j];
+            }
+          }
+        } else {
+          take(acc, [](float a, float v) { return reduce_step<kKind>(a, v); });
         }
-      }
+        r += kLoads * lanes_y;
+      });
     } else {
       for (uint32_t r = begin + ty; r < end; r += lanes_y)
         acc[0] = reduce_step<kKind>(acc[0], Traits<TIn>::load(x, base + (size_t)r * units));
@@ -340,9 +351,12 @@ void columns_launch(const void *x, void *y, uint32_t outer, uint32_t reduced, ui
   //   f32 [1024, 2048] 7.2 / 6.4 / 6.2, [586, 1072] 8.2 / 7.2 / 7.1, [2000, 2048] 8.4 / 7.8 / 8.2, [1024, 3072] 7.6 / 7.2 / 7.5
   //   f32 [64, 131072] 7.5 / 8.5 / 9.4, [3, 256, 8192] middle axis 6.6 / 7.0 / 7.1, bf16 [8192, 2048] 10.4 / 11.1 / 10.9
   //   f32 [5003, 2560] 15.1 / 14.2 / 14.4, [7000, 2048] 15.7 / 15.1 / 15.2; but [16, 2^20] 15.1 / 17.0 / 17.0
-  // An extremum is six instructions an element and gives memory time enough: two (bf16 [8192, 4096] 23.7, four 26.0).
+  // An extremum of narrow elements has the instructions of its unpacking left and is alike with both (bf16 [8192, 4096]
+  // 22.2 / 22.0, [60000, 512] 22.6 / 23.0): two.  Of f32, from more than eight rows of a lane on: four
+  //   [7000, 2048] 19.1 / 18.4, [16384, 2048] 31.6 / 30.4, [2500, 5120] 18.4 / 17.6, [3000, 8192] 26.0 / 25.8
   const uint64_t blocks = (uint64_t)grid.x * segments;
-  const int most = blocks <= 256 ? 8 : (blocks <= 512 || (blocks >= 1280 && segments > 1 && !kExtreme<kKind>) ? 4 : 2);
+  const bool long_walk = !kExtreme<kKind> || (Traits<TIn>::kSize == 4 && segment_rows > 8u * (kBlockThreads >> log2));
+  const int most = blocks <= 256 ? 8 : (blocks <= 512 || (blocks >= 1280 && segments > 1 && long_walk) ? 4 : 2);
 #define HYLE_COLUMNS(VECTOR, MOST)                                                                                            \
   note_variant<ColumnsTag<VECTOR, MOST>>();                                                                                   \
   hipLaunchKernelGGL((reduce_columns<TIn, TOut, kKind, VECTOR, MOST>), grid, dim3(kBlockThreads), 0, s, x, y, outer, reduced, \

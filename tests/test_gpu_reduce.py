@@ -300,3 +300,29 @@ def test_reduce_extrema_keep_the_bits_of_a_nan_and_tell_the_zeros_apart(dims, ax
         got = to_host(out).view(np.uint32)
         assert got[0] == (0 if kind == RK.kMaximum else 0x80000000) and got[2] == 0x7FA00123 and got[1] == 0xFFC00007
         check(kind, "f32", to_host(out), x, dims, [axis])
+
+
+@pytest.mark.parametrize("dims,axis", [([700, 2564], 1), ([300, 20480], 1), ([3, 400000], 1), ([1500, 700], 0), ([4000, 2048], 0), ([2, 300, 1 << 15], 1)])
+def test_reduce_extrema_meet_a_nan_anywhere(dims, axis):
+    """One signalling NaN per result, in every trip and at every place of a lane's elements; all its lane's later elements
+    are quiet NaNs in the first results, which must not replace it.  Results without one stay numbers."""
+    rng = np.random.default_rng(993)
+    for kind in (RK.kMaximum, RK.kMinimum):
+        x = rng.normal(0, 1, dims).astype(np.float32)
+        lanes = np.moveaxis(x.view(np.uint32), axis, -1)                     # a view: [..., reduced]
+        count, reduced = int(np.prod(dims)) // dims[axis], dims[axis]
+        wanted = np.zeros(count, np.uint32)
+        for i in range(count):
+            if i % 5 == 4:
+                continue
+            at = (i * 37) % reduced if i % 2 else reduced - 1 - (i * 11) % reduced
+            wanted[i] = 0x7FA00001 + i
+            place = np.unravel_index(i, lanes.shape[:-1])
+            lanes[(*place, at)] = wanted[i]
+            if i < 40 and axis == len(dims) - 1:
+                lanes[(*place, slice(at + 1024, None, 1024))] = 0x7FC00001   # 256 or 64 lanes of four elements: the same lane's
+        note(f"reduce {kind.name} {dims} over axis {axis}, a NaN in every trip")
+        (out,) = run(hc.Reduce(kind, hc.Axes.from_([axis]), accumulation_type=F32ACC), to_device(x, "f32"))
+        got = to_host(out).reshape(-1)
+        assert np.array_equal(got.view(np.uint32)[wanted != 0], wanted[wanted != 0])
+        check(kind, "f32", to_host(out), x, dims, [axis])
