@@ -82,19 +82,23 @@ uint32_t blocks_for(uint64_t units) {
   return (uint32_t)(blocks < 1 ? 1 : (blocks > 16384 ? 16384 : blocks));
 }
 
-template <int kUnit, uint32_t kSteps>
-void run_runs(const ConcatOperands &c, uint32_t inputs, uint32_t threads, unsigned char *out, hipStream_t s) {
+// Launch-shape labels
+template <int kUnit> struct ConcatTag {
+  static std::string text() { return "concat_general/" + std::to_string(kUnit) + "-bytes"; }
+};
+template <int kUnit, uint32_t kSteps, uint32_t kThreads> struct ConcatRunsTag {
+  static std::string text() { return "concat_runs/" + std::to_string(kUnit) + "-bytes#" + std::to_string(kSteps) + "x" + std::to_string(kThreads); }
+};
+
+template <int kUnit, uint32_t kSteps, uint32_t kThreads>
+void run_runs(const ConcatOperands &c, uint32_t inputs, unsigned char *out, hipStream_t s) {
+  note_variant<ConcatRunsTag<kUnit, kSteps, kThreads>>();
   uint64_t blocks = 1;  // of the input that needs most
-  for (uint32_t i = 0; i < inputs; ++i) blocks = std::max<uint64_t>(blocks, (c.run_bytes[i] / kUnit + kSteps * threads - 1) / (kSteps * threads) * c.outer);
-  hipLaunchKernelGGL((concat_runs<kUnit, kSteps>), dim3((uint32_t)blocks, inputs), dim3(threads), 0, s, c, out);
+  for (uint32_t i = 0; i < inputs; ++i) blocks = std::max<uint64_t>(blocks, (c.run_bytes[i] / kUnit + kSteps * kThreads - 1) / (kSteps * kThreads) * c.outer);
+  hipLaunchKernelGGL((concat_runs<kUnit, kSteps>), dim3((uint32_t)blocks, inputs), dim3(kThreads), 0, s, c, out);
 }
 
 }  // namespace
-
-// Launch-shape labels
-template <int kUnit, bool kRuns> struct ConcatTag {
-  static std::string text() { return std::string(kRuns ? "concat_runs/" : "concat_general/") + std::to_string(kUnit) + "-bytes"; }
-};
 
 hipError_t launch_concat(const ConcatParams &p, const void *const *inputs, void *out, hipStream_t stream) {
   if (p.elements == 0) return hipSuccess;
@@ -122,15 +126,14 @@ hipError_t launch_concat(const ConcatParams &p, const void *const *inputs, void 
     const uint64_t bytes = p.elements * p.size;
     switch (unit) {
       case 16:
-        note_variant<ConcatTag<16, true>>();
-        if (bytes < (16ull << 20)) run_runs<16, 1>(c, p.inputs, 256, o, stream);
-        else if (bytes < (64ull << 20)) run_runs<16, 4>(c, p.inputs, 256, o, stream);
-        else run_runs<16, 2>(c, p.inputs, 128, o, stream);
+        if (bytes < (16ull << 20)) run_runs<16, 1, 256>(c, p.inputs, o, stream);
+        else if (bytes < (64ull << 20)) run_runs<16, 4, 256>(c, p.inputs, o, stream);
+        else run_runs<16, 2, 128>(c, p.inputs, o, stream);
         break;
-      case 8: note_variant<ConcatTag<8, true>>(); run_runs<8, 4>(c, p.inputs, 256, o, stream); break;
-      case 4: note_variant<ConcatTag<4, true>>(); run_runs<4, 4>(c, p.inputs, 256, o, stream); break;
-      case 2: note_variant<ConcatTag<2, true>>(); run_runs<2, 4>(c, p.inputs, 256, o, stream); break;
-      default: note_variant<ConcatTag<1, true>>(); run_runs<1, 4>(c, p.inputs, 256, o, stream); break;
+      case 8: run_runs<8, 4, 256>(c, p.inputs, o, stream); break;
+      case 4: run_runs<4, 4, 256>(c, p.inputs, o, stream); break;
+      case 2: run_runs<2, 4, 256>(c, p.inputs, o, stream); break;
+      default: run_runs<1, 4, 256>(c, p.inputs, o, stream); break;
     }
     return hipGetLastError();
   }
@@ -147,10 +150,10 @@ hipError_t launch_concat(const ConcatParams &p, const void *const *inputs, void 
   }
   const dim3 grid(blocks_for(most), p.inputs), block(kBlockThreads);
   switch (p.size) {
-    case 8: note_variant<ConcatTag<8, false>>(); hipLaunchKernelGGL((concat_general<8>), grid, block, 0, stream, l, o); break;
-    case 4: note_variant<ConcatTag<4, false>>(); hipLaunchKernelGGL((concat_general<4>), grid, block, 0, stream, l, o); break;
-    case 2: note_variant<ConcatTag<2, false>>(); hipLaunchKernelGGL((concat_general<2>), grid, block, 0, stream, l, o); break;
-    default: note_variant<ConcatTag<1, false>>(); hipLaunchKernelGGL((concat_general<1>), grid, block, 0, stream, l, o); break;
+    case 8: note_variant<ConcatTag<8>>(); hipLaunchKernelGGL((concat_general<8>), grid, block, 0, stream, l, o); break;
+    case 4: note_variant<ConcatTag<4>>(); hipLaunchKernelGGL((concat_general<4>), grid, block, 0, stream, l, o); break;
+    case 2: note_variant<ConcatTag<2>>(); hipLaunchKernelGGL((concat_general<2>), grid, block, 0, stream, l, o); break;
+    default: note_variant<ConcatTag<1>>(); hipLaunchKernelGGL((concat_general<1>), grid, block, 0, stream, l, o); break;
   }
   return hipGetLastError();
 }

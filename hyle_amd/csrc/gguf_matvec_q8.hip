@@ -356,8 +356,8 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_lines(const unsi
 //
 // A block's rows follow one another in memory, and its loads are plain ones, by which the line that two rows or two spans
 // share is fetched once.  kStream, for weights that outgrow the caches: non-temporal loads, and a block takes every
-// gridDim.x-th four rows, so that the blocks walk the weights together.  (A row is 1680 bytes or more: row numbers stay far
-// below 2^32.)
+// gridDim.x-th four rows, so that the blocks walk the weights together.  (A row is 1088 bytes or more, and a weight has
+// fewer than 2^31 values of 1024 or more to a row: row numbers stay far below 2^32.)
 template <int kKind, class TX, int kSpans, bool kShort, bool kStream>
 __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(const unsigned char *weights, const void *x, void *y,
                                                                           uint32_t all_rows, uint32_t block_rows, uint64_t row_stride,
@@ -939,9 +939,10 @@ template <int kKind, int kM, bool kRegisters> struct LinesTag {
     return std::string("gguf_matvec_q8_lines/") + kind_word(kKind) + "/" + std::to_string(kM) + "-tokens" + (kRegisters ? "/registers" : "/lds");
   }
 };
-template <int kKind, int kSpans, bool kShort> struct SpansTag {
+template <int kKind, int kSpans, bool kShort, bool kStream> struct SpansTag {
   static std::string text() {
-    return std::string("gguf_matvec_q8_spans/") + kind_word(kKind) + "/" + std::to_string(kSpans) + "-spans" + (kShort ? "/short" : "");
+    return std::string("gguf_matvec_q8_spans/") + kind_word(kKind) + "/" + std::to_string(kSpans) + "-spans" + (kShort ? "/short" : "") +
+           (kStream ? "#stream" : "");
   }
 };
 template <int kSets, bool kOneBatch> struct TilesTag {
@@ -1391,13 +1392,15 @@ hipError_t run_spans(const MatVecParams &p, const void *w, const void *x, void *
   const unsigned char *in = static_cast<const unsigned char *>(w);
   const uint32_t rows = (uint32_t)p.rows;
 #define HYLE_SPANS(N, SHORT)                                                                                                       \
-  note_variant<SpansTag<kKind, N, SHORT>>();                                                                                       \
-  if (stream)                                                                                                                      \
+  if (stream) {                                                                                                                    \
+    note_variant<SpansTag<kKind, N, SHORT, true>>();                                                                               \
     hipLaunchKernelGGL((gguf_matvec_q8_spans<kKind, TX, N, SHORT, true>), blocks, dim3(N * kWaveLanes), 0, s, in, x, y, rows,       \
                        block_rows, p.row_stride, tail_lanes);                                                                      \
-  else                                                                                                                             \
+  } else {                                                                                                                         \
+    note_variant<SpansTag<kKind, N, SHORT, false>>();                                                                              \
     hipLaunchKernelGGL((gguf_matvec_q8_spans<kKind, TX, N, SHORT, false>), blocks, dim3(N * kWaveLanes), 0, s, in, x, y, rows,      \
-                       block_rows, p.row_stride, tail_lanes)
+                       block_rows, p.row_stride, tail_lanes);                                                                      \
+  }
   if (tail_lanes == kWaveLanes) {
     switch (spans) {
       case 1: HYLE_SPANS(1, false); break;
@@ -1505,7 +1508,7 @@ bool strips_better(const MatVecParams &p, bool vectors) {
   }
   if (!whole) return true;
   // one span of a vocabulary: the tile and quad kernels keep its codes at hand and have no tiles left over
-  const bool span_of_many = p.k > 1792 && p.k <= 2048 && p.rows >= 90000;
+  const bool span_of_many = p.k == 2048 && p.rows >= 90000;
   if (p.kind == 0) return (p.m > 4 && !span_of_many) || p.k > 2048 || p.rows < 6144;
   if (p.kind == 1 && p.m <= 4 && span_of_many) return false;
   return p.m > 2 || p.k < 8 * p.rows;

@@ -17,7 +17,7 @@ namespace hyle_hip {
 // registers itself when the library loads, so the list (hyle_hip_variant_label) holds exactly
 // the launch shapes compiled in.  A label names the shape (lanes x vectors x rows, mask form,
 // exact or masked), not the storage type: tests use it to prove that a case reached the kernel
-// it was written for.
+// it was written for.  What stands behind a '#' tells apart the forms a shape is compiled in.
 namespace variants {
 const char *add(const std::string &label);  // registers a label, returns its stable text
 void note(const char *label);               // the calling thread is about to launch this shape

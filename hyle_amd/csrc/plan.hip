@@ -44,6 +44,7 @@ hyle_hip_status hip_fail(hipError_t error, const char *what) {
 struct VariantList {
   std::mutex mutex;
   std::vector<std::string *> labels;  // never freed: the texts are handed out as C strings
+  std::vector<std::string *> forms;   // the same with what stands behind '#'
 };
 VariantList &variant_list() {
   static VariantList *list = new VariantList;  // outlives every static of the library
@@ -1458,13 +1459,17 @@ bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) &
 
 namespace hyle_hip {
 namespace variants {
+static const char *listed(std::vector<std::string *> *list, const std::string &text) {
+  for (const std::string *known : *list)
+    if (*known == text) return known->c_str();
+  list->push_back(new std::string(text));
+  return list->back()->c_str();
+}
 const char *add(const std::string &label) {
   VariantList &list = variant_list();
   std::lock_guard<std::mutex> lock(list.mutex);
-  for (const std::string *known : list.labels)
-    if (*known == label) return known->c_str();
-  list.labels.push_back(new std::string(label));
-  return list.labels.back()->c_str();
+  listed(&list.labels, label.substr(0, label.find('#')));
+  return listed(&list.forms, label);
 }
 void note(const char *label) {
   // a loop of dispatches of one shape (merge rounds) is one entry
@@ -1682,16 +1687,25 @@ const char *hyle_hip_variant_label(uint32_t index) {
   return index < list.labels.size() ? list.labels[index]->c_str() : "";
 }
 
-const char *hyle_hip_last_launch_variant(void) {
+const char *hyle_hip_launch_form_label(uint32_t index) {
+  VariantList &list = variant_list();
+  std::lock_guard<std::mutex> lock(list.mutex);
+  return index < list.forms.size() ? list.forms[index]->c_str() : "";
+}
+
+// The noted labels, each up to the first character of `end`.
+static const char *noted_text(const char *end) {
   size_t used = 0;
   g_noted_text[0] = 0;
   for (int i = 0; i < g_noted_count; ++i) {
-    const int wrote = snprintf(g_noted_text + used, sizeof g_noted_text - used, "%s%s", i ? " + " : "", g_noted[i]);
+    const int wrote = snprintf(g_noted_text + used, sizeof g_noted_text - used, "%s%.*s", i ? " + " : "", (int)strcspn(g_noted[i], end), g_noted[i]);
     if (wrote < 0 || (size_t)wrote >= sizeof g_noted_text - used) break;
     used += (size_t)wrote;
   }
   return g_noted_text;
 }
+const char *hyle_hip_last_launch_variant(void) { return noted_text("#"); }
+const char *hyle_hip_last_launch_form(void) { return noted_text(""); }
 
 hyle_hip_status hyle_hip_plan_launch(const hyle_hip_plan *plan, const void *const *inputs,
                                      uint32_t input_count, void *const *outputs, uint32_t output_count,

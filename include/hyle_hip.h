@@ -316,11 +316,15 @@ HYLE_HIP_API const char *hyle_hip_plan_route_name(const hyle_hip_plan *plan);
  * hyle_hip_variant_count / hyle_hip_variant_label list them, and hyle_hip_last_launch_variant
  * returns the label(s) of the dispatches the calling thread's last hyle_hip_plan_launch or
  * hyle_hip_plan_launch_static enqueued, joined by " + " (empty when it enqueued nothing; consecutive
- * dispatches of one shape are one entry; at most four entries).  The text stays valid until the
- * thread's next call of the same function. */
+ * dispatches of one shape are one entry; at most four entries).  A shape that is compiled in several
+ * forms, other loads or other steps of a thread, has one label; hyle_hip_launch_form_label (empty past the
+ * last) and hyle_hip_last_launch_form name the form too, behind a '#'.  The texts stay valid until the
+ * thread's next call of either last_launch function. */
 HYLE_HIP_API uint32_t hyle_hip_variant_count(void);
 HYLE_HIP_API const char *hyle_hip_variant_label(uint32_t index);
 HYLE_HIP_API const char *hyle_hip_last_launch_variant(void);
+HYLE_HIP_API const char *hyle_hip_launch_form_label(uint32_t index);
+HYLE_HIP_API const char *hyle_hip_last_launch_form(void);
 
 /* ProviderPreparedVTable::shared_submit
  * (include/hyle/compute/detail/prepared_callbacks.h:26-30): enqueue on `stream`

@@ -8,6 +8,7 @@ import sys
 import numpy as np
 import torch
 
+from hyle_amd import capi
 from hyle_amd import compute as hc
 from hyle_amd import torch_io as tio
 from oracle import lib as orc
@@ -55,10 +56,15 @@ def host_values(array: np.ndarray, tag: str) -> np.ndarray:
     return array if tag == "f32" else orc.from_f32(TYPES[tag][1], array)
 
 
+def last_launch_form() -> str:
+    return capi.load().hyle_hip_last_launch_form().decode()
+
+
 # Labels of the kernel launch shapes the tests of this session launched (hyle_hip_last_launch_variant
 # after every submit): tests/test_zy_launch_shape_coverage.py holds them against the list of shapes
 # compiled into the library.
 LAUNCHED = set()
+FORMS = set()   # the same with the form a shape was launched in (hyle_hip_last_launch_form)
 
 
 def _noting(submit):
@@ -68,6 +74,7 @@ def _noting(submit):
         chosen = hc.last_launch_variant()
         if chosen:
             LAUNCHED.update(chosen.split(" + "))
+            FORMS.update(last_launch_form().split(" + "))
     return noted
 
 

@@ -17,7 +17,7 @@ import torch
 from hyle_amd import compute as hc
 from oracle import lib as orc
 
-from gpu_support import DEVICE, TYPES, context, host_values, note, run, to_device, to_host
+from gpu_support import DEVICE, TYPES, context, host_values, last_launch_form, note, run, to_device, to_host
 from k_quant_support import random_rows
 
 pytestmark = pytest.mark.gpu
@@ -340,3 +340,28 @@ def test_q8_route_one_row_against_more_than_128_mb(tag, rows, k, kernel):
     padded[:, :raw.shape[1]] = raw
     note(f"q8 matvec {tag} rows {rows} k {k}: {rows * stride >> 20} MB")
     check(tag, "bf16", padded, rows, k, rng.normal(0, 1.5, (k,)).astype(np.float32), row_stride=stride, kernel=f"gguf_matvec_q8_spans/{tag}/{kernel}")
+
+
+STREAMED = ([("q6_k", 2048 * n, f"{n}-spans#stream") for n in range(1, 7)] + [("q8_0", 2048 * n, f"{n}-spans#stream") for n in range(1, 7)]
+            + [("q8_0", 2048 * n - (256 if n % 2 else 1792 if n > 1 else 1024), f"{n}-spans/short#stream") for n in range(1, 10)])
+
+
+@pytest.mark.parametrize("tag,k,kernel", STREAMED)
+def test_q8_route_one_row_against_more_than_128_mb_in_every_form(tag, k, kernel):
+    """Every number of spans past the caches: more fours of rows than blocks, a last four of one to three rows, and blocks
+    with one turn fewer than others.  The stride is what makes the weights large."""
+    rng = np.random.default_rng(k)
+    spans = -(-k // 2048)
+    blocks = 256 * (8 // spans if spans <= 8 else 1)
+    rows = max(4 * blocks * 5 // 4 + 1 + spans % 3, 4099)
+    size = raw_bytes_for(tag, rng, 1, k).shape[1]
+    stride = max(-(-size // 16) * 16, (129 << 20) // rows // 16 * 16 + 16)
+    raw = raw_bytes_for(tag, rng, 509, k) if spans % 2 else weights_for(tag, rng, 127, k)
+    padded = np.zeros((rows, stride), np.uint8)
+    padded[:, :size] = np.resize(raw, (rows, size))
+    padded[-3:, :size] = raw_bytes_for(tag, rng, 3, k)                         # the last ones are like no others
+    note(f"q8 matvec {tag} rows {rows} k {k}: {rows * stride >> 20} MB")
+    x_tag = ("bf16", "f32", "f16")[spans % 3] if spans % 2 == 0 else ("bf16", "f32")[spans // 2 % 2]
+    x = rng.normal(0, 1.5, (k,)).astype(np.float32)
+    check(tag, x_tag, padded, rows, k, x, row_stride=stride)
+    assert last_launch_form() == f"gguf_matvec_q8_spans/{tag}/{kernel}"

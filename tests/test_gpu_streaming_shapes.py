@@ -7,7 +7,7 @@ import pytest
 
 from hyle_amd import compute as hc
 
-from gpu_support import assert_bits_equal, note, run, to_device, to_host
+from gpu_support import assert_bits_equal, last_launch_form, note, run, to_device, to_host
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +56,17 @@ def test_concat_runs(outer, first, second, inner):
     (out,) = run(hc.Concat(1), to_device(a, "f32"), to_device(b, "f32"))
     assert hc.last_launch_variant() == "concat_runs/16-bytes"
     assert_bits_equal(to_host(out), np.concatenate([a, b], axis=1))
+
+
+# outputs on both sides of 16 and 64 MiB; units of every width have four to a thread at any size
+@pytest.mark.parametrize("outer,first,second,inner,form", [
+    (3, 5, 1, 4, "16-bytes#1x256"), (4, 8191, 8192, 64, "16-bytes#1x256"), (4, 8192, 8192, 64 * 2, "16-bytes#4x256"), (1, 1, 1 << 16, 64, "16-bytes#4x256"),
+    (4, 32767, 32768, 64, "16-bytes#4x256"), (4, 32768, 32768, 64, "16-bytes#2x128"), (9, 8000, 1333, 256, "16-bytes#2x128"), (70001, 3, 2, 52, "16-bytes#2x128"),
+    (5, 2, 7, 1001, "4-bytes#4x256"), (3, 70000, 30001, 67, "4-bytes#4x256")])
+def test_concat_runs_in_every_form(outer, first, second, inner, form):
+    rng = np.random.default_rng(first)
+    a, b = (rng.integers(0, 1 << 32, (outer, n, inner), dtype=np.uint32).view(np.float32) for n in (first, second))
+    note(f"concat [{outer}, {first} + {second}, {inner}]: {form}")
+    (out,) = run(hc.Concat(1), to_device(a, "f32"), to_device(b, "f32"))
+    assert last_launch_form() == "concat_runs/" + form
+    assert np.array_equal(to_host(out).view(np.uint32), np.concatenate([a, b], axis=1).view(np.uint32))

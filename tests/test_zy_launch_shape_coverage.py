@@ -34,3 +34,16 @@ def test_every_launch_shape_compiled_into_the_library_was_launched_by_a_test():
     compiled = set(hc.launch_variants())
     missing = sorted(compiled - gpu_support.LAUNCHED)
     assert not missing, f"{len(missing)} launch shapes compiled into the library were launched by no test: {missing}"
+
+
+def test_every_form_a_launch_shape_is_compiled_in_was_launched_by_a_test():
+    absent = [name for name in SUITE if name not in sys.modules]
+    if absent:
+        pytest.skip(f"the whole GPU suite did not run in this session (not loaded: {absent})")
+    compiled, label = [], gpu_support.capi.load().hyle_hip_launch_form_label
+    while label(len(compiled)):
+        compiled.append(label(len(compiled)))
+    compiled = {text.decode() for text in compiled}
+    assert {text.split("#")[0] for text in compiled} == set(hc.launch_variants()) and any("#" in text for text in compiled)
+    missing = sorted(compiled - gpu_support.FORMS)
+    assert not missing, f"{len(missing)} forms compiled into the library were launched by no test: {missing}"
