@@ -365,3 +365,42 @@ def test_q8_route_one_row_against_more_than_128_mb_in_every_form(tag, k, kernel)
     x = rng.normal(0, 1.5, (k,)).astype(np.float32)
     check(tag, x_tag, padded, rows, k, x, row_stride=stride)
     assert last_launch_form() == f"gguf_matvec_q8_spans/{tag}/{kernel}"
+
+
+# Products that the strip kernel took over from the kernel named here, which the oracle holds whoever serves them.
+TAKEN_OVER = (("q4_k", "f32", 600, 2048, 2), ("q4_k", "bf16", 600, 2048, 2), ("q4_k", "f32", 2100, 7680, 1), ("q4_k", "bf16", 2100, 7680, 1),
+              ("q8_0", "bf16", 8192, 4096, 4), ("q6_k", "bf16", 8192, 6144, 2), ("q4_k", "bf16", 4096, 3840, 4))
+
+
+@pytest.mark.parametrize("tag,x_tag,rows,k,m", TAKEN_OVER)
+def test_q8_route_products_that_changed_kernels(tag, x_tag, rows, k, m):
+    rng = np.random.default_rng(1821)
+    x = rng.normal(0, 1.5, (m, k) if m > 1 else (k,)).astype(np.float32)
+    note(f"q8 matvec {tag} x {x_tag} rows {rows} k {k} m {m}")
+    check(tag, x_tag, raw_bytes_for(tag, rng, rows, k), rows, k, x)
+
+
+def test_q8_route_q4_k_tiles_seeded_random_shapes_of_what_they_serve():
+    """Sixty seeded draws over every range of rows, widths and activation rows in which the tile kernel is taken: few weight
+    rows of any width, one row up to 10240 values wide, and narrow rows, many of them, against two to four."""
+    rng = np.random.default_rng(1814)
+    for case in range(60):
+        form = case % 3
+        if form == 0:
+            rows, k, m = int(rng.choice([1, 7, 16, 33, 64, 100, 257, 400, 511])), 256 * int(rng.integers(4, 41)), int(rng.integers(1, 9))
+        elif form == 1:
+            rows, k, m = int(rng.integers(512, 6000)), 2048 * int(rng.integers(1, 5)) if case % 2 else 256 * int(rng.integers(4, 9)), 1
+        else:
+            rows, k, m = int(rng.integers(6144, 9000)), 256 * int(rng.integers(4, 9)), int(rng.integers(2, 5))
+        tokens = 1 if m == 1 else (4 if m <= 4 else 8)
+        if (1 + tokens) * k + tokens * k // 256 * 36 + 1024 * max(tokens // 4, 1) > 65536:
+            m, tokens = 1, 1                                   # the codes of more rows would not fit a block's LDS
+        x_tag = ("f32", "bf16", "f16")[case // 3 % 3]
+        pad = int(rng.choice([0, 16, 48]))
+        raw = raw_bytes_for("q4_k", rng, rows, k) if x_tag != "f16" else weights_for("q4_k", rng, min(rows, 300), k)
+        padded = np.zeros((rows, raw.shape[1] + pad), np.uint8)
+        padded[:, :raw.shape[1]] = np.resize(raw, (rows, raw.shape[1]))
+        x = rng.normal(0, 1.5, (m, k) if m > 1 else (k,)).astype(np.float32)
+        note(f"q8 matvec q4_k tiles draw {case}: rows {rows} k {k} m {m} x {x_tag} pad {pad}")
+        check("q4_k", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad)
+        assert hc.last_launch_variant().startswith(f"gguf_matvec_q8_tiles/q4_k/{tokens}-tokens"), (hc.last_launch_variant(), rows, k, m)
