@@ -384,8 +384,8 @@ template <int kLanes> __device__ __forceinline__ uint32_t lanes_max(uint32_t v) 
 
 // 127 / b correctly rounded for b from 2^-60 to 2^61: the hardware's reciprocal, a Newton step and a correction of
 // the quotient by its exact remainder, right for every mantissa of b with a reciprocal up to one unit off.  It is
-// six instructions where the full division, which scales its operands, is eleven.  (1 / b is not to be had this way: for
-// a mantissa of all ones the step ends one unit short.)
+// six instructions where the full division, which scales its operands, is eleven.  (1 / b is not to be had this way
+// without knowing the reciprocal of a mantissa of all ones: from an estimate that is off the steps end one unit short.)
 __device__ __forceinline__ float quotient_of_127(float b) {
   const float rough = __builtin_amdgcn_rcpf(b);
   const float inverse = __builtin_fmaf(__builtin_fmaf(-b, rough, 1.0f), rough, rough);

@@ -382,7 +382,7 @@ def test_q8_route_products_that_changed_kernels(tag, x_tag, rows, k, m):
 
 def test_q8_route_q4_k_tiles_seeded_random_shapes_of_what_they_serve():
     """Sixty seeded draws over every range of rows, widths and activation rows in which the tile kernel is taken: few weight
-    rows of any width, one row up to 10240 values wide, and narrow rows, many of them, against two to four."""
+    rows of any width, one row up to 8192 values wide, and narrow rows, many of them, against two to four."""
     rng = np.random.default_rng(1814)
     for case in range(60):
         form = case % 3

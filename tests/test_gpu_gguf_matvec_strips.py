@@ -238,7 +238,7 @@ def test_strips_rule_for_one_span_of_a_vocabulary(tag, rows, m, kernel):
 def test_strips_scales_of_activation_blocks_are_exact_quotients():
     """A weight row picks one activation block's largest value, whose code is 127: the product is 127 times the block's
     scale, 1 / (127 / largest) in f32, rounded once.  Among the largest values those whose factor has a mantissa of all
-    ones, where a quotient by a corrected reciprocal ends one unit short."""
+    ones, where a quotient by a corrected reciprocal hangs on the reciprocal itself."""
     blocks, m, rows = 16, 8, 512
     raw = np.zeros((rows, blocks, 210), np.uint8)
     quants = np.full(256, 32)

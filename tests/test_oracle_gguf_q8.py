@@ -143,14 +143,21 @@ def test_centre_is_the_product_with_the_dequantised_activations_and_the_bound_ha
             assert np.all(np.abs(centre[i] - exact) <= slack)
 
 
+def fused(a, b, c):
+    """a * b + c of f32 arrays, rounded once: the product is exact in f64, and a sum that is not is rounded to odd there."""
+    product, c = np.asarray(a, np.float64) * np.asarray(b, np.float64), np.asarray(c, np.float64)
+    total = product + c
+    part = total - product
+    error = (product - (total - part)) + (c - part)
+    even = (total.view(np.int64) & 1) == 0
+    return np.where((error != 0) & even, np.nextafter(total, np.where(error > 0, np.inf, -np.inf)), total).astype(np.float32)
+
+
 def test_short_divisions_of_the_activation_blocks_are_exact():
     """127 / b from a reciprocal one unit off on either side, and b / 127, as the strip kernel takes them: correctly
-    rounded for every mantissa of b (the kernel's range of exponents only scales the steps by powers of two).  Each
-    fused step is taken in 64-bit mantissas, which hold its product, and rounded once more to 24."""
-    def fused(a, b, c):
-        return (a.astype(np.longdouble) * b + c).astype(np.float32)
-
-    one = np.float32(1)
+    rounded for every mantissa of b (the kernel's range of exponents only scales the steps by powers of two).  1 / b taken
+    the same way is not, where the reciprocal of a mantissa of all ones is off."""
+    one, wrong = np.float32(1), set()
     for first in range(0, 1 << 23, 1 << 21):
         b = (np.arange(first, first + (1 << 21), dtype=np.uint32) | np.uint32(0x3F800000)).view(np.float32)
         wanted = rn(127.0 / b.astype(np.float64))       # a quotient of 24-bit numbers is no closer than 2^-49 to a tie
@@ -160,7 +167,8 @@ def test_short_divisions_of_the_activation_blocks_are_exact():
             inverse = fused(fused(-b, rough, one), rough, rough)
             q = rn(127.0 * inverse.astype(np.float64))
             assert np.array_equal(fused(fused(-b, q, np.float32(127)), inverse, q), wanted), (first, unit)
-        inverse = np.float32(1) / np.float32(127)
+            wrong |= {(unit, int(v)) for v in b[fused(fused(-b, inverse, one), inverse, inverse) != nearest].view(np.uint32)}
+        inverse = one / np.float32(127)
         q = rn(b.astype(np.float64) * float(inverse))
-        got = fused(fused(np.full_like(b, -127), q, b), np.full_like(b, inverse), q)
-        assert np.array_equal(got, rn(b.astype(np.float64) / 127.0)), first
+        assert np.array_equal(fused(fused(np.float32(-127), q, b), inverse, q), rn(b.astype(np.float64) / 127.0)), first
+    assert wrong == {(-1, 0x3FFFFFFF), (1, 0x3FFFFFFF)}
