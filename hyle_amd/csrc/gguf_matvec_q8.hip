@@ -1369,16 +1369,17 @@ hipError_t run_registers(const MatVecParams &p, const void *w, const void *x, vo
 // 25 of 27 shapes (three formats, K = 2048 ... 12288, 1024 ... 151936 rows: 0-30 % below the
 // kernel that parks the codes in LDS first).
 //
-// A block takes neighbouring rows.  MI355X, bf16, us, rows dealt out one by one with non-temporal loads / neighbouring
-// rows, non-temporal / plain:
-//   Q6_K [6144 -> 2048] 5.9 / 5.6 / 5.2   [4096 -> 8192] 8.7 / 8.4 / 7.9   [2048 -> 2048] 4.7 / 4.7 / 4.2
-//   Q8_0 [5120 -> 17408] (95 MB) 18.0 / 17.9 / 16.8   [17408 -> 5120] 18.9 / 18.4 / 17.6   [7168 -> 3072] 7.8 / 7.5 / 6.8
-//   Q6_K [2048 -> 151936] (255 MB) 47.8 / 46.2 / 51.0   Q8_0 [2048 -> 100000] (218 MB) 36.5 / 36.3 / 42.2
-// Large ones non-temporally, one by one / one run of rows to a block / four rows to a block in turn:
-//   Q8_0 [2048 -> 151936] (331 MB) 53.4 / 56.7 / 52.4   [1024 -> 151936] 35.4 / 37.9 / 34.4   [2560 -> 77056] 38.6 / 37.3 / 37.0
-//   Q6_K [2048 -> 151936] 47.1 / 46.4 / 46.4   f16 [2048 -> 100001] 33.0 / 32.7 / 31.8
-// (16 waves per compute unit with plain loads: 5.6, 8.5, 4.2, 17.8, 17.6, 7.2, 52, 43, 41)
-constexpr uint64_t kSpansStream = 128ull << 20;
+// A block takes one run of neighbouring rows with plain loads, or, from 32 MiB of weights on, four rows in turn with
+// non-temporal ones.  MI355X, bf16, us, rows dealt out one by one (non-temporally) / one run / four in turn; weights that
+// come from HBM, 700 MB of them in turn, as a model's do whose every weight is read once for a token:
+//   Q6_K [2048 -> 2048] 5.4 / 4.5 / 4.8   [6144 -> 2048] 6.4 / 5.7 / 5.9   [4096 -> 8192] (26 MB) 8.5 / 8.2 / 8.3
+//     [6144 -> 8192] (39 MB) 11.6 / 11.3 / 11.0   [2048 -> 32768] 13.1 / 13.1 / 12.6   [2048 -> 70000] 23.5 / 24.5 / 22.6
+//   Q8_0 [2048 -> 6144] 6.0 / 5.3 / 5.8   [7168 -> 3072] (22 MB) 7.8 / 7.2 / 7.1   [4096 -> 8192] (34 MB) 8.7 / 9.3 / 8.5
+//     [3072 -> 20000] (62 MB) 13.1 / 16.5 / 12.8   [17408 -> 5120] (90 MB) 18.7 / 19.8 / 17.6   [5120 -> 17408] 18.0 / 18.8 / 16.6
+//   Q8_0 [2048 -> 151936] (331 MB) 53.4 / 56.7 / 52.4   Q6_K 47.1 / 46.4 / 46.4
+// Weights that the memory-side cache holds (200 MB in turn) go on to gain from plain loads up to 64 MB: Q8_0 [4096 -> 8192]
+// 8.5 / 7.9 / 8.3, [2048 -> 32768] 13.5 / 12.9 / 13.1, [5120 -> 17408] 17.7 / 16.7 / 16.3, Q6_K [2048 -> 32768] 12.8 / 11.5 / 12.4.
+constexpr uint64_t kSpansStream = 32ull << 20;
 
 template <int kKind, class TX>
 hipError_t run_spans(const MatVecParams &p, const void *w, const void *x, void *y, uint32_t spans, uint32_t tail_lanes,

@@ -367,6 +367,19 @@ def test_q8_route_one_row_against_more_than_128_mb_in_every_form(tag, k, kernel)
     assert last_launch_form() == f"gguf_matvec_q8_spans/{tag}/{kernel}"
 
 
+@pytest.mark.parametrize("tag,rows,k", [("q6_k", 4093, 2048), ("q6_k", 1031, 6144), ("q8_0", 2051, 4096), ("q8_0", 517, 5120)])
+def test_q8_route_spans_are_streamed_from_32_mib_on(tag, rows, k):
+    """Weights that come from HBM: one run of rows to a block up to 32 MiB, four rows in turn above."""
+    rng = np.random.default_rng(1815)
+    raw = weights_for(tag, rng, rows, k)
+    for stride, streamed in (((32 << 20) // rows // 16 * 16, False), ((32 << 20) // rows // 16 * 16 + 16, True)):
+        padded = np.zeros((rows, stride), np.uint8)
+        padded[:, :raw.shape[1]] = raw
+        note(f"q8 matvec {tag} rows {rows} k {k}: {rows * stride} bytes")
+        check(tag, "bf16", padded, rows, k, rng.normal(0, 1.5, (k,)).astype(np.float32), row_stride=stride)
+        assert last_launch_form().startswith("gguf_matvec_q8_spans/") and last_launch_form().endswith("#stream") == streamed
+
+
 # Products that the strip kernel took over from the kernel named here, which the oracle holds whoever serves them.
 TAKEN_OVER = (("q4_k", "f32", 600, 2048, 2), ("q4_k", "bf16", 600, 2048, 2), ("q4_k", "f32", 2100, 7680, 1), ("q4_k", "bf16", 2100, 7680, 1),
               ("q8_0", "bf16", 8192, 4096, 4), ("q6_k", "bf16", 8192, 6144, 2), ("q4_k", "bf16", 4096, 3840, 4))
