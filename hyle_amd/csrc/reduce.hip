@@ -116,8 +116,16 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_rows(const void *x, void
           return from;
         };
         const float quick = taken(acc, [](float a, float v) { return reduce_step_quick<kKind>(a, v); });
-        if (!kExtreme<kKind> || quick == quick) acc = quick;
-        else if (acc == acc) acc = taken(acc, [](float a, float v) { return reduce_step<kKind>(a, v); });
+        if (!kExtreme<kKind> || __ballot(quick != quick) == 0) {  // (branches of the wave: nothing to select, nothing done ahead)
+          acc = quick;
+        } else if (__ballot(quick != quick && acc == acc) == 0) {
+          acc = acc == acc ? quick : acc;
+        } else {
+          // unpacked again from the raw words: 109 registers instead of 70 where the unpacked ones are kept for this
+#pragma unroll
+          for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
+          acc = taken(acc, [](float a, float v) { return reduce_step<kKind>(a, v); });
+        }
         vec += kLoads * kLanes;
       });
     } else {
@@ -186,7 +194,7 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_columns(const void *x, v
           float any = quick[0];  // NaN if one of them is
 #pragma unroll
           for (int j = 1; j < kW; ++j) any = reduce_step_quick<kKind>(any, quick[j]);
-          if (any == any) {
+          if (__ballot(any != any) == 0) {
 #pragma unroll
             for (int j = 0; j < kW; ++j) acc[j] = quick[j];
           } else {
@@ -194,6 +202,8 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_columns(const void *x, v
 #pragma unroll
             for (int j = 0; j < kW; ++j) first = first || (quick[j] != quick[j] && acc[j] == acc[j]);
             if (first) {
+#pragma unroll
+              for (uint32_t i = 0; i < kLoads; ++i) loads_issued(raw[i]);
               take(acc, [](float a, float v) { return reduce_step<kKind>(a, v); });
             } else {
 #pragma unroll
