@@ -22,19 +22,19 @@ struct ConcatOperands {
 // Dense inputs: kUnit bytes per thread step (16 when every run, offset and pointer allows it,
 // otherwise the element size).  grid.y is the input; a block takes up to kSteps units per thread of
 // one run, so the run and the place in it come from one division per block.
-template <int kUnit, uint32_t kSteps>
-__global__ __launch_bounds__(kBlockThreads) void concat_runs(ConcatOperands p, unsigned char *out) {
+template <int kUnit, uint32_t kSteps, uint32_t kThreads>
+__global__ __launch_bounds__(kThreads) void concat_runs(ConcatOperands p, unsigned char *out) {
   const uint32_t input = blockIdx.y;
   const uint32_t units_per_run = (uint32_t)(p.run_bytes[input] / kUnit);
   if (units_per_run == 0) return;
-  const uint32_t blocks_per_run = (units_per_run + kSteps * blockDim.x - 1) / (kSteps * blockDim.x);
+  const uint32_t blocks_per_run = (units_per_run + kSteps * kThreads - 1) / (kSteps * kThreads);
   const uint32_t run = blockIdx.x / blocks_per_run, piece = blockIdx.x - run * blocks_per_run;
   if (run >= p.outer) return;
   const unsigned char *from = p.base[input] + (uint64_t)run * p.run_bytes[input];
   unsigned char *to = out + (uint64_t)run * p.out_pitch + p.offset_bytes[input];
 #pragma unroll
   for (uint32_t j = 0; j < kSteps; ++j) {
-    const uint32_t u = (piece * kSteps + j) * blockDim.x + threadIdx.x;
+    const uint32_t u = (piece * kSteps + j) * kThreads + threadIdx.x;
     if (u >= units_per_run) break;
     if constexpr (kUnit == 16) store16_stream(to, u, load16_stream(from, u));
     else if constexpr (kUnit == 8) reinterpret_cast<uint64_t *>(to)[u] = reinterpret_cast<const uint64_t *>(from)[u];
@@ -95,7 +95,7 @@ void run_runs(const ConcatOperands &c, uint32_t inputs, unsigned char *out, hipS
   note_variant<ConcatRunsTag<kUnit, kSteps, kThreads>>();
   uint64_t blocks = 1;  // of the input that needs most
   for (uint32_t i = 0; i < inputs; ++i) blocks = std::max<uint64_t>(blocks, (c.run_bytes[i] / kUnit + kSteps * kThreads - 1) / (kSteps * kThreads) * c.outer);
-  hipLaunchKernelGGL((concat_runs<kUnit, kSteps>), dim3((uint32_t)blocks, inputs), dim3(kThreads), 0, s, c, out);
+  hipLaunchKernelGGL((concat_runs<kUnit, kSteps, kThreads>), dim3((uint32_t)blocks, inputs), dim3(kThreads), 0, s, c, out);
 }
 
 }  // namespace
@@ -119,15 +119,22 @@ hipError_t launch_concat(const ConcatParams &p, const void *const *inputs, void 
         wide = wide && (c.run_bytes[i] | c.offset_bytes[i] | reinterpret_cast<uintptr_t>(inputs[i])) % 16 == 0;
     }
     const int unit = wide ? 16 : p.size;
-    // One unit per thread below 16 MB of output, where the launch is spread thin and each step would be a
-    // wait of its own ([10, 22 + 1132, 64] f32, 3 MB, 2.5 us against 3.8 with four); four up to 64 MB
-    // ([16, 3072 + 1024, 128] bf16, 17 MB, 7.6 us against 7.9 with two); two in blocks of 128 threads above
-    // ([32, 8000 + 3000, 256] bf16, 180 MB, 58.5 us against 63.7 with four in blocks of 256, 71 with one in blocks of 64).
+    // One unit per thread below 15 MiB of output, where the launch is spread thin and each step would be a
+    // wait of its own ([10, 22 + 1132, 64] f32, 3 MB, 2.5 us against 3.8 with four), unless many short runs give blocks
+    // enough; two in blocks of 128 threads from 64 MiB on ([32, 8000 + 3000, 256] bf16, 180 MB, 58.5 us against 63.7 with
+    // four in blocks of 256, 71 with one in blocks of 64), unless runs are so short that most of such blocks have nothing to
+    // do ([20000, 8 + 24, 64] f32 59.7 against 52.9); four otherwise ([16, 3072 + 1024, 128] bf16, 17 MB, 7.6 us against 7.9 with
+    // two, [16, 3072 + 1024, 127], 16.7 MB, against 8.0 with one).
     const uint64_t bytes = p.elements * p.size;
+    uint64_t shortest = ~0ull, quads = 0;  // bytes of a run; blocks with four units per thread
+    for (uint32_t i = 0; i < p.inputs; ++i) {
+      if (c.run_bytes[i] != 0) shortest = std::min(shortest, c.run_bytes[i]);
+      quads += (c.run_bytes[i] / 16 + 1023) / 1024 * c.outer;
+    }
     switch (unit) {
       case 16:
-        if (bytes < (16ull << 20)) run_runs<16, 1, 256>(c, p.inputs, o, stream);
-        else if (bytes < (64ull << 20)) run_runs<16, 4, 256>(c, p.inputs, o, stream);
+        if (bytes < (15ull << 20) && quads < 2048) run_runs<16, 1, 256>(c, p.inputs, o, stream);
+        else if (bytes < (64ull << 20) || shortest < 16384) run_runs<16, 4, 256>(c, p.inputs, o, stream);
         else run_runs<16, 2, 128>(c, p.inputs, o, stream);
         break;
       case 8: run_runs<8, 4, 256>(c, p.inputs, o, stream); break;

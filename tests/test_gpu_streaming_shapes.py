@@ -58,10 +58,12 @@ def test_concat_runs(outer, first, second, inner):
     assert_bits_equal(to_host(out), np.concatenate([a, b], axis=1))
 
 
-# outputs on both sides of 16 and 64 MiB; units of every width have four to a thread at any size
+# outputs on both sides of 15 and 64 MiB, runs on both sides of 16 KiB, many short ones; units of every width have four to a
+# thread at any size
 @pytest.mark.parametrize("outer,first,second,inner,form", [
-    (3, 5, 1, 4, "16-bytes#1x256"), (4, 8191, 8192, 64, "16-bytes#1x256"), (4, 8192, 8192, 64 * 2, "16-bytes#4x256"), (1, 1, 1 << 16, 64, "16-bytes#4x256"),
-    (4, 32767, 32768, 64, "16-bytes#4x256"), (4, 32768, 32768, 64, "16-bytes#2x128"), (9, 8000, 1333, 256, "16-bytes#2x128"), (70001, 3, 2, 52, "16-bytes#2x128"),
+    (3, 5, 1, 4, "16-bytes#1x256"), (4, 7679, 7680, 64, "16-bytes#1x256"), (4, 7680, 7680, 64, "16-bytes#4x256"), (1, 1, 1 << 16, 64, "16-bytes#4x256"),
+    (4, 32767, 32768, 64, "16-bytes#4x256"), (4, 32768, 32768, 64, "16-bytes#2x128"), (9, 8000, 1333, 256, "16-bytes#2x128"),
+    (70, 16, 1000, 256, "16-bytes#2x128"), (70, 15, 1000, 256, "16-bytes#4x256"), (1023, 3, 2, 52, "16-bytes#1x256"), (1024, 3, 2, 52, "16-bytes#4x256"),
     (5, 2, 7, 1001, "4-bytes#4x256"), (3, 70000, 30001, 67, "4-bytes#4x256")])
 def test_concat_runs_in_every_form(outer, first, second, inner, form):
     rng = np.random.default_rng(first)
