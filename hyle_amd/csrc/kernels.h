@@ -178,7 +178,7 @@ hipError_t launch_argmax(Elem type, const ArgmaxParams &p, const void *x, void *
 // TopK(count = k) along any axis of a plain tensor: sorted tiles, then merges of k-key lists
 // through the workspace.
 struct TopKParams {
-  uint32_t rows = 0, width = 0, count = 0, inner = 1;
+  uint32_t rows = 0, width = 0, count = 0, inner = 1, element_bytes = 4;
   bool largest = true;
   bool dense_last = false;  // dense tensor, axis innermost
   bool bytewise = false;    // strides that are not multiples of the element size

@@ -1070,6 +1070,7 @@ hyle_hip_status admit(hyle_hip_plan *p) {
       t.rank = in[0].rank;
       t.axis = axis;
       const int64_t size = (int64_t)dtype_size(in[0].dtype);
+      t.element_bytes = (uint32_t)size;
       for (int a = 0; a < in[0].rank; ++a) {
         t.dims[a] = (uint32_t)in[0].dims[a];
         t.strides[a] = in[0].byte_strides[a];

@@ -987,7 +987,15 @@ uint32_t topk_max_count() { return kTile / 2; }  // above it: sorted runs merged
 //   bf16 [3, 50001] 64 best 12.3 / 11.1, [2, 77255] 20 10.1 / 9.1, f16 [7, 62798] 40 11.8 / 10.5, f32 [1, 128000] 64 11.5 / 10.8,
 //   [16, 120000] 40 11.7 / 11.3, [64, 62800] 20 11.7 / 11.4; but f32 [3, 151936] 20 9.4 / 12.1, bf16 [1, 151936] 64 12.1 / 22.9,
 //   [60, 32000] 100 16.4 / 18.0, [30, 130000] 100 17.1 / 19.5
+// A last tile that leaves a wave without its share of the bound takes the general form, which the launch then waits for:
+// not where the halved tiles have such a last one and the whole ones do not (bf16 [1, 62800], 1360 elements in vectors
+// of eight over, 4 best 8.6 / 11.4, 64 11.6 / 13.2, [64, 62800] 20 11.8 / 14.7; both have one: bf16 [1, 9000] 13.1 / 11.7).
+bool short_last_tile(const TopKParams &p, uint32_t tile) {
+  const uint32_t vec = p.dense_last && p.width % (16 / p.element_bytes) == 0 ? 16 / p.element_bytes : 1, rest = p.width % tile;
+  return rest != 0 && rest < (kBlockThreads - kWaveLanes + (p.count + 3) / 4) * vec;
+}
 bool few_select_blocks(const TopKParams &p) {
+  if (short_last_tile(p, kBlockThreads * 16) && !short_last_tile(p, kBlockThreads * 32)) return false;
   const uint64_t tiles = (p.width + kBlockThreads * 16 - 1) / (kBlockThreads * 16);
   return p.width > kBlockThreads * 32 && tiles <= 32 && p.rows * tiles <= 1024 && p.count <= kWaveLanes;
 }

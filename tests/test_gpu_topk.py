@@ -286,3 +286,17 @@ def test_topk_tiles_of_4096_and_of_8192_elements(tag):
         outputs = run(hc.TopK(count=50, axis=0), to_device(stored, tag))
         assert "topk_select/16x256/scalar" in hc.last_launch_variant()
         check(tag, stored, dims, 50, 0, True, outputs)
+
+
+@pytest.mark.parametrize("tag,width,count,tile", [("bf16", 62800, 20, 32), ("bf16", 61440 + 1568, 20, 32), ("bf16", 61440 + 1576, 20, 16), ("f16", 12288 + 800, 40, 32),
+                                                 ("f32", 61440 + 784, 20, 32), ("f32", 61440 + 788, 20, 16), ("bf16", 9000, 20, 16), ("bf16", 62801, 20, 16),
+                                                 ("bf16", 61440 + 197, 20, 16), ("bf16", 61440 + 195, 20, 32)])
+def test_topk_halved_tiles_do_not_leave_a_last_one_that_lacks_a_wave(tag, width, count, tile):
+    """A tile's bound takes every wave's best; vectors of a short last tile reach only the first threads."""
+    rng = np.random.default_rng(1161)
+    for rows in (1, 3):
+        stored = host_values(rng.normal(0, 3, (rows, width)).astype(np.float32), tag)
+        note(f"topk {tag} [{rows}, {width}] count {count}: tiles of {256 * tile}")
+        outputs = run(hc.TopK(count=count), to_device(stored, tag))
+        assert hc.last_launch_variant().startswith(f"topk_select/{tile}x256/"), hc.last_launch_variant()
+        check(tag, stored, [rows, width], count, -1, True, outputs)
