@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kBlockThreads) void rope_vectors(RopeOperands p, co
 // The same with the phases of a step taken once for all its rows: a block owns `steps_per_block`
 // consecutive sequence steps (all `inner` rows of each, contiguous in memory), leaves cos and sin
 // of their pairs in LDS and then walks the steps' vector places, a thread per place and row.
-template <class T, bool kHalfSplit>
+template <class T, bool kHalfSplit, bool kEarly>
 __global__ __launch_bounds__(kBlockThreads) void rope_steps(RopeOperands p, const void *in, void *out, uint32_t vectors_per_row,
                                                             uint32_t places, uint32_t steps_per_block, uint32_t steps) {
   extern __shared__ float table[];  // per step of the block: cos of the pairs, then sin
@@ -147,9 +147,10 @@ __global__ __launch_bounds__(kBlockThreads) void rope_steps(RopeOperands p, cons
     }
     return unit;
   };
-  // (the first one's before the phases; a thread without one asks for the block's first)
+  // (kEarly: the first one's before the phases; a thread without one asks for the block's first)
   uint32_t u = threadIdx.x;
-  Unit current = fetch(u < total ? u : 0);
+  Unit current{};
+  if constexpr (kEarly) current = fetch(u < total ? u : 0);
   for (uint32_t i = threadIdx.x; i < own * p.pairs; i += kBlockThreads) {
     const uint32_t local = i / p.pairs, pair = i - local * p.pairs;
     const uint32_t step_index = first_step + local, step = step_index % p.sequence;
@@ -161,6 +162,7 @@ __global__ __launch_bounds__(kBlockThreads) void rope_steps(RopeOperands p, cons
   }
   __syncthreads();
   if (u >= total) return;
+  if constexpr (!kEarly) current = fetch(u);
   while (true) {
     const uint32_t following = u + kBlockThreads;
     Unit next = current;
@@ -221,8 +223,10 @@ __global__ __launch_bounds__(kBlockThreads) void rope_elements(RopeOperands p, c
 }
 
 // Launch-shape labels
-template <int kForm, bool kHalfSplit> struct RopeTag {  // 0 steps, 1 vectors
-  static std::string text() { return std::string(kForm == 0 ? "rope_steps/" : "rope_vectors/") + (kHalfSplit ? "half-split" : "interleaved"); }
+template <int kForm, bool kHalfSplit, bool kLate = false> struct RopeTag {  // 0 steps, 1 vectors
+  static std::string text() {
+    return std::string(kForm == 0 ? "rope_steps/" : "rope_vectors/") + (kHalfSplit ? "half-split" : "interleaved") + (kLate ? "#late" : "");
+  }
 };
 struct RopeElementsTag {
   static std::string text() { return "rope_elements"; }
@@ -250,19 +254,31 @@ hipError_t run_rope(const RopeParams &p, const void *in, const void *positions, 
       // rotary 32 (160 of 256 threads) 4.4 / 5.3, but [1, 6606, 20, 128] f16 (160 of 256) 15.8 / 15.1; 16.0 with 128
       // places, 14.9 us for the first when every thread takes cos and sin itself for eight rows, 31.2 us when it does
       // so for each row; the plain copy of the same bytes 11.1 us.
+      // Neighbouring pairs fill more of their places, and blocks of one step are the worse there from 8 MiB on where they
+      // are not full, from 20 MiB on where they are ([1, 4138, 14, 96] bf16 7.4 / 6.4, [1, 8192, 16, 128] 14.9 / 14.0).
+      // Loads after the phases in the half-split form of large launches and of those with idle threads, which have
+      // other blocks' loads under way while a block takes its phases: before / after them bf16 [1, 8192, 32, 128] 25.4 /
+      // 24.3, [1, 8192, 12, 256] 20.3 / 19.0, [1, 6606, 20, 128] 15.1 / 14.5, f32 [1, 8192, 16, 128] 25.0 / 24.2, [1, 3000, 20, 128]
+      // 13.4 / 12.9 (below: bf16 [1, 8192, 14, 96], 22 MB, 11.8 / 13.9, f32 [1, 8192, 8, 128] 12.8 / 13.3).
       const uint32_t per_step = p.inner * places;
-      const bool idle = 256 / per_step * per_step < 192 && p.rows * p.depth * Traits<T>::kSize > (16ull << 20);
-      uint32_t per_block = (idle ? 512 : 256) / per_step;
+      const uint64_t bytes = p.rows * p.depth * Traits<T>::kSize;
+      const bool idle = 256 / per_step * per_step < 192 && bytes > ((p.half_split ? 16ull : 8ull) << 20);
+      const bool late = p.half_split && (idle || bytes > (46ull << 20));
+      const bool pair_of_steps = !p.half_split && 256 / per_step == 1 && bytes > (20ull << 20);
+      uint32_t per_block = (idle || late || pair_of_steps ? 512 : 256) / per_step;
       per_block = per_block < 1 ? 1 : per_block;
       while (per_block > 1 && (size_t)per_block * p.rotary * sizeof(float) > 32768) --per_block;
       const size_t lds = (size_t)per_block * p.rotary * sizeof(float);
       const dim3 grid((uint32_t)((steps + per_block - 1) / per_block));
-      if (p.half_split) {
+      if (late) {
+        note_variant<RopeTag<0, true, true>>();
+        hipLaunchKernelGGL((rope_steps<T, true, false>), grid, block, lds, stream, o, in, out, per_row, places, per_block, (uint32_t)steps);
+      } else if (p.half_split) {
         note_variant<RopeTag<0, true>>();
-        hipLaunchKernelGGL((rope_steps<T, true>), grid, block, lds, stream, o, in, out, per_row, places, per_block, (uint32_t)steps);
+        hipLaunchKernelGGL((rope_steps<T, true, true>), grid, block, lds, stream, o, in, out, per_row, places, per_block, (uint32_t)steps);
       } else {
         note_variant<RopeTag<0, false>>();
-        hipLaunchKernelGGL((rope_steps<T, false>), grid, block, lds, stream, o, in, out, per_row, places, per_block, (uint32_t)steps);
+        hipLaunchKernelGGL((rope_steps<T, false, true>), grid, block, lds, stream, o, in, out, per_row, places, per_block, (uint32_t)steps);
       }
       return hipGetLastError();
     }

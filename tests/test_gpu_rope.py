@@ -12,7 +12,7 @@ import torch
 from hyle_amd import compute as hc
 from oracle import lib as orc
 
-from gpu_support import DEVICE, TYPES, context, note, to_device, to_host
+from gpu_support import DEVICE, TYPES, context, last_launch_form, note, to_device, to_host
 
 pytestmark = pytest.mark.gpu
 
@@ -129,3 +129,18 @@ def test_prefill_sized_rotation():
     values = rng.normal(0, 1, (1, 8192, 16, 128)).astype(np.float32)
     base = (1000000.0 ** (-np.arange(64) / 64.0)).astype(np.float32)
     check("bf16", values, np.arange(8192, dtype=np.int32), base, 128, 1, True)
+
+
+@pytest.mark.parametrize("tag,sequence,heads,depth,rotary,half_split,form", [
+    ("f32", 7850, 12, 128, 128, True, "half-split"), ("f32", 7851, 12, 128, 128, True, "half-split#late"),       # 46 MiB
+    ("bf16", 3276, 20, 128, 128, True, "half-split"), ("bf16", 3277, 20, 128, 128, True, "half-split#late"),     # 16 MiB, 160 of 256 places
+    ("f16", 3277, 20, 128, 96, True, "half-split"), ("bf16", 3121, 14, 96, 96, False, "interleaved"), ("f16", 5121, 16, 128, 64, False, "interleaved")])
+def test_blocks_of_one_and_two_steps_and_loads_before_and_after_the_phases(tag, sequence, heads, depth, rotary, half_split, form):
+    rng = np.random.default_rng(sequence)
+    values = rng.normal(0, 1, (1, sequence, heads, depth)).astype(np.float32)
+    positions = rng.integers(0, 1 << 14, sequence).astype(np.int32)
+    frequencies = (10000.0 ** (-np.arange(rotary // 2) / (rotary // 2))).astype(np.float32)
+    for in_place in (False, True):
+        note(f"rope {tag} [1, {sequence}, {heads}, {depth}] rotary {rotary} {form} in place {in_place}")
+        check(tag, values, positions, frequencies, rotary, sequence_axis=1, half_split=half_split, in_place=in_place)
+        assert last_launch_form() == "rope_steps/" + form
