@@ -25,7 +25,12 @@ namespace {
 // Too few rows for the waves of a row to be better spent on other rows: a row of more than 256 vectors is 256 lanes'
 // there (us, there / here: RMSNorm bf16 [5, 5120] 2.5 / 2.7, [1, 5120] 2.4 / 2.5; LayerNorm f32 [16, 3000] 2.9 / 2.75).
 // Up to 256 vectors are one wave's in any case, there of two rows: [1, 2048] 2.55 / 2.0, f32 [1, 1024] 2.3 / 1.9.
-inline bool enough_rows(uint64_t rows, uint32_t per_lane) { return per_lane <= 4 ? rows == 1 || rows >= 4 : rows >= 16; }
+// Rows of narrow elements of nine vectors a lane and more are the masked shapes' from 32 rows up to as many as a wave for each
+// vector wants (bf16 [64, 5600] 3.0 / 3.25, [501, 4112] 3.95 / 4.1, [700, 5600] 4.3 / 4.55, [1000, 5600] 5.4 / 5.2).
+inline bool enough_rows(uint64_t rows, uint32_t per_lane, int size) {
+  if (size == 2 && per_lane >= 9 && rows >= 32 && rows < 64u * per_lane) return false;
+  return per_lane <= 4 ? rows == 1 || rows >= 4 : rows >= 16;
+}
 
 template <bool kLayer, int kVpl, int kThreads, int kRows> struct TailTag {
   static std::string text() {
@@ -52,11 +57,18 @@ void launch_tail(const NormParams &p, const Bound &io, int parameters, hipStream
                        io.y, rows, row_vectors, width, p.epsilon);
 }
 
+// False: nothing was launched, the masked shapes are the faster.
 template <class T, class W, bool kLayer, int kVpl>
 bool run_tail(const NormParams &p, const Bound &io, int parameters, hipStream_t s) {
-  const uint64_t bytes = p.shape.rows * p.shape.width * Traits<T>::kSize;
-  const bool once = bytes >= (20ull << 20) && bytes <= (64ull << 20);
+  const uint64_t rows = p.shape.rows, bytes = rows * p.shape.width * Traits<T>::kSize;
+  // two rows per wave also where a smaller launch has more rows than waves find room at once (f32 LayerNorm [5000, 520],
+  // masked / one row / two rows 5.6 / 6.3 / 5.3, [5000, 1000] 8.3 / 9.6 / 7.8, [9001, 520] 8.3 / 9.5 / 8.0; [2500, 520] 4.6 / 4.0 / 4.2)
+  const bool once = (bytes >= (20ull << 20) || rows >= (Traits<T>::kSize == 4 ? 4000u : 7000u)) && bytes <= (64ull << 20);
   if constexpr (kVpl == 2) {
+    // 2048 blocks of four rows find room at once, of a LayerNorm in f32 1536, and a launch of a few more is the masked shape's, of
+    // two rows per wave, up to 20 MiB (masked / here: RMSNorm f32 [9001, 512] 7.0 / 7.75, [12000, 400] 7.2 / 8.5, [12000, 508] 11.3 / 10.1, [20001, 508]
+    // 19.4 / 15.4, [5500, 508] 5.8 / 5.2; LayerNorm bf16 [9001, 1024] 7.7 / 8.8, f32 [7000, 400] 5.35 / 6.1)
+    if (rows > (kLayer && Traits<T>::kSize == 4 ? 6144u : 8192u) && bytes < (20ull << 20)) return false;
     launch_tail<T, W, kLayer, kVpl, 256, 1>(p, io, parameters, s);
   } else if constexpr (!kLayer && kVpl == 4) {
     if (once) return false;
@@ -65,6 +77,9 @@ bool run_tail(const NormParams &p, const Bound &io, int parameters, hipStream_t 
     if (once) launch_tail<T, W, kLayer, kVpl, 64, 2>(p, io, parameters, s);
     else launch_tail<T, W, kLayer, kVpl, 64, 1>(p, io, parameters, s);
   } else {
+    // 5120 waves of these find room at once (masked / here: bf16 [6001, 1600] 7.9 / 9.4, [6001, 2000] 9.8 / 11.2, [5000, 2000]
+    // 8.7 / 8.3, [7101, 2000] alike)
+    if (kVpl == 4 && rows > 5120 && rows <= 6656) return false;
     launch_tail<T, W, kLayer, kVpl, 64, 1>(p, io, parameters, s);
   }
   return true;
@@ -75,7 +90,7 @@ bool run_tail_shape(const NormParams &p, const Bound &io, hipStream_t s) {
   constexpr uint32_t kVec = Traits<T>::kVec;
   if (p.shape.width % kVec != 0) return false;
   const uint32_t per_lane = (p.shape.width / kVec + kWaveLanes - 1) / kWaveLanes;
-  if (!enough_rows(p.shape.rows, per_lane)) return false;
+  if (!enough_rows(p.shape.rows, per_lane, Traits<T>::kSize)) return false;
   const int parameters = !p.has_weight ? kPlain : (kLayer && p.has_bias ? kScaleBias : kScale);
   switch (per_lane) {
     case 2: return run_tail<T, W, kLayer, 2>(p, io, parameters, s);

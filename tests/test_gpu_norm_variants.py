@@ -180,6 +180,18 @@ for _k in range(2, 13):
 CASES += [("rms", "f32", 1, 1024, "norm_rows_tail/rms/64x4/64/1"), ("layer", "bf16", 1, 1032, "norm_rows_tail/layer/64x3/64/1"),
           ("layer", "bf16", 5, 1536, "norm_rows_tail/layer/64x3/64/1"), ("rms", "bf16", 4097, 2568, "norm_rows_tail/rms/64x6/64/2"),
           ("rms", "bf16", 4001, 5640, "norm_rows_tail/rms/64x12/64/2")]
+# Both sides of its rules: launches a little larger than what finds room at once (2048 blocks of four rows up to 20 MiB, 5120
+# waves), rows for two rows a wave, few rows of nine narrow vectors.
+CASES += [("layer", "f32", 6144, 400, "norm_rows_tail/layer/64x2/256/1"), ("layer", "f32", 6145, 400, "norm_rows/layer/64x2/256/2/ragged"),
+          ("rms", "f32", 8192, 400, "norm_rows_tail/rms/64x2/256/1"), ("layer", "bf16", 8193, 800, "norm_rows/layer/64x2/256/2/ragged"),
+          ("rms", "f32", 13107, 400, "norm_rows/rms/64x2/256/2/ragged"), ("rms", "bf16", 13108, 800, "norm_rows_tail/rms/64x2/256/1"),
+          ("layer", "bf16", 5120, 1600, "norm_rows_tail/layer/64x4/64/1"), ("layer", "bf16", 5121, 1600, "norm_rows/layer/64x4/64/2/ragged"),
+          ("layer", "bf16", 6656, 1600, "norm_rows/layer/64x4/64/2/ragged"), ("layer", "bf16", 6657, 1600, "norm_rows_tail/layer/64x4/64/1"),
+          ("layer", "f32", 3999, 516, "norm_rows_tail/layer/64x3/64/1"), ("layer", "f32", 4001, 516, "norm_rows_tail/layer/64x3/64/2"),
+          ("rms", "f32", 3999, 1000, "norm_rows_tail/rms/64x4/64/1"), ("rms", "f32", 4001, 1000, "norm_rows/rms/64x4/256/2/ragged"),
+          ("rms", "bf16", 6999, 1032, "norm_rows_tail/rms/64x3/64/1"), ("rms", "bf16", 7001, 1032, "norm_rows_tail/rms/64x3/64/2"),
+          ("rms", "bf16", 31, 4104, "norm_rows_tail/rms/64x9/64/1"), ("rms", "bf16", 33, 4104, "norm_rows/rms/256x4/256/1/ragged"),
+          ("layer", "bf16", 575, 4104, "norm_rows/layer/256x4/256/1/ragged"), ("layer", "bf16", 577, 4104, "norm_rows_tail/layer/64x9/64/1")]
 
 reached = set()
 
