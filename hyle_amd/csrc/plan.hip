@@ -1378,7 +1378,10 @@ hyle_hip_status admit(hyle_hip_plan *p) {
       const uint64_t chunks = (row_bytes + 4095) / 4096 * row_count;
       // Rows of whole 16-byte units (if the addresses allow them) take far fewer blocks than the narrowest units, and the
       // checking dispatch costs more than index reads that hit the caches: up to 1536 indices, six loads of a thread at
-      // once, and 32 MiB (us, two dispatches / one: f16 [1037 of 2560] 5.9 / 5.0, bf16 [1400 of 704] 5.2 / 4.6).
+      // once, and 32 MiB (us, two dispatches / one: f16 [1037 of 2560] 6.6 / 5.6, [1536 of 1280] 5.9 / 4.3, [1400 of 704] 5.1 / 3.6;
+      // the source 8, 4 and 2 bytes off a boundary, with narrower units and up to eight times the blocks: [1037 of 2560] 7.8 / 7.1,
+      // 7.4 / 5.5, 7.5 / 6.0, [1400 of 704] 5.4 / 4.0, 6.7 / 6.0, 6.6 / 4.8, [1536 of 4096] 9.8 / 8.0, 9.8 / 7.9, 12.1 / 10.1).  The
+      // line is where it was looked for, not where it turns: [2048 of 704] would take 3.9 instead of 5.6, [4096 of 256] 3.5 instead of 4.8.
       const bool few = g.index_count <= 1024 && (n + 255) / 256 * index_bytes <= (8u << 20);
       const bool whole = row_bytes % 16 == 0 && g.index_count <= 1536 && (n * (uint64_t)size / 16 + 255) / 256 * index_bytes <= (32u << 20);
       const bool overlapped = row_bytes >= 4096 && chunks >= 4096 && g.index_count <= 16384 &&

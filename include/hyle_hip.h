@@ -163,7 +163,7 @@ typedef enum hyle_hip_op_kind {
   /* sampling_ops::Categorical (include/hyle/compute/sampling_ops.h:37-66): in0 dense F32 / F16 /
    * BF16 [R, V] log-weights, in1 dense U32 [R, 4] identities; out0 I32 [R] indices and, with
    * `kind2` = 1, out1 F32 [R] normalised log probabilities of the selected elements.  -Inf is
-   * zero mass.  Two dispatches and a workspace; a row with NaN, +Inf or no finite element writes
+   * zero mass.  Two dispatches (one for up to 256 rows of up to 256 elements) and a workspace; a row with NaN, +Inf or no finite element writes
    * nothing and shows as INVALID_ARGUMENT in hyle_hip_plan_device_status.  The draw is the CPU
    * provider's inverse CDF on the 52-bit uniform of the row's first Philox block; like the
    * reference's own backends it promises the distribution, not equal indices across backends. */
@@ -304,8 +304,9 @@ HYLE_HIP_API hyle_hip_status hyle_hip_plan_outputs(const hyle_hip_plan *plan,
 HYLE_HIP_API int hyle_hip_plan_alias_support(const hyle_hip_plan *plan, uint32_t output_index,
                                              uint32_t input_index);
 /* ProviderRouteCostFacts::dispatch_count
- * (include/hyle/compute/prepared_operation.h:51-67): kernels one launch enqueues (of a Categorical: at
- * most, since a few short rows take one). */
+ * (include/hyle/compute/prepared_operation.h:51-67): kernels one launch enqueues, with operands on
+ * 16-byte boundaries.  For every Categorical the two of its general form, of which up to 256 rows of up
+ * to 256 elements need one. */
 HYLE_HIP_API uint32_t hyle_hip_plan_dispatch_count(const hyle_hip_plan *plan);
 /* Name of the kernel route the plan selected (diagnostics, profiling). */
 HYLE_HIP_API const char *hyle_hip_plan_route_name(const hyle_hip_plan *plan);
