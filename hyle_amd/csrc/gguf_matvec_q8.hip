@@ -1139,9 +1139,9 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_blocks(const uns
     const uint64_t begin = (uint64_t)row * row_stride + (uint64_t)step * Step::kBytes;
     const uint64_t left = row_bytes - (uint64_t)step * Step::kBytes;
     const uint32_t bytes = left < Step::kBytes ? (uint32_t)left : Step::kBytes;
-    const uintptr_t address = reinterpret_cast<uintptr_t>(weights) + begin;
-    const uint32_t off = (uint32_t)(address & 15u);
-    const u32x4 *vectors = reinterpret_cast<const u32x4 *>(address - off);
+    // (a pointer all the way: loads from an address that was an integer are flat ones, which every wait for LDS waits for)
+    const uint32_t off = (uint32_t)(reinterpret_cast<uintptr_t>(weights + begin) & 15u);
+    const u32x4 *vectors = reinterpret_cast<const u32x4 *>(weights + begin - off);
     const uint32_t needed = (off + bytes + 15) / 16;
 #pragma unroll
     for (int i = 0; i < Step::kLoads; ++i) {

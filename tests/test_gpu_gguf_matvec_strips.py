@@ -143,6 +143,34 @@ def test_strips_every_layout_of_a_launch(tag):
         assert np.array_equal(got, np.take(got, np.arange(rows) % period, 1))
 
 
+# rows, k, activation rows, two bytes off: numbers of waves to a tile that are no powers of two
+SPLITS = [(17408, 5120, 5, 0), (17408, 5120, 3, 2),    # three waves to each of five tiles, one without a place
+          (600, 2816, 6, 0), (600, 2816, 2, 2),        # eleven to the only tile
+          (21504, 2560, 8, 0), (21504, 2560, 8, 2),    # five to each of three tiles, two rounds, one without a place
+          (9472, 1536, 7, 2), (8500, 3328, 6, 0)]      # three of eight waves; five of sixteen
+
+
+@pytest.mark.parametrize("tag", list(KINDS))
+def test_strips_any_number_of_waves_to_a_tile(tag):
+    """Held as in the test above: 257 distinct rows against the oracle, their repetitions against them bit by bit."""
+    rng = np.random.default_rng(1825)
+    kind, gguf = KINDS[tag]
+    period = 257
+    for rows, k, m, off in SPLITS:
+        raw = weights_for(tag, rng, period, k)
+        x = rng.normal(0, 1, (m, k)).astype(np.float32)
+        row_bytes = raw.shape[1]
+        storage = torch.empty(off + rows * row_bytes, dtype=torch.uint8, device=DEVICE)[off:]
+        storage.view(rows, row_bytes).copy_(torch.from_numpy(raw).to(DEVICE).repeat((rows + period - 1) // period, 1)[:rows])
+        note(f"q8 matvec {tag} [{k} -> {rows}] x {m} off {off}: waves to a tile")
+        descs = [hc.TensorDesc.gguf_weight(gguf, hc.DataType.kFloat32, k, rows), hc.TensorDesc.dense(hc.DataType.kFloat32, [m, k])]
+        (out,) = run(Q8, storage, torch.from_numpy(x).to(DEVICE), descs=descs)
+        got = out.cpu().numpy().reshape(m, rows)
+        centre, bound = orc.gguf_matvec_q8(kind, raw.reshape(-1), period, k, x)
+        assert np.all(np.abs(got[:, :period] - centre.reshape(m, period)) <= bound.reshape(m, period))
+        assert np.array_equal(got, np.take(got, np.arange(rows) % period, 1))
+
+
 @pytest.mark.parametrize("tag,k,rows,m,byte_offset", [
     ("q8_0", 5120, 2304, 6, 0), ("q8_0", 2560, 8192, 4, 0), ("q6_k", 5120, 3584, 8, 0), ("q6_k", 1024, 8192, 5, 0),
     ("q4_k", 4096, 6656, 4, 0), ("q4_k", 9984, 3072, 5, 2)])
