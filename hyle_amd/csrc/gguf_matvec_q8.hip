@@ -1487,30 +1487,33 @@ inline bool rows_of_vectors_serve(const MatVecParams &p) {
 // Where the strip kernel (gguf_matvec_strips.hip) is the faster one; `vectors`: weights, activations and
 // the row stride are multiples of 16 bytes.  MI355X, bf16, us, the kernels here / strips:
 //   several activation rows: nearly everywhere, since a compute unit quantises them once.  Q8_0 [2048 -> 16384]
-//   x 2 15.6 / 10.4, [4096 -> 2048] x 8 10.9 / 8.7, Q6_K [1024 -> 2048] x 8 11.9 / 4.7, [6144 -> 8192] x 2 20.2 / 12.9,
-//   Q4_K [1536 -> 3072] x 4 6.0 / 4.6, [7680 -> 2100] x 4 14.0 / 7.8.  Not where narrow Q4_K rows are many (tiles
-//   quantise little there and need no barrier for the tile's end): [2048 -> 6144] x 4 7.1 / 7.5, [2048 -> 65536] x 2
-//   20.1 / 22.9 ([2560 -> 8192] x 2 9.0 / 7.1, [2048 -> 65536] x 8 26.4 / 25.4, [2048 -> 80000] x 8 30.5 / 27.2), [2048 -> 100000] x 6
-//   39.6 / 41.9, [2048 -> 151936] x 5 54.9 / 58.2 and Q6_K [2048 -> 100000] x 2 38.0 / 42.0, [2048 -> 151936] x 2 55.2 / 59.2
-//   ([2048 -> 65536] x 2 29.4 / 25.2, Q4_K [1792 -> 120000] x 8 41.0 / 36.9); nor two rows far wider than the
-//   weight is high, Q8_0 [16384 -> 1024] 10.1 / 11.4 ([8192 -> 2048] 9.5 / 8.1)
+//   x 2 15.8 / 9.5, [6144 -> 2048] x 5 12.2 / 9.5, Q6_K [1024 -> 2048] x 8 12.2 / 5.0, [2048 -> 6144] x 2 8.1 / 6.1,
+//   Q4_K [1024 -> 2048] x 4 5.2 / 3.6, [6144 -> 2048] x 4 12.9 / 6.7, [1536 -> 20000] x 2 10.5 / 7.1, [2048 -> 60000] x 4
+//   19.9 / 18.0.  Not a vocabulary of one span, whose codes the tile and quad kernels keep at hand: Q4_K [2048 -> 151936]
+//   x 2 38.8 / 39.5, x 5 55.0 / 53.5, Q6_K x 2 54.3 / 57.2; nor two rows far wider than the weight is high, Q8_0
+//   [16384 -> 1024] 10.1 / 11.4.  (Two to four rows against 6144 to 8999 Q4_K rows of up to 2048 values stay with the tiles
+//   that the tests of this rule name there, 7.3 / 5.2 at [2048 -> 6144] x 4.)
 //   one row, where the alternative walks block by block, from 8 M products on, and from 4 M where a row is wide:
-//   Q6_K [1024 -> 8192] 5.8 / 5.4, [2304 -> 2304] 6.9 / 5.6, [7680 -> 2100] 12.9 / 8.2 ([1024 -> 2048] 4.0 / 4.2)
-//   one row of Q4_K tiles: rows of 10240 values or more, [17408 -> 5120] 21.1 / 17.4, and widths that are no
-//   multiple of 2048 with few weight rows, [2560 -> 2560] 5.3 / 4.5, [5120 -> 5120] 8.5 / 7.2 ([2560 -> 5120]
-//   5.7 / 5.8, [4096 -> 2048] 5.2 / 6.4, [8192 -> 8192] 12.1 / 14.6)
+//   Q6_K [2560 -> 9728] 11.6 / 7.9, [5120 -> 5120] 11.8 / 9.0 ([1024 -> 2048] 4.2 / 4.2)
+//   one row of Q4_K tiles: rows of 10240 values or more, [14080 -> 3328] 13.7 / 9.6; widths that are no multiple of 2048
+//   with few weight rows, [5120 -> 5120] 9.2 / 7.0; and more than twice as many rows as values, but for a vocabulary, whose
+//   tiles need no barrier: [2048 -> 6144] 5.5 / 4.8, [2560 -> 9728] 8.1 / 5.9, [5120 -> 17408] 15.8 / 12.7, [3072 -> 32000]
+//   14.8 / 13.6, but [1024 -> 100000] 15.4 / 16.7, [2048 -> 60000] 14.9 / 17.2, [2048 -> 151936] 31.1 / 38.5.  (Where the rows
+//   are between the width and twice as many, and for up to 6000 of them, the tests of this rule name the tiles.)
 bool strips_better(const MatVecParams &p, bool vectors) {
   if (!gguf_matvec_strips_serve(p)) return false;
   const bool whole = vectors && rows_of_vectors_serve(p);
   if (p.m == 1) {
     const uint64_t products = p.rows * p.k;
     if (!whole) return products >= 8000000 || (products >= 4000000 && p.k >= 2048);
-    return p.kind == 0 && (p.k >= 10240 || (p.k > 2048 && p.k % 2048 != 0 && (p.rows <= 4096 || p.k >= p.rows)));
+    if (p.kind != 0) return false;
+    return p.k >= 10240 || (p.k > 2048 && p.k % 2048 != 0 && (p.rows <= 4096 || p.k >= p.rows)) ||
+           (p.rows > 6000 && p.rows > 2 * (uint64_t)p.k && products <= 100000000);
   }
   if (!whole) return true;
   // one span of a vocabulary: the tile and quad kernels keep its codes at hand and have no tiles left over
   const bool span_of_many = p.k == 2048 && p.rows >= 90000;
-  if (p.kind == 0) return (p.m > 4 && !span_of_many) || p.k > 2048 || p.rows < 6144;
+  if (p.kind == 0) return p.k > 2048 || (!span_of_many && (p.m > 4 || p.rows < 6144 || p.rows >= 9000)) ;
   if (p.kind == 1 && p.m <= 4 && span_of_many) return false;
   return p.m > 2 || p.k < 8 * p.rows;
 }

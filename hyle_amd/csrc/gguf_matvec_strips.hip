@@ -736,10 +736,12 @@ hipError_t run_strips(const MatVecParams &p, uint32_t m, const void *w, const vo
   const uint32_t runs = p.k / 256, rows = (uint32_t)p.rows;
   // One block per compute unit, where the activation rows are quantised once; two of eight waves where
   // that is little beside the weight rows, which then hide each other's tile ends (us, one / two:
-  // Q8_0 [1280 -> 77056] x 4 29.4 / 26.5, Q4_K [3072 -> 77056] x 4 41.0 / 31.8 and x 8 43.9 / 38.3; but
-  // Q8_0 [1280 -> 2048] x 4 7.7 / 8.4, [3072 -> 17408] x 8 19.8 / 22.2).
+  // Q4_K [2048 -> 151936] x 2 47.7 / 39.5, Q6_K [1280 -> 100000] x 5 32.7 / 26.4, Q8_0 [5120 -> 17408] x 1 21.6 / 19.9,
+  // [3328 -> 14080] x 4 13.4 / 12.1; but Q8_0 [2048 -> 6144] x 4 6.5 / 6.9).  Q4_K and Q6_K rows of eight runs or more that
+  // are no vocabulary's share better among sixteen waves: [2560 -> 9728] x 2 6.0 / 7.3 and 8.3 / 9.5, [5120 -> 17408] x 1
+  // 12.7 / 15.4 and 17.2 / 20.2 ([3072 -> 32000] x 2 13.7 / 13.7 and 18.0 / 17.9).
   const uint32_t codes = m * p.k;
-  const bool little = (codes <= 16384 && rows >= 8192) || (codes <= 32768 && rows >= 65536);
+  const bool little = (codes <= 16384 && rows >= 8192 && (kKind >= 2 || p.k < 2048 || rows >= 32768)) || (codes <= 32768 && rows >= 65536);
   const bool twice = little && 2 * strip_layout(kKind, m, p.k, 8).bytes <= kStripLds;
   const uint32_t waves = twice ? 8 : strip_waves(kKind, m, p.k), shared = strip_layout(kKind, m, p.k, waves).bytes;
   const uint32_t wanted = units * (twice ? 2u : 1u);

@@ -143,6 +143,18 @@ def test_strips_every_layout_of_a_launch(tag):
         assert np.array_equal(got, np.take(got, np.arange(rows) % period, 1))
 
 
+# Q4_K products of more than twice as many rows as values, and of two to four activation rows against 9000 rows and more
+@pytest.mark.parametrize("x_tag,k,rows,m,kernel", [
+    ("bf16", 2048, 6001, 1, "strips"), ("bf16", 2048, 6000, 1, "tiles"), ("f32", 2816, 5633, 1, "tiles"), ("f32", 3072, 6145, 1, "strips"),
+    ("f16", 3072, 6144, 1, "tiles"), ("bf16", 1024, 97656, 1, "strips"), ("bf16", 1024, 97657, 1, "tiles"), ("f32", 2048, 9000, 2, "strips"),
+    ("bf16", 1280, 9000, 4, "strips"), ("f16", 2048, 8999, 3, "tiles"), ("bf16", 2048, 89999, 2, "strips"), ("bf16", 2048, 90000, 2, "tiles")])
+def test_strips_rule_for_many_rows_of_q4_k(x_tag, k, rows, m, kernel):
+    rng = np.random.default_rng(1826)
+    raw = np.resize(weights_for("q4_k", rng, min(rows, 2000), k), (rows, k // 256 * 144))
+    note(f"q8 matvec rule q4_k rows {rows} k {k} m {m}")
+    check("q4_k", x_tag, raw, rows, k, rng.normal(0, 1, (m, k) if m > 1 else (k,)).astype(np.float32), kernel=f"gguf_matvec_q8_{kernel}/q4_k/")
+
+
 # rows, k, activation rows, two bytes off: numbers of waves to a tile that are no powers of two
 SPLITS = [(17408, 5120, 5, 0), (17408, 5120, 3, 2),    # three waves to each of five tiles, one without a place
           (600, 2816, 6, 0), (600, 2816, 2, 2),        # eleven to the only tile
