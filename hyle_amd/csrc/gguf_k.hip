@@ -10,13 +10,15 @@
 //   Q6_K  {u8 ql[128]; u8 qh[64]; i8 scales[16]; f16 d}  y = (d * scale) * (q - 32)
 // with separate f32 roundings for the products and the subtraction, as the source writes them.
 //
-// Two kernels.  Rows made of whole 16-byte vectors with K a multiple of 2048 (the usual case)
-// take one wave per row, whole cache lines into wave-private LDS and word-wise decoding
+// Two kernels.  Q4_K rows on 16-byte boundaries and Q6_K rows at even addresses (the usual case)
+// take a wave or a block per row, whole cache lines into wave-private LDS and word-wise decoding
 // (k_quant_lines, measured 5.9 / 6.3 us for Q4_K / Q6_K [6144 x 2048] on MI355X).  Anything else
 // takes the general kernel: a block of 256 threads takes four rows at a time, eight super-blocks
 // of each (at most 1680 bytes) are staged in LDS per step with the widest loads the row's
 // address allows, and a thread decodes eight neighbouring values from LDS bytes (10.7 / 12.3 us
 // for the same shape).  Both store eight values as one 16-byte vector.
+#include <type_traits>
+
 #include "device_common.h"
 #include "gguf_decode.h"
 #include "kernels.h"
@@ -88,96 +90,129 @@ __global__ __launch_bounds__(kBlockThreads) void k_quant_rows(const unsigned cha
   }
 }
 
-// Rows made of whole 16-byte vectors, K a multiple of 2048: one wave per row and no barrier.
-// The wave reads 2048 values' worth of blocks (1152 or 1680 bytes) as 16-byte vectors, one per
-// lane and request, so that every cache line is asked for once; parks them in a region of LDS
-// that only this wave touches (LDS executes one wave's instructions in order); and each lane
+// One wave per row, or kShare waves where rows are few and wide; no barrier before the row's last.
+// The wave reads 2048 values' worth of blocks (1152 or 1680 bytes, the row's last piece what is left of it) as
+// aligned 16-byte vectors, one per lane and request, so that every cache line is asked for once; parks them in a
+// region of LDS that only this wave touches (LDS executes one wave's instructions in order); and each lane
 // decodes eight neighbouring values at a time from aligned 32-bit words, so that a store
-// instruction of the wave writes 1 KiB of consecutive bf16.  The next 2048 values are on their
-// way while these are decoded.  The loads are plain ones: with the non-temporal hint the same
-// kernel took 8.0 / 9.3 us instead of 5.9 / 6.3 us (the bf16 stores keep the hint).
-template <int kKind>  // 0 = Q4_K, 1 = Q6_K
+// instruction of the wave writes 1 KiB of consecutive bf16.  The next piece is on its
+// way while this one is decoded.  A Q6_K row may start at any even address: its vectors start at the 16-byte boundary
+// at or below it, as far below for every piece (1680 = 105 * 16), and the decoder joins words anyway.  (Q4_K headers
+// are read as words: rows on 16-byte boundaries.)  The loads are plain ones: with the non-temporal hint
+// [6144 x 2048] took 8.0 / 9.3 us instead of 5.9 / 6.3 us (the bf16 stores keep the hint).
+// Bound by HBM.  MI355X, us, before (a block to four rows, below) / here:
+//   Q4_K [1280 x 2048] 6.2 / 3.5  [2560 x 6144] 15.6 / 7.8  [5120 x 14080] 52.5 / 30.0 (6160 GB/s)
+//   Q6_K [1024 x 5120] 7.7 / 4.1  [3328 x 1280] 15.9 / 4.0  [17408 x 2048] 56.8 / 17.1 (5870 GB/s)
+// (kWhole: rows of whole pieces, which then have no bounds to look at: [2048 x 1024] 3.3 us, 3.4 with them)
+template <int kKind, int kShare, bool kWhole>  // 0 = Q4_K, 1 = Q6_K
 __global__ __launch_bounds__(kBlockThreads) void k_quant_lines(const unsigned char *blocks, void *out, float *sumsq,
                                                                uint32_t rows, uint32_t k, uint64_t row_stride) {
   constexpr uint32_t kBlockBytes = kKind == 0 ? 144 : 210;
-  constexpr uint32_t kSpan = 2048;                                  // values per step
-  constexpr uint32_t kVectors = kSpan / kSuper * kBlockBytes / 16;  // 72 or 105
-  constexpr int kLoads = (kVectors + kWaveLanes - 1) / kWaveLanes;  // 2
+  constexpr uint32_t kSpan = 2048, kSpanBytes = kSpan / kSuper * kBlockBytes;  // values and bytes per step: 72 or 105 vectors
+  constexpr int kLoads = 2;                                                    // at most 106 vectors
   constexpr int kWaves = kBlockThreads / kWaveLanes;
   __shared__ __align__(16) unsigned char slots[kWaves][kLoads * kWaveLanes * 16];
+  __shared__ float joint[kWaves];
   const uint32_t lane = threadIdx.x % kWaveLanes;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveLanes);
-  const uint32_t row = blockIdx.x * kWaves + wave;
-  if (row >= rows) return;
+  const uint32_t wanted_row = blockIdx.x * (kWaves / kShare) + wave / kShare, member = wave % kShare;
+  if (kShare == 1 && wanted_row >= rows) return;
+  const uint32_t row = min(wanted_row, rows - 1);  // (waves that share a row all have one)
   unsigned char *slot = slots[wave];
   const unsigned char *source = blocks + (size_t)row * row_stride;
-  const uint32_t steps = k / kSpan;
-  uint32_t vec[kLoads];
-#pragma unroll
-  for (int i = 0; i < kLoads; ++i) {  // past the span: its last vector again (parked, never read)
-    const uint32_t wanted = lane + i * kWaveLanes;
-    vec[i] = wanted < kVectors ? wanted : kVectors - 1;
-  }
+  const uint32_t below = kKind == 0 ? 0u : (uint32_t)reinterpret_cast<uintptr_t>(source) & 15u;
+  source -= below;
+  const uint32_t steps = (k + kSpan - 1) / kSpan;
   u32x4 raw[kLoads];
+  auto load = [&](uint32_t step) {
+    const uint32_t bytes = kWhole ? kSpanBytes : min(kSpan, k - step * kSpan) / kSuper * kBlockBytes, last = (below + bytes - 1) / 16;
 #pragma unroll
-  for (int i = 0; i < kLoads; ++i) raw[i] = load16(source, vec[i]);
+    for (int i = 0; i < kLoads; ++i)  // past the piece: its last vector again (parked, never read)
+      raw[i] = load16(source + (size_t)step * kSpanBytes, min(lane + i * kWaveLanes, last));
+  };
+  load(min(member, steps - 1));
   float squares = 0.0f;
-  for (uint32_t step = 0; step < steps; ++step) {
+  for (uint32_t step = member; step < steps; step += kShare) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) *reinterpret_cast<u32x4 *>(slot + (size_t)(lane + i * kWaveLanes) * 16) = raw[i];
-    const uint32_t following = step + 1 < steps ? step + 1 : step;
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i) raw[i] = load16(source, (size_t)following * kVectors + vec[i]);
+    load(min(step + kShare, steps - 1));
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t values = k - step * kSpan;
+    auto decode = [&](auto whole) {  // a whole piece has no branch, so that its LDS reads go out together
 #pragma unroll
-    for (uint32_t i = 0; i < kSpan / (kWaveLanes * 8); ++i) {
-      const uint32_t p = (i * kWaveLanes + lane) * 8;  // position within the span
-      float y[8];
-      if constexpr (kKind == 0) decode_q4_k_words(slot, (p / kSuper) * kBlockBytes, p % kSuper, y);
-      else decode_q6_k_words(slot, (p / kSuper) * kBlockBytes, p % kSuper, y);
+      for (uint32_t i = 0; i < kSpan / (kWaveLanes * 8); ++i) {
+        const uint32_t p = (i * kWaveLanes + lane) * 8;  // position within the span
+        if (!decltype(whole)::value && p >= values) break;
+        float y[8];
+        if constexpr (kKind == 0) decode_q4_k_words(slot, (p / kSuper) * kBlockBytes, p % kSuper, y);
+        else decode_q6_k_words(slot, below + (p / kSuper) * kBlockBytes, p % kSuper, y);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) squares = __builtin_fmaf(y[j], y[j], squares);
-      store16_stream(out, ((size_t)row * k + (size_t)step * kSpan + p) / 8, Traits<BF16>::pack(y));
-    }
+        for (int j = 0; j < 8; ++j) squares = __builtin_fmaf(y[j], y[j], squares);
+        store16_stream(out, ((size_t)row * k + (size_t)step * kSpan + p) / 8, Traits<BF16>::pack(y));
+      }
+    };
+    if (kWhole || values >= kSpan) decode(std::true_type{});
+    else decode(std::false_type{});
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
-  squares = group_sum<kWaveLanes>(squares);
-  if (lane == 0) sumsq[row] = squares;
+  if constexpr (kShare == 1) {
+    squares = group_sum<kWaveLanes>(squares);
+    if (lane == 0) sumsq[row] = squares;
+  } else {
+    static_assert(kShare == kWaves, "a row to a block");
+    squares = row_sum<kBlockThreads>(squares, joint);
+    if (threadIdx.x == 0) sumsq[row] = squares;
+  }
 }
 
 }  // namespace
 
 namespace {
-template <int kKind, bool kLines> struct KQuantTag {
-  static std::string text() { return std::string(kLines ? "k_quant_lines/" : "k_quant_rows/") + (kKind == 0 ? "q4_k" : "q6_k"); }
+enum : int { kGeneral = 0, kWholePieces = 1, kPieces = 2, kShared = 3 };  // a wave to a row, or (kShared) a block
+template <int kKind, int kForm> struct KQuantTag {
+  static std::string text() {
+    return std::string(kForm == kGeneral ? "k_quant_rows/" : "k_quant_lines/") + (kKind == 0 ? "q4_k" : "q6_k") +
+           (kForm == kShared ? "/shared" : (kForm == kPieces ? "/pieces" : ""));
+  }
 };
+
+template <int kKind> hipError_t run_lines(const KQuantParams &p, const unsigned char *in, void *out, float *sumsq, hipStream_t stream) {
+  constexpr uint32_t kWaves = kBlockThreads / kWaveLanes;
+  const uint32_t rows = (uint32_t)p.rows;
+  // A block to a row where there are at most eight rows to a compute unit and each is more than one piece (us, a wave / a
+  // block: Q6_K [17408 x 512] 9.3 / 5.9, [6144 x 1280] 5.8 / 4.7, Q4_K [5120 x 1024] 5.2 / 4.2, [2560 x 1024] 3.8 / 3.6;
+  // [3840 x 3328] 7.0 / 7.3, [5120 x 14080] 30.0 / 30.1).
+  const bool shared = p.k > 2048 && rows <= 2048;
+  const dim3 waves((rows + kWaves - 1) / kWaves), block(kBlockThreads);
+  if (shared) {
+    note_variant<KQuantTag<kKind, kShared>>();
+    hipLaunchKernelGGL((k_quant_lines<kKind, kWaves, false>), dim3(rows), block, 0, stream, in, out, sumsq, rows, p.k, p.row_stride);
+  } else if (p.k % 2048 != 0) {
+    note_variant<KQuantTag<kKind, kPieces>>();
+    hipLaunchKernelGGL((k_quant_lines<kKind, 1, false>), waves, block, 0, stream, in, out, sumsq, rows, p.k, p.row_stride);
+  } else {
+    note_variant<KQuantTag<kKind, kWholePieces>>();
+    hipLaunchKernelGGL((k_quant_lines<kKind, 1, true>), waves, block, 0, stream, in, out, sumsq, rows, p.k, p.row_stride);
+  }
+  return hipGetLastError();
+}
 }  // namespace
 
 hipError_t launch_k_quant_dequant(const KQuantParams &p, const void *blocks, void *out, float *sumsq,
                                   hipStream_t stream) {
   if (p.rows == 0) return hipSuccess;
   const unsigned char *in = static_cast<const unsigned char *>(blocks);
-  const bool lines = ((reinterpret_cast<uintptr_t>(blocks) | p.row_stride) & 15u) == 0 && p.k != 0 && p.k % 2048 == 0;
-  if (lines) {
-    constexpr int kWaves = kBlockThreads / kWaveLanes;
-    const dim3 grid(((uint32_t)p.rows + kWaves - 1) / kWaves), block(kBlockThreads);
-    if (p.kind == 0) note_variant<KQuantTag<0, true>>();
-    else note_variant<KQuantTag<1, true>>();
-    if (p.kind == 0)
-      hipLaunchKernelGGL((k_quant_lines<0>), grid, block, 0, stream, in, out, sumsq, (uint32_t)p.rows, p.k,
-                         p.row_stride);
-    else
-      hipLaunchKernelGGL((k_quant_lines<1>), grid, block, 0, stream, in, out, sumsq, (uint32_t)p.rows, p.k,
-                         p.row_stride);
-    return hipGetLastError();
-  }
+  // whole blocks on 16-byte (Q6_K: even) boundaries
+  const uint64_t together = reinterpret_cast<uintptr_t>(blocks) | p.row_stride;
+  if (p.k != 0 && p.k % kSuper == 0 && (together & (p.kind == 0 ? 15u : 1u)) == 0)
+    return p.kind == 0 ? run_lines<0>(p, in, out, sumsq, stream) : run_lines<1>(p, in, out, sumsq, stream);
   constexpr int kRows = 4;
   const dim3 grid(((uint32_t)p.rows + kRows - 1) / kRows), block(kBlockThreads);
-  if (p.kind == 0) note_variant<KQuantTag<0, false>>();
-  else note_variant<KQuantTag<1, false>>();
+  if (p.kind == 0) note_variant<KQuantTag<0, kGeneral>>();
+  else note_variant<KQuantTag<1, kGeneral>>();
   if (p.kind == 0)
     hipLaunchKernelGGL((k_quant_rows<0, kRows>), grid, block, 0, stream, in, out, sumsq, (uint32_t)p.rows, p.k,
                        p.row_stride);

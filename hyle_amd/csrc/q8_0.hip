@@ -13,10 +13,11 @@
 // stores, 1 KiB of consecutive bf16 per store instruction of a wave.  Each row's sum of squares
 // of the exact products is reduced with a wave64 butterfly.
 //
-// Three kernels: rows of K = 2048 n values made of whole 16-byte vectors take one wave per row
+// Two kernels: rows made of whole 16-byte vectors (K = 256 n) take one wave per row
 // with a region of LDS that only this wave touches and no block barrier (q8_0_lines: aligned
-// 32-bit LDS words joined by byte-wise funnel shifts); other rows of whole vectors stage
-// block-wide with 2-byte LDS reads (q8_0_rows); anything else reads bytes (q8_0_rows_bytes).
+// 32-bit LDS words joined by byte-wise funnel shifts); anything else reads bytes (q8_0_rows_bytes).
+#include <type_traits>
+
 #include "device_common.h"
 #include "gguf_decode.h"
 #include "kernels.h"
@@ -27,69 +28,18 @@ namespace {
 constexpr int kBlockBytes = 34;
 constexpr int kBlockElems = 32;
 
-// Requires row_bytes % 16 == 0, row_stride % 16 == 0 and a 16-byte aligned base.
-constexpr int kMaxRowBytes = 8704;  // 256 blocks = 8192 elements
-
-// Each wave owns `kRows` consecutive rows: all their global loads are issued first.
-template <int kWaves, int kRows>
-__global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_rows(const char *blocks, uint16_t *out,
-                                                               float *sumsq, uint32_t rows,
-                                                               uint32_t k, uint64_t row_stride,
-                                                               uint32_t row_bytes) {
-  extern __shared__ __attribute__((aligned(16))) char staged[];
-  const uint32_t wave = threadIdx.x / kWaveLanes, lane = threadIdx.x % kWaveLanes;
-  const uint32_t first_row = (blockIdx.x * kWaves + wave) * kRows;
-  char *mine = staged + (size_t)wave * kRows * row_bytes;
-  const uint32_t row_vectors = row_bytes / 16;
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const uint32_t row = first_row + r;
-    if (row < rows) {
-      const char *src = blocks + (size_t)row * row_stride;
-      for (uint32_t v = lane; v < row_vectors; v += kWaveLanes)
-        reinterpret_cast<u32x4 *>(mine + (size_t)r * row_bytes)[v] = load16_stream(src, v);
-    }
-  }
-  __syncthreads();
-  const uint32_t out_vectors = k / 8;
-#pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const uint32_t row = first_row + r;
-    float squares = 0.0f;
-    if (row < rows) {
-      const char *staged_row = mine + (size_t)r * row_bytes;
-      // output vector j holds elements [8j, 8j+8): block j/4, quants 8*(j%4) ..
-      for (uint32_t j = lane; j < out_vectors; j += kWaveLanes) {
-        const char *block = staged_row + (size_t)(j / 4) * kBlockBytes;
-        const float d = f16_to_f32(*reinterpret_cast<const uint16_t *>(block));
-        const uint16_t *q = reinterpret_cast<const uint16_t *>(block + 2 + 8 * (j % 4));
-        float y[8];
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const uint32_t pair = q[h];
-          y[2 * h] = (float)(int8_t)(pair & 0xFFu) * d;
-          y[2 * h + 1] = (float)(int8_t)(pair >> 8) * d;
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) squares = __builtin_fmaf(y[e], y[e], squares);
-        store16_stream(out, (size_t)row * out_vectors + j, Traits<BF16>::pack(y));
-      }
-    }
-    squares = group_sum<kWaveLanes>(squares);
-    if (row < rows && lane == 0) sumsq[row] = squares;
-  }
-}
-
-// Rows of K = 2048 n values, whole 16-byte vectors, 16-byte aligned: one wave per row, no barrier.
+// Rows of whole 16-byte vectors (K = 256 n), 16-byte aligned: one wave per row, no barrier.
 // A span of 2048 values is 64 blocks = 2176 bytes = 136 vectors: two per lane and a third for
-// the first eight lanes (the others repeat the span's last vector, one request for all of them);
+// the first eight lanes (the others repeat the span's last vector, one request for all of them), the row's last
+// span what is left of it: 17 vectors to 256 values;
 // plain loads: the non-temporal hint costs 10 % here, while the stores keep it.
 // The vectors are parked in LDS that only this wave touches (LDS executes one wave's
 // instructions in order); lane l then decodes output vectors l, l + 64, l + 128, l + 192 of
 // the span: eight quants at a 2-byte aligned offset come out of three aligned words and two
 // funnel shifts, the block's scale out of one 16-bit read.  The next span's loads are in flight
 // while this one is decoded.
-template <int kWaves>
+// (kWhole: rows of whole spans, which then have no bounds to look at: [2048 x 1024] 3.0 us, 3.1 with them)
+template <int kWaves, bool kWhole>
 __global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_lines(const unsigned char *blocks, void *out,
                                                                 float *sumsq, uint32_t rows, uint32_t k,
                                                                 uint64_t row_stride) {
@@ -103,43 +53,44 @@ __global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_lines(const unsigned 
   if (row >= rows) return;
   unsigned char *slot = slots[wave];
   const unsigned char *source = blocks + (size_t)row * row_stride;
-  const uint32_t steps = k / kSpan;
-  uint32_t vec[kLoads];
-#pragma unroll
-  for (int i = 0; i < kLoads; ++i) {
-    const uint32_t wanted = lane + i * kWaveLanes;
-    vec[i] = wanted < kVectors ? wanted : kVectors - 1;
-  }
+  const uint32_t steps = (k + kSpan - 1) / kSpan;
   u32x4 raw[kLoads];
+  auto load = [&](uint32_t step) {
+    const uint32_t last = (kWhole ? kVectors : min(kVectors, (k - step * kSpan) / 256 * 17)) - 1;
 #pragma unroll
-  for (int i = 0; i < kLoads; ++i) raw[i] = load16(source, vec[i]);
+    for (int i = 0; i < kLoads; ++i) raw[i] = load16(source, (size_t)step * kVectors + min(lane + i * kWaveLanes, last));
+  };
+  load(0);
   float squares = 0.0f;
   for (uint32_t step = 0; step < steps; ++step) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) *reinterpret_cast<u32x4 *>(slot + (size_t)(lane + i * kWaveLanes) * 16) = raw[i];
-    if (step + 1 < steps) {  // uniform across the wave
-#pragma unroll
-      for (int i = 0; i < kLoads; ++i) raw[i] = load16(source, (size_t)(step + 1) * kVectors + vec[i]);
-    }
+    if (step + 1 < steps) load(step + 1);  // uniform across the wave
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint32_t values = k - step * kSpan;
+    auto decode = [&](auto whole) {  // a whole span has no branch, so that its LDS reads go out together
 #pragma unroll
-    for (uint32_t i = 0; i < kSpan / (kWaveLanes * 8); ++i) {
-      const uint32_t j = i * kWaveLanes + lane;  // output vector of the span: block j / 4, quants 8 (j % 4) ..
-      const uint32_t block_offset = (j / 4) * kBlockBytes;
-      const float d = f16_to_f32(*reinterpret_cast<const uint16_t *>(slot + block_offset));
-      uint32_t q[2];
-      lds_piece(slot, block_offset + 2 + 8 * (j % 4), q);
-      float y[8];
+      for (uint32_t i = 0; i < kSpan / (kWaveLanes * 8); ++i) {
+        const uint32_t j = i * kWaveLanes + lane;  // output vector of the span: block j / 4, quants 8 (j % 4) ..
+        if (!decltype(whole)::value && 8 * j >= values) break;
+        const uint32_t block_offset = (j / 4) * kBlockBytes;
+        const float d = f16_to_f32(*reinterpret_cast<const uint16_t *>(slot + block_offset));
+        uint32_t q[2];
+        lds_piece(slot, block_offset + 2 + 8 * (j % 4), q);
+        float y[8];
 #pragma unroll
-      for (int w = 0; w < 2; ++w)
+        for (int w = 0; w < 2; ++w)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) y[4 * w + t] = (float)(int)(signed char)(q[w] >> (8 * t)) * d;
+          for (int t = 0; t < 4; ++t) y[4 * w + t] = (float)(int)(signed char)(q[w] >> (8 * t)) * d;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) squares = __builtin_fmaf(y[e], y[e], squares);
-      store16_stream(out, ((size_t)row * k + (size_t)step * kSpan) / 8 + j, Traits<BF16>::pack(y));
-    }
+        for (int e = 0; e < 8; ++e) squares = __builtin_fmaf(y[e], y[e], squares);
+        store16_stream(out, ((size_t)row * k + (size_t)step * kSpan) / 8 + j, Traits<BF16>::pack(y));
+      }
+    };
+    if (kWhole || values >= kSpan) decode(std::true_type{});
+    else decode(std::false_type{});
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
@@ -169,28 +120,12 @@ __global__ __launch_bounds__(kBlockThreads) void q8_0_rows_bytes(const uint8_t *
   if (row_ok && lane == 0) sumsq[row] = squares;
 }
 
-struct LinesTag {
-  static std::string text() { return "q8_0_lines"; }
-};
-struct RowsTag {
-  static std::string text() { return "q8_0_rows"; }
+template <bool kWhole> struct LinesTag {
+  static std::string text() { return kWhole ? "q8_0_lines" : "q8_0_lines/pieces"; }
 };
 struct BytesTag {
   static std::string text() { return "q8_0_rows_bytes"; }
 };
-
-template <int kWaves, int kRows>
-hipError_t run_rows(const Q8Params &p, const void *blocks, void *out, float *sumsq,
-                    uint32_t row_bytes, hipStream_t stream) {
-  const uint32_t rows = (uint32_t)p.rows;
-  constexpr int kRowsPerBlock = kWaves * kRows;
-  note_variant<RowsTag>();
-  hipLaunchKernelGGL((q8_0_rows<kWaves, kRows>), dim3((rows + kRowsPerBlock - 1) / kRowsPerBlock),
-                     dim3(kWaves * kWaveLanes), (size_t)kRowsPerBlock * row_bytes, stream,
-                     static_cast<const char *>(blocks), static_cast<uint16_t *>(out), sumsq, rows, p.k,
-                     p.row_stride, row_bytes);
-  return hipGetLastError();
-}
 
 }  // namespace
 
@@ -198,24 +133,23 @@ hipError_t launch_q8_0_dequant(const Q8Params &p, const void *blocks, void *out,
                                bool vectorised, hipStream_t stream) {
   if (p.rows == 0) return hipSuccess;
   const uint32_t rows = (uint32_t)p.rows;
-  const uint32_t row_bytes = p.k / kBlockElems * kBlockBytes;
-  const bool fast = vectorised && row_bytes != 0 && row_bytes % 16 == 0 &&
-                    p.row_stride % 16 == 0 && row_bytes <= kMaxRowBytes;
-  if (fast && p.k % 2048 == 0) {
+  if (vectorised && p.k != 0 && p.k % 256 == 0 && p.row_stride % 16 == 0) {
     // Measured on MI355X for W[6144 x 2048] (38.6 MB of traffic, buffers rotated): 6.7 us with
     // plain loads and non-temporal stores; 7.4 us with non-temporal loads too; 8.6 / 10.5 us with
-    // plain stores; a wave that walks several rows with the next row in flight 7.3 - 9.3 us; the
-    // block-staged kernel below 7.1 us.
+    // plain stores; a wave that walks several rows with the next row in flight 7.3 - 9.3 us.  Widths that are no multiple
+    // of 2048, in blocks that staged their rows / like this: [1280 x 14080] 13.1 / 9.4 us, [3840 x 1024] 5.3 / 3.9,
+    // [5120 x 6144] 18.5 / 16.0.
     constexpr int kWaves = 4;
-    note_variant<LinesTag>();
-    hipLaunchKernelGGL((q8_0_lines<kWaves>), dim3((rows + kWaves - 1) / kWaves), dim3(kWaves * kWaveLanes), 0, stream,
-                       static_cast<const unsigned char *>(blocks), out, sumsq, rows, p.k, p.row_stride);
+    const dim3 grid((rows + kWaves - 1) / kWaves), block(kWaves * kWaveLanes);
+    const unsigned char *in = static_cast<const unsigned char *>(blocks);
+    if (p.k % 2048 == 0) {
+      note_variant<LinesTag<true>>();
+      hipLaunchKernelGGL((q8_0_lines<kWaves, true>), grid, block, 0, stream, in, out, sumsq, rows, p.k, p.row_stride);
+    } else {
+      note_variant<LinesTag<false>>();
+      hipLaunchKernelGGL((q8_0_lines<kWaves, false>), grid, block, 0, stream, in, out, sumsq, rows, p.k, p.row_stride);
+    }
     return hipGetLastError();
-  }
-  if (fast) {
-    // Measured on MI355X for W[6144 x 2048]: 2, 4 or 8 waves per block with one row per wave
-    // all take about 8 us; two or four rows per wave are slower (9 to 13 us).
-    return run_rows<4, 1>(p, blocks, out, sumsq, row_bytes, stream);
   }
   constexpr int kWaves = kBlockThreads / kWaveLanes;
   note_variant<BytesTag>();

@@ -121,3 +121,45 @@ def test_k_quant_schema_and_benchmark_shape():
         wide, want, want_sumsq = orc.k_quant_dequant(kind, raw, 6144, 2048)
         assert np.array_equal(got, want)
         sumsq_bar(sumsq, wide)
+
+
+# rows, k: pieces of 2048 values that are not whole, a row to a wave and (at most 2048 rows of more than one piece) to a block
+@pytest.mark.parametrize("tag", ["q4_k", "q6_k"])
+def test_k_quant_rows_of_pieces(tag):
+    kind, _, block_bytes = KINDS[tag]
+    rng = np.random.default_rng(1504)
+    for rows, k in ((5, 256), (9, 1792), (2, 2304), (2048, 2304), (2049, 2304), (3, 4096), (7, 8448), (2051, 3840), (2050, 4096)):
+        row_bytes = k // 256 * block_bytes
+        raw = finite_scales(tag, rng.integers(0, 256, (min(rows, 40), row_bytes), dtype=np.uint8), block_bytes)
+        raw = np.resize(raw, (rows, row_bytes))
+        wide, want, _ = orc.k_quant_dequant(kind, raw, rows, k)
+        for pad, offset in ((0, 0), (16, 32), (16, 6), (-row_bytes % 16 + 14, 14)):
+            padded = np.zeros(offset + rows * (row_bytes + pad) + 8, np.uint8)
+            padded[offset:offset + rows * (row_bytes + pad)].reshape(rows, -1)[:, :row_bytes] = raw
+            served = (offset | (row_bytes + pad)) % (16 if tag == "q4_k" else 2) == 0
+            note(f"{tag} [{rows}, {k}] rows {row_bytes + pad} bytes apart, tensor at byte {offset}")
+            got, sumsq = dequant_on_device(tag, padded, rows, k, row_stride=row_bytes + pad, offset=offset)
+            form = "/shared" if k > 2048 and rows <= 2048 else ("/pieces" if k % 2048 else "")
+            label = f"k_quant_lines/{tag}{form}" if served else f"k_quant_rows/{tag}"
+            assert hc.last_launch_variant() == label
+            assert np.array_equal(got, want)
+            sumsq_bar(sumsq, wide)
+
+
+def test_q8_0_rows_of_pieces():
+    rng = np.random.default_rng(1505)
+    for rows, k, pad, label in ((5, 256, 0, "lines/pieces"), (9, 1792, 16, "lines/pieces"), (6, 2304, 0, "lines/pieces"), (1030, 3840, 32, "lines/pieces"),
+                                (5, 16640, 0, "lines/pieces"), (7, 10240, 16, "lines"),
+                                (4, 2304, 2, "rows_bytes"), (4, 2272, 0, "rows_bytes")):
+        blocks = rng.integers(0, 256, (rows, k // 32, 34), dtype=np.uint8)
+        blocks[:, :, 1] &= 0x3B
+        raw = blocks.reshape(rows, -1)
+        padded = np.zeros((rows, raw.shape[1] + pad), np.uint8)
+        padded[:, :raw.shape[1]] = raw
+        desc = hc.TensorDesc.gguf_weight(hc.GgufQuantizedType.kQ8_0, hc.DataType.kBFloat16, k, rows, raw.shape[1] + pad)
+        note(f"q8_0 [{rows}, {k}] rows {raw.shape[1] + pad} bytes apart")
+        out, sumsq = run(hc.GgufDequantSumSquares(), torch.from_numpy(padded).to(DEVICE), descs=[desc])
+        assert hc.last_launch_variant() == f"q8_0_{label}"
+        values = blocks[:, :, 2:].view(np.int8).astype(np.float32) * blocks[:, :, :2].copy().view(np.float16).astype(np.float32)
+        assert np.array_equal(out.contiguous().view(torch.int16).cpu().numpy().view(np.uint16), orc.from_f32(orc.BF16, values.reshape(rows, k)))
+        sumsq_bar(sumsq.cpu().numpy(), values.reshape(rows, k))
