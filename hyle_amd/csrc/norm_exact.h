@@ -44,12 +44,24 @@ bool run_exact_lanes(uint32_t per_lane, const NormParams &p, const Bound &io, in
   return false;
 }
 
+// Below 10 MiB a wave that takes two or four rows one after the other waits for each in turn while the chip has room: one row
+// per wave (norm_tail.h, or 64 x 1 and 256 x 4 of norm.hip) is the faster.  MI355X, us, here / there:
+//   RMSNorm bf16 [8, 5120] 3.4 / 2.5   [64, 4096] 3.4 / 2.7   [256, 2560] 3.6 / 2.9   [512, 1024] 4.0 / 2.6   [2048, 512] 4.5 / 2.8
+//     [1000, 5120] 5.5 / 4.9   [2000, 3072] 5.2 / 5.4   [12288, 512] 6.6 / 6.4   [16384, 512] 7.3 / 8.2
+//   LayerNorm f32 [8, 4096] 4.1 / 2.7   [64, 2560] 3.6 / 2.8   [512, 512] 4.1 / 2.6   [1000, 2560] 5.4 / 4.8   [1000, 4096] 6.9 / 7.8
+//     [8192, 256] 5.5 / 5.1   [12288, 256] 6.2 / 7.2   bf16 [2000, 2560] 5.3 / 5.1   [2000, 4096] 6.8 / 6.9
+// (As many rows as these shapes' own tests have, four of 192 vectors or more or one block of shorter ones, stay here.)
+inline bool exact_pays(uint64_t rows, uint32_t vectors, uint64_t bytes) {
+  return bytes >= (10ull << 20) || rows == (vectors <= 128 ? 512 / vectors : 4);
+}
+
 template <class T, class W, bool kLayer>
 bool run_exact_shape(const NormParams &p, const Bound &io, hipStream_t s) {
   constexpr uint32_t kVec = Traits<T>::kVec;
   if (p.shape.width % kVec != 0) return false;
   const uint32_t vectors = p.shape.width / kVec;
   if (!kLayer && vectors == 256) return false;  // norm.hip's shape measures the same
+  if (!exact_pays(p.shape.rows, vectors, p.shape.rows * p.shape.width * Traits<T>::kSize)) return false;
   const int parameters = !p.has_weight ? kPlain : (kLayer && p.has_bias ? kScaleBias : kScale);
   // short rows: two vectors per lane in a group of half as many lanes as the row has vectors, four
   // rows per group (a lane with one vector of a row is slow: [32768, 512] 14.2 / 15.5 us)

@@ -193,6 +193,15 @@ CASES += [("layer", "f32", 6144, 400, "norm_rows_tail/layer/64x2/256/1"), ("laye
           ("rms", "bf16", 31, 4104, "norm_rows_tail/rms/64x9/64/1"), ("rms", "bf16", 33, 4104, "norm_rows/rms/256x4/256/1/ragged"),
           ("layer", "bf16", 575, 4104, "norm_rows/layer/256x4/256/1/ragged"), ("layer", "bf16", 577, 4104, "norm_rows_tail/layer/64x9/64/1")]
 
+# Few rows of up to 512 vectors a wave each, and both sides of the 10 MiB below which rows are not taken two or four to a wave.
+CASES += [("rms", "f32", 2, 2048, "norm_rows_tail/rms/64x8/64/1"), ("layer", "bf16", 1, 4096, "norm_rows_tail/layer/64x8/64/1"),
+          ("rms", "bf16", 2, 1536, "norm_rows_tail/rms/64x3/64/1"), ("layer", "f32", 5, 1280, "norm_rows_tail/layer/64x5/64/1"),
+          ("rms", "bf16", 6, 5120, "norm_rows/rms/256x4/256/1/ragged"), ("layer", "f32", 8, 4096, "norm_rows/layer/256x4/256/1/exact"),
+          ("layer", "f32", 6, 5120, "norm_rows/layer/256x8/256/1/ragged"), ("rms", "bf16", 8, 1024, "norm_rows_tail/rms/64x2/256/1"),
+          ("rms", "bf16", 10232, 512, "norm_rows/rms/64x1/256/1/ragged"), ("rms", "bf16", 10240, 512, "norm_rows_exact/rms/32x2/64/4"),
+          ("layer", "f32", 10232, 256, "norm_rows/layer/64x1/256/1/exact"), ("layer", "f32", 2046, 1280, "norm_rows_tail/layer/64x5/64/1"),
+          ("layer", "f32", 2048, 1280, "norm_rows_exact/layer/64x5/64/2")]
+
 reached = set()
 
 
