@@ -103,33 +103,38 @@ __device__ __forceinline__ bool invalid_weight(float v) {
   return __builtin_amdgcn_class(v, 0x001 | 0x002 | 0x200);  // sNaN | qNaN | +inf
 }
 
-// The 16 elements of a thread in a tile: with whole 16-byte vectors, vector j of the thread holds
-// elements (j * 256 + thread) * kVec ...; element by element, step j is element j * 256 + thread.
-// Places past the row read as -inf (no mass).  `place(j, e)` is the element's index in the tile.
-template <class T, bool kVector> struct TileValues {
-  static constexpr int kVec = kVector ? Traits<T>::kVec : 1;
-  static constexpr int kSteps = kPerThread / kVec;
+// 16 bytes at any element's address.
+typedef uint32_t words4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+// The vector of elements at .. at + kVec - 1 of a tile whose first element is at `tile`, of which it has `count`; places
+// past them read as -inf (no mass).  kAligned: rows of whole 16-byte vectors on 16-byte boundaries, so that count is a
+// multiple of kVec.  Other rows (an odd vocabulary) are read as vectors at element-aligned addresses, their last elements one by one.
+// (us, both dispatches, all elements one by one / so: f16 [28, 79580] 14.9 / 9.6, [1, 85746] 10.0 / 7.3, bf16 [64, 248319] 30.3 / 17.9)
+template <class T, bool kAligned, bool kStream>
+__device__ __forceinline__ void tile_vector(const unsigned char *tile, uint32_t at, uint32_t count, float (&part)[Traits<T>::kVec]) {
+  constexpr int kVec = Traits<T>::kVec;
+  const unsigned char *from = tile + (size_t)at * Traits<T>::kSize;
+  if (kAligned ? at < count : at + kVec <= count) {
+    if constexpr (!kAligned) Traits<T>::unpack(*reinterpret_cast<const words4_any *>(from), part);
+    else Traits<T>::unpack(kStream ? load16_stream(from, 0) : load16(from, 0), part);
+  } else {
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) part[e] = !kAligned && at + e < count ? Traits<T>::load(from, e) : -__builtin_huge_valf();
+  }
+}
+
+// The 16 elements of a thread in a tile: vector j of the thread holds elements (j * 256 + thread) * kVec ...
+template <class T, bool kAligned> struct TileValues {
+  static constexpr int kVec = Traits<T>::kVec;
   float v[kPerThread];
-  static __device__ __forceinline__ uint32_t place(int j, int e) { return (uint32_t)(j * kBlockThreads + threadIdx.x) * kVec + e; }
   __device__ __forceinline__ void load(const void *row, uint32_t first, uint32_t count) {
-    constexpr float kNone = -__builtin_huge_valf();
-    if constexpr (kVector) {
+    const unsigned char *tile = static_cast<const unsigned char *>(row) + (size_t)first * Traits<T>::kSize;
 #pragma unroll
-      for (int j = 0; j < kSteps; ++j) {
-        const uint32_t at = place(j, 0);  // count is a multiple of kVec on this route
-        float part[kVec];
-        if (at < count) {
-          Traits<T>::unpack(load16_stream(static_cast<const unsigned char *>(row) + (size_t)first * Traits<T>::kSize, at / kVec), part);
-        } else {
+    for (int j = 0; j < kPerThread / kVec; ++j) {
+      float part[kVec];
+      tile_vector<T, kAligned, true>(tile, (uint32_t)(j * kBlockThreads + threadIdx.x) * kVec, count, part);
 #pragma unroll
-          for (int e = 0; e < kVec; ++e) part[e] = kNone;
-        }
-#pragma unroll
-        for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < kSteps; ++j) v[j] = place(j, 0) < count ? Traits<T>::load(row, (size_t)first + place(j, 0)) : kNone;
+      for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
     }
   }
 };
@@ -204,29 +209,17 @@ __device__ __forceinline__ double block_scan(double v, double *wave_totals, doub
 }
 
 // The 16 consecutive elements of a thread in a tile (thread t holds elements 16 t ... 16 t + 15), so
-// that one scan over the threads orders the whole tile.  Places past the row read as -inf.
-template <class T, bool kVector>
+// that one scan over the threads orders the whole tile.
+template <class T, bool kAligned>
 __device__ __forceinline__ void load_consecutive(const void *row, uint32_t first, uint32_t count, float (&v)[kPerThread]) {
-  constexpr float kNone = -__builtin_huge_valf();
-  const uint32_t mine = threadIdx.x * kPerThread;
-  if constexpr (kVector) {
-    constexpr int kVec = Traits<T>::kVec;
-    const unsigned char *base = static_cast<const unsigned char *>(row) + ((size_t)first + mine) * Traits<T>::kSize;
+  constexpr int kVec = Traits<T>::kVec;
+  const unsigned char *tile = static_cast<const unsigned char *>(row) + (size_t)first * Traits<T>::kSize;
 #pragma unroll
-    for (int j = 0; j < kPerThread / kVec; ++j) {
-      float part[kVec];
-      if (mine + j * kVec < count) {  // count is a multiple of kVec on this route
-        Traits<T>::unpack(load16(base, j), part);
-      } else {
+  for (int j = 0; j < kPerThread / kVec; ++j) {
+    float part[kVec];
+    tile_vector<T, kAligned, false>(tile, threadIdx.x * kPerThread + j * kVec, count, part);
 #pragma unroll
-        for (int e = 0; e < kVec; ++e) part[e] = kNone;
-      }
-#pragma unroll
-      for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < kPerThread; ++i) v[i] = mine + i < count ? Traits<T>::load(row, (size_t)first + mine + i) : kNone;
+    for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
   }
 }
 
@@ -413,7 +406,7 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
 
 // Rows of up to 256 elements, a few of them (what TopK leaves of a vocabulary): one wave per row does
 // the work of both dispatches above in one, with the same sums in the same order -- a lane's own first,
-// then the lanes of what would be each wave of a block (kWaves of them hold elements), then the waves --
+// then the lanes of what would be the first wave of a block, the only one with elements --
 // so that every index and score is the one the two dispatches give.  The status word is written once, by
 // the launch's last block, which looks at all rows itself: rows cannot clear a word that others set.
 // Bound by latency.  MI355X, us, two dispatches / one: [5, 40] bf16 7.7 / 3.3, [64, 100] f32 7.7 / 3.5, [250, 64] bf16
@@ -462,55 +455,44 @@ __global__ __launch_bounds__(kShortWaves *kWaveLanes) void categorical_short(con
   const void *base = static_cast<const unsigned char *>(logits) + (size_t)row * width * Traits<T>::kSize;
   const uint32_t *identity = identities + (size_t)row * 4;
   const uint32_t key0 = identity[0], key1 = identity[1], draw0 = identity[2], draw1 = identity[3];
-  // The tile's order: vector `lane`, or elements lane, 64 + lane, ...; and sixteen consecutive elements per
-  // lane for the scan.  Places past the row read as -inf.
-  constexpr int kVec = kVector ? Traits<T>::kVec : 1;
-  constexpr int kWaves = kVector ? 1 : kShortWidth / kWaveLanes;
-  float tile[kWaves][kVec], v[kPerThread];
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    const uint32_t at = (w * kWaveLanes + lane) * kVec;  // width is a multiple of kVec
-    if constexpr (kVector) {
-      Traits<T>::unpack(load16(base, at < width ? at / kVec : 0), tile[w]);
-    } else {
-      tile[w][0] = Traits<T>::load(base, at < width ? at : 0);
-    }
-#pragma unroll
-    for (int e = 0; e < kVec; ++e) tile[w][e] = at < width ? tile[w][e] : -kInfinity;
-  }
-#pragma unroll
-  for (int j = 0; j < kPerThread / kVec; ++j) {
-    const uint32_t at = lane * kPerThread + j * kVec;
-    float part[kVec];
+  // The tile's order, vector `lane`, and sixteen consecutive elements per lane for the scan.
+  constexpr int kVec = Traits<T>::kVec;
+  // No branches round these loads, so that all of them go out together: a place past the row is read inside it and
+  // counts as -inf.
+  auto vector_at = [&](uint32_t at, float (&part)[kVec]) {
     if constexpr (kVector) {
       Traits<T>::unpack(load16(base, at < width ? at / kVec : 0), part);
     } else {
-      part[0] = Traits<T>::load(base, at < width ? at : 0);
+#pragma unroll
+      for (int e = 0; e < kVec; ++e) part[e] = Traits<T>::load(base, min(at + e, width - 1));
     }
 #pragma unroll
-    for (int e = 0; e < kVec; ++e) v[j * kVec + e] = at < width ? part[e] : -kInfinity;
+    for (int e = 0; e < kVec; ++e) part[e] = (kVector ? at : at + e) < width ? part[e] : -kInfinity;
+  };
+  float tile[kVec], v[kPerThread];
+  vector_at(lane * kVec, tile);
+#pragma unroll
+  for (int j = 0; j < kPerThread / kVec; ++j) {
+    float part[kVec];
+    vector_at(lane * kPerThread + j * kVec, part);
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
   }
   const PhiloxWords draw = philox_block(key0, key1, draw0, draw1, 0);
   const double uniform = ((double)draw.x0 * 0x1p20 + (double)(draw.x1 >> 12) + 0.5) * 0x1p-52;
   bool invalid = false;
   float maximum = -kInfinity;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w)
-#pragma unroll
-    for (int e = 0; e < kVec; ++e) {
-      invalid = invalid || invalid_weight(tile[w][e]);
-      maximum = fmaxf(maximum, tile[w][e]);
-    }
+  for (int e = 0; e < kVec; ++e) {
+    invalid = invalid || invalid_weight(tile[e]);
+    maximum = fmaxf(maximum, tile[e]);
+  }
   maximum = row_max<kWaveLanes>(maximum, nullptr);
   if (__ballot(invalid) != 0 || !(maximum > -kInfinity)) return;
-  double total = 0;
+  double tile_mass = 0;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    double mass = 0;
-#pragma unroll
-    for (int e = 0; e < kVec; ++e) mass += (double)exp_nonpositive(tile[w][e] - maximum);
-    total += wave_sum(mass);
-  }
+  for (int e = 0; e < kVec; ++e) tile_mass += (double)exp_nonpositive(tile[e] - maximum);
+  const double total = wave_sum(tile_mass);
   // the row is one tile, whose scale is exp(0)
   const double threshold = total * uniform;
   if (!(total > threshold)) {
@@ -558,14 +540,14 @@ __global__ __launch_bounds__(kShortWaves *kWaveLanes) void categorical_short(con
 
 // Launch-shape labels
 template <bool kVector, bool kScored> struct CategoricalShortTag {
-  static std::string text() { return std::string("categorical_short/") + (kVector ? "vector" : "scalar") + (kScored ? "/scored" : ""); }
+  static std::string text() { return std::string("categorical_short/") + (kVector ? "vector" : "unaligned") + (kScored ? "/scored" : ""); }
 };
 template <bool kVector> struct CategoricalTilesTag {
-  static std::string text() { return std::string("categorical_tiles/") + (kVector ? "vector" : "scalar"); }
+  static std::string text() { return std::string("categorical_tiles/") + (kVector ? "vector" : "unaligned"); }
 };
 template <bool kVector, bool kScored, bool kFew> struct CategoricalRowsTag {
   static std::string text() {
-    return std::string("categorical_rows/") + (kVector ? "vector" : "scalar") + (kScored ? "/scored" : "") + (kFew ? "" : "/many-tiles");
+    return std::string("categorical_rows/") + (kVector ? "vector" : "unaligned") + (kScored ? "/scored" : "") + (kFew ? "" : "/many-tiles");
   }
 };
 template <int kForm> struct RandomBitsTag {  // 0 rows of blocks, 1 flat

@@ -732,3 +732,27 @@ def test_q8_0_other_widths_strides_and_every_scale():
     blocks = blocks.reshape(rows, 8 * 34)
     got, _ = run_q8(blocks, rows, 256)
     assert_bits_equal(got, orc.q8_0_dequant_bf16(blocks, rows, 256)[0])
+
+
+@pytest.mark.parametrize("tag", ["f32", "bf16", "f16"])
+def test_argmax_rows_of_no_whole_vectors(tag):
+    """Rows read as vectors at element-aligned addresses, the last one moved back into its neighbour: winners, ties, NaN and
+    -inf in the elements both hold, tile edges, rows shorter than a vector, and a tensor one element into its storage."""
+    rng = np.random.default_rng(113)
+    vec = 4 if tag == "f32" else 8
+    for rows, width in ((3, vec - 1), (3, vec), (9, vec + 1), (9, 2 * vec - 1), (9, 4095), (9, 4097), (9, 8191), (70, 40003)):
+        for offset in (0, 1):
+            x = rng.integers(-30, 30, (rows, width)).astype(np.float32)
+            if rows >= 9:
+                x[1, width - 1] = x[2, width - vec] = x[3, width - vec - 1] = 50.0
+                x[4, width - vec:] = 60.0                  # a tie inside the last vector
+                x[5, :], x[6, :], x[7, :], x[8, :] = np.nan, -np.inf, np.nan, -np.inf
+                x[7, width - 2], x[8, width - 1] = -np.inf, np.nan
+            note(f"argmax {tag} [{rows},{width}] {offset} elements in")
+            xs = host_values(x, tag)
+            flat = np.concatenate([np.zeros(offset, xs.dtype), xs.reshape(-1)])
+            values, indices = run(hc.TopK(), to_device(flat, tag)[offset:].view(rows, width))
+            want_values, want_indices = orc.topk1(x if tag == "f32" else orc.to_f32(TYPES[tag][1], xs))
+            assert np.array_equal(to_host(indices)[:, 0], want_indices)
+            got = to_host(values)[:, 0]
+            assert np.array_equal(got if tag == "f32" else orc.to_f32(TYPES[tag][1], got), want_values, equal_nan=True)
