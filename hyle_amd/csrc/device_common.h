@@ -17,6 +17,7 @@ constexpr int kWaveLanes = 64;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_element __attribute__((ext_vector_type(4), aligned(2)));  // at any element's address
 
 struct F32 {};
 struct F16 {};
@@ -243,6 +244,20 @@ template <int kLanes> __device__ __forceinline__ float row_sum(float v, float *j
 }
 template <int kLanes> __device__ __forceinline__ float row_max(float v, float *joint) {
   return row_reduce<kLanes>(v, joint, [](float a, float b) { return a > b ? a : b; });
+}
+// Whether `mine` holds in any thread of a block of kThreads: a ballot per wave and one barrier.  At most
+// one call per kernel (the words are not protected against the next).  (The runtime's own
+// block votes reduce over the block size that they read from the implicit arguments.)
+template <int kThreads> __device__ __forceinline__ bool block_any(bool mine) {
+  constexpr int kWaves = kThreads / kWaveLanes;
+  __shared__ uint32_t seen[kWaves];
+  const uint64_t lanes = __ballot(mine);
+  if (threadIdx.x % kWaveLanes == 0) seen[threadIdx.x / kWaveLanes] = lanes != 0 ? 1u : 0u;
+  __syncthreads();
+  uint32_t any = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) any |= seen[w];
+  return any != 0;
 }
 // NaN-propagating extrema of the reference's Reduce
 // (src/compute_provider_native/reduction.cc:34-47): the first NaN met sticks;
