@@ -42,9 +42,6 @@ __device__ __forceinline__ void consider(LaneArg &best, float value, int32_t ind
 
 constexpr int kVectorsInFlight = 2;  // loads a lane issues before it compares
 
-// 16 bytes at any element's address.
-typedef uint32_t words4_any __attribute__((ext_vector_type(4), aligned(2)));
-
 // One block per (row, tile).  A lane walks its tile two vectors at a time: both loads are issued
 // (from clamped, always valid addresses) before either is compared.
 // kAligned: rows of whole 16-byte vectors on 16-byte boundaries.  Other rows of a vector or more (an odd vocabulary, a view
@@ -85,7 +82,7 @@ __global__ __launch_bounds__(kBlockThreads) void argmax_tiles(const void *x, Can
           raw[k] = load16_stream(x, (row_first + first[k]) / kVec);
         } else {
           first[k] = min(first[k], width - kVec);
-          raw[k] = *reinterpret_cast<const words4_any *>(static_cast<const char *>(x) + (row_first + first[k]) * Traits<T>::kSize);
+          raw[k] = *reinterpret_cast<const u32x4_element *>(static_cast<const char *>(x) + (row_first + first[k]) * Traits<T>::kSize);
         }
       }
 #pragma unroll

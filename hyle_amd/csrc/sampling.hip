@@ -103,9 +103,6 @@ __device__ __forceinline__ bool invalid_weight(float v) {
   return __builtin_amdgcn_class(v, 0x001 | 0x002 | 0x200);  // sNaN | qNaN | +inf
 }
 
-// 16 bytes at any element's address.
-typedef uint32_t words4_any __attribute__((ext_vector_type(4), aligned(2)));
-
 // The vector of elements at .. at + kVec - 1 of a tile whose first element is at `tile`, of which it has `count`; places
 // past them read as -inf (no mass).  kAligned: rows of whole 16-byte vectors on 16-byte boundaries, so that count is a
 // multiple of kVec.  Other rows (an odd vocabulary) are read as vectors at element-aligned addresses, their last elements one by one.
@@ -115,7 +112,7 @@ __device__ __forceinline__ void tile_vector(const unsigned char *tile, uint32_t 
   constexpr int kVec = Traits<T>::kVec;
   const unsigned char *from = tile + (size_t)at * Traits<T>::kSize;
   if (kAligned ? at < count : at + kVec <= count) {
-    if constexpr (!kAligned) Traits<T>::unpack(*reinterpret_cast<const words4_any *>(from), part);
+    if constexpr (!kAligned) Traits<T>::unpack(*reinterpret_cast<const u32x4_element *>(from), part);
     else Traits<T>::unpack(kStream ? load16_stream(from, 0) : load16(from, 0), part);
   } else {
 #pragma unroll

@@ -32,27 +32,43 @@ namespace {
 
 constexpr uint32_t kTile = 2048;  // keys one block sorts: 16 KiB of LDS
 
+// Where the rows lie and where their k best go.  Dense tensors with the axis innermost need no strides
+// (twelve bytes for 120, nothing to branch on): bf16 [5, 248320], 40 best, both dispatches 11.6 us with the
+// general form, 11.35 with this one.
+struct DenseRows {
+  uint32_t width, count;  // extent of the axis, k
+  uint32_t largest;       // 1: largest first
+  // Byte offset of element 0 of `row`; bytes from one element to the next; the output element of the j-th best.
+  __device__ __forceinline__ int64_t base(uint32_t row, uint32_t size) const { return (int64_t)row * width * size; }
+  __device__ __forceinline__ int64_t step(uint32_t size) const { return size; }
+  __device__ __forceinline__ size_t output(uint32_t row, uint32_t j) const { return (size_t)row * count + j; }
+};
 struct Addressing {
-  uint32_t width, inner, count;  // extent of the axis, elements after it, k
-  uint32_t largest;              // 1: largest first
+  uint32_t width, count;
+  uint32_t largest;
+  uint32_t inner;                // elements after the axis
   uint32_t dense_last;           // 1: dense tensor, axis innermost
   int32_t rank, axis;
   uint32_t dims[kMaxRank];
   int64_t strides[kMaxRank];
-};
-
-// Byte offset of element 0 of `row` (row = outer * inner + position after the axis).
-__device__ __forceinline__ int64_t row_base(const Addressing &a, uint32_t row, uint32_t size) {
-  if (a.dense_last) return (int64_t)row * a.width * size;
-  int64_t base = 0;
-  uint32_t remaining = row;
-  for (int axis = a.rank - 1; axis >= 0; --axis) {
-    if (axis == a.axis) continue;
-    base += (int64_t)(remaining % a.dims[axis]) * a.strides[axis];
-    remaining /= a.dims[axis];
+  // row = outer * inner + position after the axis
+  __device__ __forceinline__ int64_t base(uint32_t row, uint32_t size) const {
+    if (dense_last) return (int64_t)row * width * size;
+    int64_t from = 0;
+    uint32_t remaining = row;
+    for (int a = rank - 1; a >= 0; --a) {
+      if (a == axis) continue;
+      from += (int64_t)(remaining % dims[a]) * strides[a];
+      remaining /= dims[a];
+    }
+    return from;
   }
-  return base;
-}
+  __device__ __forceinline__ int64_t step(uint32_t size) const { return dense_last ? size : strides[axis]; }
+  __device__ __forceinline__ size_t output(uint32_t row, uint32_t j) const {
+    const uint32_t outer = row / inner, position = row - outer * inner;
+    return ((size_t)outer * count + j) * inner + position;
+  }
+};
 
 // Element types: the three float storage types and int32 (include/hyle/compute/providers/cuda.h:108-121).
 struct I32 {};
@@ -160,15 +176,13 @@ __device__ __forceinline__ void sort_descending(uint64_t *keys, uint32_t n) {
 }
 
 // The first `count` keys of a sorted list -> outputs (kFinal) or the next list in the workspace.
-template <class T, bool kBytewise, bool kFinal>
-__device__ __forceinline__ void emit(const uint64_t *keys, const Addressing &a, uint32_t row,
+template <class T, int kThreads, bool kBytewise, bool kFinal, class A>
+__device__ __forceinline__ void emit(const uint64_t *keys, const A &a, uint32_t row,
                                      const char *x, void *values, int32_t *indices, uint64_t *list) {
   constexpr int kSize = KeyTraits<T>::kSize;
   if constexpr (kFinal) {
-    const int64_t base = row_base(a, row, kSize);
-    const int64_t step = a.dense_last ? kSize : a.strides[a.axis];
-    const uint32_t outer = row / a.inner, position = row - outer * a.inner;
-    for (uint32_t j = threadIdx.x; j < a.count; j += blockDim.x) {
+    const int64_t base = a.base(row, kSize), step = a.step(kSize);
+    for (uint32_t j = threadIdx.x; j < a.count; j += kThreads) {
       // a list always holds `count` elements of the row here; the clamp only keeps a corrupted
       // workspace from turning into a wild address
       const uint32_t index = min(~(uint32_t)keys[j], a.width - 1);
@@ -177,27 +191,27 @@ __device__ __forceinline__ void emit(const uint64_t *keys, const Addressing &a, 
       uint32_t bits;
       if (!storage_bits_of<T>((uint32_t)(keys[j] >> 32), a.largest != 0, &bits))
         bits = load_bits<T, kBytewise>(x + base + (int64_t)index * step);
-      const size_t out = ((size_t)outer * a.count + j) * a.inner + position;
+      const size_t out = a.output(row, j);
       if constexpr (kSize == 4) static_cast<uint32_t *>(values)[out] = bits;
       else static_cast<uint16_t *>(values)[out] = (uint16_t)bits;
       indices[out] = (int32_t)index;
     }
   } else {
-    for (uint32_t j = threadIdx.x; j < a.count; j += blockDim.x) list[j] = keys[j];
+    for (uint32_t j = threadIdx.x; j < a.count; j += kThreads) list[j] = keys[j];
   }
 }
 
 // One block per (row, tile): keys of up to kTile elements, sorted, best `count` kept.
-template <class T, bool kVector, bool kBytewise, bool kFinal>
+template <class T, bool kVector, bool kBytewise, bool kFinal, class A>
 __global__ __launch_bounds__(kBlockThreads) void topk_tiles(const char *x, void *values, int32_t *indices,
-                                                            uint64_t *lists, Addressing a, uint32_t tiles,
-                                                            uint32_t sort_n, uint32_t largest) {
+                                                            uint64_t *lists, A a, uint32_t tiles, uint32_t sort_n,
+                                                            uint32_t largest) {
   constexpr int kSize = KeyTraits<T>::kSize;
   constexpr int kVec = KeyTraits<T>::kVec;
   __shared__ uint64_t keys[kTile];
   const uint32_t row = blockIdx.x / tiles, tile = blockIdx.x - row * tiles;
   const uint32_t first = tile * kTile;
-  const int64_t base = row_base(a, row, kSize);
+  const int64_t base = a.base(row, kSize);
   if constexpr (kVector) {
     // dense rows whose starts are 16-byte aligned: whole vectors, a ragged end cannot occur
     const u32x4 *vectors = reinterpret_cast<const u32x4 *>(x + base);
@@ -214,7 +228,7 @@ __global__ __launch_bounds__(kBlockThreads) void topk_tiles(const char *x, void 
       }
     }
   } else {
-    const int64_t step = a.dense_last ? kSize : a.strides[a.axis];
+    const int64_t step = a.step(kSize);
     for (uint32_t i = threadIdx.x; i < sort_n; i += kBlockThreads) {
       const uint32_t element = first + i;
       keys[i] = element < a.width
@@ -223,15 +237,15 @@ __global__ __launch_bounds__(kBlockThreads) void topk_tiles(const char *x, void 
     }
   }
   sort_descending(keys, sort_n);
-  emit<T, kBytewise, kFinal>(keys, a, row, x, values, indices,
+  emit<T, kBlockThreads, kBytewise, kFinal>(keys, a, row, x, values, indices,
                              lists + ((size_t)row * tiles + tile) * a.count);
 }
 
 // One block per (row, group of `fan` lists): merge by sorting, keep the best `count`.
-template <class T, bool kBytewise, bool kFinal>
+template <class T, bool kBytewise, bool kFinal, class A>
 __global__ __launch_bounds__(kBlockThreads) void topk_merge(const char *x, void *values, int32_t *indices,
                                                             const uint64_t *in_lists, uint64_t *out_lists,
-                                                            Addressing a, uint32_t lists_in, uint32_t fan,
+                                                            A a, uint32_t lists_in, uint32_t fan,
                                                             uint32_t lists_out, uint32_t sort_n) {
   __shared__ uint64_t keys[kTile];
   const uint32_t row = blockIdx.x / lists_out, group = blockIdx.x - row * lists_out;
@@ -240,7 +254,7 @@ __global__ __launch_bounds__(kBlockThreads) void topk_merge(const char *x, void 
   const uint64_t *source = in_lists + ((size_t)row * lists_in + first_list) * a.count;
   for (uint32_t i = threadIdx.x; i < sort_n; i += kBlockThreads) keys[i] = i < taken ? source[i] : 0;
   sort_descending(keys, sort_n);
-  emit<T, kBytewise, kFinal>(keys, a, row, x, values, indices,
+  emit<T, kBlockThreads, kBytewise, kFinal>(keys, a, row, x, values, indices,
                              out_lists + ((size_t)row * lists_out + group) * a.count);
 }
 
@@ -302,17 +316,19 @@ __global__ __launch_bounds__(kBlockThreads) void topk_emit_run(const char *x, vo
   const uint32_t row = blockIdx.x / blocks_per_row;
   const uint32_t j = (blockIdx.x % blocks_per_row) * kBlockThreads + threadIdx.x;
   if (j >= a.count) return;
-  const int64_t base = row_base(a, row, kSize);
-  const int64_t step = a.dense_last ? kSize : a.strides[a.axis];
-  const uint32_t outer = row / a.inner, position = row - outer * a.inner;
+  const int64_t base = a.base(row, kSize), step = a.step(kSize);
   const uint32_t index = min(~(uint32_t)runs[(size_t)row * run_keys + j], a.width - 1);
   const uint32_t bits = load_bits<T, kBytewise>(x + base + (int64_t)index * step);
-  const size_t at = ((size_t)outer * a.count + j) * a.inner + position;
+  const size_t at = a.output(row, j);
   if constexpr (kSize == 4) static_cast<uint32_t *>(values)[at] = bits;
   else static_cast<uint16_t *>(values)[at] = (uint16_t)bits;
   indices[at] = (int32_t)index;
 }
 
+// How a tile's elements are read: one by one with the row's step, the same byte by byte, in aligned vectors, and
+// dense rows of no whole vectors (us of both dispatches, elements one by one / so: f32 [64, 151937], 40 best, 21.2 / 18.7,
+// bf16 [64, 248319], 64 best, 27.9 / 25.8, [3, 50001], 64 best, 11.0 / 10.5).
+constexpr int kElements = 0, kBytes = 1, kVectors = 2, kUnaligned = 3;
 constexpr uint32_t kSelectMax = kBlockThreads;  // largest count the select route serves
 
 // Exclusive prefix sum of `v` over the block in thread order; *total = sum over the block.
@@ -447,19 +463,20 @@ struct SelectShared {
 // data), and for int32, the tile takes the general form: ordered 32-bit values for every element,
 // the count-th largest of the 256 thread maxima as the bound, the exact count-th key bit by bit
 // if need be.
-template <class T, int kE, bool kVector, bool kBytewise, bool kFinal>
-__device__ __forceinline__ void select_tile(uint32_t (&bits)[kE], uint32_t first, const Addressing &a, uint32_t row,
+template <class T, int kE, int kAccess, bool kFinal, class A>
+__device__ __forceinline__ void select_tile(uint32_t (&bits)[kE], uint32_t first, const A &a, uint32_t row,
                                             uint32_t largest, const char *x, void *values, int32_t *indices,
                                             uint64_t *list, SelectShared &shared) {
   constexpr int kVec = KeyTraits<T>::kVec;
-  constexpr bool kFloat = !std::is_same<T, I32>::value;
+  constexpr bool kFloat = !std::is_same<T, I32>::value, kBytewise = kAccess == kBytes;
   uint64_t *keys = shared.keys;
   const uint32_t lane = threadIdx.x % kWaveLanes, wave = threadIdx.x / kWaveLanes;
-  auto element_of = [&](int j) -> uint32_t {
-    if constexpr (kVector) return first + (threadIdx.x + (j / kVec) * kBlockThreads) * kVec + (j % kVec);
-    else return first + threadIdx.x + j * kBlockThreads;
-  };
   const bool whole = first + kBlockThreads * kE <= a.width;  // no slot lies past the row's end
+  const bool vectors = kAccess == kVectors || (kAccess == kUnaligned && whole);
+  auto element_of = [&](int j) -> uint32_t {
+    if (vectors) return first + (threadIdx.x + (j / kVec) * kBlockThreads) * kVec + (j % kVec);
+    return first + threadIdx.x + j * kBlockThreads;
+  };
 
   if constexpr (kFloat) {
     // storage bits with the sign flipped when the smallest are wanted, so that "better" is
@@ -516,7 +533,7 @@ __device__ __forceinline__ void select_tile(uint32_t (&bits)[kE], uint32_t first
         __syncthreads();
         rank_candidates<kBlockThreads, 4>(keys, kCompact, total, a.count);
         __syncthreads();
-        emit<T, kBytewise, kFinal>(keys + kRanked, a, row, x, values, indices, list);
+        emit<T, kBlockThreads, kBytewise, kFinal>(keys + kRanked, a, row, x, values, indices, list);
         done = true;
       }
     }
@@ -621,7 +638,7 @@ __device__ __forceinline__ void select_tile(uint32_t (&bits)[kE], uint32_t first
     __syncthreads();
     rank_candidates<kBlockThreads, 4>(keys, 0, total, a.count);
     __syncthreads();
-    emit<T, kBytewise, kFinal>(keys + kRanked, a, row, x, values, indices, list);
+    emit<T, kBlockThreads, kBytewise, kFinal>(keys + kRanked, a, row, x, values, indices, list);
     __syncthreads();
     return;
   }
@@ -633,7 +650,7 @@ __device__ __forceinline__ void select_tile(uint32_t (&bits)[kE], uint32_t first
   for (int j = 0; j < kE; ++j)
     if (candidate(j) && position < kTile) keys[position++] = key_of(j);  // the guard never binds
   sort_descending(keys, sort_n);
-  emit<T, kBytewise, kFinal>(keys, a, row, x, values, indices, list);
+  emit<T, kBlockThreads, kBytewise, kFinal>(keys, a, row, x, values, indices, list);
   __syncthreads();
 }
 
@@ -641,21 +658,22 @@ __device__ __forceinline__ void select_tile(uint32_t (&bits)[kE], uint32_t first
 // one tile, the outputs).  Measured on MI355X for TopK(64) over [64, 151936] f32: tiles of 8192
 // elements 15.3 us, of 16384 (64 registers of elements per thread) 16.3 us; two tiles per block
 // with every load issued up front, so that one tile is selected while the next arrives, 17.9 us.
-template <class T, int kE, bool kVector, bool kBytewise, bool kFinal>
+template <class T, int kE, int kAccess, bool kFinal, class A>
 __global__ __launch_bounds__(kBlockThreads) void topk_select(const char *x, void *values, int32_t *indices,
-                                                             uint64_t *out_lists, Addressing a, uint32_t tiles,
+                                                             uint64_t *out_lists, A a, uint32_t tiles,
                                                              uint32_t largest) {
   constexpr int kSize = KeyTraits<T>::kSize;
   constexpr int kVec = KeyTraits<T>::kVec;
   __shared__ SelectShared shared;
   const uint32_t row = blockIdx.x / tiles, tile = blockIdx.x - row * tiles;
   const uint32_t first = tile * (kBlockThreads * kE);
-  const int64_t base = row_base(a, row, kSize);
+  const int64_t base = a.base(row, kSize);
   // Every load is issued before the first value is looked at: addresses past the row's end are
   // clamped to its last vector or element (a load inside a branch would wait for itself there).
   uint32_t bits[kE];
-  if constexpr (kVector) {
-    static_assert(kE % kVec == 0, "whole vectors per thread");
+  static_assert(kE % kVec == 0, "whole vectors per thread");
+  static_assert(!std::is_reference<A>::value, "arguments of a kernel go by value");
+  if constexpr (kAccess == kVectors) {
     const u32x4 *vectors = reinterpret_cast<const u32x4 *>(x + base);
     const uint32_t last_vector = a.width / kVec - 1;
     u32x4 raw[kE / kVec];
@@ -671,23 +689,38 @@ __global__ __launch_bounds__(kBlockThreads) void topk_select(const char *x, void
 #pragma unroll
       for (int j = 0; j < kVec; ++j) bits[v * kVec + j] = piece[j];
     }
+  } else if (kAccess == kUnaligned && first + kBlockThreads * kE <= a.width) {
+    // Rows of no whole vectors, a whole tile of one: vectors at element-aligned addresses.  The row's last
+    // tile goes element by element, which also deals its elements to all waves (each adds to the bound).
+    const char *tile_start = x + base + (size_t)first * kSize;
+    u32x4 raw[kE / kVec];
+#pragma unroll
+    for (int v = 0; v < kE / kVec; ++v)
+      raw[v] = *reinterpret_cast<const u32x4_element *>(tile_start + (size_t)(threadIdx.x + v * kBlockThreads) * 16);
+#pragma unroll
+    for (int v = 0; v < kE / kVec; ++v) {
+      uint32_t piece[kVec];
+      vector_bits<T>(raw[v], piece);
+#pragma unroll
+      for (int j = 0; j < kVec; ++j) bits[v * kVec + j] = piece[j];
+    }
   } else {
-    const int64_t step = a.dense_last ? kSize : a.strides[a.axis];
+    const int64_t step = a.step(kSize);
     const uint32_t last = a.width - 1;
 #pragma unroll
     for (int j = 0; j < kE; ++j)
-      bits[j] = load_bits<T, kBytewise>(x + base + (int64_t)min(first + threadIdx.x + j * kBlockThreads, last) * step);
+      bits[j] = load_bits<T, kAccess == kBytes>(x + base + (int64_t)min(first + threadIdx.x + j * kBlockThreads, last) * step);
   }
-  select_tile<T, kE, kVector, kBytewise, kFinal>(bits, first, a, row, largest, x, values, indices,
+  select_tile<T, kE, kAccess, kFinal>(bits, first, a, row, largest, x, values, indices,
                                                  out_lists + ((size_t)row * tiles + tile) * a.count, shared);
 }
 
 constexpr int kMergeThreads = 1024;  // one block per row: the work of a merge is latency, spread over 16 waves
 
-template <class T, bool kBytewise, bool kFinal>
+template <class T, bool kBytewise, bool kFinal, class A>
 __global__ __launch_bounds__(kMergeThreads) void topk_rank_lists(const char *x, void *values, int32_t *indices,
                                                                  const uint64_t *in_lists, uint64_t *out_lists,
-                                                                 Addressing a, uint32_t units_in, uint32_t fan,
+                                                                 A a, uint32_t units_in, uint32_t fan,
                                                                  uint32_t units_out) {
   extern __shared__ uint64_t merged[];  // fan * count keys
   __shared__ uint64_t chosen[kTile];    // candidates in [0, kRanked), the ranked result above
@@ -772,7 +805,7 @@ __global__ __launch_bounds__(kMergeThreads) void topk_rank_lists(const char *x, 
       __syncthreads();
       rank_candidates<kMergeThreads, 16>(chosen, 0, total, a.count);
       __syncthreads();
-      emit<T, kBytewise, kFinal>(ranked, a, row, x, values, indices, list);
+      emit<T, kMergeThreads, kBytewise, kFinal>(ranked, a, row, x, values, indices, list);
       return;
     }
   }
@@ -794,18 +827,21 @@ __global__ __launch_bounds__(kMergeThreads) void topk_rank_lists(const char *x, 
     if (rank < a.count && key != 0) ranked[rank] = key;
   }
   __syncthreads();
-  emit<T, kBytewise, kFinal>(ranked, a, row, x, values, indices, list);
+  emit<T, kMergeThreads, kBytewise, kFinal>(ranked, a, row, x, values, indices, list);
 }
 
 // Launch-shape labels: topk_<kernel>/<form>...
 inline std::string access_word(bool vector, bool bytewise) { return vector ? "vector" : (bytewise ? "bytes" : "scalar"); }
-template <int kE, bool kVector, bool kBytewise, bool kFinal> struct SelectTag {
+template <int kE, int kAccess, bool kFinal> struct SelectTag {
   static std::string text() {
-    return "topk_select/" + std::to_string(kE) + "x256/" + access_word(kVector, kBytewise) + (kFinal ? "/final" : "/lists");
+    return "topk_select/" + std::to_string(kE) + "x256/" + (kAccess == kUnaligned ? "unaligned" : access_word(kAccess == kVectors, kAccess == kBytes)) +
+           (kFinal ? "/final" : "/lists");
   }
 };
-template <bool kBytewise, bool kFinal> struct RankListsTag {
-  static std::string text() { return std::string("topk_rank_lists") + (kBytewise ? "/bytes" : "") + (kFinal ? "/final" : "/lists"); }
+template <bool kBytewise, bool kFinal, bool kDense> struct RankListsTag {  // #strided: the last round's outputs of other rows
+  static std::string text() {
+    return std::string("topk_rank_lists") + (kBytewise ? "/bytes" : "") + (kFinal ? "/final" : "/lists") + (kFinal && !kBytewise && !kDense ? "#strided" : "");
+  }
 };
 template <bool kVector, bool kBytewise, bool kFinal> struct TilesTag {
   static std::string text() { return "topk_tiles/" + access_word(kVector, kBytewise) + (kFinal ? "/final" : "/lists"); }
@@ -825,20 +861,24 @@ void select_tiles_launch(const TopKParams &p, const Addressing &a, const char *i
                          int32_t *indices, uint64_t *lists, bool vector, hipStream_t s) {
   const dim3 grid(p.rows * p.tiles), block(kBlockThreads);
   const uint32_t largest = p.largest ? 1u : 0u;
-  const bool final = p.tiles == 1;
-#define HYLE_SELECT(VEC, BYTES, FINAL)                                                                   \
-  note_variant<SelectTag<kE, VEC, BYTES, FINAL>>();                                                         \
-  hipLaunchKernelGGL((topk_select<T, kE, VEC, BYTES, FINAL>), grid, block, 0, s, in, values, indices, lists, a, \
-                     p.tiles, largest)
+  const bool final = p.tiles == 1, unaligned = p.dense_last && !kBytewise;
+  const DenseRows dense{a.width, a.count, a.largest};
+  constexpr int kOther = kBytewise ? kBytes : kElements;
+#define HYLE_SELECT(ACCESS, FINAL, ROWS)                                                              \
+  note_variant<SelectTag<kE, ACCESS, FINAL>>();                                                       \
+  hipLaunchKernelGGL((topk_select<T, kE, ACCESS, FINAL, std::decay_t<decltype(ROWS)>>), grid, block, 0, s, in, values, \
+                     indices, lists, ROWS, p.tiles, largest)
   // tiles of 2048 elements are chosen only for rows that one of them covers (topk_plan): no lists there; tiles of
   // 4096 only for rows of three or more
   if constexpr (kE != 16) {
-    if (final && vector) { HYLE_SELECT(true, false, true); }
-    else if (final) { HYLE_SELECT(false, kBytewise, true); }
+    if (final && vector) { HYLE_SELECT(kVectors, true, dense); }
+    else if (final && unaligned) { HYLE_SELECT(kUnaligned, true, dense); }
+    else if (final) { HYLE_SELECT(kOther, true, a); }
   }
   if constexpr (kE != 8) {
-    if (!final && vector) { HYLE_SELECT(true, false, false); }
-    else if (!final) { HYLE_SELECT(false, kBytewise, false); }
+    if (!final && vector) { HYLE_SELECT(kVectors, false, dense); }
+    else if (!final && unaligned) { HYLE_SELECT(kUnaligned, false, dense); }
+    else if (!final) { HYLE_SELECT(kOther, false, a); }
   }
 #undef HYLE_SELECT
 }
@@ -849,14 +889,19 @@ void rank_lists_launch(const TopKParams &p, const Addressing &a, const char *in,
                        hipStream_t s) {
   const dim3 grid(p.rows * out), block(kMergeThreads);
   const size_t shared = (size_t)fan * p.count * sizeof(uint64_t);
-  if (out == 1) {
-    note_variant<RankListsTag<kBytewise, true>>();
-    hipLaunchKernelGGL((topk_rank_lists<T, kBytewise, true>), grid, block, shared, s, in, values, indices, from, to,
-                       a, lists, fan, out);
-  } else {
-    note_variant<RankListsTag<kBytewise, false>>();
-    hipLaunchKernelGGL((topk_rank_lists<T, kBytewise, false>), grid, block, shared, s, in, values, indices, from,
+  const DenseRows dense{a.width, a.count, a.largest};
+  if (out > 1) {
+    note_variant<RankListsTag<kBytewise, false, true>>();
+    hipLaunchKernelGGL((topk_rank_lists<T, kBytewise, false, DenseRows>), grid, block, shared, s, in, values, indices, from,
+                       to, dense, lists, fan, out);
+  } else if (kBytewise || !p.dense_last) {
+    note_variant<RankListsTag<kBytewise, true, false>>();
+    hipLaunchKernelGGL((topk_rank_lists<T, kBytewise, true, Addressing>), grid, block, shared, s, in, values, indices, from,
                        to, a, lists, fan, out);
+  } else {
+    note_variant<RankListsTag<false, true, true>>();
+    hipLaunchKernelGGL((topk_rank_lists<T, false, true, DenseRows>), grid, block, shared, s, in, values, indices, from, to,
+                       dense, lists, fan, out);
   }
 }
 
@@ -881,6 +926,7 @@ hipError_t run(const TopKParams &p, const void *x, void *values, int32_t *indice
     a.dims[d] = p.dims[d];
     a.strides[d] = p.strides[d];
   }
+  const DenseRows dense{a.width, a.count, a.largest};
   const char *in = static_cast<const char *>(x);
   uint64_t *lists_a = static_cast<uint64_t *>(workspace);
   uint64_t *lists_b = lists_a + (size_t)p.rows * p.tiles * p.count;
@@ -909,14 +955,15 @@ hipError_t run(const TopKParams &p, const void *x, void *values, int32_t *indice
     // whole tiles sorted (every key kept), then runs merged in pairs until one is left per row
     Addressing whole = a;
     whole.count = kTile;
+    const DenseRows whole_dense{whole.width, whole.count, whole.largest};
     uint64_t *from = lists_a, *to = lists_a + (size_t)p.rows * p.tiles * kTile;
     if (vector) {
       note_variant<TilesTag<true, false, false>>();
-      hipLaunchKernelGGL((topk_tiles<T, true, false, false>), dim3(p.rows * p.tiles), block, 0, s, in, values, indices,
-                         from, whole, p.tiles, kTile, largest);
+      hipLaunchKernelGGL((topk_tiles<T, true, false, false, DenseRows>), dim3(p.rows * p.tiles), block, 0, s, in, values, indices,
+                         from, whole_dense, p.tiles, kTile, largest);
     } else {
       note_variant<TilesTag<false, kBytewise, false>>();
-      hipLaunchKernelGGL((topk_tiles<T, false, kBytewise, false>), dim3(p.rows * p.tiles), block, 0, s, in, values,
+      hipLaunchKernelGGL((topk_tiles<T, false, kBytewise, false, Addressing>), dim3(p.rows * p.tiles), block, 0, s, in, values,
                          indices, from, whole, p.tiles, kTile, largest);
     }
     const uint32_t limit = (p.count + kTile - 1) / kTile * kTile;  // no run needs more keys than this
@@ -939,22 +986,22 @@ hipError_t run(const TopKParams &p, const void *x, void *values, int32_t *indice
   if (p.tiles == 1) {
     if (vector) {
       note_variant<TilesTag<true, false, true>>();
-      hipLaunchKernelGGL((topk_tiles<T, true, false, true>), dim3(p.rows), block, 0, s, in, values, indices,
-                         lists_a, a, 1u, tile_n, largest);
+      hipLaunchKernelGGL((topk_tiles<T, true, false, true, DenseRows>), dim3(p.rows), block, 0, s, in, values, indices,
+                         lists_a, dense, 1u, tile_n, largest);
     } else {
       note_variant<TilesTag<false, kBytewise, true>>();
-      hipLaunchKernelGGL((topk_tiles<T, false, kBytewise, true>), dim3(p.rows), block, 0, s, in, values,
+      hipLaunchKernelGGL((topk_tiles<T, false, kBytewise, true, Addressing>), dim3(p.rows), block, 0, s, in, values,
                          indices, lists_a, a, 1u, tile_n, largest);
     }
     return hipGetLastError();
   }
   if (vector) {
     note_variant<TilesTag<true, false, false>>();
-    hipLaunchKernelGGL((topk_tiles<T, true, false, false>), dim3(p.rows * p.tiles), block, 0, s, in, values,
-                       indices, lists_a, a, p.tiles, kTile, largest);
+    hipLaunchKernelGGL((topk_tiles<T, true, false, false, DenseRows>), dim3(p.rows * p.tiles), block, 0, s, in, values,
+                       indices, lists_a, dense, p.tiles, kTile, largest);
   } else {
     note_variant<TilesTag<false, kBytewise, false>>();
-    hipLaunchKernelGGL((topk_tiles<T, false, kBytewise, false>), dim3(p.rows * p.tiles), block, 0, s, in,
+    hipLaunchKernelGGL((topk_tiles<T, false, kBytewise, false, Addressing>), dim3(p.rows * p.tiles), block, 0, s, in,
                        values, indices, lists_a, a, p.tiles, kTile, largest);
   }
   uint32_t lists = p.tiles;
@@ -964,12 +1011,12 @@ hipError_t run(const TopKParams &p, const void *x, void *values, int32_t *indice
     const uint32_t sort_n = pow2_at_least(std::min(lists, p.fan) * p.count, 64);
     if (out == 1) {
       note_variant<MergeTag<kBytewise, true>>();
-      hipLaunchKernelGGL((topk_merge<T, kBytewise, true>), dim3(p.rows), block, 0, s, in, values, indices, from,
+      hipLaunchKernelGGL((topk_merge<T, kBytewise, true, Addressing>), dim3(p.rows), block, 0, s, in, values, indices, from,
                          to, a, lists, p.fan, 1u, sort_n);
     } else {
       note_variant<MergeTag<kBytewise, false>>();
-      hipLaunchKernelGGL((topk_merge<T, kBytewise, false>), dim3(p.rows * out), block, 0, s, in, values,
-                         indices, from, to, a, lists, p.fan, out, sort_n);
+      hipLaunchKernelGGL((topk_merge<T, kBytewise, false, DenseRows>), dim3(p.rows * out), block, 0, s, in, values,
+                         indices, from, to, dense, lists, p.fan, out, sort_n);
     }
     std::swap(from, to);
     lists = out;

@@ -300,3 +300,30 @@ def test_topk_halved_tiles_do_not_leave_a_last_one_that_lacks_a_wave(tag, width,
         outputs = run(hc.TopK(count=count), to_device(stored, tag))
         assert hc.last_launch_variant().startswith(f"topk_select/{tile}x256/"), hc.last_launch_variant()
         check(tag, stored, [rows, width], count, -1, True, outputs)
+
+
+@pytest.mark.parametrize("tag", ["f32", "bf16"])
+def test_topk_dense_rows_of_no_whole_vectors(tag):
+    """Whole tiles are read as vectors at element-aligned addresses, a row's last one element by element: one tile and several, a
+    base one element in, a last tile of one element and of all but one; and the same rows with the axis in front."""
+    rng = np.random.default_rng(1162)
+    for rows, width, count, label in ((3, 2047, 17, "8x256/unaligned/final"), (2, 2049, 40, "32x256/unaligned/final"), (3, 8191, 256, "32x256/unaligned/final"),
+                                      (3, 8193, 41, "16x256/unaligned/lists"), (2, 12287, 64, "16x256/unaligned/lists"),
+                                      (2, 131073, 20, "32x256/unaligned/lists"), (3, 3 * 8192 + 1, 100, "32x256/unaligned/lists"), (2, 140001, 256, "32x256/unaligned/lists")):
+        stored = tied_values(rng, [rows, width], tag)
+        for largest in (True, False):
+            note(f"topk {tag} [{rows}, {width}] count {count} largest {largest}: {label}")
+            outputs = run(hc.TopK(count=count, largest=largest), to_device(stored, tag))
+            assert hc.last_launch_variant().startswith("topk_select/" + label), hc.last_launch_variant()
+            check(tag, stored, [rows, width], count, -1, largest, outputs)
+        note(f"topk {tag} axis 0 of [{width}, {rows}] count {count}")
+        across = np.ascontiguousarray(stored.T)
+        outputs = run(hc.TopK(count=count, axis=0), to_device(across, tag))
+        assert hc.last_launch_variant().startswith("topk_select/" + label.replace("unaligned", "scalar")), hc.last_launch_variant()
+        check(tag, across, [width, rows], count, 0, True, outputs)
+    for width, label in ((2048, "8x256/unaligned/final"), (8192, "32x256/unaligned/final"), (24576, "16x256/unaligned/lists")):
+        stored = tied_values(rng, [2 * width + 1], tag)
+        note(f"topk {tag} [2, {width}] one element in")
+        outputs = run(hc.TopK(count=9), to_device(stored, tag)[1:].view(2, width))
+        assert hc.last_launch_variant().startswith("topk_select/" + label), hc.last_launch_variant()
+        check(tag, stored[1:].copy(), [2, width], 9, -1, True, outputs)
