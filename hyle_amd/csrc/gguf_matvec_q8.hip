@@ -34,6 +34,7 @@
 #include "gguf_decode.h"
 #include "gguf_lines.h"
 #include "gguf_q8_math.h"
+#include "gguf_q8_quantise.h"
 #include "kernels.h"
 
 namespace hyle_hip {
@@ -75,38 +76,45 @@ struct LaneCodes {
   float scale;
 };
 
-// Quantises the lane's share of span `span` of the activation row at `x` (k values of type TX).
-// Every lane of a wave calls it; lanes that share an activation block agree on its scale through
-// a cross-lane maximum.
+// The lane's share of span `span` of the activation row at `x` (k values of type TX), 32 values.
 // `live`: the lane's positions exist (a Q8_0 row's last span may be short: lanes past it read the
-// row's first values and come back with zero codes and a zero scale).
+// row's first values and come back from quantise_span with zero codes and a zero scale).
 template <int kKind, class TX>
-__device__ __forceinline__ LaneCodes quantise_span(const void *x, size_t row_offset, uint32_t span, uint32_t lane, bool live = true) {
+__device__ __forceinline__ BlockValues<TX, 32> fetch_span(const void *x, size_t row_offset, uint32_t span, uint32_t lane, bool live = true) {
   using Kind = Lines<kKind>;
   // the lane's positions come in runs of eight neighbours (Lines<kind>::position), each a whole
   // 16-byte vector of a narrow type or two of f32: x starts on a 16-byte boundary (run_m)
-  float values[32];
+  BlockValues<TX, 32> fetched;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const size_t at = row_offset + (live ? Kind::position(span, lane, 8 * g) : (uint32_t)(8 * g));
-    if constexpr (Traits<TX>::kVec == 8) {
-      float piece[8];
-      Traits<TX>::unpack(load16(x, at / 8), piece);
+    constexpr int kPieces = 8 / Traits<TX>::kVec;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) values[8 * g + t] = piece[t];
-    } else {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        float piece[4];
-        Traits<TX>::unpack(load16(x, at / 4 + h), piece);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) values[8 * g + 4 * h + t] = piece[t];
-      }
-    }
+    for (int h = 0; h < kPieces; ++h) fetched.raw[kPieces * g + h] = load16(x, at / Traits<TX>::kVec + h);
   }
+  return fetched;
+}
+// Quantises it.  Every lane of a wave calls it; lanes that share an activation block agree on its scale through a
+// cross-lane maximum.  A wave of regular blocks takes the short form of gguf_q8_quantise.h: what precedes a span kernel's
+// first row is about 160 instructions then, 390 the long way (us: Q6_K [2048 -> 2560] 5.0 with the long way alone and the
+// activations asked for behind the weights, 4.05 now; [6144 -> 2048] 6.25 / 5.75; Q8_0 [2048 -> 2048] 4.0 / 3.85).
+template <int kKind, class TX>
+__device__ __forceinline__ LaneCodes quantise_span(const BlockValues<TX, 32> &fetched, uint32_t span, uint32_t lane, bool live = true) {
+  using Kind = Lines<kKind>;
+  float values[32];
+  fetched.values(values);
   LaneCodes out;
   // Q8_0: the lane's 32 values are one block.  Q6_K: eight lanes share a block of 256.
   constexpr int kLanesPerBlock = kKind == 1 ? 8 : 1;
+  const BlockTop block = block_top<kKind == 2, kLanesPerBlock>(fetched, values);
+  if (__builtin_expect(__ballot(!block.regular()) == 0, 1)) {
+    float factor;
+    short_factors<kKind == 2>(block, factor, out.scale);
+    if (!live) factor = out.scale = 0.0f;  // 0 * finite: codes of 0
+#pragma unroll
+    for (int w = 0; w < 8; ++w) out.codes[w] = short_codes(values[4 * w], values[4 * w + 1], values[4 * w + 2], values[4 * w + 3], factor);
+    return out;
+  }
   LaneMax mine{0.0f, 0.0f, 0u};
 #pragma unroll
   for (int e = 0; e < 32; ++e) {  // positions rise with e, so ">" keeps the first
@@ -256,7 +264,7 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_lines(const unsi
   const uint32_t k = spans * 2048;
   // every wave quantises its share of the (activation row, span) pairs; the block then shares them
   for (uint32_t pair = wave; pair < m * spans; pair += kWavesPerBlock)
-    park(staged, pair, lane, quantise_span<kKind, TX>(x, (size_t)(pair / spans) * k, pair % spans, lane));
+    park(staged, pair, lane, quantise_span<kKind, TX>(fetch_span<kKind, TX>(x, (size_t)(pair / spans) * k, pair % spans, lane), pair % spans, lane));
   __syncthreads();
   LaneCodes held[kRegisters ? kM : 1];
   if constexpr (kRegisters) {
@@ -379,13 +387,14 @@ __global__ __launch_bounds__(kSpans * kWaveLanes) void gguf_matvec_q8_spans(cons
   const uint32_t live_lanes = kShort && span == (uint32_t)kSpans - 1 ? tail_lanes : (uint32_t)kWaveLanes;
   const bool live = !kShort || lane < live_lanes;
   const uint32_t vectors = kShort ? (live_lanes * 34u + 15u) / 16u : (uint32_t)Kind::kPassVectors;
+  const BlockValues<TX, 32> fetched = fetch_span<kKind, TX>(x, 0, span, lane, live);  // before the weights: loads return in order
   Row ring[kLinesDepth];
 #pragma unroll
   for (int d = 0; d < kLinesDepth; ++d) {
     const uint32_t wanted = first + d;
     ring[d] = Row::template load<kStream>(mine + (size_t)(wanted < rows ? wanted : first) * row_stride, lane, vectors);
   }
-  const LaneCodes held = quantise_span<kKind, TX>(x, 0, span, lane, live);  // while the first rows are on their way
+  const LaneCodes held = quantise_span<kKind, TX>(fetched, span, lane, live);  // while the first rows are on their way
   for (uint32_t base = first; base < rows; base += step) {
     float totals[kLinesDepth] = {};
 #pragma unroll
@@ -507,7 +516,7 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_quads(const unsi
   const uint32_t quad = lane / 4, own = lane % 4;  // positions of lanes 4 quad .. + 3; weight row and activation row `own`
   const uint32_t k = spans * 2048;
   for (uint32_t pair = wave; pair < m * spans; pair += kWavesPerBlock)
-    park(staged, pair, lane, quantise_span<kKind, TX>(x, (size_t)(pair / spans) * k, pair % spans, lane));
+    park(staged, pair, lane, quantise_span<kKind, TX>(fetch_span<kKind, TX>(x, (size_t)(pair / spans) * k, pair % spans, lane), pair % spans, lane));
   __syncthreads();
   uint32_t token[kSets];
 #pragma unroll
@@ -623,67 +632,6 @@ __host__ __device__ inline size_t tile_shared_bytes(uint32_t tokens, uint32_t bl
          (size_t)kWavesPerBlock * kWaveLanes * (tokens >= 4 ? tokens / 4 : 1) * 4;
 }
 
-// Half a wave quantises an activation block of 256 values (Q8_K), eight values per lane.
-struct TileValues {
-  u32x4 raw[2];
-};
-template <class TX> __device__ __forceinline__ TileValues tile_fetch(const void *x, size_t first, uint32_t u) {
-  TileValues out;
-  if constexpr (Traits<TX>::kVec == 8) {
-    out.raw[0] = load16(x, first / 8 + u);
-    out.raw[1] = out.raw[0];
-  } else {
-    out.raw[0] = load16(x, first / 4 + 2 * (size_t)u);
-    out.raw[1] = load16(x, first / 4 + 2 * (size_t)u + 1);
-  }
-  return out;
-}
-template <class TX>
-__device__ __forceinline__ void tile_quantise(const TileValues &fetched, uint32_t u, unsigned char *codes, int *sums,
-                                              float *scale) {
-  float values[8];
-  if constexpr (Traits<TX>::kVec == 8) {
-    Traits<TX>::unpack(fetched.raw[0], values);
-  } else {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      float piece[4];
-      Traits<TX>::unpack(fetched.raw[h], piece);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) values[4 * h + e] = piece[e];
-    }
-  }
-  LaneMax mine{0.0f, 0.0f, 0u};
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {  // positions rise with e, so ">" keeps the first
-    const float magnitude = __builtin_fabsf(values[e]);
-    if (magnitude > mine.magnitude) mine = LaneMax{magnitude, values[e], 8 * u + (uint32_t)e};
-  }
-  if (mine.magnitude == 0.0f) mine.position = 0xFFFFFFFFu;
-  const LaneMax top = block_largest<32>(mine);
-  float factor = 0.0f, stored = 0.0f;
-  if (top.magnitude != 0.0f) {
-    factor = -127.0f / top.value;
-    stored = 1.0f / factor;
-  }
-  uint32_t words[2];
-#pragma unroll
-  for (int w = 0; w < 2; ++w) {
-    uint32_t word = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) word |= code_of(values[4 * w + e] * factor) << (8 * e);
-    words[w] = top.magnitude != 0.0f ? word : 0u;
-  }
-  int sum = dot4(0x01010101u, words[0], dot4(0x01010101u, words[1], 0));
-  sum += dpp_move<kDppSwap1>(sum);
-  sum += dpp_move<kDppSwap2>(sum);  // the four lanes of a 32-value sub-block
-  uint32_t *at = reinterpret_cast<uint32_t *>(codes) + 2 * u;
-  at[0] = words[0];
-  at[1] = words[1];
-  if (u % 4 == 0) sums[u / 4] = sum;
-  if (u == 0) *scale = stored;
-}
-
 // The sixteen six-bit factors of a block: sc[s] and mn[s] of sub-block s.
 struct TileFactors {
   int sc[8], mn[8];
@@ -748,35 +696,38 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_tiles(const unsi
     return out;
   };
   auto clamped = [&](uint32_t g) { return g < groups ? g : groups - 1; };
-  // activation blocks go round the block's eight half waves, four (eight) of a half wave's loads in flight;
+  // (sixteen lanes to an activation block and the short form: [6144 -> 2048] 6.15 us, 7.05 with 32 lanes that each carry
+  // value, magnitude and place through the maximum; [8192 -> 2048] 6.55 and 7.9)
+  // activation blocks go round the block's sixteen groups of sixteen lanes, two (four) of a group's loads in flight;
   // the first round is asked for before the weights: loads return in order
-  constexpr uint32_t kHalves = kBlockThreads / 32, kBatch = kSets == 2 ? 8 : 4;  // (eight activation rows of 2048 values are 64 blocks)
-  const uint32_t half = threadIdx.x / 32, u = threadIdx.x % 32;
-  const uint32_t units = kTokens * blocks;
-  auto fetch_batch = [&](uint32_t first, TileValues (&fetched)[kBatch]) {
+  constexpr uint32_t kGroups = kBlockThreads / 16, kBatch = kSets == 2 ? 4 : 2;  // (eight activation rows of 2048 values are 64 blocks)
+  const uint32_t own_unit = threadIdx.x / 16, units = kTokens * blocks;
+  auto clamped_unit = [&](uint32_t unit) { return unit < units ? unit : units - 1; };  // the last one again: the same values to the same places
+  auto fetch_batch = [&](uint32_t first, BlockValues<TX> (&fetched)[kBatch]) {
 #pragma unroll
     for (uint32_t j = 0; j < kBatch; ++j) {
-      const uint32_t unit = first + j * kHalves < units ? first + j * kHalves : units - 1;
+      const uint32_t unit = clamped_unit(first + j * kGroups);
       const uint32_t token = unit / blocks, block = unit - token * blocks;
-      fetched[j] = tile_fetch<TX>(x, (size_t)(token < m ? token : m - 1) * k + (size_t)block * 256, u);
+      fetched[j].load(x, (size_t)(token < m ? token : m - 1) * k + (size_t)block * 256 + 16 * (lane % 16));
     }
   };
-  auto quantise_batch = [&](uint32_t first, const TileValues (&fetched)[kBatch]) {
+  auto quantise_batch = [&](uint32_t first, const BlockValues<TX> (&fetched)[kBatch]) {
 #pragma unroll
     for (uint32_t j = 0; j < kBatch; ++j) {
-      const uint32_t unit = first + j * kHalves;
-      if (unit < units) tile_quantise<TX>(fetched[j], u, codes + (size_t)unit * 256, sums + (size_t)unit * 8, scales + unit);
+      const uint32_t unit = clamped_unit(first + j * kGroups);
+      if (first - lane / 16 + j * kGroups < units)  // the same for the whole wave
+        quantise_block<0, TX>(fetched[j], lane, codes + (size_t)unit * 256, scales + unit, 0, sums + (size_t)unit * 8, 1);
     }
   };
-  TileValues fetched[kBatch];
-  fetch_batch(half, fetched);
+  BlockValues<TX> fetched[kBatch];
+  fetch_batch(own_unit, fetched);
   TileGroup ring[2];
   ring[0] = load_group(clamped(member));
   ring[1] = load_group(clamped(member + split));
   for (uint32_t at = threadIdx.x * 16; at < k; at += kBlockThreads * 16) *reinterpret_cast<u32x4 *>(shared + at) = u32x4{0u, 0u, 0u, 0u};
-  quantise_batch(half, fetched);
+  quantise_batch(own_unit, fetched);
   if constexpr (!kOneBatch) {  // more activation blocks than one round takes: the rest wait for the weights before them
-    for (uint32_t first = half + kHalves * kBatch; first < units; first += kHalves * kBatch) {
+    for (uint32_t first = own_unit + kGroups * kBatch; first - lane / 16 < units; first += kGroups * kBatch) {
       fetch_batch(first, fetched);
       quantise_batch(first, fetched);
     }
@@ -1152,14 +1103,10 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_blocks(const uns
   };
   u32x4 ring[kBlocksDepth][Step::kLoads];
   uint32_t shifts[kBlocksDepth] = {};
-  if (segments != 0) {  // the wave's first steps are on their way while the block quantises the activations
-#pragma unroll
-    for (int d = 0; d < kBlocksDepth; ++d) next_load(ring[d], &shifts[d]);
-  }
-
   // ---- the activation rows, quantised once per block ------------------------------------------
   // A thread takes eight neighbouring values at a time (one 16-byte vector of a narrow type, two of
-  // f32, when x allows vector loads), the next eight already on their way.
+  // f32, when x allows vector loads), the next eight already on their way; the first before
+  // the weights: loads return in order.
   auto fetch_values = [&](uint32_t r, uint32_t p, float (&values)[8]) {
     const bool inside = p < k;
     const size_t at = (size_t)r * k + (inside ? p : 0u);  // a thread past the row reads its start and keeps nothing
@@ -1188,6 +1135,10 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_blocks(const uns
   const uint32_t turns = m * pieces;
   float ahead[8];
   if (turns != 0) fetch_values(0, threadIdx.x * 8, ahead);
+  if (segments != 0) {  // the wave's first steps are on their way while the block quantises the activations
+#pragma unroll
+    for (int d = 0; d < kBlocksDepth; ++d) next_load(ring[d], &shifts[d]);
+  }
   for (uint32_t turn = 0; turn < turns; ++turn) {
     const uint32_t r = turn / pieces, p = (turn % pieces) * (kBlockThreads * 8) + threadIdx.x * 8;
     const bool inside = p < k;  // the same for all lanes that share an activation block
@@ -1196,28 +1147,36 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_blocks(const uns
     for (int e = 0; e < 8; ++e) values[e] = ahead[e];
     if (turn + 1 < turns)
       fetch_values((turn + 1) / pieces, ((turn + 1) % pieces) * (kBlockThreads * 8) + threadIdx.x * 8, ahead);
-    LaneMax mine{0.0f, 0.0f, 0u};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {  // positions rise with e, so ">" keeps the first
-      const float magnitude = __builtin_fabsf(values[e]);
-      if (magnitude > mine.magnitude) mine = LaneMax{magnitude, values[e], p + e};
-    }
-    if (mine.magnitude == 0.0f) mine.position = 0xFFFFFFFFu;  // no candidate: any lane with one goes first
-    const LaneMax top = block_largest<kQuantiseLanes>(mine);
     float factor = 0.0f, stored = 0.0f;
-    if (top.magnitude != 0.0f) {
-      if constexpr (kKind == 2) {
-        stored = f16_to_f32(f32_to_f16(top.magnitude / 127.0f));
-        factor = 127.0f / top.magnitude;
-      } else {
-        factor = -127.0f / top.value;
-        stored = 1.0f / factor;
-      }
-    }
     uint32_t words[2] = {0u, 0u};
-    if (top.magnitude != 0.0f) {
+    BlockValues<F32, 8> widened;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) words[e / 4] |= code_of(values[e] * factor) << (8 * (e % 4));
+    for (int e = 0; e < 8; ++e) widened.raw[e / 4][e % 4] = f32_bits(values[e]);
+    const BlockTop block = block_top<kKind == 2, kQuantiseLanes>(widened, values);
+    if (__builtin_expect(__ballot(inside && !block.regular()) == 0, 1)) {
+      short_factors<kKind == 2>(block, factor, stored);
+#pragma unroll
+      for (int w = 0; w < 2; ++w) words[w] = short_codes(values[4 * w], values[4 * w + 1], values[4 * w + 2], values[4 * w + 3], factor);
+    } else {
+      LaneMax mine{0.0f, 0.0f, 0u};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {  // positions rise with e, so ">" keeps the first
+        const float magnitude = __builtin_fabsf(values[e]);
+        if (magnitude > mine.magnitude) mine = LaneMax{magnitude, values[e], p + e};
+      }
+      if (mine.magnitude == 0.0f) mine.position = 0xFFFFFFFFu;  // no candidate: any lane with one goes first
+      const LaneMax top = block_largest<kQuantiseLanes>(mine);
+      if (top.magnitude != 0.0f) {
+        if constexpr (kKind == 2) {
+          stored = f16_to_f32(f32_to_f16(top.magnitude / 127.0f));
+          factor = 127.0f / top.magnitude;
+        } else {
+          factor = -127.0f / top.value;
+          stored = 1.0f / factor;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) words[e / 4] |= code_of(values[e] * factor) << (8 * (e % 4));
+      }
     }
     if (inside) {
       uint32_t *to = reinterpret_cast<uint32_t *>(codes + (size_t)r * k + p);

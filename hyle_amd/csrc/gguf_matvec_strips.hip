@@ -54,6 +54,7 @@
 
 #include "device_common.h"
 #include "gguf_q8_math.h"
+#include "gguf_q8_quantise.h"
 #include "kernels.h"
 
 namespace hyle_hip {
@@ -64,10 +65,7 @@ constexpr size_t kStripLds = 160 * 1024;  // of a compute unit, and the most one
 constexpr uint32_t kZeroBytes = 384;      // a lane's operands of one run lie within 384 bytes of its base
 constexpr uint32_t kCodePad = 16;         // between activation rows: neighbours start on other LDS banks
 
-// 16 bytes at any even address.
-typedef uint32_t words4_even __attribute__((ext_vector_type(4), aligned(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef short short2v __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // kWords words of LDS from any even offset.
@@ -322,183 +320,6 @@ template <int kSets> struct StripDotInPlace {
 template <int kSets> struct StripDot<3, kSets> : StripDotInPlace<kSets> {};
 template <int kSets> struct StripDot<4, kSets> : StripDotInPlace<kSets> {};
 
-// Sixteen neighbouring values of an activation row at any element's address.
-template <class TX> struct StripValues {
-  static constexpr int kVectors = Traits<TX>::kSize;
-  u32x4 raw[kVectors];
-  __device__ __forceinline__ void load(const void *x, size_t first) {
-#pragma unroll
-    for (int h = 0; h < kVectors; ++h)
-      raw[h] = *reinterpret_cast<const words4_even *>(static_cast<const char *>(x) + first * Traits<TX>::kSize + 16 * h);
-  }
-  __device__ __forceinline__ void values(float (&v)[16]) const {
-#pragma unroll
-    for (int h = 0; h < kVectors; ++h) {
-      float piece[Traits<TX>::kVec];
-      Traits<TX>::unpack(raw[h], piece);
-#pragma unroll
-      for (int e = 0; e < Traits<TX>::kVec; ++e) v[Traits<TX>::kVec * h + e] = piece[e];
-    }
-  }
-  // f32 bits of the largest value that is not negative and of the largest magnitude among the others, 0 where
-  // there is none.  Compared as stored: bit patterns of one sign are in the order of their magnitudes, NaN last.
-  __device__ __forceinline__ void extremes(uint32_t &positive, uint32_t &negative) const {
-    if constexpr (Traits<TX>::kSize == 4) {
-      int above = (int)raw[0].x;
-      uint32_t below = raw[0].x;
-#pragma unroll
-      for (int i = 1; i < 16; ++i) {
-        above = max(above, (int)raw[i / 4][i % 4]);
-        below = max(below, raw[i / 4][i % 4]);
-      }
-      positive = above < 0 ? 0u : (uint32_t)above;
-      negative = (int)below < 0 ? below & 0x7FFFFFFFu : 0u;
-    } else {
-      typedef short i16x2 __attribute__((ext_vector_type(2)));
-      typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-      i16x2 above = __builtin_bit_cast(i16x2, (uint32_t)raw[0].x);
-      u16x2 below = __builtin_bit_cast(u16x2, (uint32_t)raw[0].x);
-#pragma unroll
-      for (int i = 1; i < 8; ++i) {
-        above = __builtin_elementwise_max(above, __builtin_bit_cast(i16x2, (uint32_t)raw[i / 4][i % 4]));
-        below = __builtin_elementwise_max(below, __builtin_bit_cast(u16x2, (uint32_t)raw[i / 4][i % 4]));
-      }
-      const int high = max((int)above.x, (int)above.y);
-      const uint32_t low = max((uint32_t)below.x, (uint32_t)below.y);
-      positive = f32_bits(widened((uint32_t)max(high, 0)));
-      negative = f32_bits(widened((low & 0x8000u) != 0 ? low & 0x7FFFu : 0u));
-    }
-  }
-  static __device__ __forceinline__ float widened(uint32_t half) {
-    if constexpr (std::is_same_v<TX, BF16>) return bits_f32(half << 16);
-    else return f16_to_f32((uint16_t)half);
-  }
-};
-
-// The larger of both over 2 or 16 neighbouring lanes.
-template <int kLanes> __device__ __forceinline__ uint32_t lanes_max(uint32_t v) {
-  v = max(v, (uint32_t)dpp_move<kDppSwap1>((int)v));
-  if constexpr (kLanes == 16) {
-    v = max(v, (uint32_t)dpp_move<kDppSwap2>((int)v));
-    v = max(v, (uint32_t)dpp_move<kDppHalfMirror>((int)v));
-    v = max(v, (uint32_t)dpp_move<kDppRowMirror>((int)v));
-  }
-  return v;
-}
-
-// 127 / b correctly rounded for b from 2^-60 to 2^61: the hardware's reciprocal, a Newton step and a correction of
-// the quotient by its exact remainder, right for every mantissa of b with a reciprocal up to one unit off.  It is
-// six instructions where the full division, which scales its operands, is eleven.  (1 / b is not to be had this way
-// without knowing the reciprocal of a mantissa of all ones: from an estimate that is off the steps end one unit short.)
-__device__ __forceinline__ float quotient_of_127(float b) {
-  const float rough = __builtin_amdgcn_rcpf(b);
-  const float inverse = __builtin_fmaf(__builtin_fmaf(-b, rough, 1.0f), rough, rough);
-  const float q = 127.0f * inverse;
-  return __builtin_fmaf(__builtin_fmaf(-b, q, 127.0f), inverse, q);
-}
-// b / 127 the same way
-__device__ __forceinline__ float over_127(float b) {
-  constexpr float kInverse = 1.0f / 127.0f;
-  const float q = b * kInverse;
-  return __builtin_fmaf(__builtin_fmaf(-127.0f, q, b), kInverse, q);
-}
-
-// Sixteen lanes quantise a run of 256 values of an activation row, sixteen values per lane u: one Q8_K block, or eight
-// Q8_0 blocks of two lanes each.  A block whose largest magnitude lies between 2^-60 and 2^61 and (Q8_K, where its sign
-// counts) is not met with both signs takes the short form, in which a code is the low byte of value * factor + 1.5 * 2^23:
-// rounded to the nearest integer, ties to even, and no more than 127 in magnitude.  Any other block (zeros, NaN,
-// infinities) sends the wave the long way.
-template <int kKind, class TX>
-__device__ __forceinline__ void strip_quantise(const StripValues<TX> &fetched, uint32_t lane, unsigned char *codes, float *scale, uint32_t scale_step,
-                                               int *sums, uint32_t sum_step) {
-  constexpr bool kSmall = kKind >= 2;  // blocks of 32
-  constexpr int kLanes = kSmall ? 2 : 16;
-  const uint32_t u = lane % 16;
-  float v[16];
-  fetched.values(v);
-  uint32_t positive, negative, top_bits;
-  if constexpr (kSmall) {  // no sign to keep: the largest magnitude, NaN if there is one
-    float largest = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; e += 2)
-      largest = __builtin_elementwise_maximum(__builtin_elementwise_maximum(__builtin_fabsf(v[e]), __builtin_fabsf(v[e + 1])), largest);
-    positive = negative = top_bits = lanes_max<kLanes>(f32_bits(largest) & 0x7FFFFFFFu);
-  } else {
-    fetched.extremes(positive, negative);
-    positive = lanes_max<kLanes>(positive), negative = lanes_max<kLanes>(negative);
-    top_bits = max(positive, negative);
-  }
-  const bool regular = top_bits >= (67u << 23) && top_bits < (188u << 23) && (kSmall || positive != negative);
-  float factor = 0.0f, stored = 0.0f;
-  uint32_t words[4];
-  if (__builtin_expect(__ballot(!regular) == 0, 1)) {
-    const float top = bits_f32(top_bits);
-    if constexpr (kSmall) {
-      stored = f16_to_f32(f32_to_f16(over_127(top)));
-      factor = quotient_of_127(top);
-    } else {
-      factor = quotient_of_127(top);
-      factor = positive > negative ? -factor : factor;
-      stored = 1.0f / factor;
-    }
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      uint32_t code[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) code[e] = f32_bits(v[4 * w + e] * factor + 12582912.0f);
-      words[w] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(code[3], code[2], 0x0C0C0400u), __builtin_amdgcn_perm(code[1], code[0], 0x0C0C0400u), 0x05040100u);
-    }
-  } else {
-    float largest = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) largest = __builtin_fmaxf(largest, __builtin_fabsf(v[e]));  // a NaN is no candidate
-    const float top = bits_f32(lanes_max<kLanes>(f32_bits(largest)));
-    if constexpr (kSmall) {
-      if (top != 0.0f) {
-        stored = f16_to_f32(f32_to_f16(top / 127.0f));
-        factor = 127.0f / top;
-      }
-    } else {
-      // the sign of the block's first value of that magnitude: of the lowest lane that has one
-      bool below_zero = false;
-#pragma unroll
-      for (int e = 15; e >= 0; --e) below_zero = __builtin_fabsf(v[e]) == top ? v[e] < 0.0f : below_zero;
-      const uint64_t has = __ballot(largest == top), below = __ballot(below_zero);
-      const uint32_t own_has = (uint32_t)(has >> (lane & 48u)) & 0xFFFFu, own_below = (uint32_t)(below >> (lane & 48u));
-      if (top != 0.0f) {
-        const float value = (own_below >> __builtin_ctz(own_has)) & 1u ? -top : top;
-        factor = -127.0f / value;
-        stored = 1.0f / factor;
-      }
-    }
-    // nearest integer, ties to even, at most 127 (a block of zeros: factor 0); only the low bytes are kept
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      int code[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) code[e] = (int)__builtin_rintf(v[4 * w + e] * factor);
-      const short2v most = {127, 127};
-      const short2v low = __builtin_elementwise_min(__builtin_bit_cast(short2v, __builtin_amdgcn_cvt_pk_i16(code[0], code[1])), most);
-      const short2v high = __builtin_elementwise_min(__builtin_bit_cast(short2v, __builtin_amdgcn_cvt_pk_i16(code[2], code[3])), most);
-      words[w] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, high), __builtin_bit_cast(uint32_t, low), 0x06040200u);
-    }
-  }
-  const u32x4 whole = {words[0], words[1], words[2], words[3]};
-  // Q8_0 in place: 48 bytes per block, its codes where its quants lie in the 48 bytes from its first vector
-  if constexpr (kKind >= 3) *reinterpret_cast<words4_even *>(codes + 50 * (u / 2) + 2 + 16 * (u % 2)) = whole;
-  else reinterpret_cast<u32x4 *>(codes)[u] = whole;
-  if constexpr (kKind == 0) {
-    int sum = dot4(0x01010101u, words[0], dot4(0x01010101u, words[1], dot4(0x01010101u, words[2], dot4(0x01010101u, words[3], 0))));
-    sum += dpp_move<kDppSwap1>(sum);  // the two lanes of a sub-block
-    if (u % 2 == 0) sums[(u / 2) * sum_step] = sum;
-  }
-  if constexpr (kSmall) {
-    if (u % 2 == 0) scale[(u / 2) * scale_step] = stored;
-  } else {
-    if (u == 0) *scale = stored;
-  }
-}
-
 // Orders a wave's own LDS accesses.
 __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -583,9 +404,9 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
   const uint32_t units = m * runs, step = blockDim.x / 16, u = lane % 16;
   const uint32_t inverse = (1u << 20) / runs + 1;  // unit / runs = unit * inverse >> 20 while units * runs < 2^20 (units <= 8 runs, runs <= 224)
   // a unit past the last is the last one again: the same values to the same places
-  auto fetch = [&](uint32_t first, StripValues<TX> &into) { into.load(x, (size_t)min(first + lane / 16, units - 1) * 256 + 16 * u); };  // rows are dense
+  auto fetch = [&](uint32_t first, BlockValues<TX> &into) { into.load(x, (size_t)min(first + lane / 16, units - 1) * 256 + 16 * u); };  // rows are dense
   uint32_t unit = 4 * wave;  // of the wave's first sixteen lanes
-  StripValues<TX> ahead[kBatch];
+  BlockValues<TX> ahead[kBatch];
 #pragma unroll
   for (int j = 0; j < kBatch; ++j)
     if (unit + j * step < units) fetch(unit + j * step, ahead[j]);
@@ -604,10 +425,10 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
       if (unit >= units) break;
-      const StripValues<TX> now = ahead[j];
+      const BlockValues<TX> now = ahead[j];
       if (unit + kBatch * step < units) fetch(unit + kBatch * step, ahead[j]);
       const uint32_t mine = min(unit + lane / 16, units - 1), token = __umul24(mine, inverse) >> 20, run = mine - __umul24(token, runs);
-      strip_quantise<kKind, TX>(now, lane, shared + kZeroBytes + __umul24(token, strip_code_pitch(kKind, k)) + __umul24(run, strip_run_codes(kKind)),
+      quantise_block<kKind, TX>(now, lane, shared + kZeroBytes + __umul24(token, strip_code_pitch(kKind, k)) + __umul24(run, strip_run_codes(kKind)),
                                 scales + (size_t)(kKind >= 2 ? 8 * run : run) * kSets * 4 + token, kSets * 4,
                                 sums + (size_t)8 * run * kSets * 4 + token, kSets * 4);
       unit += step;
@@ -750,11 +571,12 @@ hipError_t run_strips(const MatVecParams &p, uint32_t m, const void *w, const vo
   const uint32_t tiles = (block_rows + kStripRows - 1) / kStripRows, tile_rows = (block_rows + tiles - 1) / tiles;
   // waves to a tile: the fewest of those whose busiest wave has the fewest runs, whatever their number (Q8_0 [5120 -> 17408]
   // has five tiles of twenty runs to a block: seven runs with three waves to a tile, nine with eight; 24.3 -> 24.0 us, Q6_K
-  // 23.5 -> 21.7)
+  // 23.5 -> 21.7); joining the shares of a round counts as a quarter of a run (Q8_0 [1792 -> 105243] x 7, thirteen tiles of seven
+  // runs to a block of eight waves: 48.4 one wave to a tile, 50.6 with eight)
   uint32_t split = 1, least = 0xFFFFFFFFu;
   for (uint32_t candidate = 1; candidate <= waves && candidate <= runs; ++candidate) {
     const uint32_t slots = waves / candidate;
-    const uint32_t cost = ((tiles + slots - 1) / slots) * ((runs + candidate - 1) / candidate);
+    const uint32_t cost = ((tiles + slots - 1) / slots) * (4 * ((runs + candidate - 1) / candidate) + (candidate > 1 ? 1 : 0));
     if (cost < least) {
       least = cost;
       split = candidate;

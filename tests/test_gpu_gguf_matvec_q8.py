@@ -417,3 +417,29 @@ def test_q8_route_q4_k_tiles_seeded_random_shapes_of_what_they_serve():
         note(f"q8 matvec q4_k tiles draw {case}: rows {rows} k {k} m {m} x {x_tag} pad {pad}")
         check("q4_k", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad)
         assert hc.last_launch_variant().startswith(f"gguf_matvec_q8_tiles/q4_k/{tokens}-tokens"), (hc.last_launch_variant(), rows, k, m)
+
+
+@pytest.mark.parametrize("x_tag", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("tag,rows,k,m,kernel", [("q4_k", 70, 4096, 1, "tiles/q4_k/1"), ("q4_k", 70, 2048, 3, "tiles/q4_k/4"), ("q4_k", 40, 1280, 6, "tiles/q4_k/8"),
+                                                ("q6_k", 70, 4096, 1, "spans/q6_k/2"), ("q6_k", 70, 2048, 2, "quads/q6_k"), ("q6_k", 40, 1280, 2, "blocks/q6_k/2"),
+                                                ("q8_0", 70, 4096, 1, "spans/q8_0/2"), ("q8_0", 70, 2304, 1, "spans/q8_0/2-spans/short"),
+                                                ("q8_0", 70, 2048, 3, "quads/q8_0"), ("q8_0", 40, 1312, 2, "blocks/q8_0/2")])
+def test_q8_route_activation_blocks_on_both_sides_of_the_short_form(tag, rows, k, m, kernel, x_tag):
+    """Blocks of zeros, of magnitudes near and past what the short form takes, and with one magnitude of both signs (the first
+    one's counts) quantise the long way: whole waves of them, and blocks that share a wave with ordinary ones.  f16 has
+    zeros, subnormals and equal magnitudes only."""
+    rng = np.random.default_rng(1827)
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    group = k // 8
+    x[0, :256] = 0.0
+    x[0, 256:288] = np.where(np.arange(32) % 2 == 0, 1.25, -1.25)
+    x[0, 512:768] = np.where(np.arange(256) % 3 == 0, -2.5, 2.5)
+    x[0, 768:800] = -3.0
+    if x_tag != "f16":
+        scale = np.float32([1, 2.0 ** -62, 2.0 ** -59, 2.0 ** -61, 2.0 ** 58, 2.0 ** 61, 2.0 ** 20, 2.0 ** -70])
+        if tag == "q8_0":
+            scale = np.minimum(scale, np.float32(2.0 ** 19))   # its scales are f16
+        x[m - 1, :8 * group] *= np.repeat(scale, group)
+    x = x if m > 1 else x[0]
+    note(f"q8 matvec {tag} x {x_tag} [{k} -> {rows}] x {m}: activation blocks that quantise the long way")
+    check(tag, x_tag, weights_for(tag, rng, rows, k), rows, k, x, kernel="gguf_matvec_q8_" + kernel)
