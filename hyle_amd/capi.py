@@ -210,6 +210,17 @@ def launcher():
     return functools.partial(_submit.launch, C.cast(load().hyle_hip_plan_launch, C.c_void_p).value)
 
 
+@functools.lru_cache(maxsize=None)
+def tensor_launcher(current_device, current_stream):
+    """launch(plan, input tensors, output tensors, workspace, workspace size) -> status code, on the stream that
+    current_stream(current_device()) names; None where the extension was not built."""
+    launch = launcher()
+    if launch is launch_through_ctypes:
+        return None
+    from . import _submit
+    return functools.partial(_submit.launch_tensors, launch.args[0], current_device, current_stream)
+
+
 def last_error() -> str:
     return load().hyle_hip_last_error().decode()
 

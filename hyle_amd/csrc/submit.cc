@@ -68,7 +68,65 @@ PyObject *launch(PyObject *, PyObject *const *args, Py_ssize_t count) {
   return PyLong_FromLong(static_cast<long>(status));
 }
 
-PyMethodDef methods[] = {{"launch", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(launch)), METH_FASTCALL, nullptr},
+PyObject *data_ptr_name = nullptr;  // "data_ptr"
+
+// The addresses of a list or tuple of tensors: what their data_ptr() answers.
+bool storage_of(PyObject *tensors, void **out, Py_ssize_t most, uint32_t *count) {
+  const Py_ssize_t size = PySequence_Fast_GET_SIZE(tensors);
+  if (size > most) {
+    PyErr_SetString(PyExc_IndexError, "more bindings than an operation can have");
+    return false;
+  }
+  for (Py_ssize_t i = 0; i < size; ++i) {
+    // (data_ptr() of a tensor subclass is Python: it may change the list)
+    if (i >= PySequence_Fast_GET_SIZE(tensors)) {
+      PyErr_SetString(PyExc_RuntimeError, "bindings changed while they were read");
+      return false;
+    }
+    PyObject *tensor = PySequence_Fast_GET_ITEM(tensors, i);
+    Py_INCREF(tensor);
+    PyObject *address = PyObject_CallMethodNoArgs(tensor, data_ptr_name);
+    Py_DECREF(tensor);
+    if (address == nullptr) return false;
+    const bool fine = address_of(address, &out[i]);
+    Py_DECREF(address);
+    if (!fine) return false;
+  }
+  *count = static_cast<uint32_t>(size);
+  return true;
+}
+
+// launch_tensors(function, current device, current stream of a device, plan, inputs, outputs, workspace, workspace size)
+// -> status code: launch with lists or tuples of tensors, on the current device's current stream.
+PyObject *launch_tensors(PyObject *, PyObject *const *args, Py_ssize_t count) {
+  if (count != 8 || !(PyList_Check(args[4]) || PyTuple_Check(args[4])) || !(PyList_Check(args[5]) || PyTuple_Check(args[5]))) {
+    PyErr_SetString(PyExc_TypeError, "launch_tensors takes eight arguments, bindings as lists or tuples");
+    return nullptr;
+  }
+  void *function, *plan, *workspace, *stream, *inputs[kMostInputs], *outputs[kMostOutputs];
+  uint32_t input_count, output_count;
+  PyObject *device = PyObject_CallNoArgs(args[1]);
+  if (device == nullptr) return nullptr;
+  PyObject *handle = PyObject_CallOneArg(args[2], device);
+  Py_DECREF(device);
+  if (handle == nullptr) return nullptr;
+  const bool found = address_of(handle, &stream);
+  Py_DECREF(handle);
+  if (!found || !address_of(args[0], &function) || !address_of(args[3], &plan) || !storage_of(args[4], inputs, kMostInputs, &input_count) ||
+      !storage_of(args[5], outputs, kMostOutputs, &output_count) || !address_of(args[6], &workspace))
+    return nullptr;
+  const size_t size = PyLong_AsSize_t(args[7]);
+  if (size == static_cast<size_t>(-1) && PyErr_Occurred()) return nullptr;
+  hyle_hip_status status;
+  Py_BEGIN_ALLOW_THREADS
+  status = reinterpret_cast<decltype(&hyle_hip_plan_launch)>(function)(static_cast<const hyle_hip_plan *>(plan), inputs, input_count, outputs,
+                                                                       output_count, workspace, size, stream);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong(static_cast<long>(status));
+}
+
+PyMethodDef methods[] = {{"launch_tensors", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(launch_tensors)), METH_FASTCALL, nullptr},
+                         {"launch", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(launch)), METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_submit", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
@@ -79,5 +137,6 @@ PyMODINIT_FUNC PyInit__submit() {
   if (ctypes == nullptr) return nullptr;
   pointer_type = PyObject_GetAttrString(ctypes, "c_void_p");
   Py_DECREF(ctypes);
-  return pointer_type == nullptr ? nullptr : PyModule_Create(&module);
+  data_ptr_name = PyUnicode_InternFromString("data_ptr");
+  return pointer_type == nullptr || data_ptr_name == nullptr ? nullptr : PyModule_Create(&module);
 }

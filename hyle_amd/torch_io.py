@@ -51,6 +51,9 @@ def current_stream_handle(device=None) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_BINDINGS = (list, tuple)
+
+
 class Bound:
     """A prepared operation with its workspace, ready to be submitted repeatedly."""
 
@@ -63,11 +66,22 @@ class Bound:
         ptr = self.workspace.data_ptr() if self.workspace is not None else 0
         self.invocation = self.prepared.create_invocation(ptr, req.size)
         self.device = device
+        self._launch = None
 
     def outputs(self) -> list:
         return [empty_like_desc(d, self.device) for d in self.prepared.output_descriptions()]
 
     def submit(self, inputs: Sequence[torch.Tensor], outputs: Sequence[torch.Tensor], stream: Optional[int] = None):
+        launch = self._launch
+        if launch is not None and stream is None and type(inputs) in _BINDINGS and type(outputs) in _BINDINGS:
+            # the stream and the addresses are asked for natively: 0.3 us of the 3.7 of a small submit
+            invocation = self.invocation
+            code = launch(invocation._prepared._handle, inputs, outputs, invocation._workspace, invocation._workspace_size)
+            if code != hc.capi.OK:
+                hc._check(code)
+            return
+        if launch is None and _raw_stream is not None and torch.cuda.is_initialized():
+            self._launch = hc.capi.tensor_launcher(_current_device, _raw_stream)
         handle = current_stream_handle() if stream is None else stream
         self.invocation.submit(handle, [t.data_ptr() for t in inputs], [t.data_ptr() for t in outputs])
 

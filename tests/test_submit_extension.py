@@ -44,3 +44,43 @@ def test_what_cannot_be_an_address_is_refused():
     with pytest.raises(TypeError):
         extension.launch(NOTING, 1)
     assert SEEN == []
+
+
+class Tensor:
+    """What launch_tensors asks a tensor for."""
+
+    def __init__(self, address, also=None):
+        self.address, self.also = address, also
+
+    def data_ptr(self):
+        if self.also is not None:
+            self.also()
+        return self.address
+
+
+def test_tensors_arrive_with_the_current_stream_and_what_fails_is_not_launched():
+    asked = []
+
+    def stream_of(device):
+        asked.append(device)
+        return 0x55
+
+    for inputs, outputs in (([], ()), ([Tensor(1), Tensor(0)], (Tensor((1 << 64) - 256),)), ((Tensor(3),) * 4, [Tensor(5), Tensor(6)])):
+        SEEN.clear()
+        assert extension.launch_tensors(NOTING, lambda: 3, stream_of, 0x1234, inputs, outputs, 0x100, 512) == 7
+        assert SEEN == [(0x1234, [t.address or None for t in inputs], [t.address for t in outputs], 0x100, 512, 0x55)]
+    assert asked == [3, 3, 3]
+    SEEN.clear()
+    shrinking = [Tensor(1), Tensor(2)]
+    shrinking[0].also = shrinking.clear
+
+    def no_device():
+        raise RuntimeError("no device")
+
+    for device, inputs, outputs, size, error in ((lambda: 3, [1], [], 0, AttributeError), (lambda: 3, [Tensor("1")], [], 0, TypeError),
+                                                 (lambda: 3, [], iter([]), 0, TypeError), (lambda: 3, [Tensor(1)] * (capi.MAX_INPUTS + 1), [], 0, IndexError),
+                                                 (lambda: 3, [], [Tensor(1)] * (capi.MAX_OUTPUTS + 1), 0, IndexError), (lambda: 3, shrinking, [], 0, RuntimeError),
+                                                 (no_device, [], [], 0, RuntimeError), (lambda: 3, [], [], "8", TypeError)):
+        with pytest.raises(error):
+            extension.launch_tensors(NOTING, device, stream_of, 1, inputs, outputs, 0, size)
+    assert SEEN == []
