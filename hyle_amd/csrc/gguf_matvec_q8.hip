@@ -661,7 +661,7 @@ struct TileFactors {
 // (rows past m repeat the last one and are not stored).  1 << split_log2 waves share a tile of
 // sixteen weight rows: wave w of them walks the groups w, w + split, ... and the first adds the
 // shares in wave order.
-template <class TX, int kSets, bool kOneBatch>
+template <class TX, int kSets, bool kOneBatch, uint32_t kRows>
 __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_tiles(const unsigned char *weights, const void *x, void *y,
                                                                       uint32_t rows, uint64_t row_stride, uint32_t blocks,
                                                                       uint32_t m, uint32_t split_log2) {
@@ -677,7 +677,8 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_tiles(const unsi
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveLanes);
   const uint32_t column = lane % 16, part = lane / 16;
   const uint32_t split = 1u << split_log2, member = wave & (split - 1);
-  const uint32_t row = ((blockIdx.x * kWavesPerBlock + wave) >> split_log2) * kTileRows + column;
+  // (kRows == 8: the other eight columns are the same rows again)
+  const uint32_t row = ((blockIdx.x * kWavesPerBlock + wave) >> split_log2) * kRows + column % kRows;
   // rows past the last repeat it (valid addresses) and are not stored
   const unsigned char *mine = weights + (size_t)(row < rows ? row : rows - 1) * row_stride;
   const uint32_t groups = (blocks + 3) / 4;
@@ -867,7 +868,7 @@ __global__ __launch_bounds__(kBlockThreads) void gguf_matvec_q8_tiles(const unsi
     for (int t = 0; t < kTotals; ++t)
       for (uint32_t other = 1; other < split; ++other) totals[t] += shares[((size_t)(wave + other) * kWaveLanes + lane) * kTotals + t];
   }
-  if (row < rows) {
+  if (row < rows && column < kRows) {
     if constexpr (kSets == 0) {
       if (part == 0) Traits<TX>::store(y, (size_t)row, totals[0]);
     } else {
@@ -896,9 +897,9 @@ template <int kKind, int kSpans, bool kShort, bool kStream> struct SpansTag {
            (kStream ? "#stream" : "");
   }
 };
-template <int kSets, bool kOneBatch> struct TilesTag {
+template <int kSets, bool kOneBatch, uint32_t kRows> struct TilesTag {
   static std::string text() {
-    return "gguf_matvec_q8_tiles/q4_k/" + std::to_string(kSets == 0 ? 1 : 4 * kSets) + "-tokens" + (kOneBatch ? "" : "/long");
+    return "gguf_matvec_q8_tiles/q4_k/" + std::to_string(kSets == 0 ? 1 : 4 * kSets) + "-tokens" + (kOneBatch ? "" : "/long") + (kRows == 8 ? "#8-rows" : "");
   }
 };
 template <int kKind, int kM> struct BlocksTag {
@@ -1400,26 +1401,38 @@ inline bool tiles_serve(const MatVecParams &p) {
 template <class TX, int kSets>
 hipError_t run_tiles_m(const MatVecParams &p, const void *w, const void *x, void *y, int compute_units, hipStream_t s) {
   const uint32_t blocks = p.k / 256, groups = (blocks + 3) / 4;
-  const uint32_t tiles = (uint32_t)((p.rows + kTileRows - 1) / kTileRows);
+  uint32_t tiles = (uint32_t)((p.rows + kTileRows - 1) / kTileRows);
   // few rows: up to four waves share a tile, each walking every second or fourth group of four blocks,
   // until there are eight waves per compute unit
   const uint64_t wanted = 8ull * (uint64_t)(compute_units > 0 ? compute_units : 256);
   uint32_t split_log2 = 0;
   while (split_log2 < 2 && (2u << split_log2) <= groups && ((uint64_t)tiles << split_log2) < wanted) ++split_log2;
+  // one activation row: tiles of eight rows where blocks with one of sixteen leave half the compute units without a block and
+  // waves have several groups to walk (us, sixteen / eight: [6144 -> 2048] 6.15 / 5.65, [8192 -> 2048] 6.4 / 5.8, [6144 -> 1024]
+  // 5.45 / 5.2, but [5120 -> 500], five groups, 5.0 / 5.1)
+  const bool half = kSets == 0 && split_log2 == 2 && groups >= 6 && 2 * (uint64_t)tiles <= wanted / 8;
+  if (half) tiles = (uint32_t)((p.rows + kTileRows / 2 - 1) / (kTileRows / 2));
   const uint32_t waves = tiles << split_log2;
   const size_t shared = tile_shared_bytes(kSets == 0 ? 1 : 4 * kSets, blocks);
   const dim3 grid((waves + kWavesPerBlock - 1) / kWavesPerBlock);
   const unsigned char *in = static_cast<const unsigned char *>(w);
-  // at most 32 activation blocks in all (64 with eight rows): one round of the block's half waves, no loop around it
-  if ((kSets == 0 ? 1u : 4u * kSets) * blocks <= (kSets == 2 ? 64u : 32u)) {
-    note_variant<TilesTag<kSets, true>>();
-    hipLaunchKernelGGL((gguf_matvec_q8_tiles<TX, kSets, true>), grid, dim3(kBlockThreads), shared, s, in, x, y, (uint32_t)p.rows,
+  // at most 32 activation blocks in all (64 with eight rows): one round of the block's groups of lanes, no loop around it
+  const bool one_batch = (kSets == 0 ? 1u : 4u * kSets) * blocks <= (kSets == 2 ? 64u : 32u);
+  auto go = [&](auto batch, auto tile) {
+    constexpr bool kOneBatch = decltype(batch)::value;
+    constexpr uint32_t kRows = decltype(tile)::value;
+    note_variant<TilesTag<kSets, kOneBatch, kRows>>();
+    hipLaunchKernelGGL((gguf_matvec_q8_tiles<TX, kSets, kOneBatch, kRows>), grid, dim3(kBlockThreads), shared, s, in, x, y, (uint32_t)p.rows,
                        p.row_stride, blocks, p.m, split_log2);
-  } else {
-    note_variant<TilesTag<kSets, false>>();
-    hipLaunchKernelGGL((gguf_matvec_q8_tiles<TX, kSets, false>), grid, dim3(kBlockThreads), shared, s, in, x, y, (uint32_t)p.rows,
-                       p.row_stride, blocks, p.m, split_log2);
+  };
+  using Whole = std::integral_constant<uint32_t, kTileRows>;
+  if constexpr (kSets == 0) {
+    using Half = std::integral_constant<uint32_t, kTileRows / 2>;
+    if (half && one_batch) go(std::true_type{}, Half{});
+    else if (half) go(std::false_type{}, Half{});
   }
+  if (!half && one_batch) go(std::true_type{}, Whole{});
+  else if (!half) go(std::false_type{}, Whole{});
   return hipGetLastError();
 }
 template <class TX>

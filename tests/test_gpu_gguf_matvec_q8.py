@@ -443,3 +443,14 @@ def test_q8_route_activation_blocks_on_both_sides_of_the_short_form(tag, rows, k
     x = x if m > 1 else x[0]
     note(f"q8 matvec {tag} x {x_tag} [{k} -> {rows}] x {m}: activation blocks that quantise the long way")
     check(tag, x_tag, weights_for(tag, rng, rows, k), rows, k, x, kernel="gguf_matvec_q8_" + kernel)
+
+
+@pytest.mark.parametrize("x_tag", ["f32", "bf16"])
+def test_q8_route_q4_k_tiles_of_eight_rows(x_tag):
+    """Few rows of six groups of four blocks or more: a tile has eight rows, on both sides of its edges and of the rule."""
+    rng = np.random.default_rng(1828)
+    for rows, k, form in ((1, 6144, "#8-rows"), (7, 6144, "#8-rows"), (8, 5376, "#8-rows"), (9, 8192, "#8-rows"), (17, 9984, "/long#8-rows"), (511, 8448, "/long#8-rows"),
+                          (2048, 6144, "#8-rows"), (2049, 6144, ""), (2048, 4096, ""), (33, 5120, ""), (8450, 8448, "/long")):
+        note(f"q8 matvec q4_k tiles x {x_tag} rows {rows} k {k}: 1-tokens{form}")
+        check("q4_k", x_tag, raw_bytes_for("q4_k", rng, rows, k), rows, k, rng.normal(0, 1.5, k).astype(np.float32), kernel="gguf_matvec_q8_tiles/q4_k/1-tokens")
+        assert last_launch_form() == f"gguf_matvec_q8_tiles/q4_k/1-tokens{form}"
