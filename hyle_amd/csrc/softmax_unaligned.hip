@@ -54,9 +54,11 @@ template <class T, bool kLog> __device__ __forceinline__ float row_exp(float t) 
   }
 }
 
-template <class T, int kLanes, int kVpl, int kThreads, int kMask, bool kLog>
+// kShared: rows `inner` apart have the same mask row (the heads of a layer), and a lane takes up to `each` of them one after
+// another: the mask is loaded once, and a row's loads are under way while the row before is worked on.
+template <class T, int kLanes, int kVpl, int kThreads, int kMask, bool kLog, bool kShared>
 __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x, const char *mask, char *y, uint32_t rows,
-                                                                  uint32_t width, float scale, MaskRows mrows) {
+                                                                  uint32_t width, float scale, MaskRows mrows, uint32_t inner, uint32_t each) {
   constexpr uint32_t kVec = Traits<T>::kVec, kSize = Traits<T>::kSize;
   constexpr int kWords = kVec / 4;
   constexpr int kGroupsPerBlock = kThreads / kLanes;
@@ -66,11 +68,17 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x
   uint32_t group = threadIdx.x / kLanes;
   if constexpr (kLanes >= kWaveLanes) group = __builtin_amdgcn_readfirstlane(group);  // the row's address stays scalar
   const uint32_t wanted_row = blockIdx.x * kGroupsPerBlock + group;
-  const bool row_ok = wanted_row < rows;
-  const uint32_t row = row_ok ? wanted_row : rows - 1;
+  const uint32_t places = kShared ? inner : rows;
+  const bool row_ok = wanted_row < places;
+  uint32_t row = row_ok ? wanted_row : places - 1, left = 1;
+  if constexpr (kShared) {
+    row += blockIdx.y * each * inner;
+    left = min(each, rows / inner - blockIdx.y * each);
+  }
   const char *mask_row = nullptr;
   if constexpr (kMask != kMaskNone) mask_row = mask + mask_row_offset(mrows, row);
   const char *row_x = x + (size_t)row * width * kSize;
+  char *row_y = y + (size_t)row * width * kSize;
 
   // Vector `lane + k * kLanes` of the row, moved back to end at the row's end where it would pass
   // it: `skip` of its elements belong to the vector before it (all of them: nothing is left).
@@ -89,126 +97,159 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x
       for (int q = 0; q < kWords; ++q) bits[k][q] = reinterpret_cast<const word_any *>(mask_row + start[k])[q];
   }
   u32x4 raw[kVpl], added[kVpl];
+  uint32_t from[kVpl];
 #pragma unroll
   for (int k = 0; k < kVpl; ++k) {
-    uint32_t from = start[k];
+    from[k] = start[k];
     if constexpr (kMask == kMaskBoolean) {
       uint32_t any = 0;
 #pragma unroll
       for (int q = 0; q < kWords; ++q) any |= bits[k][q];
-      from = any != 0 ? from : 0u;  // nothing kept: no new line is asked for
+      from[k] = any != 0 ? from[k] : 0u;  // nothing kept: no new line is asked for
     }
-    raw[k] = *reinterpret_cast<const words4_any *>(row_x + (size_t)from * kSize);
+    raw[k] = *reinterpret_cast<const words4_any *>(row_x + (size_t)from[k] * kSize);
     if constexpr (kMask == kMaskAdditive) added[k] = *reinterpret_cast<const words4_any *>(mask_row + (size_t)start[k] * kSize);
   }
 #pragma unroll
   for (int k = 0; k < kVpl; ++k) loads_issued(raw[k]);
 
-  float v[kVpl][kVec];
-  float peak = -INFINITY;
+  while (true) {
+    float v[kVpl][kVec];
 #pragma unroll
-  for (int k = 0; k < kVpl; ++k) {
-    Traits<T>::unpack(raw[k], v[k]);
-    if constexpr (kMask == kMaskAdditive) {
-      float addend[kVec];
-      Traits<T>::unpack(added[k], addend);
+    for (int k = 0; k < kVpl; ++k) Traits<T>::unpack(raw[k], v[k]);
+    if constexpr (kShared) {
+      row_x += (size_t)inner * width * kSize;
+      if (left > 1) {
 #pragma unroll
-      for (int j = 0; j < (int)kVec; ++j) v[k][j] = v[k][j] * scale + addend[j];
-    } else if constexpr (kMask == kMaskBoolean) {
-#pragma unroll
-      for (int j = 0; j < (int)kVec; ++j) {
-        const bool keep = ((bits[k][j / 4] >> (8 * (j % 4))) & 0xFFu) != 0;
-        v[k][j] = keep ? v[k][j] * scale : -INFINITY;
+        for (int k = 0; k < kVpl; ++k) raw[k] = *reinterpret_cast<const words4_any *>(row_x + (size_t)from[k] * kSize);
+        asm volatile("" ::: "memory");
       }
-    } else {
-#pragma unroll
-      for (int j = 0; j < (int)kVec; ++j) v[k][j] *= scale;
     }
+    float peak = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < (int)kVec; j += 2) {
-      peak = __builtin_elementwise_maximum(__builtin_elementwise_maximum(v[k][j], v[k][j + 1]), peak);  // a NaN stays
-    }
-  }
-  // an infinite maximum of either sign marks the row: +inf poisoned, -inf nothing finite
-  peak = row_max<kLanes>(peak != peak ? INFINITY : peak, joint_max);
-  const bool invalid = __builtin_fabsf(peak) == INFINITY;
-  float total = 0.0f, maxima = 0.0f;
+    for (int k = 0; k < kVpl; ++k) {
+      if constexpr (kMask == kMaskAdditive) {
+        float addend[kVec];
+        Traits<T>::unpack(added[k], addend);
 #pragma unroll
-  for (int k = 0; k < kVpl; ++k) {
-    float sum = 0.0f, count = 0.0f;
+        for (int j = 0; j < (int)kVec; ++j) v[k][j] = v[k][j] * scale + addend[j];
+      } else if constexpr (kMask == kMaskBoolean) {
 #pragma unroll
-    for (int j = 0; j < (int)kVec; ++j) {
-      const float shifted = v[k][j] - peak;
-      if constexpr (kLog) {  // the maxima are counted, not summed (src/compute_provider_cuda/reduction_kernel.cu:178-196)
-        const bool at_peak = shifted == 0.0f;
-        sum += at_peak ? 0.0f : row_exp<T, kLog>(shifted);
-        count += at_peak ? 1.0f : 0.0f;
-        v[k][j] = shifted;
+        for (int j = 0; j < (int)kVec; ++j) {
+          const bool keep = ((bits[k][j / 4] >> (8 * (j % 4))) & 0xFFu) != 0;
+          v[k][j] = keep ? v[k][j] * scale : -INFINITY;
+        }
       } else {
-        v[k][j] = row_exp<T, kLog>(shifted);
-        sum += v[k][j];
+#pragma unroll
+        for (int j = 0; j < (int)kVec; ++j) v[k][j] *= scale;
+      }
+#pragma unroll
+      for (int j = 0; j < (int)kVec; j += 2) {
+        peak = __builtin_elementwise_maximum(__builtin_elementwise_maximum(v[k][j], v[k][j + 1]), peak);  // a NaN stays
       }
     }
-    if (skip[k] != 0) {  // the row's last vectors: elements of two vectors count once
-      sum = 0.0f;
-      count = 0.0f;
+    // an infinite maximum of either sign marks the row: +inf poisoned, -inf nothing finite
+    peak = row_max<kLanes>(peak != peak ? INFINITY : peak, joint_max);
+    const bool invalid = __builtin_fabsf(peak) == INFINITY;
+    float total = 0.0f, maxima = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kVpl; ++k) {
+      float sum = 0.0f, count = 0.0f;
 #pragma unroll
       for (int j = 0; j < (int)kVec; ++j) {
-        const bool mine = (uint32_t)j >= skip[k];
-        if constexpr (kLog) {
-          sum += mine && v[k][j] != 0.0f ? row_exp<T, kLog>(v[k][j]) : 0.0f;
-          count += mine && v[k][j] == 0.0f ? 1.0f : 0.0f;
+        const float shifted = v[k][j] - peak;
+        if constexpr (kLog) {  // the maxima are counted, not summed (src/compute_provider_cuda/reduction_kernel.cu:178-196)
+          const bool at_peak = shifted == 0.0f;
+          sum += at_peak ? 0.0f : row_exp<T, kLog>(shifted);
+          count += at_peak ? 1.0f : 0.0f;
+          v[k][j] = shifted;
         } else {
-          sum += mine ? v[k][j] : 0.0f;
+          v[k][j] = row_exp<T, kLog>(shifted);
+          sum += v[k][j];
         }
       }
-    }
-    total += sum;
-    maxima += count;
-  }
-  total = row_sum<kLanes>(total, joint_sum);  // = 2^32 * sum(exp)
-  // joint_max is free again: every wave read it before the barrier of the sum above
-  if constexpr (kLog) maxima = row_sum<kLanes>(maxima, joint_max);
-  float normaliser = kLog ? log1pf((maxima - 1.0f) + total * 2.3283064365386963e-10f) : 1.0f / total;
-  if (invalid) normaliser = __builtin_nanf("");
-  char *row_y = y + (size_t)row * width * kSize;
+      if (skip[k] != 0) {  // the row's last vectors: elements of two vectors count once
+        sum = 0.0f;
+        count = 0.0f;
 #pragma unroll
-  for (int k = 0; k < kVpl; ++k) {
-    if (row_ok && skip[k] < kVec) {
-      float out[kVec];
-#pragma unroll
-      for (int j = 0; j < (int)kVec; ++j) out[j] = kLog ? v[k][j] - normaliser : v[k][j] * normaliser;
-      const u32x4 packed = Traits<T>::pack(out);
-      __builtin_nontemporal_store(packed, reinterpret_cast<words4_any *>(row_y + (size_t)start[k] * kSize));
+        for (int j = 0; j < (int)kVec; ++j) {
+          const bool mine = (uint32_t)j >= skip[k];
+          if constexpr (kLog) {
+            sum += mine && v[k][j] != 0.0f ? row_exp<T, kLog>(v[k][j]) : 0.0f;
+            count += mine && v[k][j] == 0.0f ? 1.0f : 0.0f;
+          } else {
+            sum += mine ? v[k][j] : 0.0f;
+          }
+        }
+      }
+      total += sum;
+      maxima += count;
     }
+    total = row_sum<kLanes>(total, joint_sum);  // = 2^32 * sum(exp)
+    // joint_max is free again: every wave read it before the barrier of the sum above
+    if constexpr (kLog) maxima = row_sum<kLanes>(maxima, joint_max);
+    float normaliser = kLog ? log1pf((maxima - 1.0f) + total * 2.3283064365386963e-10f) : 1.0f / total;
+    if (invalid) normaliser = __builtin_nanf("");
+#pragma unroll
+    for (int k = 0; k < kVpl; ++k) {
+      if (row_ok && skip[k] < kVec) {
+        float out[kVec];
+#pragma unroll
+        for (int j = 0; j < (int)kVec; ++j) out[j] = kLog ? v[k][j] - normaliser : v[k][j] * normaliser;
+        const u32x4 packed = Traits<T>::pack(out);
+        __builtin_nontemporal_store(packed, reinterpret_cast<words4_any *>(row_y + (size_t)start[k] * kSize));
+      }
+    }
+    if constexpr (!kShared) break;
+    if (--left == 0) break;  // the same for the whole block
+    row_y += (size_t)inner * width * kSize;
+    if constexpr (kLanes > kWaveLanes) __syncthreads();  // the joint words are free again
   }
 }
 
-// softmax_unaligned/<lanes>x<vectors per lane>/<threads per block>/<mask>
-template <int kLanes, int kVpl, int kThreads, int kMask> struct UnalignedTag {
+// softmax_unaligned/<lanes>x<vectors per lane>/<threads per block>/<mask>[#shared: several rows to a mask row]
+template <int kLanes, int kVpl, int kThreads, int kMask, bool kShared> struct UnalignedTag {
   static std::string text() {
-    return "softmax_unaligned/" + std::to_string(kLanes) + "x" + std::to_string(kVpl) + "/" + std::to_string(kThreads) + "/" + mask_word(kMask);
+    return "softmax_unaligned/" + std::to_string(kLanes) + "x" + std::to_string(kVpl) + "/" + std::to_string(kThreads) + "/" + mask_word(kMask) +
+           (kShared ? "#shared" : "");
   }
 };
 
-template <class T, int kLanes, int kVpl, int kThreads, int kMask>
-void run_mask(const SoftmaxParams &p, const MaskRows &m, const void *x, const void *mask, void *y, hipStream_t s) {
-  constexpr uint32_t kGroupsPerBlock = kThreads / kLanes;
-  const uint32_t rows = (uint32_t)p.shape.rows;
-  const dim3 grid((rows + kGroupsPerBlock - 1) / kGroupsPerBlock);
-  const char *in = static_cast<const char *>(x), *in_mask = static_cast<const char *>(mask);
-  char *out = static_cast<char *>(y);
-  note_variant<UnalignedTag<kLanes, kVpl, kThreads, kMask>>();
-  if (p.log)
-    hipLaunchKernelGGL((softmax_rows_unaligned<T, kLanes, kVpl, kThreads, kMask, true>), grid, dim3(kThreads), 0, s, in, in_mask, out, rows,
-                       p.shape.width, p.scale, m);
-  else
-    hipLaunchKernelGGL((softmax_rows_unaligned<T, kLanes, kVpl, kThreads, kMask, false>), grid, dim3(kThreads), 0, s, in, in_mask, out, rows,
-                       p.shape.width, p.scale, m);
+// Three rows to a mask row in large launches of masked rows of several waves: the mask is asked for once instead of three times,
+// and a row's loads are under way during the exponentials of the row before.  us, one row / three: additive bf16
+// [19, 1932, 6908] 216 / 181, [16, 1500, 5001] 126 / 110, [46, 1495, 2094] 118 / 109, f16 [9, 3800, 4081] 116 / 107, f32
+// [16, 1500, 2501] 102 / 87; Boolean bf16 [19, 1932, 6908] 183 / 169, [24, 2200, 3100] 119 / 111.  Not below 100 MB, where it
+// leaves too few waves (bf16 [16, 800, 2201] 28.2 / 30.6, [64, 260, 2500] 32.9 / 35.6), nor with a mask that every
+// L2 holds beside the rows ([64, 300, 2700] 40.1 / 40.8); rows of one wave gain nothing
+// (bf16 [30, 2000, 1700] 77 / 82 with five vectors a lane, [24, 777, 1013] 18.4 / 19.5), nor do rows without a mask ([24, 777, 2094] 30.9 / 32.6).
+constexpr uint32_t kSharedRows = 3;
+constexpr uint64_t kSharedBytes = 100000000, kSharedMask = 2000000;
+// Rows between two that have the same mask row (0: none that a launch could share).
+inline uint32_t shared_inner(const SoftmaxParams &p, uint32_t size) {
+  if ((int)p.mask_kind == kMaskNone || (uint64_t)p.shape.rows * p.shape.width * size < kSharedBytes) return 0;
+  uint64_t outer = 1;
+  for (int i = 0; i < p.outer_rank && (p.mask_outer_strides[i] == 0 || p.outer_dims[i] == 1); ++i) outer *= p.outer_dims[i];
+  const uint64_t inner = p.shape.rows / outer, mask_bytes = inner * p.shape.width * ((int)p.mask_kind == kMaskBoolean ? 1 : size);
+  return outer >= kSharedRows && mask_bytes >= kSharedMask && (outer + kSharedRows - 1) / kSharedRows <= 65535u ? (uint32_t)inner : 0u;
 }
 
-template <class T, int kLanes, int kVpl, int kThreads>
-void run_shape(const SoftmaxParams &p, const void *x, const void *mask, void *y, hipStream_t s) {
+template <class T, int kLanes, int kVpl, int kThreads, int kMask, bool kShared = false>
+void run_mask(const SoftmaxParams &p, const MaskRows &m, const void *x, const void *mask, void *y, hipStream_t s) {
+  constexpr uint32_t kGroupsPerBlock = kThreads / kLanes;
+  const uint32_t rows = (uint32_t)p.shape.rows, inner = kShared ? shared_inner(p, Traits<T>::kSize) : rows, outer = rows / inner;
+  const dim3 grid((inner + kGroupsPerBlock - 1) / kGroupsPerBlock, kShared ? (outer + kSharedRows - 1) / kSharedRows : 1);
+  const char *in = static_cast<const char *>(x), *in_mask = static_cast<const char *>(mask);
+  char *out = static_cast<char *>(y);
+  note_variant<UnalignedTag<kLanes, kVpl, kThreads, kMask, kShared>>();
+  if (p.log)
+    hipLaunchKernelGGL((softmax_rows_unaligned<T, kLanes, kVpl, kThreads, kMask, true, kShared>), grid, dim3(kThreads), 0, s, in, in_mask, out, rows,
+                       p.shape.width, p.scale, m, inner, kSharedRows);
+  else
+    hipLaunchKernelGGL((softmax_rows_unaligned<T, kLanes, kVpl, kThreads, kMask, false, kShared>), grid, dim3(kThreads), 0, s, in, in_mask, out, rows,
+                       p.shape.width, p.scale, m, inner, kSharedRows);
+}
+
+inline MaskRows mask_rows(const SoftmaxParams &p) {
   MaskRows m{};
   m.outer_rank = p.outer_rank;
   for (int i = 0; i < kMaxRank; ++i) {
@@ -216,6 +257,18 @@ void run_shape(const SoftmaxParams &p, const void *x, const void *mask, void *y,
     m.outer_strides[i] = p.mask_outer_strides[i];
   }
   m.inner_stride = p.mask_inner_stride;
+  return m;
+}
+
+template <class T, int kLanes, int kVpl, int kThreads>
+void run_shape(const SoftmaxParams &p, const void *x, const void *mask, void *y, hipStream_t s) {
+  const MaskRows m = mask_rows(p);
+  if constexpr (kLanes == 128 || kLanes == 256) {
+    if (shared_inner(p, Traits<T>::kSize) != 0) {
+      if ((int)p.mask_kind == kMaskBoolean) return run_mask<T, kLanes, kVpl, kThreads, kMaskBoolean, true>(p, m, x, mask, y, s);
+      return run_mask<T, kLanes, kVpl, kThreads, kMaskAdditive, true>(p, m, x, mask, y, s);
+    }
+  }
   switch ((int)p.mask_kind) {
     case kMaskBoolean: return run_mask<T, kLanes, kVpl, kThreads, kMaskBoolean>(p, m, x, mask, y, s);
     case kMaskAdditive: return run_mask<T, kLanes, kVpl, kThreads, kMaskAdditive>(p, m, x, mask, y, s);

@@ -9,7 +9,7 @@ import torch
 
 from hyle_amd import compute as hc
 
-from gpu_support import DEVICE, TYPES, note, run
+from gpu_support import DEVICE, TYPES, last_launch_form, note, run
 from test_gpu_softmax_variants import MASKS, compare_on_device, make_inputs, oracle_softmax
 
 pytestmark = pytest.mark.gpu
@@ -92,3 +92,20 @@ def test_narrow_rows_are_no_further_from_64_bits_than_the_strided_kernel(tag, lo
         assert hc.last_launch_variant().startswith(label)
         wrong.append(int((out.view(torch.int16) != exact.view(torch.int16)).sum()))
     assert wrong[0] <= wrong[1] + 3.0 * (rows * width * 2.0 ** -15) ** 0.5, wrong
+
+
+@pytest.mark.parametrize("tag,heads,q,width,mask_word,shape", [
+    ("bf16", 7, 3487, 2049, "additive", "128x3/256"), ("f16", 4, 4071, 3071, "boolean", "128x3/256"), ("f32", 5, 4864, 1031, "boolean", "128x3/256"),
+    ("bf16", 8, 2036, 3073, "boolean", "128x4/256"), ("f16", 4, 3058, 4089, "additive", "128x4/256"), ("f32", 3, 4200, 2047, "additive", "128x4/256"),
+    ("f16", 3, 4070, 4097, "additive", "256x3/256"), ("bf16", 5, 2001, 5001, "boolean", "256x3/256"), ("f32", 4, 2048, 3067, "additive", "256x3/256"),
+    ("f16", 3, 2720, 6145, "boolean", "256x4/256"), ("bf16", 7, 900, 8191, "additive", "256x4/256"), ("f32", 3, 2200, 4091, "boolean", "256x4/256")])
+def test_heads_that_share_a_mask_row(tag, heads, q, width, mask_word, shape):
+    """Three heads to a block's mask row, one, two or three in the last, at both ends of each width: odd and even numbers of rows,
+    in place, and LogSoftmax; a tensor below the least size, and two heads, go the other way."""
+    log_form = heads % 2 == 0
+    check(tag, q, width, mask_word, shape, log_form, False, in_place=not log_form, heads=heads)
+    assert last_launch_form() == f"softmax_unaligned/{shape}/{mask_word}#shared"
+    if (heads, width) == (4, 4089):
+        for other_heads, rows in ((4, q - 2), (2, 2 * q)):
+            check(tag, rows, width, mask_word, shape, False, False, in_place=False, heads=other_heads)
+            assert not last_launch_form().endswith("#shared")
