@@ -178,6 +178,60 @@ constexpr int kDppSwap2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141;  // lane i <-> 7 - i within 8
 constexpr int kDppRowMirror = 0x140;   // lane i <-> 15 - i within 16
 
+// The value of the lane kStep places below, as __shfl_up has it but without a trip through LDS (about a hundred
+// cycles each, in a row in a scan): neighbours by the wavefront shift, rows of sixteen and halves by the lane
+// swaps.  Lanes below kStep come back with some lane's value.
+template <int kStep> __device__ __forceinline__ uint32_t lane_up(uint32_t v) {
+  static_assert(kStep == 1 || kStep == 2 || kStep == 4 || kStep == 8 || kStep == 16 || kStep == 32, "a step of a scan");
+  if constexpr (kStep == 32) {
+    return __builtin_amdgcn_permlane32_swap(v, v, false, false)[0];  // the lower half in both
+  } else if constexpr (kStep == 16) {
+    const auto rows = __builtin_amdgcn_permlane16_swap(v, v, false, false);  // rows 0 0 2 2 and 1 1 3 3
+    const auto first = __builtin_amdgcn_permlane32_swap(rows[1], rows[1], false, false);
+    return (threadIdx.x & 48u) == 32u ? first[0] : rows[0];
+  } else if constexpr (kStep == 8) {
+    const uint32_t turned = (uint32_t)dpp_move<0x128>((int)v);  // row_ror:8
+    const uint32_t above = lane_up<16>(turned);
+    return (threadIdx.x & 8u) != 0 ? turned : above;
+  } else {
+#pragma unroll
+    for (int i = 0; i < kStep; ++i) v = (uint32_t)dpp_move<0x138>((int)v);  // wave_shr:1
+    return v;
+  }
+}
+template <int kStep> __device__ __forceinline__ double lane_up(double v) {
+  const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, ((uint64_t)lane_up<kStep>((uint32_t)(bits >> 32)) << 32) | lane_up<kStep>((uint32_t)bits));
+}
+// One lane's value, the same lane for the whole wave.
+__device__ __forceinline__ float lane_value(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(bits >> 32), lane) << 32) |
+                                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, lane));
+}
+// v of this lane + v of lane ^ kStep (addition commutes: the sums of the two are the same bits)
+template <int kStep> __device__ __forceinline__ double add_xor(double v) {
+  const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+  const uint32_t low = (uint32_t)bits, high = (uint32_t)(bits >> 32);
+  auto joined = [](uint32_t h, uint32_t l) { return __builtin_bit_cast(double, ((uint64_t)h << 32) | l); };
+  if constexpr (kStep == 32) {
+    const auto h = __builtin_amdgcn_permlane32_swap(high, high, false, false), l = __builtin_amdgcn_permlane32_swap(low, low, false, false);
+    return joined(h[0], l[0]) + joined(h[1], l[1]);
+  } else if constexpr (kStep == 16) {
+    const auto h = __builtin_amdgcn_permlane16_swap(high, high, false, false), l = __builtin_amdgcn_permlane16_swap(low, low, false, false);
+    return joined(h[0], l[0]) + joined(h[1], l[1]);
+  } else {
+    auto moved = [](uint32_t w) {
+      if constexpr (kStep == 1) return (uint32_t)dpp_move<kDppSwap1>((int)w);
+      else if constexpr (kStep == 2) return (uint32_t)dpp_move<kDppSwap2>((int)w);
+      else if constexpr (kStep == 4) return (uint32_t)dpp_move<0x1B>(dpp_move<kDppHalfMirror>((int)w));  // and quad_perm [3,2,1,0]
+      else return (uint32_t)dpp_move<0x128>((int)w);                                                     // row_ror:8
+    };
+    return v + joined(moved(high), moved(low));
+  }
+}
+
 // Combine across `kLanes` adjacent lanes (4, 8, 16, 32 or 64) with `op`.
 template <int kLanes, class V, class Op>
 __device__ __forceinline__ V group_reduce(V v, Op op) {

@@ -137,9 +137,7 @@ template <class T, bool kAligned> struct TileValues {
 };
 
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int step = 1; step < kWaveLanes; step *= 2) v += __shfl_xor(v, step, kWaveLanes);
-  return v;
+  return add_xor<32>(add_xor<16>(add_xor<8>(add_xor<4>(add_xor<2>(add_xor<1>(v))))));
 }
 
 template <class T, bool kVector>
@@ -178,18 +176,29 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_tiles(const void *l
   }
 }
 
+// Inclusive sums over the lanes of a wave, in lane order, of its first kLanes lanes.
+template <int kLanes> __device__ __forceinline__ double wave_scan(double v) {
+  const int lane = threadIdx.x & (kWaveLanes - 1);
+  auto step = [&](auto places) {
+    constexpr int kStep = decltype(places)::value;
+    if constexpr (kStep < kLanes) {
+      const double below = lane_up<kStep>(v);
+      if (lane >= kStep) v += below;
+    }
+  };
+  step(std::integral_constant<int, 1>{}), step(std::integral_constant<int, 2>{}), step(std::integral_constant<int, 4>{});
+  step(std::integral_constant<int, 8>{}), step(std::integral_constant<int, 16>{}), step(std::integral_constant<int, 32>{});
+  return v;
+}
+
 // Scan of one double per thread over the block, in thread order: returns the sum of the threads
 // below (exactly the inclusive value the thread below holds) and leaves the inclusive value and
 // the block's total in `through` and `total`.  Two barriers; `vote` comes between them, with both sums known.
 template <class Vote>
 __device__ __forceinline__ double block_scan(double v, double *wave_totals, double *through, double *total, Vote vote) {
   const int lane = threadIdx.x & (kWaveLanes - 1), wave = threadIdx.x / kWaveLanes;
-#pragma unroll
-  for (int step = 1; step < kWaveLanes; step *= 2) {
-    const double below = __shfl_up(v, step, kWaveLanes);
-    if (lane >= step) v += below;
-  }
-  const double previous = __shfl_up(v, 1, kWaveLanes);
+  v = wave_scan<kWaveLanes>(v);
+  const double previous = lane_up<1>(v);
   if (lane == kWaveLanes - 1) wave_totals[wave] = v;
   __syncthreads();
   double before = 0, all = 0;
@@ -277,19 +286,15 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
     const float scale = exp_nonpositive(held.maximum - maximum);
     const double own = lane < tiles ? held.mass * (double)scale : 0.0;
     double through = own;
-#pragma unroll
-    for (int step = 1; step < kWaveLanes; step *= 2) {
-      const double below = __shfl_up(through, step, kWaveLanes);
-      if (lane >= (uint32_t)step) through += below;
-    }
-    const double previous = __shfl_up(through, 1, kWaveLanes), before = lane == 0 ? 0.0 : previous;
-    total = __shfl(through, kWaveLanes - 1, kWaveLanes);
+    through = wave_scan<kWaveLanes>(through);
+    const double previous = lane_up<1>(through), before = lane == 0 ? 0.0 : previous;
+    total = lane_value(through, kWaveLanes - 1);
     const double threshold = total * uniform;
     const uint64_t candidates = __ballot(own > 0 && through > threshold);
     const int holder = candidates != 0 ? __builtin_ctzll(candidates) : 0;
     const double residual = before + own > threshold ? threshold - before : 0.0;
-    crossing = Crossing{__shfl(residual, holder, kWaveLanes), candidates != 0 ? (uint32_t)holder : 0xFFFFFFFFu,
-                        __shfl(held.maximum, holder, kWaveLanes), __shfl(scale, holder, kWaveLanes)};
+    crossing = Crossing{lane_value(residual, holder), candidates != 0 ? (uint32_t)holder : 0xFFFFFFFFu,
+                        lane_value(held.maximum, holder), lane_value(scale, holder)};
   } else {
     // the row's maximum; a tile with NaN or +inf counts as +inf, which no valid tile reaches
     for (uint32_t t = threadIdx.x; t < tiles; t += kBlockThreads) maximum = fmaxf(maximum, mine[t].invalid ? kInfinity : mine[t].maximum);
@@ -513,12 +518,8 @@ __global__ __launch_bounds__(kShortWaves *kWaveLanes) void categorical_short(con
     mass += (double)weights[i];
   }
   double through = mass;
-#pragma unroll
-  for (int step = 1; step < kShortWidth / kPerThread; step *= 2) {  // sixteen lanes hold the row
-    const double below = __shfl_up(through, step, kWaveLanes);
-    if (lane >= (uint32_t)step) through += below;
-  }
-  const double previous = __shfl_up(through, 1, kWaveLanes), before = lane == 0 ? 0 : previous;
+  through = wave_scan<kShortWidth / kPerThread>(through);  // sixteen lanes hold the row
+  const double previous = lane_up<1>(through), before = lane == 0 ? 0 : previous;
   // (lanes past the sixteen have no mass)  None crossed: rounding left the threshold at the scan's total, the last with mass
   const uint64_t crossed = __ballot(mass > 0 && through > threshold), massive = __ballot(mass > 0);
   if (lane == (uint32_t)(crossed != 0 ? __builtin_ctzll(crossed) : kWaveLanes - 1 - __builtin_clzll(massive))) {

@@ -734,7 +734,7 @@ __global__ __launch_bounds__(kMergeThreads) void topk_rank_lists(const char *x, 
   uint64_t *list = out_lists + ((size_t)row * units_out + unit) * a.count;
   for (uint32_t i = threadIdx.x; i < taken; i += kMergeThreads) merged[i] = source[i];
   for (uint32_t i = threadIdx.x; i < a.count; i += kMergeThreads) ranked[i] = 0;  // a short last tile leaves "no element" keys
-  if (threadIdx.x == 0) reached = 0;
+  if (threadIdx.x == 0) reached = 0, bound_slot = 0;
   __syncthreads();
   // The bound comes from samples of the lists.  A sample at place p of its list stands for the
   // keys above it down to the list's previous sample: p + 1 keys of that list reach it.  Walking
@@ -745,8 +745,6 @@ __global__ __launch_bounds__(kMergeThreads) void topk_rank_lists(const char *x, 
   // compared (equal values of other indices come along).  A weak list (a row's short last tile)
   // sends weak samples and does not pull the bound down.  More than 64 lists: one sample per list
   // at the same place in each, ranked by counting.
-  if (threadIdx.x == 0) bound_slot = 0;
-  __syncthreads();
   if (lists <= kWaveLanes) {
     if (threadIdx.x < kWaveLanes) {
       uint32_t per_list = kWaveLanes / lists;
@@ -754,14 +752,19 @@ __global__ __launch_bounds__(kMergeThreads) void topk_rank_lists(const char *x, 
       const uint32_t own_list = threadIdx.x / per_list, nth = threadIdx.x - own_list * per_list;
       // places: share * {0.4, 0.8, 1.2, 1.7, 2.4, 3.4, 5, 8}, stretched so that the last one used
       // is at least 2.5 shares deep; strictly increasing, inside the list
-      const float factors[8] = {0.4f, 0.8f, 1.2f, 1.7f, 2.4f, 3.4f, 5.0f, 8.0f};
-      const float stretch = factors[per_list - 1] < 2.5f ? 2.5f / factors[per_list - 1] : 1.0f;
+      // (constants of an unrolled loop: a table would be fetched from memory step by step)
+      constexpr float factors[8] = {0.4f, 0.8f, 1.2f, 1.7f, 2.4f, 3.4f, 5.0f, 8.0f};
+      float last_factor = factors[0];
+#pragma unroll
+      for (uint32_t i = 1; i < 8; ++i) last_factor = i < per_list ? factors[i] : last_factor;
+      const float stretch = last_factor < 2.5f ? 2.5f / last_factor : 1.0f;
       const float share = (float)a.count / (float)lists * stretch;
       uint32_t place = 0, previous = 0, weight = 0, value = 0;
-      for (uint32_t i = 0; i <= nth; ++i) {
-        const uint32_t wanted_place = (uint32_t)ceilf(share * factors[i]);
-        previous = place;                                                  // keys before this sample's span
-        place = wanted_place > previous ? wanted_place : previous + 1;     // place = p + 1
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) {
+        const uint32_t wanted_place = (uint32_t)ceilf(share * factors[i]), next = wanted_place > place ? wanted_place : place + 1;
+        previous = i <= nth ? place : previous;  // keys before this sample's span
+        place = i <= nth ? next : place;         // place = p + 1
       }
       if (own_list < lists && place <= a.count) {
         weight = place - previous;
@@ -771,11 +774,13 @@ __global__ __launch_bounds__(kMergeThreads) void topk_rank_lists(const char *x, 
       uint64_t pair = ((uint64_t)value << 32) | weight;
       pair = wave_sort_descending(pair, threadIdx.x);
       uint32_t reached_by = (uint32_t)pair;
-#pragma unroll
-      for (int d = 1; d < kWaveLanes; d <<= 1) {
-        const uint32_t other = __shfl_up(reached_by, d, kWaveLanes);
-        if (threadIdx.x >= (uint32_t)d) reached_by += other;
-      }
+      auto gather = [&](auto step) {
+        constexpr int kStep = decltype(step)::value;
+        const uint32_t other = lane_up<kStep>(reached_by);
+        if (threadIdx.x >= (uint32_t)kStep) reached_by += other;
+      };
+      gather(std::integral_constant<int, 1>{}), gather(std::integral_constant<int, 2>{}), gather(std::integral_constant<int, 4>{});
+      gather(std::integral_constant<int, 8>{}), gather(std::integral_constant<int, 16>{}), gather(std::integral_constant<int, 32>{});
       const uint64_t enough = __ballot(reached_by >= a.count && (uint32_t)(pair >> 32) != 0);
       if (enough != 0 && threadIdx.x == (uint32_t)__ffsll((long long)enough) - 1) bound_slot = pair & 0xFFFFFFFF00000000ull;
     }
