@@ -78,7 +78,6 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x
   const char *mask_row = nullptr;
   if constexpr (kMask != kMaskNone) mask_row = mask + mask_row_offset(mrows, row);
   const char *row_x = x + (size_t)row * width * kSize;
-  char *row_y = y + (size_t)row * width * kSize;
 
   // Vector `lane + k * kLanes` of the row, moved back to end at the row's end where it would pass
   // it: `skip` of its elements belong to the vector before it (all of them: nothing is left).
@@ -115,9 +114,9 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x
 
   while (true) {
     float v[kVpl][kVec];
-#pragma unroll
-    for (int k = 0; k < kVpl; ++k) Traits<T>::unpack(raw[k], v[k]);
     if constexpr (kShared) {
+#pragma unroll
+      for (int k = 0; k < kVpl; ++k) Traits<T>::unpack(raw[k], v[k]);
       row_x += (size_t)inner * width * kSize;
       if (left > 1) {
 #pragma unroll
@@ -128,6 +127,7 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x
     float peak = -INFINITY;
 #pragma unroll
     for (int k = 0; k < kVpl; ++k) {
+      if constexpr (!kShared) Traits<T>::unpack(raw[k], v[k]);
       if constexpr (kMask == kMaskAdditive) {
         float addend[kVec];
         Traits<T>::unpack(added[k], addend);
@@ -190,6 +190,7 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x
     if constexpr (kLog) maxima = row_sum<kLanes>(maxima, joint_max);
     float normaliser = kLog ? log1pf((maxima - 1.0f) + total * 2.3283064365386963e-10f) : 1.0f / total;
     if (invalid) normaliser = __builtin_nanf("");
+    char *row_y = y + (size_t)row * width * kSize;
 #pragma unroll
     for (int k = 0; k < kVpl; ++k) {
       if (row_ok && skip[k] < kVec) {
@@ -202,7 +203,7 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_unaligned(const char *x
     }
     if constexpr (!kShared) break;
     if (--left == 0) break;  // the same for the whole block
-    row_y += (size_t)inner * width * kSize;
+    row += inner;
     if constexpr (kLanes > kWaveLanes) __syncthreads();  // the joint words are free again
   }
 }
