@@ -1462,7 +1462,8 @@ inline bool rows_of_vectors_serve(const MatVecParams &p) {
 //   x 2 15.8 / 9.5, [6144 -> 2048] x 5 12.2 / 9.5, Q6_K [1024 -> 2048] x 8 12.2 / 5.0, [2048 -> 6144] x 2 8.1 / 6.1,
 //   Q4_K [1024 -> 2048] x 4 5.2 / 3.6, [6144 -> 2048] x 4 12.9 / 6.7, [1536 -> 20000] x 2 10.5 / 7.1, [2048 -> 60000] x 4
 //   19.9 / 18.0.  Not a vocabulary of one span, whose codes the tile and quad kernels keep at hand: Q4_K [2048 -> 151936]
-//   x 2 38.8 / 39.5, x 5 55.0 / 53.5, Q6_K x 2 54.3 / 57.2; nor two rows far wider than the weight is high, Q8_0
+//   x 2 38.8 / 39.5, x 5 55.0 / 53.5, two rows of Q6_K 54.3 / 57.2 (three 62.1 / 55.7, four 59.4 / 53.3, [2048 -> 91000] x 4
+//   39.0 / 34.4); nor two rows far wider than the weight is high, Q8_0
 //   [16384 -> 1024] 10.1 / 11.4.  (Two to four rows against 6144 to 8999 Q4_K rows of up to 2048 values stay with the tiles
 //   that the tests of this rule name there, 7.3 / 5.2 at [2048 -> 6144] x 4.)
 //   one row, where the alternative walks block by block, from 8 M products on, and from 4 M where a row is wide:
@@ -1486,7 +1487,7 @@ bool strips_better(const MatVecParams &p, bool vectors) {
   // one span of a vocabulary: the tile and quad kernels keep its codes at hand and have no tiles left over
   const bool span_of_many = p.k == 2048 && p.rows >= 90000;
   if (p.kind == 0) return p.k > 2048 || (!span_of_many && (p.m > 4 || p.rows < 6144 || p.rows >= 9000)) ;
-  if (p.kind == 1 && p.m <= 4 && span_of_many) return false;
+  if (p.kind == 1 && p.m <= 2 && span_of_many) return false;
   return p.m > 2 || p.k < 8 * p.rows;
 }
 

@@ -303,3 +303,11 @@ def test_strips_scales_of_activation_blocks_are_exact_quotients():
         assert hc.last_launch_variant().startswith("gguf_matvec_q8_strips/q6_k/8")
         wanted = np.float32(-127) * (np.float32(1) / factor)
         assert np.array_equal(out.cpu().numpy(), np.tile(wanted, (1, rows // blocks)))
+
+
+@pytest.mark.parametrize("rows,m,kernel", [(90000, 1, "spans/q6_k/1"), (90000, 3, "strips/q6_k/4"), (90001, 4, "strips/q6_k/4")])
+def test_strips_rule_for_one_span_of_a_vocabulary_and_three_rows_or_more(rows, m, kernel):
+    rng = np.random.default_rng(1829)
+    note(f"q8 matvec rule q6_k rows {rows} k 2048 m {m}")
+    check("q6_k", "bf16", raw_bytes_for("q6_k", rng, rows, 2048), rows, 2048, rng.normal(0, 1, (m, 2048) if m > 1 else (2048,)).astype(np.float32),
+          kernel="gguf_matvec_q8_" + kernel)
