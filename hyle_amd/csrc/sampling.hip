@@ -411,7 +411,7 @@ __global__ __launch_bounds__(kBlockThreads) void categorical_rows(const void *lo
 // then the lanes of what would be the first wave of a block, the only one with elements --
 // so that every index and score is the one the two dispatches give.  The status word is written once, by
 // the launch's last block, which looks at all rows itself: rows cannot clear a word that others set.
-// Bound by latency.  MI355X, us, two dispatches / one: [5, 40] bf16 7.7 / 3.3, [64, 100] f32 7.7 / 3.5, [250, 64] bf16
+// Bound by latency.  MI355X, us, two dispatches / one: [5, 40] bf16 7.7 / 3.15, [64, 100] f32 7.7 / 3.35, [250, 64] bf16
 // 8.0 / 5.9.
 constexpr int kShortWidth = 256;             // TopK's select route serves as many
 constexpr int kShortWaves = 16;              // that share the status block's rows

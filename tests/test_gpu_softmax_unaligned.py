@@ -9,7 +9,8 @@ import torch
 
 from hyle_amd import compute as hc
 
-from gpu_support import DEVICE, TYPES, last_launch_form, note, run
+from gpu_support import DEVICE, TYPES, note, run
+from gpu_support import last_launch_form
 from test_gpu_softmax_variants import MASKS, compare_on_device, make_inputs, oracle_softmax
 
 pytestmark = pytest.mark.gpu
