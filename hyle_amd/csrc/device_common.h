@@ -232,6 +232,21 @@ template <int kStep> __device__ __forceinline__ double add_xor(double v) {
   }
 }
 
+// Lanes 0 to 31: a of this lane + a of the lane 32 above; lanes 32 to 63: b of the lane 32 below + b of this lane.
+__device__ __forceinline__ double add_halves_apart(double a, double b) {
+  const uint64_t first = __builtin_bit_cast(uint64_t, a), second = __builtin_bit_cast(uint64_t, b);
+  const auto h = __builtin_amdgcn_permlane32_swap((uint32_t)(first >> 32), (uint32_t)(second >> 32), false, false);
+  const auto l = __builtin_amdgcn_permlane32_swap((uint32_t)first, (uint32_t)second, false, false);
+  return __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) + __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+}
+// The same for rows of sixteen lanes: rows 0 and 2 add their a and the next row's, rows 1 and 3 the previous row's b and theirs.
+__device__ __forceinline__ double add_rows_apart(double a, double b) {
+  const uint64_t first = __builtin_bit_cast(uint64_t, a), second = __builtin_bit_cast(uint64_t, b);
+  const auto h = __builtin_amdgcn_permlane16_swap((uint32_t)(first >> 32), (uint32_t)(second >> 32), false, false);
+  const auto l = __builtin_amdgcn_permlane16_swap((uint32_t)first, (uint32_t)second, false, false);
+  return __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) + __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+}
+
 // Combine across `kLanes` adjacent lanes (4, 8, 16, 32 or 64) with `op`.
 template <int kLanes, class V, class Op>
 __device__ __forceinline__ V group_reduce(V v, Op op) {

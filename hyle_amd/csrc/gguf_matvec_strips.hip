@@ -24,12 +24,11 @@
 // A block of sixteen waves (eight where the codes leave no room for more slots) has a compute unit's
 // LDS, quantises the activation rows once, while its first weight bytes are on their way, and walks its
 // share of the weight rows in tiles of at most sixteen; `split` waves share a tile, each
-// taking every split-th run, and the first adds the shares.  A lane's chain of up to 224 runs, and the
-// sum over the shares, run in 64 bits: in 32, a chain that is several times as long as one of the
-// kernels that spread a row over 64 lanes was further from the 64-bit sum than theirs in a third of
-// the shapes (f32 Q8_0 [5120 -> 2304] x 6 9.6e-8 relative against 8.2e-8 there, Q4_K [4096 -> 6656] x 4
-// 7.6e-8 against 6.2e-8; in 64 bits 5.3e-8 and 4.5e-8, at most 0.75 of theirs over 87 shapes, for about
-// 1 % of the time).  Q8_0 and Q6_K runs are loaded as the aligned vectors that cover them and
+// taking every split-th run, and the first adds the shares.  A lane's chain of up to 224 runs, the sums
+// over the lanes of a column and the sum over the shares run in 64 bits: in 32, a chain that is several times as long
+// as one of the kernels that spread a row over 64 lanes was further from the 64-bit sum than theirs in a third of the
+// shapes (f32 Q8_0 [5120 -> 2304] x 6 9.6e-8 relative against 8.4e-8 there, Q4_K [4096 -> 6656] x 4 7.6e-8 against 7.1e-8;
+// in 64 bits 3.5e-8 for both, at most 4.3e-8 over 300 shapes, for about 1 % of the time).  Q8_0 and Q6_K runs are loaded as the aligned vectors that cover them and
 // redistributed through a wave-private slot: lanes that load their own 16 bytes at 2-byte addresses keep the
 // memory pipe busy several times as long (Q8_0 [2048 -> 151936] 111 us that way, 63 us through the slot), and lanes
 // that load their own aligned vectors ask for sixteen half lines at a time (in place, [5120 -> 17408] x 4 24.6 us,
@@ -453,33 +452,27 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
   // Lane (c, p) of the tile's first wave ends with activation row 4 set + p against weight row c.
   auto finish = [&]() {
     const uint32_t lane = opaque(threadIdx.x % kWaveLanes), column = lane % 16, part = lane / 16;
-    float mine[kSets];
+    // 64-bit sums over the lanes of a column, one rounding for a share and one for the product (with the lanes' sums rounded
+    // first: Q4_K [2304 -> 12800] x 3 6.2e-8 off the 64-bit product in f32, 3.5e-8 like this)
+    double mine[kSets];
 #pragma unroll
     for (int set = 0; set < kSets; ++set) {
-      const bool upper = part >= 2, odd = part % 2 != 0;
-      float own_sum[4], pair[2];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) own_sum[i] = (float)totals[set][i];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        pair[i] = (upper ? own_sum[2 + i] : own_sum[i]) + __shfl_xor(upper ? own_sum[i] : own_sum[2 + i], 32, kWaveLanes);
-      mine[set] = (odd ? pair[1] : pair[0]) + __shfl_xor(odd ? pair[0] : pair[1], 16, kWaveLanes);
+      mine[set] = add_rows_apart(add_halves_apart(totals[set][0], totals[set][2]), add_halves_apart(totals[set][1], totals[set][3]));
 #pragma unroll
       for (int i = 0; i < 4; ++i) totals[set][i] = 0.0;
     }
     if (split != 1) {
       // the wave's own share; those of the waves behind it follow, kSets * kWaveLanes apart
       float *share = reinterpret_cast<float *>(shared + opaque(layout.shares + (wave * kSets * kWaveLanes + lane) * 4));
+      if (member != 0) {
 #pragma unroll
-      for (int set = 0; set < kSets; ++set) share[set * kWaveLanes] = mine[set];
+        for (int set = 0; set < kSets; ++set) share[set * kWaveLanes] = (float)mine[set];
+      }
       lds_barrier();
       if (member == 0) {
 #pragma unroll
-        for (int set = 0; set < kSets; ++set) {
-          double whole = (double)mine[set];
-          for (uint32_t other = 1; other < split; ++other) whole += (double)share[(other * kSets + set) * kWaveLanes];
-          mine[set] = (float)whole;
-        }
+        for (int set = 0; set < kSets; ++set)
+          for (uint32_t other = 1; other < split; ++other) mine[set] += (double)share[(other * kSets + set) * kWaveLanes];
       }
       if (++round < rounds) lds_barrier();  // before the shares of the next round
     }
@@ -487,7 +480,7 @@ __global__ __launch_bounds__(kMostWaves * kWaveLanes) void gguf_matvec_q8_strips
     if (member == 0 && row < tile_end(tile)) {
 #pragma unroll
       for (uint32_t set = 0; set < (uint32_t)kSets; ++set)
-        if (4 * set + part < m) Traits<TX>::store(y, (size_t)(4 * set + part) * rows + row, mine[set]);
+        if (4 * set + part < m) Traits<TX>::store(y, (size_t)(4 * set + part) * rows + row, (float)mine[set]);
     }
   };
   for (uint32_t done = 0; done < items; ++done) {

@@ -213,6 +213,27 @@ def test_strips_are_no_further_from_64_bit_sums(tag, k, rows, m, byte_offset):
     assert own <= others, f"{own / others:.3f} of the error of the kernels for few rows"
 
 
+@pytest.mark.parametrize("tag,k,rows,m", [
+    ("q4_k", 4352, 1280, 1), ("q4_k", 2560, 12544, 1), ("q4_k", 2304, 12800, 3), ("q6_k", 1792, 2560, 5), ("q6_k", 5632, 3072, 1),
+    ("q8_0", 3328, 4352, 8), ("q8_0", 5120, 4608, 5)])
+def test_strips_round_a_product_twice(tag, k, rows, m):
+    """f32 products against the oracle's float64 sums over the same 8-bit codes.  A product is the sum in 64 bits of its waves'
+    shares, each rounded to f32 but the first, and is rounded once itself.  A rounding moves a value by 2^-24 / sqrt(3) of it
+    in root mean square, at the foot of a binade, and the shares' squares add up to the product's in the mean: sqrt(2 / 3) * 2^-24 =
+    4.9e-8 of the products (2-norm) at most.  (With the lanes' sums rounded first 5.2e-8 to 6.9e-8 at these sizes.)"""
+    rng = np.random.default_rng(1827)
+    raw = weights_for(tag, rng, rows, k)
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    kind, gguf = KINDS[tag]
+    note(f"q8 matvec {tag} [{k} -> {rows}] x {m}: strips against float64")
+    descs = [hc.TensorDesc.gguf_weight(gguf, hc.DataType.kFloat32, k, rows), hc.TensorDesc.dense(hc.DataType.kFloat32, [m, k])]
+    (out,) = run(Q8, torch.from_numpy(raw.reshape(-1)).to(DEVICE), torch.from_numpy(x).to(DEVICE), descs=descs)
+    assert hc.last_launch_variant().startswith("gguf_matvec_q8_strips"), hc.last_launch_variant()
+    centre, _ = orc.gguf_matvec_q8(kind, raw.reshape(-1), rows, k, x)
+    off = np.linalg.norm(out.cpu().numpy().astype(np.float64).reshape(m, rows) - centre.reshape(m, rows)) / np.linalg.norm(centre)
+    assert off <= np.sqrt(2 / 3) * 2.0 ** -24, f"{off:.3e}"
+
+
 @pytest.mark.parametrize("tag", list(KINDS))
 def test_strips_activations_that_are_no_numbers(tag):
     """A NaN is no candidate for a block's magnitude and has the code of a zero; an infinity leaves its block no finite
