@@ -557,7 +557,7 @@ hipError_t run_strips(const MatVecParams &p, uint32_t m, const void *w, const vo
   const uint32_t codes = m * p.k;
   const bool little = (codes <= 16384 && rows >= 8192 && (kKind >= 2 || p.k < 2048 || rows >= 32768)) || (codes <= 32768 && rows >= 65536);
   const bool twice = little && 2 * strip_layout(kKind, m, p.k, 8).bytes <= kStripLds;
-  const uint32_t waves = twice ? 8 : strip_waves(kKind, m, p.k), shared = strip_layout(kKind, m, p.k, waves).bytes;
+  const uint32_t waves = twice ? 8 : strip_waves(kKind, m, p.k);
   const uint32_t wanted = units * (twice ? 2u : 1u);
   const uint32_t block_rows = (rows + wanted - 1) / wanted;
   const uint32_t grid = (rows + block_rows - 1) / block_rows;
@@ -575,6 +575,11 @@ hipError_t run_strips(const MatVecParams &p, uint32_t m, const void *w, const vo
       split = candidate;
     }
   }
+  // No more waves than have a tile's runs to walk or activations to quantise: a wave without an item loads as much as another,
+  // and up to fifteen of them keep a compute unit's memory pipe for 0.2 to 0.8 us (sixteen waves always / like this: Q8_0
+  // [1024 -> 768] x 4 4.6 / 3.8, [1536 -> 1280] x 3 4.9 / 4.3, [2048 -> 2816] x 2 5.15 / 4.5, Q4_K [1792 -> 1792] x 3 4.2 / 4.0).
+  const uint32_t busy = std::min(tiles, waves / split) * split, quantising = (m * runs + 3) / 4;
+  const uint32_t block_waves = std::min(waves, std::max(busy, quantising)), shared = strip_layout(kKind, m, p.k, block_waves).bytes;
   if constexpr (kKind == 3) {
     note_variant<StripsTag<kKind, kSets, kSixteen>>();
   } else {
@@ -586,7 +591,7 @@ hipError_t run_strips(const MatVecParams &p, uint32_t m, const void *w, const vo
     else if (waves == kMostWaves && split != 1) note_variant<StripsTag<kKind, kSets, kSixteenShared>>();
     else if (waves == kMostWaves) note_variant<StripsTag<kKind, kSets, kSixteen>>();
   }
-  hipLaunchKernelGGL((gguf_matvec_q8_strips<kKind, TX, kSets>), dim3(grid), dim3(waves * kWaveLanes), shared, s, static_cast<const unsigned char *>(w), x, y,
+  hipLaunchKernelGGL((gguf_matvec_q8_strips<kKind, TX, kSets>), dim3(grid), dim3(block_waves * kWaveLanes), shared, s, static_cast<const unsigned char *>(w), x, y,
                      rows, p.row_stride, p.k, m, block_rows, tile_rows, split, (255 + split) / split);
   return hipGetLastError();
 }

@@ -183,6 +183,20 @@ def test_strips_any_number_of_waves_to_a_tile(tag):
         assert np.array_equal(got, np.take(got, np.arange(rows) % period, 1))
 
 
+@pytest.mark.parametrize("x_tag", ["f32", "bf16"])
+@pytest.mark.parametrize("tag", list(KINDS))
+def test_strips_blocks_of_few_waves(tag, x_tag):
+    """One tile to a block and few activations: a block has only the waves that walk or quantise, one to fifteen."""
+    rng = np.random.default_rng(1830)
+    for rows, k, m in ((700, 256, 2), (530, 256, 8), (513, 512, 8), (601, 768, 3), (1027, 1280, 5), (600, 1792, 2), (4100, 1792, 8),
+                       (600, 2304, 7), (515, 2816, 4), (5200, 1024, 2), (520, 3840, 3), (9300, 768, 4)):
+        raw = raw_bytes_for(tag, rng, rows, k)
+        for byte_offset in (0, 2):
+            note(f"q8 matvec strips few waves {tag} x {x_tag} rows {rows} k {k} m {m} off {byte_offset}")
+            check(tag, x_tag, raw, rows, k, rng.normal(0, 1.5, (m, k)).astype(np.float32), byte_offset=byte_offset)
+        assert hc.last_launch_variant().startswith(f"gguf_matvec_q8_strips/{tag}/{4 if m <= 4 else 8}-tokens")   # two bytes off: no kernel of whole vectors
+
+
 @pytest.mark.parametrize("tag,k,rows,m,byte_offset", [
     ("q8_0", 5120, 2304, 6, 0), ("q8_0", 2560, 8192, 4, 0), ("q6_k", 5120, 3584, 8, 0), ("q6_k", 1024, 8192, 5, 0),
     ("q4_k", 4096, 6656, 4, 0), ("q4_k", 9984, 3072, 5, 2)])
