@@ -50,10 +50,9 @@ bool run_exact_lanes(uint32_t per_lane, const NormParams &p, const Bound &io, in
 //     [1000, 5120] 5.5 / 4.9   [2000, 3072] 5.2 / 5.4   [12288, 512] 6.6 / 6.4   [16384, 512] 7.3 / 8.2
 //   LayerNorm f32 [8, 4096] 4.1 / 2.7   [64, 2560] 3.6 / 2.8   [512, 512] 4.1 / 2.6   [1000, 2560] 5.4 / 4.8   [1000, 4096] 6.9 / 7.8
 //     [8192, 256] 5.5 / 5.1   [12288, 256] 6.2 / 7.2   bf16 [2000, 2560] 5.3 / 5.1   [2000, 4096] 6.8 / 6.9
-// (As many rows as these shapes' own tests have, four of 192 vectors or more or one block of shorter ones, stay here.)
-inline bool exact_pays(uint64_t rows, uint32_t vectors, uint64_t bytes) {
-  return bytes >= (10ull << 20) || rows == (vectors <= 128 ? 512 / vectors : 4);
-}
+//   four rows, one after another in a graph: RMSNorm bf16 [4, 1024] 2.5 / 1.7   [4, 5120] 3.2 / 2.2   [4, 10240] 2.7 / 2.75
+//     LayerNorm f32 [4, 1024] 2.1 / 1.8   [4, 8192] 3.65 / 2.65   bf16 [4, 6144] 4.7 / 2.7
+inline bool exact_pays(uint64_t bytes) { return bytes >= (10ull << 20); }
 
 template <class T, class W, bool kLayer>
 bool run_exact_shape(const NormParams &p, const Bound &io, hipStream_t s) {
@@ -61,7 +60,7 @@ bool run_exact_shape(const NormParams &p, const Bound &io, hipStream_t s) {
   if (p.shape.width % kVec != 0) return false;
   const uint32_t vectors = p.shape.width / kVec;
   if (!kLayer && vectors == 256) return false;  // norm.hip's shape measures the same
-  if (!exact_pays(p.shape.rows, vectors, p.shape.rows * p.shape.width * Traits<T>::kSize)) return false;
+  if (!exact_pays(p.shape.rows * p.shape.width * Traits<T>::kSize)) return false;
   const int parameters = !p.has_weight ? kPlain : (kLayer && p.has_bias ? kScaleBias : kScale);
   // short rows: two vectors per lane in a group of half as many lanes as the row has vectors, four
   // rows per group (a lane with one vector of a row is slow: [32768, 512] 14.2 / 15.5 us)

@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from hyle_amd import compute as hc
 from oracle import lib as orc
@@ -61,43 +62,43 @@ CASES = [
     ("rms", "f32", 3, 16372, "norm_rows/rms/1024x4/1024/1/ragged"),
     ("rms", "f32", 3, 32756, "norm_rows/rms/1024x8/1024/1/ragged"),
     ("rms", "f32", 3, 1027, "norm_generic/rms"),
-    ("rms", "f32", 32, 64, "norm_rows_exact/rms/8x2/64/4"),
-    ("rms", "f32", 16, 128, "norm_rows_exact/rms/16x2/64/4"),
-    ("rms", "f32", 8, 256, "norm_rows_exact/rms/32x2/64/4"),
-    ("rms", "f32", 4, 512, "norm_rows_exact/rms/64x2/64/4"),
-    ("rms", "f32", 4, 768, "norm_rows_exact/rms/64x3/64/2"),
-    ("rms", "f32", 4, 1280, "norm_rows_exact/rms/64x5/64/2"),
-    ("rms", "f32", 4, 1536, "norm_rows_exact/rms/64x6/64/2"),
-    ("rms", "f32", 4, 1792, "norm_rows_exact/rms/64x7/64/2"),
-    ("rms", "f32", 4, 2048, "norm_rows_exact/rms/64x8/64/2"),
-    ("rms", "f32", 4, 2304, "norm_rows_exact/rms/64x9/64/2"),
-    ("rms", "f32", 4, 2560, "norm_rows_exact/rms/64x10/64/2"),
-    ("rms", "f32", 4, 3072, "norm_rows_exact/rms/64x12/64/2"),
-    ("rms", "f32", 4, 3584, "norm_rows_exact/rms/128x7/128/2"),
-    ("rms", "f32", 4, 4096, "norm_rows_exact/rms/128x8/128/2"),
-    ("rms", "f32", 4, 5120, "norm_rows_exact/rms/256x5/256/2"),
-    ("rms", "f32", 4, 6144, "norm_rows_exact/rms/256x6/256/2"),
-    ("rms", "f32", 4, 7168, "norm_rows_exact/rms/256x7/256/2"),
-    ("rms", "f32", 4, 8192, "norm_rows_exact/rms/256x8/256/2"),
-    ("layer", "f32", 32, 64, "norm_rows_exact/layer/8x2/64/4"),
-    ("layer", "f32", 16, 128, "norm_rows_exact/layer/16x2/64/4"),
-    ("layer", "f32", 8, 256, "norm_rows_exact/layer/32x2/64/4"),
-    ("layer", "f32", 4, 512, "norm_rows_exact/layer/64x2/64/4"),
-    ("layer", "f32", 4, 768, "norm_rows_exact/layer/64x3/64/2"),
-    ("layer", "f32", 4, 1024, "norm_rows_exact/layer/64x4/64/2"),
-    ("layer", "f32", 4, 1280, "norm_rows_exact/layer/64x5/64/2"),
-    ("layer", "f32", 4, 1536, "norm_rows_exact/layer/64x6/64/2"),
-    ("layer", "f32", 4, 1792, "norm_rows_exact/layer/64x7/64/2"),
-    ("layer", "f32", 4, 2048, "norm_rows_exact/layer/64x8/64/2"),
-    ("layer", "f32", 4, 2304, "norm_rows_exact/layer/64x9/64/2"),
-    ("layer", "f32", 4, 2560, "norm_rows_exact/layer/64x10/64/2"),
-    ("layer", "f32", 4, 3072, "norm_rows_exact/layer/64x12/64/2"),
-    ("layer", "f32", 4, 3584, "norm_rows_exact/layer/128x7/128/2"),
-    ("layer", "f32", 4, 4096, "norm_rows_exact/layer/128x8/128/2"),
-    ("layer", "f32", 4, 5120, "norm_rows_exact/layer/256x5/256/2"),
-    ("layer", "f32", 4, 6144, "norm_rows_exact/layer/256x6/256/2"),
-    ("layer", "f32", 4, 7168, "norm_rows_exact/layer/256x7/256/2"),
-    ("layer", "f32", 4, 8192, "norm_rows_exact/layer/256x8/256/2"),
+    ("rms", "f32", 32, 64, "norm_rows/rms/16x1/256/1/ragged"),
+    ("rms", "f32", 16, 128, "norm_rows/rms/32x1/256/1/ragged"),
+    ("rms", "f32", 8, 256, "norm_rows/rms/64x1/256/1/ragged"),
+    ("rms", "f32", 4, 512, "norm_rows_tail/rms/64x2/256/1"),
+    ("rms", "f32", 4, 768, "norm_rows_tail/rms/64x3/64/1"),
+    ("rms", "f32", 4, 1280, "norm_rows_tail/rms/64x5/64/1"),
+    ("rms", "f32", 4, 1536, "norm_rows_tail/rms/64x6/64/1"),
+    ("rms", "f32", 4, 1792, "norm_rows_tail/rms/64x7/64/1"),
+    ("rms", "f32", 4, 2048, "norm_rows_tail/rms/64x8/64/1"),
+    ("rms", "f32", 4, 2304, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "f32", 4, 2560, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "f32", 4, 3072, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "f32", 4, 3584, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "f32", 4, 4096, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "f32", 4, 5120, "norm_rows/rms/256x8/256/1/ragged"),
+    ("rms", "f32", 4, 6144, "norm_rows/rms/256x8/256/1/ragged"),
+    ("rms", "f32", 4, 7168, "norm_rows/rms/256x8/256/1/ragged"),
+    ("rms", "f32", 4, 8192, "norm_rows/rms/256x8/256/1/ragged"),
+    ("layer", "f32", 32, 64, "norm_rows/layer/16x1/256/1/exact"),
+    ("layer", "f32", 16, 128, "norm_rows/layer/32x1/256/1/exact"),
+    ("layer", "f32", 8, 256, "norm_rows/layer/64x1/256/1/exact"),
+    ("layer", "f32", 4, 512, "norm_rows_tail/layer/64x2/256/1"),
+    ("layer", "f32", 4, 768, "norm_rows_tail/layer/64x3/64/1"),
+    ("layer", "f32", 4, 1024, "norm_rows_tail/layer/64x4/64/1"),
+    ("layer", "f32", 4, 1280, "norm_rows_tail/layer/64x5/64/1"),
+    ("layer", "f32", 4, 1536, "norm_rows_tail/layer/64x6/64/1"),
+    ("layer", "f32", 4, 1792, "norm_rows_tail/layer/64x7/64/1"),
+    ("layer", "f32", 4, 2048, "norm_rows_tail/layer/64x8/64/1"),
+    ("layer", "f32", 4, 2304, "norm_rows/layer/256x4/256/1/ragged"),
+    ("layer", "f32", 4, 2560, "norm_rows/layer/256x4/256/1/ragged"),
+    ("layer", "f32", 4, 3072, "norm_rows/layer/256x4/256/1/ragged"),
+    ("layer", "f32", 4, 3584, "norm_rows/layer/256x4/256/1/ragged"),
+    ("layer", "f32", 4, 4096, "norm_rows/layer/256x4/256/1/exact"),
+    ("layer", "f32", 4, 5120, "norm_rows/layer/256x8/256/1/ragged"),
+    ("layer", "f32", 4, 6144, "norm_rows/layer/256x8/256/1/ragged"),
+    ("layer", "f32", 4, 7168, "norm_rows/layer/256x8/256/1/ragged"),
+    ("layer", "f32", 4, 8192, "norm_rows/layer/256x8/256/1/exact"),
     ("layer", "bf16", 32, 64, "norm_rows/layer/8x1/256/1/exact"),
     ("layer", "bf16", 3, 40, "norm_rows/layer/8x1/256/1/ragged"),
     ("layer", "bf16", 16, 128, "norm_rows/layer/16x1/256/1/exact"),
@@ -130,43 +131,43 @@ CASES = [
     ("rms", "bf16", 3, 32744, "norm_rows/rms/1024x4/1024/1/ragged"),
     ("rms", "bf16", 3, 65512, "norm_rows/rms/1024x8/1024/1/ragged"),
     ("rms", "bf16", 3, 1027, "norm_generic/rms"),
-    ("rms", "bf16", 32, 128, "norm_rows_exact/rms/8x2/64/4"),
-    ("rms", "bf16", 16, 256, "norm_rows_exact/rms/16x2/64/4"),
-    ("rms", "bf16", 8, 512, "norm_rows_exact/rms/32x2/64/4"),
-    ("rms", "bf16", 4, 1024, "norm_rows_exact/rms/64x2/64/4"),
-    ("rms", "bf16", 4, 1536, "norm_rows_exact/rms/64x3/64/2"),
-    ("rms", "bf16", 4, 2560, "norm_rows_exact/rms/64x5/64/2"),
-    ("rms", "bf16", 4, 3072, "norm_rows_exact/rms/64x6/64/2"),
-    ("rms", "bf16", 4, 3584, "norm_rows_exact/rms/64x7/64/2"),
-    ("rms", "bf16", 4, 4096, "norm_rows_exact/rms/64x8/64/2"),
-    ("rms", "bf16", 4, 4608, "norm_rows_exact/rms/64x9/64/2"),
-    ("rms", "bf16", 4, 5120, "norm_rows_exact/rms/64x10/64/2"),
-    ("rms", "bf16", 4, 6144, "norm_rows_exact/rms/64x12/64/2"),
-    ("rms", "bf16", 4, 7168, "norm_rows_exact/rms/128x7/128/2"),
-    ("rms", "bf16", 4, 8192, "norm_rows_exact/rms/128x8/128/2"),
-    ("rms", "bf16", 4, 10240, "norm_rows_exact/rms/256x5/256/2"),
-    ("rms", "bf16", 4, 12288, "norm_rows_exact/rms/256x6/256/2"),
-    ("rms", "bf16", 4, 14336, "norm_rows_exact/rms/256x7/256/2"),
-    ("rms", "bf16", 4, 16384, "norm_rows_exact/rms/256x8/256/2"),
-    ("layer", "bf16", 32, 128, "norm_rows_exact/layer/8x2/64/4"),
-    ("layer", "bf16", 16, 256, "norm_rows_exact/layer/16x2/64/4"),
-    ("layer", "bf16", 8, 512, "norm_rows_exact/layer/32x2/64/4"),
-    ("layer", "bf16", 4, 1024, "norm_rows_exact/layer/64x2/64/4"),
-    ("layer", "bf16", 4, 1536, "norm_rows_exact/layer/64x3/64/2"),
-    ("layer", "bf16", 4, 2048, "norm_rows_exact/layer/64x4/64/2"),
-    ("layer", "bf16", 4, 2560, "norm_rows_exact/layer/64x5/64/2"),
-    ("layer", "bf16", 4, 3072, "norm_rows_exact/layer/64x6/64/2"),
-    ("layer", "bf16", 4, 3584, "norm_rows_exact/layer/64x7/64/2"),
-    ("layer", "bf16", 4, 4096, "norm_rows_exact/layer/64x8/64/2"),
-    ("layer", "bf16", 4, 4608, "norm_rows_exact/layer/64x9/64/2"),
-    ("layer", "bf16", 4, 5120, "norm_rows_exact/layer/64x10/64/2"),
-    ("layer", "bf16", 4, 6144, "norm_rows_exact/layer/64x12/64/2"),
-    ("layer", "bf16", 4, 7168, "norm_rows_exact/layer/128x7/128/2"),
-    ("layer", "bf16", 4, 8192, "norm_rows_exact/layer/128x8/128/2"),
-    ("layer", "bf16", 4, 10240, "norm_rows_exact/layer/256x5/256/2"),
-    ("layer", "bf16", 4, 12288, "norm_rows_exact/layer/256x6/256/2"),
-    ("layer", "bf16", 4, 14336, "norm_rows_exact/layer/256x7/256/2"),
-    ("layer", "bf16", 4, 16384, "norm_rows_exact/layer/256x8/256/2"),
+    ("rms", "bf16", 32, 128, "norm_rows/rms/16x1/256/1/ragged"),
+    ("rms", "bf16", 16, 256, "norm_rows/rms/32x1/256/1/ragged"),
+    ("rms", "bf16", 8, 512, "norm_rows/rms/64x1/256/1/ragged"),
+    ("rms", "bf16", 4, 1024, "norm_rows_tail/rms/64x2/256/1"),
+    ("rms", "bf16", 4, 1536, "norm_rows_tail/rms/64x3/64/1"),
+    ("rms", "bf16", 4, 2560, "norm_rows_tail/rms/64x5/64/1"),
+    ("rms", "bf16", 4, 3072, "norm_rows_tail/rms/64x6/64/1"),
+    ("rms", "bf16", 4, 3584, "norm_rows_tail/rms/64x7/64/1"),
+    ("rms", "bf16", 4, 4096, "norm_rows_tail/rms/64x8/64/1"),
+    ("rms", "bf16", 4, 4608, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "bf16", 4, 5120, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "bf16", 4, 6144, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "bf16", 4, 7168, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "bf16", 4, 8192, "norm_rows/rms/256x4/256/1/ragged"),
+    ("rms", "bf16", 4, 10240, "norm_rows/rms/256x8/256/1/ragged"),
+    ("rms", "bf16", 4, 12288, "norm_rows/rms/256x8/256/1/ragged"),
+    ("rms", "bf16", 4, 14336, "norm_rows/rms/256x8/256/1/ragged"),
+    ("rms", "bf16", 4, 16384, "norm_rows/rms/256x8/256/1/ragged"),
+    ("layer", "bf16", 32, 128, "norm_rows/layer/16x1/256/1/exact"),
+    ("layer", "bf16", 16, 256, "norm_rows/layer/32x1/256/1/exact"),
+    ("layer", "bf16", 8, 512, "norm_rows/layer/64x1/256/1/exact"),
+    ("layer", "bf16", 4, 1024, "norm_rows_tail/layer/64x2/256/1"),
+    ("layer", "bf16", 4, 1536, "norm_rows_tail/layer/64x3/64/1"),
+    ("layer", "bf16", 4, 2048, "norm_rows_tail/layer/64x4/64/1"),
+    ("layer", "bf16", 4, 2560, "norm_rows_tail/layer/64x5/64/1"),
+    ("layer", "bf16", 4, 3072, "norm_rows_tail/layer/64x6/64/1"),
+    ("layer", "bf16", 4, 3584, "norm_rows_tail/layer/64x7/64/1"),
+    ("layer", "bf16", 4, 4096, "norm_rows_tail/layer/64x8/64/1"),
+    ("layer", "bf16", 4, 4608, "norm_rows/layer/256x4/256/1/ragged"),
+    ("layer", "bf16", 4, 5120, "norm_rows/layer/256x4/256/1/ragged"),
+    ("layer", "bf16", 4, 6144, "norm_rows/layer/256x4/256/1/ragged"),
+    ("layer", "bf16", 4, 7168, "norm_rows/layer/256x4/256/1/ragged"),
+    ("layer", "bf16", 4, 8192, "norm_rows/layer/256x4/256/1/exact"),
+    ("layer", "bf16", 4, 10240, "norm_rows/layer/256x8/256/1/ragged"),
+    ("layer", "bf16", 4, 12288, "norm_rows/layer/256x8/256/1/ragged"),
+    ("layer", "bf16", 4, 14336, "norm_rows/layer/256x8/256/1/ragged"),
+    ("layer", "bf16", 4, 16384, "norm_rows/layer/256x8/256/1/exact"),
 ]
 
 # One wave per row (norm_tail.h): widths on both sides of a lane's last vector, few rows, and for two rows per wave an
@@ -191,6 +192,7 @@ CASES += [("layer", "f32", 6144, 400, "norm_rows_tail/layer/64x2/256/1"), ("laye
           ("rms", "f32", 3999, 1000, "norm_rows_tail/rms/64x4/64/1"), ("rms", "f32", 4001, 1000, "norm_rows/rms/64x4/256/2/ragged"),
           ("rms", "bf16", 6999, 1032, "norm_rows_tail/rms/64x3/64/1"), ("rms", "bf16", 7001, 1032, "norm_rows_tail/rms/64x3/64/2"),
           ("rms", "bf16", 31, 4104, "norm_rows_tail/rms/64x9/64/1"), ("rms", "bf16", 33, 4104, "norm_rows/rms/256x4/256/1/ragged"),
+          ("rms", "bf16", 8193, 800, "norm_rows/rms/64x2/256/2/ragged"), ("rms", "bf16", 7001, 1544, "norm_rows/rms/64x4/256/2/ragged"),
           ("layer", "bf16", 575, 4104, "norm_rows/layer/256x4/256/1/ragged"), ("layer", "bf16", 577, 4104, "norm_rows_tail/layer/64x9/64/1")]
 
 # Few rows of up to 512 vectors a wave each, and both sides of the 10 MiB below which rows are not taken two or four to a wave.
@@ -202,14 +204,28 @@ CASES += [("rms", "f32", 2, 2048, "norm_rows_tail/rms/64x8/64/1"), ("layer", "bf
           ("layer", "f32", 10232, 256, "norm_rows/layer/64x1/256/1/exact"), ("layer", "f32", 2046, 1280, "norm_rows_tail/layer/64x5/64/1"),
           ("layer", "f32", 2048, 1280, "norm_rows_exact/layer/64x5/64/2")]
 
+# The shapes that cover the tensor exactly: 16-byte vectors to a row, shape, rows to a block; they serve from 10 MiB on.
+EXACT_SHAPES = [(16, "8x2/64/4", 32), (32, "16x2/64/4", 16), (64, "32x2/64/4", 8), (128, "64x2/64/4", 4)]
+EXACT_SHAPES += [(64 * _k, f"64x{_k}/64/2", 2) for _k in (3, 4, 5, 6, 7, 8, 9, 10, 12)]
+EXACT_SHAPES += [(128 * _k, f"128x{_k}/128/2", 2) for _k in (7, 8)] + [(256 * _k, f"256x{_k}/256/2", 2) for _k in (5, 6, 7, 8)]
+EXACT = []
+for _vectors, _shape, _block in EXACT_SHAPES:
+    _rows = -((-10 << 20) // (16 * _vectors * _block)) * _block   # the fewest whole blocks of 10 MiB
+    for _operator in ("layer", "rms"):
+        if (_operator, _vectors) != ("rms", 256):                 # norm.hip's
+            EXACT += [(_operator, _tag, _rows, _vectors * (4 if _tag == "f32" else 8), f"norm_rows_exact/{_operator}/{_shape}", _block)
+                      for _tag in ("f32", "bf16")]
+
 reached = set()
 
 
-def run_case(operator, tag, weight_tag, rows, width, label, parameters, seed):
-    """parameters: 0 none, 1 scale, 2 scale and bias (LayerNorm only)."""
+def run_case(operator, tag, weight_tag, rows, width, label, parameters, seed, distinct=None):
+    """parameters: 0 none, 1 scale, 2 scale and bias (LayerNorm only).  distinct: that many rows over and over, the first of
+    each held against the oracle and the others against those, bit by bit (a row's sums do not depend on its place)."""
     oid, wid = TYPES[tag][1], TYPES[weight_tag][1]
     rng = np.random.default_rng(seed)
-    values = (rng.normal(0, 1, (rows, width)) * rng.uniform(0.1, 10, (rows, 1))).astype(np.float32)
+    own = distinct or rows
+    values = (rng.normal(0, 1, (own, width)) * rng.uniform(0.1, 10, (own, 1))).astype(np.float32)
     if rows > 1 and operator == "rms":
         values[1] = 2.0   # a constant row (tests/compute_provider_native/normalization_test.cc:186-199)
     xs = host_values(values, tag)
@@ -217,6 +233,8 @@ def run_case(operator, tag, weight_tag, rows, width, label, parameters, seed):
     bias = host_values(rng.normal(0, 0.5, width).astype(np.float32), weight_tag)
     note(f"{operator} norm {tag}/{weight_tag} [{rows}, {width}] parameters={parameters}: expecting {label}")
     operands = [to_device(xs, tag)]
+    if distinct:
+        operands[0] = operands[0].repeat(((rows + own - 1) // own, 1))[:rows].contiguous()
     if parameters >= 1:
         operands.append(to_device(scale, weight_tag))
     if parameters == 2:
@@ -229,9 +247,15 @@ def run_case(operator, tag, weight_tag, rows, width, label, parameters, seed):
         want = orc.layer_norm(oid, xs, scale if parameters else None, bias if parameters == 2 else None, 1e-5,
                               param_type=wid if parameters else None)
     chosen = hc.last_launch_variant()
-    assert chosen == label, f"{operator} [{rows}, {width}] {tag}: launched {chosen}, the table says {label}"
-    reached.add(chosen)
-    got = to_host(out)
+    if label is None:
+        assert not chosen.startswith("norm_rows_exact"), f"{operator} [{rows}, {width}] {tag}: launched {chosen}"
+    else:
+        assert chosen == label, f"{operator} [{rows}, {width}] {tag}: launched {chosen}, the table says {label}"
+        reached.add(chosen)
+    if distinct:
+        bits = out.view(torch.int32 if tag == "f32" else torch.int16)
+        assert torch.equal(bits[own:], bits[:-own]), f"{operator} [{rows}, {width}] {tag}: equal rows, other results"
+    got = to_host(out[:own])
     if operator == "layer":
         layer_bar(got, want, tag, bias if parameters == 2 else None)
     elif tag == "f32":
@@ -251,11 +275,23 @@ def test_norm_case_reaches_its_launch_shape_and_matches_the_oracle(case):
         run_case(operator, "f16", "f16", rows, width, label, 1, seed + 8)
 
 
+@pytest.mark.parametrize("case", EXACT, ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}x{c[3]}")
+def test_norm_exact_shapes_serve_from_10_mib_on(case):
+    operator, tag, rows, width, label, block = case
+    seed = 5000 + EXACT.index(case)
+    forms = [(tag, tag, parameters) for parameters in ((0, 1) if operator == "rms" else (0, 1, 2))]
+    if tag == "bf16":
+        forms += [("bf16", "f32", 2 if operator == "layer" else 1), ("f16", "f16", 1)]
+    for form, (own_tag, weight_tag, parameters) in enumerate(forms):
+        run_case(operator, own_tag, weight_tag, rows, width, label, parameters, seed + form, distinct=61)
+    run_case(operator, tag, tag, rows - block, width, None, 1, seed, distinct=61)
+
+
 def test_every_norm_launch_shape_in_the_library_is_reached():
     """Runs after the cases above (file order): a norm launch shape compiled into the library that no
     case reached is either dead code or an untested kernel."""
     compiled = {label for label in hc.launch_variants() if label.startswith("norm")}
-    tabled = {case[4] for case in CASES}
+    tabled = {case[4] for case in CASES + EXACT}
     assert compiled == tabled, f"not in the table: {sorted(compiled - tabled)}; not in the library: {sorted(tabled - compiled)}"
     if reached:
         assert tabled <= reached, f"tabled but not reached: {sorted(tabled - reached)}"
