@@ -54,8 +54,8 @@ template <bool kLayer> struct GenericTag {
   static std::string text() { return std::string("norm_generic/") + (kLayer ? "layer" : "rms"); }
 };
 
-// kExactElsewhere: whenever this shape would cover the tensor exactly, a shape of norm_exact.h has
-// already taken the launch (same width, a row count it divides), so no exact form is built here.
+// kExactElsewhere: whenever this shape would cover the tensor exactly, norm_exact.h (from 10 MiB on, the same width, a row
+// count it divides) or norm_tail.h has already taken the launch, so no exact form is built here.
 template <class T, class W, bool kLayer, int kLanes, int kVpl, int kThreads = kBlockThreads, int kRows = 1,
           bool kExactElsewhere = false>
 hipError_t run_rows(const NormParams &p, const Bound &io, int parameters, hipStream_t s) {
@@ -108,10 +108,11 @@ hipError_t run(const NormParams &p, const Bound &io, bool vectorised, hipStream_
       // LayerNorm 11.3 us in blocks of one wave (11.5-11.8 us in blocks of 2-8 waves, 12.2 us
       // with four rows per wave, 13.5 us with one, 14.3 us for two waves per row); RMSNorm
       // 11.2 us in blocks of four waves (11.6-11.9 us for two waves per row).
-      if constexpr (kLayer) return run_rows<T, W, kLayer, 64, 4, 64, 2, true>(p, io, parameters, s);
-      else return run_rows<T, W, kLayer, 64, 4, 256, 2>(p, io, parameters, s);
+      // (a LayerNorm of f32 of this width is norm_tail.h's at any number of rows)
+      if constexpr (!kLayer) return run_rows<T, W, kLayer, 64, 4, 256, 2>(p, io, parameters, s);
+      else if constexpr (Traits<T>::kSize == 2) return run_rows<T, W, kLayer, 64, 4, 64, 2, true>(p, io, parameters, s);
     }
-    if (vectors <= 512) return run_rows<T, W, kLayer, 256, 2, 256, 2, true>(p, io, parameters, s);
+    // (257 to 512 vectors are norm_tail.h's at any number of rows)
     if (vectors <= 1024) return run_rows<T, W, kLayer, 256, 4>(p, io, parameters, s);
     if (vectors <= 2048) return run_rows<T, W, kLayer, 256, 8>(p, io, parameters, s);
     if (vectors <= 4096) return run_rows<T, W, kLayer, 1024, 4, 1024>(p, io, parameters, s);

@@ -25,12 +25,13 @@ namespace {
 // Too few rows for the waves of a row to be better spent on other rows: a row of more than 256 vectors is 256 lanes'
 // there (us, there / here: RMSNorm bf16 [5, 5120] 2.5 / 2.7, [1, 5120] 2.4 / 2.5; LayerNorm f32 [16, 3000] 2.9 / 2.75).
 // Up to 512 vectors a row is a wave's here however few there are, there of two rows: RMSNorm bf16 [1, 2048] 2.55 / 2.0, f32
-// [1, 1024] 2.3 / 1.9, bf16 [5, 2560] 2.8 / 2.2, f32 [15, 1280] 3.0 / 2.2, [2, 2048] 2.5 / 2.1, LayerNorm f32 [15, 1792] 3.2 / 2.3.  (Three rows are what the tests of the masked shapes have.)
+// [1, 1024] 2.3 / 1.9, bf16 [5, 2560] 2.8 / 2.2, f32 [15, 1280] 3.0 / 2.2, [2, 2048] 2.5 / 2.1, LayerNorm f32 [15, 1792] 3.2 / 2.3;
+// one after another in a graph RMSNorm bf16 [3, 2048] 2.7 / 1.8, [3, 4096] 2.4 / 2.2, LayerNorm f32 [3, 1024] 2.7 / 1.7.
 // Rows of narrow elements of nine vectors a lane and more are the masked shapes' from 32 rows up to as many as a wave for each
 // vector wants (bf16 [64, 5600] 3.0 / 3.25, [501, 4112] 3.95 / 4.1, [700, 5600] 4.3 / 4.55, [1000, 5600] 5.4 / 5.2).
 inline bool enough_rows(uint64_t rows, uint32_t per_lane, int size) {
   if (size == 2 && per_lane >= 9 && rows >= 32 && rows < 64u * per_lane) return false;
-  return per_lane <= 8 ? rows != 3 : rows >= 16;
+  return per_lane <= 8 || rows >= 16;
 }
 
 template <bool kLayer, int kVpl, int kThreads, int kRows> struct TailTag {

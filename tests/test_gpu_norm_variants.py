@@ -38,9 +38,9 @@ CASES = [
     ("layer", "f32", 3, 116, "norm_rows/layer/32x1/256/1/ragged"),
     ("layer", "f32", 4, 256, "norm_rows/layer/64x1/256/1/exact"),
     ("layer", "f32", 3, 244, "norm_rows/layer/64x1/256/1/ragged"),
-    ("layer", "f32", 3, 500, "norm_rows/layer/64x2/256/2/ragged"),
-    ("layer", "f32", 3, 768, "norm_rows/layer/64x4/64/2/ragged"),
-    ("layer", "f32", 3, 1280, "norm_rows/layer/256x2/256/2/ragged"),
+    ("layer", "f32", 3, 500, "norm_rows_tail/layer/64x2/256/1"),
+    ("layer", "f32", 3, 768, "norm_rows_tail/layer/64x3/64/1"),
+    ("layer", "f32", 3, 1280, "norm_rows_tail/layer/64x5/64/1"),
     ("layer", "f32", 3, 4096, "norm_rows/layer/256x4/256/1/exact"),
     ("layer", "f32", 3, 2304, "norm_rows/layer/256x4/256/1/ragged"),
     ("layer", "f32", 3, 8192, "norm_rows/layer/256x8/256/1/exact"),
@@ -54,9 +54,9 @@ CASES = [
     ("rms", "f32", 3, 52, "norm_rows/rms/16x1/256/1/ragged"),
     ("rms", "f32", 3, 116, "norm_rows/rms/32x1/256/1/ragged"),
     ("rms", "f32", 3, 244, "norm_rows/rms/64x1/256/1/ragged"),
-    ("rms", "f32", 3, 500, "norm_rows/rms/64x2/256/2/ragged"),
-    ("rms", "f32", 3, 768, "norm_rows/rms/64x4/256/2/ragged"),
-    ("rms", "f32", 3, 1280, "norm_rows/rms/256x2/256/2/ragged"),
+    ("rms", "f32", 3, 500, "norm_rows_tail/rms/64x2/256/1"),
+    ("rms", "f32", 3, 768, "norm_rows_tail/rms/64x3/64/1"),
+    ("rms", "f32", 3, 1280, "norm_rows_tail/rms/64x5/64/1"),
     ("rms", "f32", 3, 2304, "norm_rows/rms/256x4/256/1/ragged"),
     ("rms", "f32", 3, 5120, "norm_rows/rms/256x8/256/1/ragged"),
     ("rms", "f32", 3, 16372, "norm_rows/rms/1024x4/1024/1/ragged"),
@@ -107,9 +107,9 @@ CASES = [
     ("layer", "bf16", 3, 232, "norm_rows/layer/32x1/256/1/ragged"),
     ("layer", "bf16", 4, 512, "norm_rows/layer/64x1/256/1/exact"),
     ("layer", "bf16", 3, 488, "norm_rows/layer/64x1/256/1/ragged"),
-    ("layer", "bf16", 3, 1000, "norm_rows/layer/64x2/256/2/ragged"),
-    ("layer", "bf16", 3, 1536, "norm_rows/layer/64x4/64/2/ragged"),
-    ("layer", "bf16", 3, 2560, "norm_rows/layer/256x2/256/2/ragged"),
+    ("layer", "bf16", 3, 1000, "norm_rows_tail/layer/64x2/256/1"),
+    ("layer", "bf16", 3, 1536, "norm_rows_tail/layer/64x3/64/1"),
+    ("layer", "bf16", 3, 2560, "norm_rows_tail/layer/64x5/64/1"),
     ("layer", "bf16", 3, 8192, "norm_rows/layer/256x4/256/1/exact"),
     ("layer", "bf16", 3, 4608, "norm_rows/layer/256x4/256/1/ragged"),
     ("layer", "bf16", 3, 16384, "norm_rows/layer/256x8/256/1/exact"),
@@ -123,9 +123,9 @@ CASES = [
     ("rms", "bf16", 3, 104, "norm_rows/rms/16x1/256/1/ragged"),
     ("rms", "bf16", 3, 232, "norm_rows/rms/32x1/256/1/ragged"),
     ("rms", "bf16", 3, 488, "norm_rows/rms/64x1/256/1/ragged"),
-    ("rms", "bf16", 3, 1000, "norm_rows/rms/64x2/256/2/ragged"),
-    ("rms", "bf16", 3, 1536, "norm_rows/rms/64x4/256/2/ragged"),
-    ("rms", "bf16", 3, 2560, "norm_rows/rms/256x2/256/2/ragged"),
+    ("rms", "bf16", 3, 1000, "norm_rows_tail/rms/64x2/256/1"),
+    ("rms", "bf16", 3, 1536, "norm_rows_tail/rms/64x3/64/1"),
+    ("rms", "bf16", 3, 2560, "norm_rows_tail/rms/64x5/64/1"),
     ("rms", "bf16", 3, 4608, "norm_rows/rms/256x4/256/1/ragged"),
     ("rms", "bf16", 3, 10240, "norm_rows/rms/256x8/256/1/ragged"),
     ("rms", "bf16", 3, 32744, "norm_rows/rms/1024x4/1024/1/ragged"),
