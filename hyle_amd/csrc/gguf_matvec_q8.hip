@@ -1460,12 +1460,13 @@ inline bool rows_of_vectors_serve(const MatVecParams &p) {
 // the row stride are multiples of 16 bytes.  MI355X, bf16, us, the kernels here / strips:
 //   several activation rows: nearly everywhere, since a compute unit quantises them once.  Q8_0 [2048 -> 16384]
 //   x 2 15.8 / 9.5, [6144 -> 2048] x 5 12.2 / 9.5, Q6_K [1024 -> 2048] x 8 12.2 / 5.0, [2048 -> 6144] x 2 8.1 / 6.1,
-//   Q4_K [1024 -> 2048] x 4 5.2 / 3.6, [6144 -> 2048] x 4 12.9 / 6.7, [1536 -> 20000] x 2 10.5 / 7.1, [2048 -> 60000] x 4
-//   19.9 / 18.0.  Not a vocabulary of one span, whose codes the tile and quad kernels keep at hand: Q4_K [2048 -> 151936]
-//   x 2 38.8 / 39.5, x 5 55.0 / 53.5, two rows of Q6_K 54.3 / 57.2 (three 62.1 / 55.7, four 59.4 / 53.3, [2048 -> 91000] x 4
-//   39.0 / 34.4); nor two rows far wider than the weight is high, Q8_0
-//   [16384 -> 1024] 10.1 / 11.4.  (Two to four rows against 6144 to 8999 Q4_K rows of up to 2048 values stay with the tiles
-//   that the tests of this rule name there, 7.3 / 5.2 at [2048 -> 6144] x 4.)
+//   Q4_K [1024 -> 2048] x 4 5.2 / 3.6, [6144 -> 2048] x 4 12.9 / 6.7, [2048 -> 6144] x 4 6.3 / 5.0, [1536 -> 8192] x 3 5.7 / 5.5,
+//   [2048 -> 32000] x 2 13.2 / 9.9.  Not the vocabularies whose codes the tile and quad kernels keep at hand: two to four rows
+//   of Q4_K from about 115 M products on ([2048 -> 45000] x 2 13.5 / 13.2, [2048 -> 60000] x 2 16.7 / 17.3, [1536 -> 151936] x 2
+//   27.6 / 30.0), of five blocks or fewer from 150 M ([1280 -> 89999] x 3 16.3 / 15.8, [1280 -> 151936] x 3 23.6 / 24.8), and five
+//   to eight rows against one span of 90000 rows and more, which are alike ([2048 -> 151936] x 5 43.7 / 43.0); two rows of one span of Q6_K,
+//   [2048 -> 151936] 54.3 / 57.2 (three 62.1 / 55.7, four 59.4 / 53.3, [2048 -> 91000] x 4 39.0 / 34.4); nor two rows far wider than
+//   the weight is high, Q8_0 [16384 -> 1024] 10.1 / 11.4.
 //   one row, where the alternative walks block by block, from 8 M products on, and from 4 M where a row is wide:
 //   Q6_K [2560 -> 9728] 11.6 / 7.9, [5120 -> 5120] 11.8 / 9.0 ([1024 -> 2048] 4.2 / 4.2)
 //   one row of Q4_K tiles: rows of 10240 values or more, [14080 -> 3328] 13.7 / 9.6; widths that are no multiple of 2048
@@ -1476,8 +1477,8 @@ inline bool rows_of_vectors_serve(const MatVecParams &p) {
 bool strips_better(const MatVecParams &p, bool vectors) {
   if (!gguf_matvec_strips_serve(p)) return false;
   const bool whole = vectors && rows_of_vectors_serve(p);
+  const uint64_t products = p.rows * p.k;
   if (p.m == 1) {
-    const uint64_t products = p.rows * p.k;
     if (!whole) return products >= 8000000 || (products >= 4000000 && p.k >= 2048);
     if (p.kind != 0) return false;
     return p.k >= 10240 || (p.k > 2048 && p.k % 2048 != 0 && (p.rows <= 4096 || p.k >= p.rows)) ||
@@ -1486,7 +1487,7 @@ bool strips_better(const MatVecParams &p, bool vectors) {
   if (!whole) return true;
   // one span of a vocabulary: the tile and quad kernels keep its codes at hand and have no tiles left over
   const bool span_of_many = p.k == 2048 && p.rows >= 90000;
-  if (p.kind == 0) return p.k > 2048 || (!span_of_many && (p.m > 4 || p.rows < 6144 || p.rows >= 9000)) ;
+  if (p.kind == 0) return p.k > 2048 || (p.m > 4 ? !span_of_many : products <= (p.k <= 1280 ? 150000000u : 115000000u));
   if (p.kind == 1 && p.m <= 2 && span_of_many) return false;
   return p.m > 2 || p.k < 8 * p.rows;
 }

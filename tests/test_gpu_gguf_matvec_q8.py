@@ -394,8 +394,8 @@ def test_q8_route_products_that_changed_kernels(tag, x_tag, rows, k, m):
 
 
 def test_q8_route_q4_k_tiles_seeded_random_shapes_of_what_they_serve():
-    """Sixty seeded draws over every range of rows, widths and activation rows in which the tile kernel is taken: few weight
-    rows of any width, one row up to 8192 values wide, and narrow rows, many of them, against two to four."""
+    """Sixty seeded draws over ranges of rows, widths and activation rows of the tile kernel and next to them: few weight
+    rows of any width, one row up to 8192 values wide, and narrow rows, many of them, against two to four (the strip kernel)."""
     rng = np.random.default_rng(1814)
     for case in range(60):
         form = case % 3
@@ -416,7 +416,8 @@ def test_q8_route_q4_k_tiles_seeded_random_shapes_of_what_they_serve():
         x = rng.normal(0, 1.5, (m, k) if m > 1 else (k,)).astype(np.float32)
         note(f"q8 matvec q4_k tiles draw {case}: rows {rows} k {k} m {m} x {x_tag} pad {pad}")
         check("q4_k", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad)
-        assert hc.last_launch_variant().startswith(f"gguf_matvec_q8_tiles/q4_k/{tokens}-tokens"), (hc.last_launch_variant(), rows, k, m)
+        kernel = "strips/q4_k/4-tokens" if form == 2 else f"tiles/q4_k/{tokens}-tokens"
+        assert hc.last_launch_variant().startswith("gguf_matvec_q8_" + kernel), (hc.last_launch_variant(), rows, k, m)
 
 
 @pytest.mark.parametrize("x_tag", ["f32", "bf16", "f16"])
