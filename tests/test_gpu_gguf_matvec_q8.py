@@ -135,14 +135,14 @@ def test_q8_route_the_reference_s_own_projection_shapes():
     """The shapes of the reference's Q8_0 / Q4_K projection cases
     (tests/compute_models/cpu_c5_gguf_inputs.h:231,237,259,287,314): none is a multiple of 2048 wide.
     The Q8_0 ones of 256 n values take the span kernel with a short last span (128 values: the kernel
-    that walks a row block by block), the Q4_K one the matrix-unit kernel."""
+    that walks a row block by block), the Q4_K one the strip kernel (more rows than values)."""
     rng = np.random.default_rng(1803)
     for tag, k, rows in (("q8_0", 1024, 32768), ("q4_k", 5120, 10240), ("q8_0", 7168, 3072), ("q8_0", 17408, 5120),
                          ("q8_0", 128, 512)):
         raw = weights_for(tag, rng, rows, k)
         x = rng.normal(0, 1.5, (k,)).astype(np.float32)
         note(f"q8 matvec {tag} [{k} -> {rows}], one activation row")
-        kernel = {1024: "gguf_matvec_q8_spans/q8_0/1-spans/short", 5120: "gguf_matvec_q8_tiles/q4_k/1-tokens",
+        kernel = {1024: "gguf_matvec_q8_spans/q8_0/1-spans/short", 5120: "gguf_matvec_q8_strips/q4_k/4-tokens",
                   7168: "gguf_matvec_q8_spans/q8_0/4-spans/short", 17408: "gguf_matvec_q8_spans/q8_0/9-spans/short",
                   128: "gguf_matvec_q8_blocks/q8_0/1-tokens"}[k]
         check(tag, "f32", raw, rows, k, x, kernel=kernel)
@@ -266,7 +266,7 @@ def test_q8_route_q4_k_matrix_unit_widths_tokens_and_shared_tiles(x_tag):
             x[m - 1, 256:512] = 0.0
         tokens = 1 if m == 1 else (4 if m <= 4 else 8)
         note(f"q8 matvec q4_k tiles x {x_tag} rows {rows} k {k} m {m}")
-        family = "strips" if (rows, m) in ((600, 2), (2100, 1)) else "tiles"   # many weight rows: the strip kernel
+        family = "strips" if (rows, m) in ((600, 2), (2100, 1), (10240, 1)) else "tiles"   # many weight rows: the strip kernel
         check("q4_k", x_tag, raw, rows, k, x, kernel=f"gguf_matvec_q8_{family}/q4_k/{4 if family == 'strips' else tokens}-tokens")
     note("q8 matvec q4_k: fewer than four blocks per row, an odd row stride and unaligned activations keep the block-walking kernel")
     raw = raw_bytes_for("q4_k", rng, 20, 768)
@@ -324,7 +324,7 @@ def test_q8_route_q4_k_matrix_unit_seeded_random_shapes():
         padded[:, :raw.shape[1]] = raw
         x = rng.normal(0, 1.5, (m, k) if m > 1 else (k,)).astype(np.float32)
         note(f"q8 matvec q4_k tiles draw {case}: rows {rows} k {k} m {m} x {x_tag} pad {pad}")
-        strips = rows >= 512 and (m > 1 or k >= 10240 or (k > 2048 and k % 2048 != 0))   # several rows or wide ones against many
+        strips = rows >= 512 and (m > 1 or k >= 10240 or (k > 2048 and k % 2048 != 0) or rows > k)   # several rows or wide ones against many
         kernel = f"gguf_matvec_q8_strips/q4_k/{4 if m <= 4 else 8}-tokens" if strips else f"gguf_matvec_q8_tiles/q4_k/{tokens}-tokens"
         check("q4_k", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad, kernel=kernel)
 
@@ -395,7 +395,8 @@ def test_q8_route_products_that_changed_kernels(tag, x_tag, rows, k, m):
 
 def test_q8_route_q4_k_tiles_seeded_random_shapes_of_what_they_serve():
     """Sixty seeded draws over ranges of rows, widths and activation rows of the tile kernel and next to them: few weight
-    rows of any width, one row up to 8192 values wide, and narrow rows, many of them, against two to four (the strip kernel)."""
+    rows of any width, one row up to 8192 values wide (against more weight rows than that the strip kernel), and narrow rows,
+    many of them, against two to four (the strip kernel)."""
     rng = np.random.default_rng(1814)
     for case in range(60):
         form = case % 3
@@ -416,7 +417,7 @@ def test_q8_route_q4_k_tiles_seeded_random_shapes_of_what_they_serve():
         x = rng.normal(0, 1.5, (m, k) if m > 1 else (k,)).astype(np.float32)
         note(f"q8 matvec q4_k tiles draw {case}: rows {rows} k {k} m {m} x {x_tag} pad {pad}")
         check("q4_k", x_tag, padded, rows, k, x, row_stride=raw.shape[1] + pad)
-        kernel = "strips/q4_k/4-tokens" if form == 2 else f"tiles/q4_k/{tokens}-tokens"
+        kernel = "strips/q4_k/4-tokens" if form == 2 or (form == 1 and rows > k) else f"tiles/q4_k/{tokens}-tokens"
         assert hc.last_launch_variant().startswith("gguf_matvec_q8_" + kernel), (hc.last_launch_variant(), rows, k, m)
 
 
@@ -448,10 +449,11 @@ def test_q8_route_activation_blocks_on_both_sides_of_the_short_form(tag, rows, k
 
 @pytest.mark.parametrize("x_tag", ["f32", "bf16"])
 def test_q8_route_q4_k_tiles_of_eight_rows(x_tag):
-    """Few rows of six groups of four blocks or more: a tile has eight rows, on both sides of its edges and of the rule."""
+    """Few rows of six groups of four blocks or more: a tile has eight rows, on both sides of its edges and of the rule
+    (the last shape, of more than 100 M products, is too many for the strip kernel)."""
     rng = np.random.default_rng(1828)
     for rows, k, form in ((1, 6144, "#8-rows"), (7, 6144, "#8-rows"), (8, 5376, "#8-rows"), (9, 8192, "#8-rows"), (17, 9984, "/long#8-rows"), (511, 8448, "/long#8-rows"),
-                          (2048, 6144, "#8-rows"), (2049, 6144, ""), (2048, 4096, ""), (33, 5120, ""), (8450, 8448, "/long")):
+                          (2048, 6144, "#8-rows"), (2049, 6144, ""), (2048, 4096, ""), (33, 5120, ""), (12000, 8448, "/long")):
         note(f"q8 matvec q4_k tiles x {x_tag} rows {rows} k {k}: 1-tokens{form}")
         check("q4_k", x_tag, raw_bytes_for("q4_k", rng, rows, k), rows, k, rng.normal(0, 1.5, k).astype(np.float32), kernel="gguf_matvec_q8_tiles/q4_k/1-tokens")
         assert last_launch_form() == f"gguf_matvec_q8_tiles/q4_k/1-tokens{form}"

@@ -92,7 +92,7 @@ def test_strips_decoded_q8_0_off_a_boundary_in_every_form():
     ("q8_0", 4096, 8192, 4, "strips/q8_0/4"), ("q8_0", 16384, 1024, 2, "lines/q8_0/2"), ("q6_k", 6144, 8192, 4, "strips/q6_k/4"),
     ("q6_k", 6144, 511, 2, "quads/q6_k/4"), ("q6_k", 2304, 2304, 1, "strips/q6_k/4"), ("q6_k", 4096, 8192, 1, "spans/q6_k/2"),
     ("q4_k", 4096, 4096, 2, "strips/q4_k/4"), ("q4_k", 2048, 8192, 4, "strips/q4_k/4"), ("q4_k", 2048, 8192, 5, "strips/q4_k/8"),
-    ("q4_k", 3840, 4096, 1, "strips/q4_k/4"), ("q4_k", 2560, 5120, 1, "tiles/q4_k/1"), ("q4_k", 10240, 16384, 1, "strips/q4_k/4")])
+    ("q4_k", 3840, 4096, 1, "strips/q4_k/4"), ("q4_k", 2560, 5120, 1, "strips/q4_k/4"), ("q4_k", 10240, 16384, 1, "strips/q4_k/4")])
 def test_strips_rule(tag, k, rows, m, kernel):
     rng = np.random.default_rng(1821)
     note(f"q8 matvec rule {tag} rows {rows} k {k} m {m}")
@@ -143,11 +143,15 @@ def test_strips_every_layout_of_a_launch(tag):
         assert np.array_equal(got, np.take(got, np.arange(rows) % period, 1))
 
 
-# Q4_K products of more than twice as many rows as values, and of two to four activation rows up to 115 or 150 M products
+# Q4_K products on both sides of the limits: more rows than values up to 64, 80 or 100 M products, two to four activation rows up
+# to 115 or 150 M
 @pytest.mark.parametrize("x_tag,k,rows,m,kernel", [
-    ("bf16", 2048, 6001, 1, "strips"), ("bf16", 2048, 6000, 1, "tiles"), ("f32", 2816, 5633, 1, "tiles"), ("f32", 3072, 6145, 1, "strips"),
-    ("f16", 3072, 6144, 1, "tiles"), ("bf16", 1024, 97656, 1, "strips"), ("bf16", 1024, 97657, 1, "tiles"), ("f32", 2048, 9000, 2, "strips"),
+    ("bf16", 2048, 6001, 1, "strips"), ("bf16", 2048, 6000, 1, "strips"), ("f32", 2816, 5633, 1, "strips"), ("f32", 3072, 6145, 1, "strips"),
+    ("f16", 3072, 6144, 1, "strips"), ("bf16", 1024, 97656, 1, "tiles"), ("bf16", 1024, 97657, 1, "tiles"), ("f32", 2048, 9000, 2, "strips"),
     ("bf16", 1280, 9000, 4, "strips"), ("f16", 2048, 8999, 3, "strips"), ("bf16", 2048, 89999, 2, "tiles"), ("bf16", 2048, 90000, 2, "tiles"),
+    ("bf16", 2048, 2049, 1, "strips"), ("f32", 2048, 2048, 1, "tiles"), ("f16", 1024, 1025, 1, "strips"), ("bf16", 1024, 1024, 1, "tiles"),
+    ("bf16", 4096, 4097, 1, "strips"), ("bf16", 4096, 4096, 1, "tiles"), ("bf16", 2048, 31250, 1, "strips"), ("f32", 2048, 31251, 1, "tiles"),
+    ("bf16", 4096, 19531, 1, "strips"), ("bf16", 4096, 19532, 1, "tiles"), ("bf16", 5120, 19531, 1, "strips"), ("bf16", 5120, 19532, 1, "tiles"),
     ("f32", 2048, 6144, 2, "strips"), ("bf16", 2048, 6143, 3, "strips"), ("f16", 1024, 7000, 4, "strips"), ("bf16", 2048, 6144, 4, "strips"),
     ("bf16", 2048, 56152, 2, "strips"), ("bf16", 2048, 56153, 4, "tiles"), ("bf16", 1280, 117187, 3, "strips"), ("bf16", 1280, 117188, 2, "tiles")])
 def test_strips_rule_for_many_rows_of_q4_k(x_tag, k, rows, m, kernel):
