@@ -208,13 +208,14 @@ CASES += [("rms", "f32", 2, 2048, "norm_rows_tail/rms/64x8/64/1"), ("layer", "bf
 EXACT_SHAPES = [(16, "8x2/64/4", 32), (32, "16x2/64/4", 16), (64, "32x2/64/4", 8), (128, "64x2/64/4", 4)]
 EXACT_SHAPES += [(64 * _k, f"64x{_k}/64/2", 2) for _k in (3, 4, 5, 6, 7, 8, 9, 10, 12)]
 EXACT_SHAPES += [(128 * _k, f"128x{_k}/128/2", 2) for _k in (7, 8)] + [(256 * _k, f"256x{_k}/256/2", 2) for _k in (5, 6, 7, 8)]
-EXACT = []
+EXACT_BLOCKS = {}   # case: rows to a block
 for _vectors, _shape, _block in EXACT_SHAPES:
     _rows = -((-10 << 20) // (16 * _vectors * _block)) * _block   # the fewest whole blocks of 10 MiB
     for _operator in ("layer", "rms"):
         if (_operator, _vectors) != ("rms", 256):                 # norm.hip's
-            EXACT += [(_operator, _tag, _rows, _vectors * (4 if _tag == "f32" else 8), f"norm_rows_exact/{_operator}/{_shape}", _block)
-                      for _tag in ("f32", "bf16")]
+            EXACT_BLOCKS.update({(_operator, _tag, _rows, _vectors * (4 if _tag == "f32" else 8), f"norm_rows_exact/{_operator}/{_shape}"): _block
+                                 for _tag in ("f32", "bf16")})
+CASES += list(EXACT_BLOCKS)
 
 reached = set()
 
@@ -266,32 +267,24 @@ def run_case(operator, tag, weight_tag, rows, width, label, parameters, seed, di
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}x{c[3]}")
 def test_norm_case_reaches_its_launch_shape_and_matches_the_oracle(case):
+    """An exact shape at the fewest rows that it serves, of which 61 are distinct, leaves a block's rows fewer to another."""
     operator, tag, rows, width, label = case
     seed = 3000 + CASES.index(case)
+    distinct = 61 if case in EXACT_BLOCKS else None
     for parameters in ((0, 1) if operator == "rms" else (0, 1, 2)):
-        run_case(operator, tag, tag, rows, width, label, parameters, seed + parameters)
+        run_case(operator, tag, tag, rows, width, label, parameters, seed + parameters, distinct)
     if tag == "bf16":   # f32 parameters under narrow storage (the cast + norm + cast of the decoder graph), and f16
-        run_case(operator, "bf16", "f32", rows, width, label, 2 if operator == "layer" else 1, seed + 7)
-        run_case(operator, "f16", "f16", rows, width, label, 1, seed + 8)
-
-
-@pytest.mark.parametrize("case", EXACT, ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}x{c[3]}")
-def test_norm_exact_shapes_serve_from_10_mib_on(case):
-    operator, tag, rows, width, label, block = case
-    seed = 5000 + EXACT.index(case)
-    forms = [(tag, tag, parameters) for parameters in ((0, 1) if operator == "rms" else (0, 1, 2))]
-    if tag == "bf16":
-        forms += [("bf16", "f32", 2 if operator == "layer" else 1), ("f16", "f16", 1)]
-    for form, (own_tag, weight_tag, parameters) in enumerate(forms):
-        run_case(operator, own_tag, weight_tag, rows, width, label, parameters, seed + form, distinct=61)
-    run_case(operator, tag, tag, rows - block, width, None, 1, seed, distinct=61)
+        run_case(operator, "bf16", "f32", rows, width, label, 2 if operator == "layer" else 1, seed + 7, distinct)
+        run_case(operator, "f16", "f16", rows, width, label, 1, seed + 8, distinct)
+    if case in EXACT_BLOCKS:
+        run_case(operator, tag, tag, rows - EXACT_BLOCKS[case], width, None, 1, seed, distinct)
 
 
 def test_every_norm_launch_shape_in_the_library_is_reached():
     """Runs after the cases above (file order): a norm launch shape compiled into the library that no
     case reached is either dead code or an untested kernel."""
     compiled = {label for label in hc.launch_variants() if label.startswith("norm")}
-    tabled = {case[4] for case in CASES + EXACT}
+    tabled = {case[4] for case in CASES}
     assert compiled == tabled, f"not in the table: {sorted(compiled - tabled)}; not in the library: {sorted(tabled - compiled)}"
     if reached:
         assert tabled <= reached, f"tabled but not reached: {sorted(tabled - reached)}"
