@@ -54,6 +54,14 @@ def current_stream_handle(device=None) -> int:
 _BINDINGS = (list, tuple)
 
 
+def _tensor_launcher():
+    """capi.tensor_launcher on torch's current stream; None where torch offers no bare handle, has not initialised the
+    device yet, or the extension was not built."""
+    if _raw_stream is None or not torch.cuda.is_initialized():
+        return None
+    return hc.capi.tensor_launcher(_current_device, _raw_stream)
+
+
 class Bound:
     """A prepared operation with its workspace, ready to be submitted repeatedly."""
 
@@ -66,7 +74,7 @@ class Bound:
         ptr = self.workspace.data_ptr() if self.workspace is not None else 0
         self.invocation = self.prepared.create_invocation(ptr, req.size)
         self.device = device
-        self._launch = None
+        self._launch = _tensor_launcher()  # (here and not at the first submit, which is the only one that some programs make)
 
     def outputs(self) -> list:
         return [empty_like_desc(d, self.device) for d in self.prepared.output_descriptions()]
@@ -80,8 +88,8 @@ class Bound:
             if code != hc.capi.OK:
                 hc._check(code)
             return
-        if launch is None and _raw_stream is not None and torch.cuda.is_initialized():
-            self._launch = hc.capi.tensor_launcher(_current_device, _raw_stream)
+        if launch is None:
+            self._launch = _tensor_launcher()
         handle = current_stream_handle() if stream is None else stream
         self.invocation.submit(handle, [t.data_ptr() for t in inputs], [t.data_ptr() for t in outputs])
 

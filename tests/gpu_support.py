@@ -78,9 +78,11 @@ def _noting(submit):
     return noted
 
 
-# every launch a GPU test makes goes through one of these two, whichever helper it uses
+# every launch a GPU test makes goes through one of these, whichever helper it uses (a Bound's without a stream of the
+# caller's go past the invocation)
 hc.OperationInvocation.submit = _noting(hc.OperationInvocation.submit)
 hc.OperationInvocation.submit_without_workspace = _noting(hc.OperationInvocation.submit_without_workspace)
+tio.Bound.submit = _noting(tio.Bound.submit)
 
 
 def run(operation, *tensors, descs=None, outputs=None):
