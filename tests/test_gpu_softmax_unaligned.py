@@ -9,8 +9,7 @@ import torch
 
 from hyle_amd import compute as hc
 
-from gpu_support import DEVICE, TYPES, note, run
-from gpu_support import last_launch_form
+from gpu_support import DEVICE, TYPES, last_launch_form, note, run
 from test_gpu_softmax_variants import MASKS, compare_on_device, make_inputs, oracle_softmax
 
 pytestmark = pytest.mark.gpu
@@ -110,3 +109,29 @@ def test_heads_that_share_a_mask_row(tag, heads, q, width, mask_word, shape):
         for other_heads, rows in ((4, q - 2), (2, 2 * q)):
             check(tag, rows, width, mask_word, shape, False, False, in_place=False, heads=other_heads)
             assert not last_launch_form().endswith("#shared")
+
+
+@pytest.mark.parametrize("tag,mask_word,q,width,shape", [("bf16", "additive", 2036, 3073, "128x4/256"), ("f32", "boolean", 2048, 3067, "256x3/256")])
+@pytest.mark.parametrize("layout", ["for all", "a batch of one", "off a boundary", "a batch"])
+def test_masks_shared_by_leading_axes(tag, mask_word, q, width, shape, layout):
+    """[batch, heads, q, k]: a mask [q, k] for both leading axes, one whose batch axis of extent 1 has a stride of its own, one
+    that starts one element behind a boundary; a mask for each batch is shared by its heads alone and no block takes three."""
+    batches, heads = (1, 8) if layout == "a batch of one" else (2, 4)
+    note(f"softmax {tag} [{batches}, {heads}, {q}, {width}] {mask_word}, the mask {layout}")
+    x, x_host, mask, mask_host = make_inputs(tag, 8, q, width, mask_word, seed=width)
+    want = oracle_softmax(tag, x_host, mask_word, mask_host, 0.125, False)
+    if layout == "a batch of one":
+        padded = torch.zeros((1, 1, q + 1, width), dtype=mask.dtype, device=DEVICE)
+        padded[0, 0, :q] = mask
+        mask = padded[:, :, :q]              # the axes of extent 1 keep the strides of q + 1 rows
+        assert mask.stride(0) != q * width
+    elif layout == "off a boundary":
+        mask = offset_by_one(mask)
+    elif layout == "a batch":
+        other, other_host = make_inputs(tag, 1, q, width, mask_word, seed=width + 1)[2:]
+        mask = torch.stack([mask, other])[:, None]
+        want[4:] = oracle_softmax(tag, x_host[4:], mask_word, other_host, 0.125, False)
+    (out,) = run(hc.Softmax(scale=0.125, mask=MASKS[mask_word]), x.view(batches, heads, q, width), mask)
+    assert last_launch_form() == f"softmax_unaligned/{shape}/{mask_word}" + ("" if layout == "a batch" else "#shared")
+    count, text = compare_on_device(tag, out.view(8, q, width), want, False)
+    assert count == 0, f"{count} elements outside the bar, {text}"
