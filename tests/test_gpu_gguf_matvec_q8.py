@@ -428,8 +428,8 @@ def test_q8_route_q4_k_tiles_seeded_random_shapes_of_what_they_serve():
                                                 ("q8_0", 70, 2048, 3, "quads/q8_0"), ("q8_0", 40, 1312, 2, "blocks/q8_0/2")])
 def test_q8_route_activation_blocks_on_both_sides_of_the_short_form(tag, rows, k, m, kernel, x_tag):
     """Blocks of zeros, of magnitudes near and past what the short form takes, and with one magnitude of both signs (the first
-    one's counts) quantise the long way: whole waves of them, and blocks that share a wave with ordinary ones.  f16 has
-    zeros, subnormals and equal magnitudes only."""
+    one's counts) quantise the long way: whole waves of them, and blocks that share a wave with ordinary ones.  Nothing that
+    f16 holds is too small or too large for the short form: its subnormals, down to a block of none but 2^-24 and zeros, take it."""
     rng = np.random.default_rng(1827)
     x = rng.normal(0, 1, (m, k)).astype(np.float32)
     group = k // 8
@@ -437,7 +437,10 @@ def test_q8_route_activation_blocks_on_both_sides_of_the_short_form(tag, rows, k
     x[0, 256:288] = np.where(np.arange(32) % 2 == 0, 1.25, -1.25)
     x[0, 512:768] = np.where(np.arange(256) % 3 == 0, -2.5, 2.5)
     x[0, 768:800] = -3.0
-    if x_tag != "f16":
+    if x_tag == "f16":
+        scale = np.float32([1, 2.0 ** -20, 1, 2.0 ** -25, 2.0 ** -15, 2.0 ** -24, 2.0 ** -22, 1])
+        x[m - 1, :8 * group] *= np.repeat(scale, group)
+    else:
         scale = np.float32([1, 2.0 ** -62, 2.0 ** -59, 2.0 ** -61, 2.0 ** 58, 2.0 ** 61, 2.0 ** 20, 2.0 ** -70])
         if tag == "q8_0":
             scale = np.minimum(scale, np.float32(2.0 ** 19))   # its scales are f16
@@ -457,3 +460,40 @@ def test_q8_route_q4_k_tiles_of_eight_rows(x_tag):
         note(f"q8 matvec q4_k tiles x {x_tag} rows {rows} k {k}: 1-tokens{form}")
         check("q4_k", x_tag, raw_bytes_for("q4_k", rng, rows, k), rows, k, rng.normal(0, 1.5, k).astype(np.float32), kernel="gguf_matvec_q8_tiles/q4_k/1-tokens")
         assert last_launch_form() == f"gguf_matvec_q8_tiles/q4_k/1-tokens{form}"
+
+
+@pytest.mark.parametrize("x_tag", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("tag,rows,k,m,kernel", [
+    ("q4_k", 70, 4096, 1, "tiles/q4_k/1-tokens"), ("q4_k", 40, 6144, 1, "tiles/q4_k/1-tokens#8-rows"), ("q4_k", 70, 2048, 3, "tiles/q4_k/4"),
+    ("q4_k", 40, 1280, 6, "tiles/q4_k/8"), ("q6_k", 70, 4096, 1, "spans/q6_k/2"), ("q8_0", 70, 4096, 1, "spans/q8_0/2"),
+    ("q8_0", 70, 2304, 1, "spans/q8_0/2-spans/short"), ("q6_k", 70, 2048, 2, "quads/q6_k"), ("q8_0", 70, 2048, 3, "quads/q8_0"),
+    ("q8_0", 1024, 16384, 2, "lines/q8_0/2"), ("q6_k", 40, 1280, 2, "blocks/q6_k/2"), ("q8_0", 40, 1312, 2, "blocks/q8_0/2")])
+def test_q8_route_activations_that_are_no_numbers(tag, rows, k, m, kernel, x_tag):
+    """A NaN is no candidate for a block's magnitude and has the code of a zero: the products are those of zeros in its place, also
+    those of a block without a number, and an infinity makes its activation row's products NaN.  The other activation rows keep
+    their bits."""
+    rng = np.random.default_rng(1831)
+    dtype = TYPES[x_tag][2]
+    weights = torch.from_numpy(weights_for(tag, rng, rows, k).reshape(-1)).to(DEVICE)
+    descs = [hc.TensorDesc.gguf_weight(KINDS[tag][1], TYPES[x_tag][0], k, rows), hc.TensorDesc.dense(TYPES[x_tag][0], [m, k] if m > 1 else [k])]
+
+    def products(x):
+        (out,) = run(Q8, weights, x if m > 1 else x[0], descs=descs)
+        assert last_launch_form().startswith("gguf_matvec_q8_" + kernel) and ("#8-rows" in last_launch_form()) == ("#8-rows" in kernel), last_launch_form()
+        return out.view(m, rows)
+
+    values = torch.from_numpy(rng.normal(0, 1, (m, k)).astype(np.float32)).to(DEVICE).to(dtype)
+    same = torch.int32 if x_tag == "f32" else torch.int16
+    for number, (what, at, value) in enumerate((("NaN", [5], float("nan")), ("NaN in three blocks", [k - 1, 300, 900], -float("nan")),
+                                                ("a block of NaN", list(range(512, 768)), float("nan")), ("infinity", [700], float("inf")),
+                                                ("minus infinity", [k - 256], -float("inf")))):
+        token = (number + 1) % m
+        clean, odd = values.clone(), values.clone()
+        clean[token, at], odd[token, at] = 0.0, value
+        note(f"q8 matvec {tag} x {x_tag} [{k} -> {rows}] x {m}: {what} in activation row {token}")
+        want, got = products(clean), products(odd)
+        assert not torch.isnan(want).any()
+        if "infinity" in what:
+            assert torch.isnan(got[token]).all()
+            want[token], got[token] = 0.0, 0.0
+        assert torch.equal(got.view(same), want.view(same))
