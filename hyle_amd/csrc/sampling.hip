@@ -107,11 +107,13 @@ __device__ __forceinline__ bool invalid_weight(float v) {
 // past them read as -inf (no mass).  kAligned: rows of whole 16-byte vectors on 16-byte boundaries, so that count is a
 // multiple of kVec.  Other rows (an odd vocabulary) are read as vectors at element-aligned addresses, their last elements one by one.
 // (us, both dispatches, all elements one by one / so: f16 [28, 79580] 14.9 / 9.6, [1, 85746] 10.0 / 7.3, bf16 [64, 248319] 30.3 / 17.9)
-template <class T, bool kAligned, bool kStream>
+// kWhole: no place is past the row, and the loads have no branch round them, so that a thread's go out together (f32, four vectors
+// a thread, all elements one by one / vectors in branches / so: [64, 146861] 16.8 / 17.9 / 13.9, [64, 248321] 19.7 / 20.8 / 17.0).
+template <class T, bool kAligned, bool kStream, bool kWhole>
 __device__ __forceinline__ void tile_vector(const unsigned char *tile, uint32_t at, uint32_t count, float (&part)[Traits<T>::kVec]) {
   constexpr int kVec = Traits<T>::kVec;
   const unsigned char *from = tile + (size_t)at * Traits<T>::kSize;
-  if (kAligned ? at < count : at + kVec <= count) {
+  if (kWhole || (kAligned ? at < count : at + kVec <= count)) {
     if constexpr (!kAligned) Traits<T>::unpack(*reinterpret_cast<const u32x4_element *>(from), part);
     else Traits<T>::unpack(kStream ? load16_stream(from, 0) : load16(from, 0), part);
   } else {
@@ -126,13 +128,17 @@ template <class T, bool kAligned> struct TileValues {
   float v[kPerThread];
   __device__ __forceinline__ void load(const void *row, uint32_t first, uint32_t count) {
     const unsigned char *tile = static_cast<const unsigned char *>(row) + (size_t)first * Traits<T>::kSize;
+    auto all = [&](auto whole) {
 #pragma unroll
-    for (int j = 0; j < kPerThread / kVec; ++j) {
-      float part[kVec];
-      tile_vector<T, kAligned, true>(tile, (uint32_t)(j * kBlockThreads + threadIdx.x) * kVec, count, part);
+      for (int j = 0; j < kPerThread / kVec; ++j) {
+        float part[kVec];
+        tile_vector<T, kAligned, true, decltype(whole)::value>(tile, (uint32_t)(j * kBlockThreads + threadIdx.x) * kVec, count, part);
 #pragma unroll
-      for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
-    }
+        for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
+      }
+    };
+    if (!kAligned && count == (uint32_t)kCategoricalTile) all(std::true_type{});  // the same for the whole block
+    else all(std::false_type{});
   }
 };
 
@@ -220,13 +226,17 @@ template <class T, bool kAligned>
 __device__ __forceinline__ void load_consecutive(const void *row, uint32_t first, uint32_t count, float (&v)[kPerThread]) {
   constexpr int kVec = Traits<T>::kVec;
   const unsigned char *tile = static_cast<const unsigned char *>(row) + (size_t)first * Traits<T>::kSize;
+  auto all = [&](auto whole) {
 #pragma unroll
-  for (int j = 0; j < kPerThread / kVec; ++j) {
-    float part[kVec];
-    tile_vector<T, kAligned, false>(tile, threadIdx.x * kPerThread + j * kVec, count, part);
+    for (int j = 0; j < kPerThread / kVec; ++j) {
+      float part[kVec];
+      tile_vector<T, kAligned, false, decltype(whole)::value>(tile, threadIdx.x * kPerThread + j * kVec, count, part);
 #pragma unroll
-    for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
-  }
+      for (int e = 0; e < kVec; ++e) v[j * kVec + e] = part[e];
+    }
+  };
+  if (!kAligned && count == (uint32_t)kCategoricalTile) all(std::true_type{});
+  else all(std::false_type{});
 }
 
 // Who holds the crossing.  A scan's running sums are associated differently from lane to lane, so they need not be
