@@ -179,13 +179,17 @@ template <int kKind, int kForm> struct KQuantTag {
   }
 };
 
-template <int kKind> hipError_t run_lines(const KQuantParams &p, const unsigned char *in, void *out, float *sumsq, hipStream_t stream) {
+template <int kKind>
+hipError_t run_lines(const KQuantParams &p, const unsigned char *in, void *out, float *sumsq, int compute_units, hipStream_t stream) {
   constexpr uint32_t kWaves = kBlockThreads / kWaveLanes;
   const uint32_t rows = (uint32_t)p.rows;
-  // A block to a row where there are at most eight rows to a compute unit and each is more than one piece (us, a wave / a
-  // block: Q6_K [17408 x 512] 9.3 / 5.9, [6144 x 1280] 5.8 / 4.7, Q4_K [5120 x 1024] 5.2 / 4.2, [2560 x 1024] 3.8 / 3.6;
-  // [3840 x 3328] 7.0 / 7.3, [5120 x 14080] 30.0 / 30.1).
-  const bool shared = p.k > 2048 && rows <= 2048;
+  // A block to a row of more than one piece where the compute units find room for all rows at once, eight to a unit; Q4_K
+  // rows, with more to decode per byte, gain up to seven of one or two pieces, seven and a half of three or four, six and a half of more (us, a
+  // wave / a block: Q6_K [17408 x 512] 9.1 / 5.55, [6144 x 1280] 6.4 / 4.9, [3840 x 2048] 5.5 / 5.0, [3840 x 2560] 5.9 / 6.1; Q4_K
+  // [5120 x 1024] 4.9 / 3.9, [4096 x 1792] 4.6 / 4.5, [4096 x 2048] 4.8 / 5.5, [2304 x 2048] 4.1 / 4.8, [6144 x 1793] 6.0 / 5.7,
+  // [6144 x 2047] 6.2 / 6.4, [9728 x 1537] 8.5 / 7.7, [17408 x 1793] 13.8 / 14.8).
+  const uint32_t halves = kKind == 1 ? 16 : (p.k <= 4096 ? 14 : (p.k <= 8192 ? 15 : 13));
+  const bool shared = p.k > 2048 && rows <= halves * (compute_units > 0 ? (uint32_t)compute_units : 256u) / 2;
   const dim3 waves((rows + kWaves - 1) / kWaves), block(kBlockThreads);
   if (shared) {
     note_variant<KQuantTag<kKind, kShared>>();
@@ -201,14 +205,14 @@ template <int kKind> hipError_t run_lines(const KQuantParams &p, const unsigned 
 }
 }  // namespace
 
-hipError_t launch_k_quant_dequant(const KQuantParams &p, const void *blocks, void *out, float *sumsq,
+hipError_t launch_k_quant_dequant(const KQuantParams &p, const void *blocks, void *out, float *sumsq, int compute_units,
                                   hipStream_t stream) {
   if (p.rows == 0) return hipSuccess;
   const unsigned char *in = static_cast<const unsigned char *>(blocks);
   // whole blocks on 16-byte (Q6_K: even) boundaries
   const uint64_t together = reinterpret_cast<uintptr_t>(blocks) | p.row_stride;
   if (p.k != 0 && p.k % kSuper == 0 && (together & (p.kind == 0 ? 15u : 1u)) == 0)
-    return p.kind == 0 ? run_lines<0>(p, in, out, sumsq, stream) : run_lines<1>(p, in, out, sumsq, stream);
+    return p.kind == 0 ? run_lines<0>(p, in, out, sumsq, compute_units, stream) : run_lines<1>(p, in, out, sumsq, compute_units, stream);
   constexpr int kRows = 4;
   const dim3 grid(((uint32_t)p.rows + kRows - 1) / kRows), block(kBlockThreads);
   if (p.kind == 0) note_variant<KQuantTag<0, kGeneral>>();

@@ -206,7 +206,7 @@ struct KQuantParams {
   uint64_t row_stride = 0;  // bytes between physical rows
   uint8_t kind = 0;
 };
-hipError_t launch_k_quant_dequant(const KQuantParams &p, const void *blocks, void *out, float *sumsq,
+hipError_t launch_k_quant_dequant(const KQuantParams &p, const void *blocks, void *out, float *sumsq, int compute_units,
                                   hipStream_t stream);
 
 // y[m][n] = sum_k w[n][k] * x[m][k], w a GGUF weight (kind 0 Q4_K, 1 Q6_K, 2 Q8_0), x [m, k] dense.

@@ -1809,7 +1809,8 @@ hyle_hip_status hyle_hip_plan_launch(const hyle_hip_plan *plan, const void *cons
                                 aligned(inputs[0], 16) && aligned(outputs[0], 16), stream);
       break;
     case Route::kKQuantDequant:
-      err = launch_k_quant_dequant(plan->kquant, inputs[0], outputs[0], static_cast<float *>(outputs[1]), stream);
+      err = launch_k_quant_dequant(plan->kquant, inputs[0], outputs[0], static_cast<float *>(outputs[1]), plan->context->compute_units,
+                                   stream);
       break;
     case Route::kGgufMatVec:
       if (plan->matvec.codec == HYLE_HIP_ACTIVATIONS_GGML_Q8)

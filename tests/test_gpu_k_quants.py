@@ -123,12 +123,14 @@ def test_k_quant_schema_and_benchmark_shape():
         sumsq_bar(sumsq, wide)
 
 
-# rows, k: pieces of 2048 values that are not whole, a row to a wave and (at most 2048 rows of more than one piece) to a block
+# rows, k: pieces of 2048 values that are not whole, a row to a wave and (rows of more than one piece, at most eight to a compute unit,
+# of Q4_K up to seven and a half) to a block
 @pytest.mark.parametrize("tag", ["q4_k", "q6_k"])
 def test_k_quant_rows_of_pieces(tag):
     kind, _, block_bytes = KINDS[tag]
     rng = np.random.default_rng(1504)
-    for rows, k in ((5, 256), (9, 1792), (2, 2304), (2048, 2304), (2049, 2304), (3, 4096), (7, 8448), (2051, 3840), (2050, 4096)):
+    for rows, k in ((5, 256), (9, 1792), (2, 2304), (2048, 2304), (2049, 2304), (3, 4096), (7, 8448), (2051, 3840), (2050, 4096),
+                    (1792, 4096), (1793, 2304), (1920, 4352), (1921, 4352), (1664, 8448), (1665, 8448)):
         row_bytes = k // 256 * block_bytes
         raw = finite_scales(tag, rng.integers(0, 256, (min(rows, 40), row_bytes), dtype=np.uint8), block_bytes)
         raw = np.resize(raw, (rows, row_bytes))
@@ -139,7 +141,9 @@ def test_k_quant_rows_of_pieces(tag):
             served = (offset | (row_bytes + pad)) % (16 if tag == "q4_k" else 2) == 0
             note(f"{tag} [{rows}, {k}] rows {row_bytes + pad} bytes apart, tensor at byte {offset}")
             got, sumsq = dequant_on_device(tag, padded, rows, k, row_stride=row_bytes + pad, offset=offset)
-            form = "/shared" if k > 2048 and rows <= 2048 else ("/pieces" if k % 2048 else "")
+            halves = 16 if tag == "q6_k" else (14 if k <= 4096 else (15 if k <= 8192 else 13))
+            together = torch.cuda.get_device_properties(0).multi_processor_count * halves // 2
+            form = "/shared" if k > 2048 and rows <= together else ("/pieces" if k % 2048 else "")
             label = f"k_quant_lines/{tag}{form}" if served else f"k_quant_rows/{tag}"
             assert hc.last_launch_variant() == label
             assert np.array_equal(got, want)
