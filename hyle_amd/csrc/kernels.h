@@ -242,7 +242,7 @@ struct Q8Params {
   uint64_t row_stride = 0;  // bytes between physical rows
 };
 hipError_t launch_q8_0_dequant(const Q8Params &p, const void *blocks, void *out, float *sumsq,
-                               bool vectorised, hipStream_t stream);
+                               bool vectorised, int compute_units, hipStream_t stream);
 
 // Cast between storage types, or Copy (copy_size = element bytes, types ignored): any plain
 // input (dims + byte strides, elements need not be aligned) to a dense output.

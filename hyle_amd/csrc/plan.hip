@@ -1806,7 +1806,7 @@ hyle_hip_status hyle_hip_plan_launch(const hyle_hip_plan *plan, const void *cons
       break;
     case Route::kQ8Dequant:
       err = launch_q8_0_dequant(plan->q8, inputs[0], outputs[0], static_cast<float *>(outputs[1]),
-                                aligned(inputs[0], 16) && aligned(outputs[0], 16), stream);
+                                aligned(inputs[0], 16) && aligned(outputs[0], 16), plan->context->compute_units, stream);
       break;
     case Route::kKQuantDequant:
       err = launch_k_quant_dequant(plan->kquant, inputs[0], outputs[0], static_cast<float *>(outputs[1]), plan->context->compute_units,

@@ -13,9 +13,11 @@
 // stores, 1 KiB of consecutive bf16 per store instruction of a wave.  Each row's sum of squares
 // of the exact products is reduced with a wave64 butterfly.
 //
-// Two kernels: rows made of whole 16-byte vectors (K = 256 n) take one wave per row
+// Three kernels: rows made of whole 16-byte vectors (K = 256 n) take one wave per row
 // with a region of LDS that only this wave touches and no block barrier (q8_0_lines: aligned
-// 32-bit LDS words joined by byte-wise funnel shifts); anything else reads bytes (q8_0_rows_bytes).
+// 32-bit LDS words joined by byte-wise funnel shifts), or, where a launch of rows of no whole spans is resident at
+// once, whole rows staged by blocks (q8_0_rows); anything else reads bytes (q8_0_rows_bytes).
+#include <algorithm>
 #include <type_traits>
 
 #include "device_common.h"
@@ -98,6 +100,44 @@ __global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_lines(const unsigned 
   if (lane == 0) sumsq[row] = squares;
 }
 
+// Rows of whole 16-byte vectors, 16-byte aligned: a block stages a whole row for each of its waves, and decodes once all
+// are there.  Few registers, and no piece of a row left over: where all blocks of a launch are resident at once, their reads end
+// before their writes begin, and a short last span does not cost a step of its own.
+template <int kWaves>
+__global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_rows(const unsigned char *blocks, void *out, float *sumsq, uint32_t rows, uint32_t k,
+                                                               uint64_t row_stride) {
+  extern __shared__ __align__(16) unsigned char staged[];
+  const uint32_t wave = threadIdx.x / kWaveLanes, lane = threadIdx.x % kWaveLanes;
+  const uint32_t row = blockIdx.x * kWaves + wave;
+  const uint32_t row_vectors = k / 256 * 17, out_vectors = k / 8;
+  unsigned char *mine = staged + (size_t)wave * row_vectors * 16;
+  if (row < rows) {
+    const unsigned char *source = blocks + (size_t)row * row_stride;
+    for (uint32_t v = lane; v < row_vectors; v += kWaveLanes) reinterpret_cast<u32x4 *>(mine)[v] = load16_stream(source, v);
+  }
+  __syncthreads();
+  float squares = 0.0f;
+  if (row < rows) {
+    for (uint32_t j = lane; j < out_vectors; j += kWaveLanes) {  // block j / 4, quants 8 (j % 4) ..
+      const unsigned char *block = mine + (size_t)(j / 4) * kBlockBytes;
+      const float d = f16_to_f32(*reinterpret_cast<const uint16_t *>(block));
+      const uint16_t *q = reinterpret_cast<const uint16_t *>(block + 2 + 8 * (j % 4));
+      float y[8];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const uint32_t pair = q[h];
+        y[2 * h] = (float)(int8_t)(pair & 0xFFu) * d;
+        y[2 * h + 1] = (float)(int8_t)(pair >> 8) * d;
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) squares = __builtin_fmaf(y[e], y[e], squares);
+      store16_stream(out, (size_t)row * out_vectors + j, Traits<BF16>::pack(y));
+    }
+  }
+  squares = group_sum<kWaveLanes>(squares);
+  if (row < rows && lane == 0) sumsq[row] = squares;
+}
+
 // Any k (multiple of 32), any stride or alignment: one wave per row, byte loads.
 __global__ __launch_bounds__(kBlockThreads) void q8_0_rows_bytes(const uint8_t *blocks, uint16_t *out,
                                                                  float *sumsq, uint32_t rows,
@@ -123,26 +163,45 @@ __global__ __launch_bounds__(kBlockThreads) void q8_0_rows_bytes(const uint8_t *
 template <bool kWhole> struct LinesTag {
   static std::string text() { return kWhole ? "q8_0_lines" : "q8_0_lines/pieces"; }
 };
+struct RowsTag {
+  static std::string text() { return "q8_0_rows"; }
+};
 struct BytesTag {
   static std::string text() { return "q8_0_rows_bytes"; }
 };
 
+// Where q8_0_rows is the faster one: rows of more than one span and no whole number of them, in launches that are resident at once
+// (a compute unit holds eight blocks of four waves, or as many as have room in its LDS) and have more than four blocks to a unit, three
+// and a half of rows of more than two spans.  MI355X, us, lines / rows: [2304 x 6144] 9.8 / 8.3, [2816 x 4352] 8.2 / 6.9, [4608 x 8192] 22.3 / 20.3,
+// [4864 x 7168] 21.9 / 19.9, [5888 x 6144] 22.2 / 20.3, [7424 x 3584] 17.0 / 16.0; one block more than fit: [4608 x 8448] 22.9 / 24.7,
+// [4864 x 7680] 23.0 / 23.9, [6656 x 6144] 24.9 / 26.3; fewer: [3072 x 3072] 6.4 / 7.2, [8960 x 3073] 17.0 / 19.6, [8960 x 3328] alike.
+constexpr uint32_t kUnitLds = 160 * 1024;
+inline bool rows_pay(const Q8Params &p, int compute_units) {
+  if (p.k <= 2048 || p.k % 2048 == 0) return false;
+  const uint32_t fit = std::min(8u, kUnitLds / (4 * (p.k / kBlockElems) * kBlockBytes));
+  const uint64_t units = compute_units > 0 ? (uint64_t)compute_units : 256u, blocks = (p.rows + 3) / 4;
+  return (p.k <= 4096 ? blocks > 4 * units : 2 * blocks >= 7 * units) && blocks <= fit * units;
+}
+
 }  // namespace
 
 hipError_t launch_q8_0_dequant(const Q8Params &p, const void *blocks, void *out, float *sumsq,
-                               bool vectorised, hipStream_t stream) {
+                               bool vectorised, int compute_units, hipStream_t stream) {
   if (p.rows == 0) return hipSuccess;
   const uint32_t rows = (uint32_t)p.rows;
   if (vectorised && p.k != 0 && p.k % 256 == 0 && p.row_stride % 16 == 0) {
     // Measured on MI355X for W[6144 x 2048] (38.6 MB of traffic, buffers rotated): 6.7 us with
     // plain loads and non-temporal stores; 7.4 us with non-temporal loads too; 8.6 / 10.5 us with
     // plain stores; a wave that walks several rows with the next row in flight 7.3 - 9.3 us.  Widths that are no multiple
-    // of 2048, in blocks that staged their rows / like this: [1280 x 14080] 13.1 / 9.4 us, [3840 x 1024] 5.3 / 3.9,
-    // [5120 x 6144] 18.5 / 16.0.
+    // of 2048, in blocks that stage their rows / like this: [1280 x 14080] 13.1 / 9.4 us, [3840 x 1024] 5.2 / 3.8, [5120 x 16000] 49 / 40.
     constexpr int kWaves = 4;
     const dim3 grid((rows + kWaves - 1) / kWaves), block(kWaves * kWaveLanes);
     const unsigned char *in = static_cast<const unsigned char *>(blocks);
-    if (p.k % 2048 == 0) {
+    if (rows_pay(p, compute_units)) {
+      note_variant<RowsTag>();
+      hipLaunchKernelGGL((q8_0_rows<kWaves>), grid, block, (size_t)kWaves * (p.k / kBlockElems) * kBlockBytes, stream, in, out, sumsq, rows, p.k,
+                         p.row_stride);
+    } else if (p.k % 2048 == 0) {
       note_variant<LinesTag<true>>();
       hipLaunchKernelGGL((q8_0_lines<kWaves, true>), grid, block, 0, stream, in, out, sumsq, rows, p.k, p.row_stride);
     } else {

@@ -151,9 +151,13 @@ def test_k_quant_rows_of_pieces(tag):
 
 
 def test_q8_0_rows_of_pieces():
+    """The larger ones on both sides of the launches that are resident at once on 256 compute units, where blocks stage whole rows."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
     rng = np.random.default_rng(1505)
     for rows, k, pad, label in ((5, 256, 0, "lines/pieces"), (9, 1792, 16, "lines/pieces"), (6, 2304, 0, "lines/pieces"), (1030, 3840, 32, "lines/pieces"),
-                                (5, 16640, 0, "lines/pieces"), (7, 10240, 16, "lines"),
+                                (5, 16640, 0, "lines/pieces"), (7, 10240, 16, "lines"), (4096, 2304, 0, "lines/pieces"), (4097, 2304, 16, "rows"),
+                                (8192, 4608, 0, "rows"), (8193, 2560, 0, "lines/pieces"), (7168, 4864, 0, "rows"), (7169, 4864, 0, "lines/pieces"),
+                                (3580, 7936, 0, "lines/pieces"), (3581, 7936, 32, "rows"), (4096, 9472, 0, "rows"), (4099, 8192, 0, "lines"), (5000, 9984, 0, "lines/pieces"),
                                 (4, 2304, 2, "rows_bytes"), (4, 2272, 0, "rows_bytes")):
         blocks = rng.integers(0, 256, (rows, k // 32, 34), dtype=np.uint8)
         blocks[:, :, 1] &= 0x3B
