@@ -232,6 +232,11 @@ template <int kStep> __device__ __forceinline__ double add_xor(double v) {
   }
 }
 
+// The sum over a wave, the same in every lane.
+__device__ __forceinline__ double wave_sum(double v) {
+  return add_xor<32>(add_xor<16>(add_xor<8>(add_xor<4>(add_xor<2>(add_xor<1>(v))))));
+}
+
 // Lanes 0 to 31: a of this lane + a of the lane 32 above; lanes 32 to 63: b of the lane 32 below + b of this lane.
 __device__ __forceinline__ double add_halves_apart(double a, double b) {
   const uint64_t first = __builtin_bit_cast(uint64_t, a), second = __builtin_bit_cast(uint64_t, b);

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_quant_lines(const unsigned ch
   constexpr int kLoads = 2;                                                    // at most 106 vectors
   constexpr int kWaves = kBlockThreads / kWaveLanes;
   __shared__ __align__(16) unsigned char slots[kWaves][kLoads * kWaveLanes * 16];
-  __shared__ float joint[kWaves];
+  __shared__ double joint[kShare];
   const uint32_t lane = threadIdx.x % kWaveLanes;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveLanes);
   const uint32_t wanted_row = blockIdx.x * (kWaves / kShare) + wave / kShare, member = wave % kShare;
@@ -148,8 +148,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_quant_lines(const unsigned ch
         float y[8];
         if constexpr (kKind == 0) decode_q4_k_words(slot, (p / kSuper) * kBlockBytes, p % kSuper, y);
         else decode_q6_k_words(slot, below + (p / kSuper) * kBlockBytes, p % kSuper, y);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) squares = __builtin_fmaf(y[j], y[j], squares);
+        squares += sum_of_squares(y);
         store16_stream(out, ((size_t)row * k + (size_t)step * kSpan + p) / 8, Traits<BF16>::pack(y));
       }
     };
@@ -158,13 +157,18 @@ __global__ __launch_bounds__(kBlockThreads) void k_quant_lines(const unsigned ch
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
+  // the lanes' sums are added in 64 bits and rounded once
+  double total = wave_sum((double)squares);
   if constexpr (kShare == 1) {
-    squares = group_sum<kWaveLanes>(squares);
-    if (lane == 0) sumsq[row] = squares;
+    if (lane == 0) sumsq[row] = (float)total;
   } else {
     static_assert(kShare == kWaves, "a row to a block");
-    squares = row_sum<kBlockThreads>(squares, joint);
-    if (threadIdx.x == 0) sumsq[row] = squares;
+    if (lane == 0) joint[wave] = total;
+    __syncthreads();
+    total = joint[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) total += joint[w];
+    if (threadIdx.x == 0) sumsq[row] = (float)total;
   }
 }
 

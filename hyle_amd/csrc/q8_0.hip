@@ -86,8 +86,7 @@ __global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_lines(const unsigned 
         for (int w = 0; w < 2; ++w)
 #pragma unroll
           for (int t = 0; t < 4; ++t) y[4 * w + t] = (float)(int)(signed char)(q[w] >> (8 * t)) * d;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) squares = __builtin_fmaf(y[e], y[e], squares);
+        squares += sum_of_squares(y);
         store16_stream(out, ((size_t)row * k + (size_t)step * kSpan) / 8 + j, Traits<BF16>::pack(y));
       }
     };
@@ -96,8 +95,8 @@ __global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_lines(const unsigned 
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
-  squares = group_sum<kWaveLanes>(squares);
-  if (lane == 0) sumsq[row] = squares;
+  const double total = wave_sum((double)squares);  // the lanes' sums are added in 64 bits and rounded once
+  if (lane == 0) sumsq[row] = (float)total;
 }
 
 // Rows of whole 16-byte vectors, 16-byte aligned: a block stages a whole row for each of its waves, and decodes once all
@@ -129,13 +128,12 @@ __global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_rows(const unsigned c
         y[2 * h] = (float)(int8_t)(pair & 0xFFu) * d;
         y[2 * h + 1] = (float)(int8_t)(pair >> 8) * d;
       }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) squares = __builtin_fmaf(y[e], y[e], squares);
+      squares += sum_of_squares(y);
       store16_stream(out, (size_t)row * out_vectors + j, Traits<BF16>::pack(y));
     }
   }
-  squares = group_sum<kWaveLanes>(squares);
-  if (row < rows && lane == 0) sumsq[row] = squares;
+  const double total = wave_sum((double)squares);
+  if (row < rows && lane == 0) sumsq[row] = (float)total;
 }
 
 // Any k (multiple of 32), any stride or alignment: one wave per row, byte loads.

@@ -142,10 +142,6 @@ template <class T, bool kAligned> struct TileValues {
   }
 };
 
-__device__ __forceinline__ double wave_sum(double v) {
-  return add_xor<32>(add_xor<16>(add_xor<8>(add_xor<4>(add_xor<2>(add_xor<1>(v))))));
-}
-
 template <class T, bool kVector>
 __global__ __launch_bounds__(kBlockThreads) void categorical_tiles(const void *logits, uint32_t width, uint32_t tiles,
                                                                    CategoricalTile *out, uint32_t *status) {

@@ -150,6 +150,36 @@ def test_k_quant_rows_of_pieces(tag):
             sumsq_bar(sumsq, wide)
 
 
+@pytest.mark.parametrize("tag,rows,k", [("q4_k", 2100, 14080), ("q4_k", 2100, 17408), ("q4_k", 300, 17408), ("q4_k", 2100, 7168), ("q6_k", 2100, 17408),
+                                        ("q6_k", 300, 14080), ("q6_k", 2100, 8192), ("q8_0", 300, 17408), ("q8_0", 6144, 2304), ("q8_0", 300, 8192)])
+def test_row_sums_of_squares_round_seldom(tag, rows, k):
+    """Against the float64 sums of the same f32 values, 2-norm over 300 distinct rows.  The last rounding moves a sum by
+    2^-24 / sqrt(3) of it in root mean square, at the foot of a binade.  Each of 64 lanes adds K / 512 sums of eight squares, a
+    rounding of the part there is so far each time (a third of so many whole ones in the mean square) and two whole ones at
+    most within the eights, independent of the other lanes'.  300 rows give the mean square of an even distribution within
+    0.155 of it, three standard deviations.  (One chain of squares a lane: 5.2e-8 to 7.0e-8 at these widths of Q4_K.)"""
+    rng = np.random.default_rng(1506)
+    distinct = 300
+    if tag == "q8_0":
+        blocks = rng.integers(0, 256, (distinct, k // 32, 34), dtype=np.uint8)
+        blocks[:, :, 1] = blocks[:, :, 1] & 0x07 | 0x10
+        raw = blocks.reshape(distinct, -1)
+        wide = (blocks[:, :, 2:].view(np.int8).astype(np.float32) * blocks[:, :, :2].copy().view(np.float16).astype(np.float32)).reshape(distinct, k)
+    else:
+        kind, _, block_bytes = KINDS[tag]
+        raw = finite_scales(tag, rng.integers(0, 256, (distinct, k // 256 * block_bytes), dtype=np.uint8), block_bytes)
+        wide = orc.k_quant_dequant(kind, raw, distinct, k)[0]
+    gguf = {"q8_0": hc.GgufQuantizedType.kQ8_0, "q4_k": hc.GgufQuantizedType.kQ4K, "q6_k": hc.GgufQuantizedType.kQ6K}[tag]
+    desc = hc.TensorDesc.gguf_weight(gguf, hc.DataType.kBFloat16, k, rows)
+    note(f"{tag} [{rows}, {k}]: row sums of squares against float64")
+    _, sumsq = run(hc.GgufDequantSumSquares(), torch.from_numpy(np.resize(raw, (rows, raw.shape[1]))).to(DEVICE), descs=[desc])
+    got = sumsq.cpu().numpy()
+    assert np.array_equal(got, np.resize(got[:distinct], rows))
+    want = (np.asarray(wide, np.float64).reshape(distinct, k) ** 2).sum(1)
+    off = np.linalg.norm((got[:distinct] - want) / want) / np.sqrt(distinct)
+    assert off <= np.sqrt(1.155 * (1 / 3 + (k / 512 / 3 + 2) / (3 * 64))) * 2.0 ** -24, f"{off:.3e}"
+
+
 def test_q8_0_rows_of_pieces():
     """The larger ones on both sides of the launches that are resident at once on 256 compute units, where blocks stage whole rows."""
     assert torch.cuda.get_device_properties(0).multi_processor_count == 256
