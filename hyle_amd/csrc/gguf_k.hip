@@ -12,11 +12,12 @@
 //
 // Two kernels.  Q4_K rows on 16-byte boundaries and Q6_K rows at even addresses (the usual case)
 // take a wave or a block per row, whole cache lines into wave-private LDS and word-wise decoding
-// (k_quant_lines, measured 5.9 / 6.3 us for Q4_K / Q6_K [6144 x 2048] on MI355X).  Anything else
+// (k_quant_lines, measured 5.9 / 6.3 us for Q4_K / Q6_K [6144 x 2048] on MI355X).  Anything else, Q4_K rows off a
+// 16-byte boundary and Q6_K rows at odd addresses or an odd number of bytes apart,
 // takes the general kernel: a block of 256 threads takes four rows at a time, eight super-blocks
 // of each (at most 1680 bytes) are staged in LDS per step with the widest loads the row's
-// address allows, and a thread decodes eight neighbouring values from LDS bytes (10.7 / 12.3 us
-// for the same shape).  Both store eight values as one 16-byte vector.
+// address allows, and a thread decodes eight neighbouring values from LDS bytes (Q4_K [6144 x 2048] four bytes off 10.8 us,
+// Q6_K one byte off 17.1).  Both store eight values as one 16-byte vector.
 #include <type_traits>
 
 #include "device_common.h"
@@ -28,8 +29,8 @@ namespace {
 
 constexpr int kChunkBlocks = kBlockThreads * 8 / kSuper;  // super-blocks decoded per step: 8
 
-// Bytes -> LDS with the widest loads the address allows (Q4_K rows of a 16-byte aligned tensor
-// always take words; Q6_K blocks are only 2-byte aligned as a rule).
+// Bytes -> LDS with the widest loads the address allows: words, pairs or single bytes for Q4_K rows, whatever boundary they are
+// off; single bytes for a chunk of Q6_K blocks at an odd address, pairs for the rows between whose addresses are even.
 __device__ __forceinline__ void stage(unsigned char *to, const unsigned char *from, uint32_t bytes) {
   if (((reinterpret_cast<uintptr_t>(from) | bytes) & 3u) == 0) {
     for (uint32_t i = threadIdx.x; i < bytes / 4; i += kBlockThreads)

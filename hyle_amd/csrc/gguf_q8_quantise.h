@@ -1,5 +1,6 @@
-// The activation rows of the ggml route, quantised by sixteen lanes per run of 256 values: what the tile and strip
-// kernels (gguf_matvec_q8.hip, gguf_matvec_strips.hip) do before they touch a weight.
+// The activation rows of the ggml route, quantised: sixteen lanes per run of 256 values in the tile and strip kernels
+// (gguf_matvec_q8.hip, gguf_matvec_strips.hip), before they touch a weight; the span, quad, line and block kernels of
+// gguf_matvec_q8.hip have lanes of 32 or eight values and take the maxima and the short form from here.
 #pragma once
 
 #include <type_traits>
