@@ -98,9 +98,9 @@ template <> struct Strip<0> {  // rows are whole 16-byte vectors as a rule: load
   using Pending = Strip;
   u32x4 head, q[2];
   __device__ __forceinline__ void load(const unsigned char *at, uint32_t part) {
-    head = *reinterpret_cast<const words4_even *>(at);
+    head = *reinterpret_cast<const u32x4_element *>(at);
 #pragma unroll
-    for (int s = 0; s < 2; ++s) q[s] = *reinterpret_cast<const words4_even *>(at + 16 + 32 * part + 16 * s);
+    for (int s = 0; s < 2; ++s) q[s] = *reinterpret_cast<const u32x4_element *>(at + 16 + 32 * part + 16 * s);
   }
 };
 template <> struct Strip<1> : StripStage<210> {

@@ -11,8 +11,6 @@
 namespace hyle_hip {
 namespace {
 
-// 16 bytes at any even address.
-typedef uint32_t words4_even __attribute__((ext_vector_type(4), aligned(2)));
 typedef short short2v __attribute__((ext_vector_type(2)));
 
 // kCount values of an activation row, sixteen as a rule: neighbours, at any element's address.
@@ -22,7 +20,7 @@ template <class TX, int kCount = 16> struct BlockValues {
   __device__ __forceinline__ void load(const void *x, size_t first) {
 #pragma unroll
     for (int h = 0; h < kVectors; ++h)
-      raw[h] = *reinterpret_cast<const words4_even *>(static_cast<const char *>(x) + first * Traits<TX>::kSize + 16 * h);
+      raw[h] = *reinterpret_cast<const u32x4_element *>(static_cast<const char *>(x) + first * Traits<TX>::kSize + 16 * h);
   }
   __device__ __forceinline__ void values(float (&v)[kCount]) const {
 #pragma unroll
@@ -193,7 +191,7 @@ __device__ __forceinline__ void quantise_block(const BlockValues<TX> &fetched, u
   }
   const u32x4 whole = {words[0], words[1], words[2], words[3]};
   // Q8_0 in place: 48 bytes per block, its codes where its quants lie in the 48 bytes from its first vector
-  if constexpr (kKind >= 3) *reinterpret_cast<words4_even *>(codes + 50 * (u / 2) + 2 + 16 * (u % 2)) = whole;
+  if constexpr (kKind >= 3) *reinterpret_cast<u32x4_element *>(codes + 50 * (u / 2) + 2 + 16 * (u % 2)) = whole;
   else reinterpret_cast<u32x4 *>(codes)[u] = whole;
   if constexpr (kKind == 0) {
     int sum = dot4(0x01010101u, words[0], dot4(0x01010101u, words[1], dot4(0x01010101u, words[2], dot4(0x01010101u, words[3], 0))));
