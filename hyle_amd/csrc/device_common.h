@@ -237,6 +237,14 @@ __device__ __forceinline__ double wave_sum(double v) {
   return add_xor<32>(add_xor<16>(add_xor<8>(add_xor<4>(add_xor<2>(add_xor<1>(v))))));
 }
 
+// The sum over a wave of f32 values, its last three steps in 64 bits: those before them round at an eighth of the sum and below.
+__device__ __forceinline__ double wave_sum_of_eighths(float v) {
+  v += __int_as_float(dpp_move<kDppSwap1>(__float_as_int(v)));
+  v += __int_as_float(dpp_move<kDppSwap2>(__float_as_int(v)));
+  v += __int_as_float(dpp_move<kDppHalfMirror>(__float_as_int(v)));
+  return add_xor<32>(add_xor<16>(add_xor<8>((double)v)));
+}
+
 // Lanes 0 to 31: a of this lane + a of the lane 32 above; lanes 32 to 63: b of the lane 32 below + b of this lane.
 __device__ __forceinline__ double add_halves_apart(double a, double b) {
   const uint64_t first = __builtin_bit_cast(uint64_t, a), second = __builtin_bit_cast(uint64_t, b);

@@ -21,17 +21,15 @@ __device__ __forceinline__ float lds_f16(const unsigned char *p) {
   return f16_to_f32((uint16_t)(p[0] | ((uint16_t)p[1] << 8)));
 }
 
-// The sum of eight squares, in two chains: a lane that adds the sums of its vectors, and not square after square, rounds
-// an eighth as often along its way (f32 row sums of Q4_K [17408 x 3000] against 64 bits, 2-norm: 7.0e-8 off in one chain a lane, 4.5e-8
-// in eights, 3.0e-8 with the lanes' sums added in 64 bits; over 195 shapes of the three formats 3.4e-8 at most).
+// The sum of eight squares: a lane that adds the sums of its vectors, and not square after square, rounds at the size of what
+// it has an eighth as often (f32 row sums of Q4_K [17408 x 3000] against 64 bits, 2-norm: 7.0e-8 off in one chain a lane, 4.5e-8
+// in eights, 3.3e-8 with the last steps over the lanes in 64 bits; over 195 shapes of the three formats 3.8e-8 at most.  All six steps in
+// 64 bits: 3.4e-8, and 2 to 6 % of the time of many rows of 256 to 1024 values).
 __device__ __forceinline__ float sum_of_squares(const float (&y)[8]) {
-  float even = y[0] * y[0], odd = y[1] * y[1];
+  float sum = y[0] * y[0];
 #pragma unroll
-  for (int j = 2; j < 8; j += 2) {
-    even = __builtin_fmaf(y[j], y[j], even);
-    odd = __builtin_fmaf(y[j + 1], y[j + 1], odd);
-  }
-  return even + odd;
+  for (int j = 1; j < 8; ++j) sum = __builtin_fmaf(y[j], y[j], sum);
+  return sum;
 }
 
 // Eight values of a Q4_K block starting at position p (a multiple of 8).

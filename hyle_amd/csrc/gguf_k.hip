@@ -158,8 +158,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_quant_lines(const unsigned ch
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
-  // the lanes' sums are added in 64 bits and rounded once
-  double total = wave_sum((double)squares);
+  double total = wave_sum_of_eighths(squares);
   if constexpr (kShare == 1) {
     if (lane == 0) sumsq[row] = (float)total;
   } else {

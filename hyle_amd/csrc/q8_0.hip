@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_lines(const unsigned 
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
-  const double total = wave_sum((double)squares);  // the lanes' sums are added in 64 bits and rounded once
+  const double total = wave_sum_of_eighths(squares);
   if (lane == 0) sumsq[row] = (float)total;
 }
 
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(kWaves *kWaveLanes) void q8_0_rows(const unsigned c
       store16_stream(out, (size_t)row * out_vectors + j, Traits<BF16>::pack(y));
     }
   }
-  const double total = wave_sum((double)squares);
+  const double total = wave_sum_of_eighths(squares);
   if (row < rows && lane == 0) sumsq[row] = (float)total;
 }
 
