@@ -1473,8 +1473,9 @@ inline bool rows_of_vectors_serve(const MatVecParams &p) {
 //   one row of Q4_K tiles: rows of 10240 values or more, [14080 -> 3328] 13.7 / 9.6; widths that are no multiple of 2048
 //   with few weight rows, [5120 -> 5120] 9.2 / 7.0; and more rows than values, [1024 -> 2048] 3.7 / 3.15, [2048 -> 6144] 5.5 / 4.8,
 //   [2560 -> 5120] 5.4 / 4.7, [4096 -> 8192] 7.9 / 6.75, [5120 -> 17408] 15.8 / 12.7, until the tiles, which need no barrier,
-//   catch up: [2048 -> 29297] 12.1 / 9.3, [2048 -> 33203] 11.1 / 11.3, [2048 -> 48828] 12.0 / 13.5, [1536 -> 65104] 12.6 / 14.7;
-//   [4096 -> 18555] 11.8 / 10.9, [4096 -> 24414] 12.5 / 13.6 ([8192 -> 12200] 13.2 / 13.6); of other widths
+//   catch up, at more tiles to a block than its eight waves have places for, one to a tile of six runs or fewer, two of seven or
+//   eight: [1280 -> 53125] 10.9 / 10.0, [1536 -> 52201] 10.8 / 10.2, [1536 -> 65104] 12.6 / 14.7, [1024 -> 66406] 11.0 / 11.4; [2048 -> 29297]
+//   12.1 / 9.3, [2048 -> 33203] 11.1 / 11.3, [2048 -> 48828] 12.0 / 13.5; wider ones by products, [4096 -> 18555] 11.8 / 10.9, [4096 -> 24414] 12.5 / 13.6 ([8192 -> 12200] 13.2 / 13.6); of other widths
 //   [3072 -> 32552] 13.8 / 13.0, [6144 -> 32552] 22.6 / 24.1.
 bool strips_better(const MatVecParams &p, bool vectors) {
   if (!gguf_matvec_strips_serve(p)) return false;
@@ -1483,8 +1484,8 @@ bool strips_better(const MatVecParams &p, bool vectors) {
   if (p.m == 1) {
     if (!whole) return products >= 8000000 || (products >= 4000000 && p.k >= 2048);
     if (p.kind != 0) return false;
-    const uint64_t most = p.k <= 2048 ? 64000000 : (p.k % 4096 == 0 ? 80000000 : 100000000);
-    return p.k >= 10240 || (p.k > 2048 && p.k % 2048 != 0 && (p.rows <= 4096 || p.k >= p.rows)) || (p.rows > p.k && products <= most);
+    const bool held = p.k <= 2048 ? p.rows < (p.k <= 1536 ? 56000u : 32768u) : products <= (p.k % 4096 == 0 ? 80000000u : 100000000u);
+    return p.k >= 10240 || (p.k > 2048 && p.k % 2048 != 0 && (p.rows <= 4096 || p.k >= p.rows)) || (p.rows > p.k && held);
   }
   if (!whole) return true;
   // one span of a vocabulary: the tile and quad kernels keep its codes at hand and have no tiles left over

@@ -143,14 +143,15 @@ def test_strips_every_layout_of_a_launch(tag):
         assert np.array_equal(got, np.take(got, np.arange(rows) % period, 1))
 
 
-# Q4_K products on both sides of the limits: more rows than values up to 64, 80 or 100 M products, two to four activation rows up
-# to 115 or 150 M
+# Q4_K products on both sides of the limits: more rows than values below 56000 or 32768 rows, of more than 2048 values up to 80 or 100 M
+# products, and two to four activation rows up to 115 or 150 M
 @pytest.mark.parametrize("x_tag,k,rows,m,kernel", [
     ("bf16", 2048, 6001, 1, "strips"), ("bf16", 2048, 6000, 1, "strips"), ("f32", 2816, 5633, 1, "strips"), ("f32", 3072, 6145, 1, "strips"),
     ("f16", 3072, 6144, 1, "strips"), ("bf16", 1024, 97656, 1, "tiles"), ("bf16", 1024, 97657, 1, "tiles"), ("f32", 2048, 9000, 2, "strips"),
     ("bf16", 1280, 9000, 4, "strips"), ("f16", 2048, 8999, 3, "strips"), ("bf16", 2048, 89999, 2, "tiles"), ("bf16", 2048, 90000, 2, "tiles"),
     ("bf16", 2048, 2049, 1, "strips"), ("f32", 2048, 2048, 1, "tiles"), ("f16", 1024, 1025, 1, "strips"), ("bf16", 1024, 1024, 1, "tiles"),
-    ("bf16", 4096, 4097, 1, "strips"), ("bf16", 4096, 4096, 1, "tiles"), ("bf16", 2048, 31250, 1, "strips"), ("f32", 2048, 31251, 1, "tiles"),
+    ("bf16", 4096, 4097, 1, "strips"), ("bf16", 4096, 4096, 1, "tiles"), ("bf16", 2048, 32767, 1, "strips"), ("f32", 2048, 32768, 1, "tiles"),
+    ("bf16", 1536, 55999, 1, "strips"), ("f16", 1536, 56000, 1, "tiles"), ("f32", 1792, 32768, 1, "tiles"),
     ("bf16", 4096, 19531, 1, "strips"), ("bf16", 4096, 19532, 1, "tiles"), ("bf16", 5120, 19531, 1, "strips"), ("bf16", 5120, 19532, 1, "tiles"),
     ("f32", 2048, 6144, 2, "strips"), ("bf16", 2048, 6143, 3, "strips"), ("f16", 1024, 7000, 4, "strips"), ("bf16", 2048, 6144, 4, "strips"),
     ("bf16", 2048, 56152, 2, "strips"), ("bf16", 2048, 56153, 4, "tiles"), ("bf16", 1280, 117187, 3, "strips"), ("bf16", 1280, 117188, 2, "tiles")])
@@ -256,7 +257,7 @@ def test_strips_round_a_product_twice(tag, k, rows, m):
     assert off <= np.sqrt(2 / 3) * 2.0 ** -24, f"{off:.3e}"
 
 
-@pytest.mark.parametrize("k,rows,m", [(1024, 500, 1), (2048, 2048, 1), (6144, 300, 1), (8192, 1500, 1), (2048, 32000, 1), (4096, 400, 3), (1280, 511, 8),
+@pytest.mark.parametrize("k,rows,m", [(1024, 500, 1), (2048, 2048, 1), (6144, 300, 1), (8192, 1500, 1), (2048, 32769, 1), (4096, 400, 3), (1280, 511, 8),
                                      (2048, 57000, 2)])
 def test_tiles_round_a_product_twice(k, rows, m):
     """The same of the tile kernel, whose waves share a tile by two or four.  (Closed and summed in 32 bits 6.1e-8 to 8.0e-8.)"""
