@@ -3,9 +3,9 @@ against the CPU oracle.
 
 Which kernel serves a norm depends on the row width and on the number of rows: widths that a lane
 group holds in whole vectors have launch shapes that cover the tensor exactly when the row count is
-a multiple of the rows a block takes (norm_exact.h, and for LayerNorm the exact forms of norm.hip);
-other widths and row counts take the masked shapes of norm.hip, and widths that are no whole
-number of 16-byte vectors the generic kernel.  CASES is the table (operator, type, rows, width) ->
+a multiple of the rows a block takes (norm_exact.h, from 10 MiB on, and for LayerNorm the exact forms of norm.hip);
+rows of 65 to 768 vectors take a wave each (norm_tail.h), other widths and row counts the masked shapes of norm.hip, and
+widths that are no whole number of 16-byte vectors the generic kernel.  CASES is the table (operator, type, rows, width) ->
 label of the launch shape the library must choose; `hyle_hip_last_launch_variant` reports the
 shape actually launched.  The last test fails when a norm shape compiled into the library
 (`hyle_hip_variant_label`) is reached by no case.
